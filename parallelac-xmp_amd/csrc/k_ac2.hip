@@ -737,13 +737,16 @@ __device__ __forceinline__ bool low_setup(const GridP& g, const Ball* v,
 }
 
 /* KIND 0: triangles (items = alpha triangle ids), 1: edges (alpha edge ids).
- * Simplices already in the closure (in_flag) pass without a test.  Same
- * phase A / phase B split as the tet kernel. */
+ * Simplices already in the closure (in_flag) pass without a test, those
+ * with an edge that one ball covers (kDeadBit in tkd, edead) fail without
+ * one: a third of the 100k globule's alpha triangles and half of its alpha
+ * edges are left to scan.  Same phase A / phase B split as the tet kernel. */
 template <class R, int KIND, bool PHASE_B, bool FINE, bool MOL>
 __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     Stage S, Cnt c_nitems, const uint32_t* ecol, const uint32_t* eleft,
-    const uint32_t* tk, const uint32_t* tedge, const uint8_t* in_flag,
-    uint8_t* flag, Queue q1, uint32_t* rest, unsigned* nrest, int budget) {
+    const uint32_t* tkd, const uint32_t* tedge, const uint8_t* edead,
+    const uint8_t* in_flag, uint8_t* flag, Queue q1, uint32_t* rest,
+    unsigned* nrest, int budget) {
   unsigned evals = 0, pairs = 0;
   __shared__ uint32_t s_pre[LSLOTS + 1];
   if (PHASE_B) list_table(nrest, S.lcap, s_pre);
@@ -759,10 +762,19 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     uint32_t vid[3];
     if (KIND == 0) {
       uint32_t e = tedge[id];
+      const uint32_t kd = tkd[id];
+      if (!PHASE_B && (kd & kDeadBit)) { /* an edge of it is covered */
+        flag[id] = 0;
+        return;
+      }
       vid[0] = eleft[e];
       vid[1] = ecol[e];
-      vid[2] = tk[id];
+      vid[2] = kd & ~kDeadBit;
     } else {
+      if (!PHASE_B && edead && edead[id]) {
+        flag[id] = 0;
+        return;
+      }
       vid[0] = eleft[id];
       vid[1] = ecol[id];
       vid[2] = vid[1];
@@ -1228,70 +1240,74 @@ void launch_tet_ac2_exact_sorted(const Stage& S, const uint32_t* item,
 }
 template <class R, int KIND, bool FINE, bool MOL>
 static void low_hot4(const Stage& S, Cnt nitems, const uint32_t* ecol,
-                     const uint32_t* eleft, const uint32_t* tk,
-                     const uint32_t* tedge, const uint8_t* in_flag,
-                     uint8_t* flag, Queue q1, uint32_t* rest, unsigned* nrest,
-                     int budget, PipeLaunch L) {
+                     const uint32_t* eleft, const uint32_t* tkd,
+                     const uint32_t* tedge, const uint8_t* edead,
+                     const uint8_t* in_flag, uint8_t* flag, Queue q1,
+                     uint32_t* rest, unsigned* nrest, int budget,
+                     PipeLaunch L) {
   dim3 gr((unsigned)((nitems.cap + kBlock - 1) / kBlock)), gb((unsigned)S.bgrid);
   hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, false, FINE, MOL>), gr,
-                     dim3(kBlock), 0, L.s, S, nitems, ecol, eleft, tk, tedge,
-                     in_flag, flag, q1, rest, nrest, budget);
+                     dim3(kBlock), 0, L.s, S, nitems, ecol, eleft, tkd, tedge,
+                     edead, in_flag, flag, q1, rest, nrest, budget);
   if (budget > 0) {
     hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, true, FINE, MOL>), gb,
                        dim3((unsigned)S.bblock), 0, L.s, S, nitems, ecol, eleft,
-                       tk, tedge, in_flag, flag, q1, rest, nrest, budget);
+                       tkd, tedge, edead, in_flag, flag, q1, rest, nrest,
+                       budget);
   }
 }
 template <class R, int KIND, bool FINE>
 static void low_hot3(const Stage& S, Cnt nitems, const uint32_t* ecol,
-                     const uint32_t* eleft, const uint32_t* tk,
-                     const uint32_t* tedge, const uint8_t* in_flag,
-                     uint8_t* flag, Queue q1, uint32_t* rest, unsigned* nrest,
-                     int budget, PipeLaunch L) {
+                     const uint32_t* eleft, const uint32_t* tkd,
+                     const uint32_t* tedge, const uint8_t* edead,
+                     const uint8_t* in_flag, uint8_t* flag, Queue q1,
+                     uint32_t* rest, unsigned* nrest, int budget,
+                     PipeLaunch L) {
   if (S.mol)
-    low_hot4<R, KIND, FINE, true>(S, nitems, ecol, eleft, tk, tedge, in_flag,
-                                  flag, q1, rest, nrest, budget, L);
+    low_hot4<R, KIND, FINE, true>(S, nitems, ecol, eleft, tkd, tedge, edead,
+                                  in_flag, flag, q1, rest, nrest, budget, L);
   else
-    low_hot4<R, KIND, FINE, false>(S, nitems, ecol, eleft, tk, tedge, in_flag,
-                                   flag, q1, rest, nrest, budget, L);
+    low_hot4<R, KIND, FINE, false>(S, nitems, ecol, eleft, tkd, tedge, edead,
+                                   in_flag, flag, q1, rest, nrest, budget, L);
 }
 template <class R, int KIND>
 static void low_hot2(const Stage& S, Cnt nitems, const uint32_t* ecol,
-                     const uint32_t* eleft, const uint32_t* tk,
-                     const uint32_t* tedge, const uint8_t* in_flag,
-                     uint8_t* flag, Queue q1, uint32_t* rest, unsigned* nrest,
-                     int budget, PipeLaunch L) {
+                     const uint32_t* eleft, const uint32_t* tkd,
+                     const uint32_t* tedge, const uint8_t* edead,
+                     const uint8_t* in_flag, uint8_t* flag, Queue q1,
+                     uint32_t* rest, unsigned* nrest, int budget,
+                     PipeLaunch L) {
   if (S.fine)
-    low_hot3<R, KIND, true>(S, nitems, ecol, eleft, tk, tedge, in_flag, flag,
-                            q1, rest, nrest, budget, L);
+    low_hot3<R, KIND, true>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
+                            flag, q1, rest, nrest, budget, L);
   else
-    low_hot3<R, KIND, false>(S, nitems, ecol, eleft, tk, tedge, in_flag, flag,
-                             q1, rest, nrest, budget, L);
+    low_hot3<R, KIND, false>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
+                             flag, q1, rest, nrest, budget, L);
 }
 void launch_low_ac2_hot(const Stage& S, int kind, Cnt nitems,
                         const uint32_t* ecol, const uint32_t* eleft,
-                        const uint32_t* tk, const uint32_t* tedge,
-                        const uint8_t* in_flag, uint8_t* flag, Queue q1,
-                        uint32_t* rest, unsigned* nrest, int budget,
-                        PipeLaunch L) {
+                        const uint32_t* tkd, const uint32_t* tedge,
+                        const uint8_t* edead, const uint8_t* in_flag,
+                        uint8_t* flag, Queue q1, uint32_t* rest,
+                        unsigned* nrest, int budget, PipeLaunch L) {
   if (nitems.cap <= 0) return;
   if constexpr (!kBallF64) {
     if (S.staged) {
       if (kind == 0)
-        low_hot2<float, 0>(S, nitems, ecol, eleft, tk, tedge, in_flag, flag, q1,
-                           rest, nrest, budget, L);
+        low_hot2<float, 0>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
+                           flag, q1, rest, nrest, budget, L);
       else
-        low_hot2<float, 1>(S, nitems, ecol, eleft, tk, tedge, in_flag, flag, q1,
-                           rest, nrest, budget, L);
+        low_hot2<float, 1>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
+                           flag, q1, rest, nrest, budget, L);
       return;
     }
   }
   if (kind == 0)
-    low_hot2<double, 0>(S, nitems, ecol, eleft, tk, tedge, in_flag, flag, q1,
-                        rest, nrest, budget, L);
+    low_hot2<double, 0>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
+                        flag, q1, rest, nrest, budget, L);
   else
-    low_hot2<double, 1>(S, nitems, ecol, eleft, tk, tedge, in_flag, flag, q1,
-                        rest, nrest, budget, L);
+    low_hot2<double, 1>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
+                        flag, q1, rest, nrest, budget, L);
 }
 void launch_low_ac2_esc(const Stage& S, int kind, QRef q,
                         const uint32_t* ecol, const uint32_t* eleft,

@@ -415,9 +415,25 @@ __device__ __forceinline__ int edge_code_ss(const Ball& a, const Ball& b,
   const R Vp = ((R)4 * uu) * (wa + fabs(al)) + Ap * Ap;
   return code_of(fe_sign(ss_fe(SS<R>{V, Vp}, 8)));
 }
+/* A rejected triangle (a, b, c) also tells which of its edges one ball
+ * covers.  The points of equal power to a and b with that power <= alpha
+ * are a disk around the edge's centre; c's power minus theirs is affine on
+ * the disk's plane and vanishes nowhere on the disk (such a point would be
+ * a common orthocentre of value <= alpha), so its sign at the edge's
+ * centre, the sign of c's barycentric coordinate of the triangle's
+ * orthocentre, is its sign on the whole disk.  Negative: every alpha
+ * simplex with the edge ab has its orthocentre on the disk, where c's
+ * power is strictly below the simplex's value, and is not empty.
+ * The coordinates (times 2 |n|^2 > 0): b: A |v|^2 - B u.v, c: B |u|^2 -
+ * A u.v, a: 2 |n|^2 minus both; at most 18 roundings on any path of the
+ * last (14 of the others), bounded by 24 u times the permanent.
+ * cover: bit q set when vertex q (a, b, c) certainly covers the opposite
+ * edge; set only with the result REJECT. */
 template <class R>
 __device__ __forceinline__ int tri_code_ss(const Ball& a, const Ball& b,
-                                           const Ball& c, Real alpha) {
+                                           const Ball& c, Real alpha,
+                                           unsigned& cover) {
+  cover = 0u;
   const R ax = a.x, ay = a.y, az = a.z;
   const R ux = (R)b.x - ax, uy = (R)b.y - ay, uz = (R)b.z - az;
   const R vx = (R)c.x - ax, vy = (R)c.y - ay, vz = (R)c.z - az;
@@ -438,7 +454,17 @@ __device__ __forceinline__ int tri_code_ss(const Ball& a, const Ball& b,
   const R al = (R)alpha;
   const R V = ((R)4 * nn) * (wa + al) - lhs;
   const R Vp = ((R)4 * nnp) * (wa + fabs(al)) + lhsp;
-  return code_of(fe_sign(ss_fe(SS<R>{V, Vp}, 11)));
+  const int r = code_of(fe_sign(ss_fe(SS<R>{V, Vp}, 11)));
+  if (r == REJECT) {
+    const SS<R> lb{A * vv - B * uv, Ap * vv + Bp * uvp};
+    const SS<R> lc{B * uu - A * uv, Bp * uu + Ap * uvp};
+    const SS<R> la{(A * (uv - vv) + B * (uv - uu)) + (R)2 * nn,
+                   (Ap * (uvp + vv) + Bp * (uvp + uu)) + (R)2 * nnp};
+    cover = (fe_sign(ss_fe(la, 22)) < 0 ? 1u : 0u) |
+            (fe_sign(ss_fe(lb, 22)) < 0 ? 2u : 0u) |
+            (fe_sign(ss_fe(lc, 22)) < 0 ? 4u : 0u);
+  }
+  return r;
 }
 /* the first stage of the tet filter: D and N with a-priori error bounds
  * (tet_dn_ss: one extra operation per operation, on absolute values),
@@ -702,7 +728,12 @@ constexpr int fam_of(int KIND) {
  * round robin (uniform work per lane), writes every slot's flag coalesced
  * and the four vertex ids only of the slots that are kept or undecided
  * (the later stages read no others).  Slots past the LDS stage were
- * written to global memory during the merges and are filtered from there. */
+ * written to global memory during the merges and are filtered from there.
+ * A candidate with a covered edge (kDeadBit of one of its triangles in
+ * tkd, carried through the merge in the slot's first id) is filtered like
+ * any other, but an alpha tet among them is only counted (CTR_DROP), not
+ * written: it cannot be empty.  On the 100k globule 4.6M of the 19.1M
+ * alpha tets are written. */
 /* First slot of alpha triangle q without a per-triangle offset array:
  * the triangles of edge e occupy rows trow[e] .. trow[e+1]-1 and each has
  * its row's tail after it as slots, so triangle s + k of a row of L = trow
@@ -720,7 +751,7 @@ __device__ __forceinline__ uint64_t tet_slot_off(const uint64_t* roff,
 template <class R, bool BUF>
 __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_filter(
-    Stage S, Cnt c_nt, const uint64_t* trow, const uint32_t* tk,
+    Stage S, Cnt c_nt, const uint64_t* trow, const uint32_t* tkd,
     const uint32_t* tedge, const uint32_t* teik, const uint32_t* tejk,
     const uint32_t* eleft, const uint32_t* ecol, const uint64_t* off,
     const uint64_t* roff, uint64_t* bbase, uint4* ctet, uint8_t* flag,
@@ -767,38 +798,45 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
   unsigned found = 0;
   if (q < nt) {
     const uint32_t eik = teik[q], ejk = tejk[q];
-    const uint32_t i = eleft[eij], j = ecol[eij], k = tk[q];
+    const uint32_t kd = tkd[q], k = kd & ~kDeadBit;
+    const uint32_t i = eleft[eij], j = ecol[eij];
     if constexpr (BUF) {
-      /* the same merge over byte offsets into tk (below 4 GiB): no 64-bit
+      /* the same merge over byte offsets into tkd (below 4 GiB): no 64-bit
        * address arithmetic per load.  A triangle's slots are its row's
        * tail after it, so o < oe holds while a < ae, unless it was given
        * none (chunk sub-inputs): then the merge is empty. */
-      const BufU32 K{tk, (uint32_t)(c_nt.cap * 4)};
+      const BufU32 K{tkd, (uint32_t)(c_nt.cap * 4)};
       uint32_t a = ((uint32_t)q + 1u) << 2, ae = (uint32_t)trow[eij + 1] << 2;
       uint32_t b = (uint32_t)trow[eik] << 2, be = (uint32_t)trow[eik + 1] << 2;
       uint32_t c = (uint32_t)trow[ejk] << 2, ce = (uint32_t)trow[ejk + 1] << 2;
       if (o == oe) ae = a;
       /* two merge steps a round: each list's next element is loaded with
-       * its current one (~0u past the row's end, above every ball id) */
+       * its current one (kEnd past the row's end, above every ball id) */
+      constexpr uint32_t kEnd = ~kDeadBit;
       while (a < ae && b < be && c < ce) {
-        const uint32_t x0 = K.at(a), y0 = K.at(b), z0 = K.at(c);
-        const uint32_t x1 = a + 4u < ae ? K.at(a + 4u) : ~0u;
-        const uint32_t y1 = b + 4u < be ? K.at(b + 4u) : ~0u;
-        const uint32_t z1 = c + 4u < ce ? K.at(c + 4u) : ~0u;
+        const uint32_t xd0 = K.at(a), yd0 = K.at(b), zd0 = K.at(c);
+        const uint32_t xd1 = a + 4u < ae ? K.at(a + 4u) : kEnd;
+        const uint32_t yd1 = b + 4u < be ? K.at(b + 4u) : kEnd;
+        const uint32_t zd1 = c + 4u < ce ? K.at(c + 4u) : kEnd;
+        const uint32_t x0 = xd0 & kEnd, y0 = yd0 & kEnd, z0 = zd0 & kEnd;
         const uint32_t m0 = max(x0, max(y0, z0));
         const bool all0 = x0 == m0 && y0 == m0 && z0 == m0;
         if (all0) {
-          B.put(ctet, o, make_uint4(i, j, k, m0));
+          const uint32_t dead = (kd | xd0 | yd0 | zd0) & kDeadBit;
+          B.put(ctet, o, make_uint4(i | dead, j, k, m0));
           ++o;
           ++found;
         }
         const bool sa = all0 || x0 < m0, sb = all0 || y0 < m0,
                    sc = all0 || z0 < m0;
-        const uint32_t x = sa ? x1 : x0, y = sb ? y1 : y0, z = sc ? z1 : z0;
+        const uint32_t xd = sa ? xd1 : xd0, yd = sb ? yd1 : yd0,
+                       zd = sc ? zd1 : zd0;
+        const uint32_t x = xd & kEnd, y = yd & kEnd, z = zd & kEnd;
         const uint32_t m = max(x, max(y, z));
         const bool all = x == m && y == m && z == m;
-        if (all && m != ~0u) {
-          B.put(ctet, o, make_uint4(i, j, k, m));
+        if (all && m != kEnd) {
+          const uint32_t dead = (kd | xd | yd | zd) & kDeadBit;
+          B.put(ctet, o, make_uint4(i | dead, j, k, m));
           ++o;
           ++found;
         }
@@ -815,10 +853,13 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
       uint32_t b = (uint32_t)trow[eik], be = (uint32_t)trow[eik + 1];
       uint32_t c = (uint32_t)trow[ejk], ce = (uint32_t)trow[ejk + 1];
       while (a < ae && b < be && c < ce && o < oe) {
-        const uint32_t x = tk[a], y = tk[b], z = tk[c];
+        const uint32_t xd = tkd[a], yd = tkd[b], zd = tkd[c];
+        const uint32_t x = xd & ~kDeadBit, y = yd & ~kDeadBit,
+                       z = zd & ~kDeadBit;
         const uint32_t m = max(x, max(y, z));
         if (x == m && y == m && z == m) {
-          B.put(ctet, o, make_uint4(i, j, k, m));
+          const uint32_t dead = (kd | xd | yd | zd) & kDeadBit;
+          B.put(ctet, o, make_uint4(i | dead, j, k, m));
           ++o;
           ++found;
           ++a;
@@ -846,6 +887,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
   uint32_t run = 0; /* kept + undecided written so far (block-uniform) */
+  unsigned dropped = 0;
   for (uint64_t r0 = 0; r0 < m; r0 += kBlock) {
     const uint64_t t = r0 + threadIdx.x;
     uint4 v = make_uint4(0xffffffffu, 0u, 0u, 0u);
@@ -853,6 +895,8 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
     if (t < m) {
       v = t < (uint64_t)CAP ? s_out[t] : ctet[base + t];
       if (v.x != 0xffffffffu) {
+        const bool dead = (v.x & kDeadBit) != 0;
+        v.x &= ~kDeadBit;
         const Ball bv[4] = {S.ball[v.x], S.ball[v.y], S.ball[v.z], S.ball[v.w]};
         /* the weights are first used after the test of D's sign; left
          * alone, the compiler loads them there, a second round trip per
@@ -860,6 +904,10 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
 #pragma unroll
         for (int k = 0; k < 4; ++k) asm volatile("" ::"v"(bv[k].w));
         r = tet_code_ss<R>(bv, S.alpha);
+        if (dead && r == KEEP) { /* an alpha tet, certainly not empty */
+          ++dropped;
+          r = REJECT;
+        }
       }
     }
     const uint64_t bm = __ballot(r != REJECT);
@@ -889,9 +937,10 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
     bkeep[blockIdx.x] = s_und ? kRecount : run;
   }
   block_flush(S.ctr, CTR_CAND + 2, found);
+  block_flush(S.ctr, CTR_DROP, dropped);
 }
 void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
-                            const uint32_t* tk, const uint32_t* tedge,
+                            const uint32_t* tkd, const uint32_t* tedge,
                             const uint32_t* teik, const uint32_t* tejk,
                             const uint32_t* eleft, const uint32_t* ecol,
                             const uint64_t* off, const uint64_t* roff,
@@ -900,13 +949,13 @@ void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
                             PipeLaunch L, uint64_t lim) {
   if (nt.cap <= 0) return;
   dim3 gr((unsigned)((nt.cap + kBlock - 1) / kBlock));
-  /* byte offsets into tk while it stays below 4 GiB */
+  /* byte offsets into tkd while it stays below 4 GiB */
   const bool buf = nt.cap < ((int64_t)1 << 30);
   if constexpr (!kBallF64) {
     if (S.staged) {
       auto kf = buf ? k_tet_enum_filter<float, true>
                     : k_tet_enum_filter<float, false>;
-      hipLaunchKernelGGL(kf, gr, dim3(kBlock), 0, L.s, S, nt, trow, tk, tedge,
+      hipLaunchKernelGGL(kf, gr, dim3(kBlock), 0, L.s, S, nt, trow, tkd, tedge,
                          teik, tejk, eleft, ecol, off, roff, bbase, ctet, flag,
                          bcnt, bkeep, q1, lim);
       return;
@@ -914,7 +963,7 @@ void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
   }
   auto kd = buf ? k_tet_enum_filter<double, true>
                 : k_tet_enum_filter<double, false>;
-  hipLaunchKernelGGL(kd, gr, dim3(kBlock), 0, L.s, S, nt, trow, tk, tedge, teik,
+  hipLaunchKernelGGL(kd, gr, dim3(kBlock), 0, L.s, S, nt, trow, tkd, tedge, teik,
                      tejk, eleft, ecol, off, roff, bbase, ctet, flag, bcnt,
                      bkeep, q1, lim);
 }
@@ -1121,11 +1170,12 @@ void launch_seg_keep(int64_t n, const uint64_t* off, const uint32_t* bcnt,
   hipLaunchKernelGGL(k_seg_keep, dim3((unsigned)((n + kBlock - 1) / kBlock)),
                      dim3(kBlock), 0, L.s, n, off, bcnt, flag, keep);
 }
-/* ball i's kept edges (one wave per ball) to (ecol, eleft)[erow[i], ...) */
+/* ball i's kept edges (one wave per ball) to (ecol, eleft)[erow[i], ...),
+ * their marks in edead (if given) cleared for the triangle stage */
 __global__ __launch_bounds__(kBlock) void k_edge_copy(
     int64_t n, const uint64_t* off, const uint32_t* bcnt, const uint32_t* cval,
     const uint8_t* flag, const uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
-    uint64_t ocap) {
+    uint8_t* edead, uint64_t ocap) {
   const int64_t iw = (int64_t)blockIdx.x * kEdgeBallsPerBlock + (threadIdx.x >> 6);
   if (iw >= n) return;
   const uint32_t i = __builtin_amdgcn_readfirstlane((uint32_t)iw);
@@ -1143,6 +1193,7 @@ __global__ __launch_bounds__(kBlock) void k_edge_copy(
       if (w < ocap) {
         ecol[w] = cval[base + t];
         eleft[w] = i;
+        if (edead) edead[w] = 0;
       }
     }
     o += (uint64_t)__popcll(bm);
@@ -1151,12 +1202,13 @@ __global__ __launch_bounds__(kBlock) void k_edge_copy(
 void launch_edge_copy(int64_t n, const uint64_t* off, const uint32_t* bcnt,
                       const uint32_t* cval, const uint8_t* flag,
                       const uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
-                      PipeLaunch L, uint64_t ocap) {
+                      uint8_t* edead, PipeLaunch L, uint64_t ocap) {
   if (n <= 0) return;
   hipLaunchKernelGGL(
       k_edge_copy,
       dim3((unsigned)((n + kEdgeBallsPerBlock - 1) / kEdgeBallsPerBlock)),
-      dim3(kBlock), 0, L.s, n, off, bcnt, cval, flag, erow, ecol, eleft, ocap);
+      dim3(kBlock), 0, L.s, n, off, bcnt, cval, flag, erow, ecol, eleft, edead,
+      ocap);
 }
 
 /* Triangles of alpha edge q = (i, j) -- k in row(i) after j and in row(j),
@@ -1167,13 +1219,16 @@ void launch_edge_copy(int64_t n, const uint64_t* off, const uint32_t* bcnt,
  * filtered round robin (uniform work per lane) and the kept and undecided
  * ones written compacted, in slot order, from the block's first slot on
  * (as in k_tet_enum_filter), four arrays and the flag; the filter never
- * reads an array the enumeration wrote for every slot. */
+ * reads an array the enumeration wrote for every slot.
+ * edead (alpha edges, cleared; may be null): set for the edges a rejected
+ * candidate shows covered by one ball (tri_code_ss): no simplex with such
+ * an edge is empty. */
 template <class R, bool BUF>
 __global__ __launch_bounds__(kBlock) void k_tri_enum_filter(
     Stage S, Cnt c_ne, const uint64_t* erow, const uint32_t* ecol,
     const uint32_t* eleft, const uint64_t* off, uint32_t* cval,
     uint32_t* cseg, uint32_t* cea, uint32_t* ceb, uint8_t* flag,
-    uint32_t* bcnt, uint32_t* bkeep, Queue q1, uint64_t lim) {
+    uint32_t* bcnt, uint32_t* bkeep, uint8_t* edead, Queue q1, uint64_t lim) {
   const int64_t ne = c_ne.get();
   /* 6 blocks per CU fit in LDS with the edge table and block_flush's 16 B
    * (a block averages ~1,800 slots on the 100k globule; the rest go to
@@ -1260,7 +1315,13 @@ __global__ __launch_bounds__(kBlock) void k_tri_enum_filter(
       const Ball b0 = S.ball[ij.x], b1 = S.ball[ij.y], b2 = S.ball[v[0]];
       /* weights used here: one 16-byte load per ball (as for tets) */
       asm volatile("" ::"v"(b0.w), "v"(b1.w), "v"(b2.w));
-      r = tri_code_ss<R>(b0, b1, b2, S.alpha);
+      unsigned cover;
+      r = tri_code_ss<R>(b0, b1, b2, S.alpha, cover);
+      if (cover && edead) { /* opposite edges: (j, k), (i, k), (i, j) */
+        if (cover & 1u) edead[v[3]] = 1;
+        if (cover & 2u) edead[v[2]] = 1;
+        if (cover & 4u) edead[v[1]] = 1;
+      }
     }
     const uint64_t bm = __ballot(r != REJECT);
     if (lane == 0) s_wsum[w] = (unsigned)__popcll(bm);
@@ -1296,7 +1357,8 @@ void launch_tri_enum_filter(const Stage& S, Cnt ne, const uint64_t* erow,
                             const uint64_t* off, uint32_t* cval,
                             uint32_t* cseg, uint32_t* cea, uint32_t* ceb,
                             uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep,
-                            Queue q1, PipeLaunch L, uint64_t lim) {
+                            uint8_t* edead, Queue q1, PipeLaunch L,
+                            uint64_t lim) {
   if (ne.cap <= 0) return;
   dim3 gr((unsigned)((ne.cap + kBlock - 1) / kBlock));
   /* byte offsets into ecol while it stays below 4 GiB */
@@ -1306,19 +1368,21 @@ void launch_tri_enum_filter(const Stage& S, Cnt ne, const uint64_t* erow,
                      : (buf ? k_tri_enum_filter<double, true>
                             : k_tri_enum_filter<double, false>);
   hipLaunchKernelGGL(kf, gr, dim3(kBlock), 0, L.s, S, ne, erow, ecol, eleft, off,
-                     cval, cseg, cea, ceb, flag, bcnt, bkeep, q1, lim);
+                     cval, cseg, cea, ceb, flag, bcnt, bkeep, edead, q1, lim);
 }
 /* the kept triangles of block b to (tk, tedge, teik, tejk)[bout[b], ...)
  * in order; trow[e] for the block's edges e (and trow[ne], by the block
  * holding index ne) = bout[b] + the block's kept triangles of edges
- * before e (counted per edge in LDS, then scanned).  Grid: nblk + 1
- * blocks, nblk = ceil(ne.cap / 256); bout has nblk + 1 entries. */
+ * before e (counted per edge in LDS, then scanned).  tkd: tk with
+ * kDeadBit set where one of the triangle's edges is marked in edead (null:
+ * none).  Grid: nblk + 1 blocks, nblk = ceil(ne.cap / 256); bout has
+ * nblk + 1 entries. */
 __global__ __launch_bounds__(kBlock) void k_tri_block_copy(
     Cnt c_ne, const uint64_t* off, const uint32_t* bcnt, const uint32_t* cval,
     const uint32_t* cseg, const uint32_t* cea, const uint32_t* ceb,
-    const uint8_t* flag, const uint64_t* bout, uint32_t* tk, uint32_t* tedge,
-    uint32_t* teik, uint32_t* tejk, uint64_t* trow, uint64_t* tpair,
-    uint64_t ocap) {
+    const uint8_t* flag, const uint64_t* bout, const uint8_t* edead,
+    uint32_t* tk, uint32_t* tkd, uint32_t* tedge, uint32_t* teik,
+    uint32_t* tejk, uint64_t* trow, uint64_t* tpair, uint64_t ocap) {
   const int64_t ne = c_ne.get();
   const int64_t b = blockIdx.x;
   const int64_t q0 = b * kBlock;
@@ -1354,6 +1418,8 @@ __global__ __launch_bounds__(kBlock) void k_tri_block_copy(
       }
       const bool keep = t < n && fv == KEEP;
       const uint32_t seg = keep ? sv : 0xffffffffu;
+      uint32_t xd = xv;
+      if (edead && keep && (edead[sv] | edead[av] | edead[bv])) xd |= kDeadBit;
       /* entries come in edge order: one LDS add per run of lanes with
        * the same edge (its first lane adds the run's length) instead of
        * one per lane on the same counter */
@@ -1369,6 +1435,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_block_copy(
         if (keep && o + t - r0 < ocap) {
           const uint64_t at = o + t - r0;
           tk[at] = xv;
+          tkd[at] = xd;
           tedge[at] = seg;
           teik[at] = av;
           tejk[at] = bv;
@@ -1388,6 +1455,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_block_copy(
       }
       if (keep && pre < ocap) {
         tk[pre] = xv;
+        tkd[pre] = xd;
         tedge[pre] = seg;
         teik[pre] = av;
         tejk[pre] = bv;
@@ -1423,13 +1491,14 @@ void launch_tri_block_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
                            const uint32_t* cval, const uint32_t* cseg,
                            const uint32_t* cea, const uint32_t* ceb,
                            const uint8_t* flag, const uint64_t* bout,
-                           uint32_t* tk, uint32_t* tedge, uint32_t* teik,
-                           uint32_t* tejk, uint64_t* trow, uint64_t* tpair,
-                           PipeLaunch L, uint64_t ocap) {
+                           const uint8_t* edead, uint32_t* tk, uint32_t* tkd,
+                           uint32_t* tedge, uint32_t* teik, uint32_t* tejk,
+                           uint64_t* trow, uint64_t* tpair, PipeLaunch L,
+                           uint64_t ocap) {
   const int64_t nblk = (std::max<int64_t>(ne.cap, 0) + kBlock - 1) / kBlock;
   hipLaunchKernelGGL(k_tri_block_copy, dim3((unsigned)(nblk + 1)), dim3(kBlock),
                      0, L.s, ne, off, bcnt, cval, cseg, cea, ceb, flag, bout,
-                     tk, tedge, teik, tejk, trow, tpair, ocap);
+                     edead, tk, tkd, tedge, teik, tejk, trow, tpair, ocap);
 }
 
 template <int KIND>

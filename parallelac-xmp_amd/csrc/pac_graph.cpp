@@ -237,7 +237,11 @@ void graph_create(const float* xyzr, const int64_t* offsets, int64_t nmol,
     const pac_result& pr = *probe->groups[g];
     for (int q = 0; q < RC_COUNT; ++q) {
       p.probe[q] = pr.sizes[q];
-      p.cap[q] = with_headroom(pr.sizes[q], headroom);
+      /* alpha tets: room for all of them, also those a covered edge kept
+       * out of the list, so that a changed input is accepted as long as
+       * its alpha tets keep within the headroom */
+      p.cap[q] = with_headroom(
+          q == RC_KALPHA ? pr.st.tet_alpha : pr.sizes[q], headroom);
       if (p.cap[q] >= ((int64_t)1 << 32) - 1)
         p.cap[q] = ((int64_t)1 << 32) - 2; /* survivors index with uint32 */
     }

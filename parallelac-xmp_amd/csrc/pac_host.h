@@ -378,6 +378,7 @@ inline void stats_from_counters(const unsigned long long* hs, bool staged,
   const int hot = staged ? 0 : 1;
   st.tri_candidates += (int64_t)h[CTR_CAND + 1];
   st.tet_candidates += (int64_t)h[CTR_CAND + 2];
+  st.tet_alpha += (int64_t)h[CTR_DROP]; /* beside the listed ones */
   st.stage_evals[0][hot] += edge_candidates;
   st.stage_evals[1][hot] += (int64_t)h[CTR_CAND + 1];
   st.stage_evals[2][hot] += (int64_t)h[CTR_CAND + 2];

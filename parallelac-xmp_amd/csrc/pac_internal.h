@@ -63,6 +63,9 @@ struct Cnt {
   }
 };
 
+/* set in a triangle's third vertex (ball ids stay below 2^31 - 1) when one
+ * of its edges is covered by a single ball (k_tri_enum_filter) */
+constexpr uint32_t kDeadBit = 0x80000000u;
 struct QEntry {
   uint32_t item;  /* candidate / simplex index */
   uint32_t aux;   /* segment (ball / edge / triangle) or ball index */
@@ -74,7 +77,8 @@ enum {
   CTR_SOS = 24,
   CTR_PAIRS = 25,       /* [3] tet, tri, edge pairs */
   CTR_CAND = 28,        /* [3] candidates: (unused), triangles, tets */
-  CTR_COUNT = 31
+  CTR_DROP = 31,        /* alpha tets with a covered edge (not listed) */
+  CTR_COUNT = 32
 };
 constexpr int CTR_SLOTS = 32;   /* copies of each counter (see flush_ctr) */
 enum { FAM_EDGE = 0, FAM_TRI = 1, FAM_TET = 2, FAM_TET_AC2 = 3,
@@ -416,7 +420,7 @@ void launch_seg_keep(int64_t n, const uint64_t* off, const uint32_t* bcnt,
 void launch_edge_copy(int64_t n, const uint64_t* off, const uint32_t* bcnt,
                       const uint32_t* cval, const uint8_t* flag,
                       const uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
-                      PipeLaunch L, uint64_t ocap = ~0ull);
+                      uint8_t* edead, PipeLaunch L, uint64_t ocap = ~0ull);
 /* slot capacity of item q = row[owner[q] + 1] - q - 1 */
 void launch_tail_caps(Cnt m, const uint64_t* row, const uint32_t* owner,
                       uint32_t* cap, PipeLaunch L);
@@ -434,35 +438,42 @@ void launch_tri_count(Cnt ne, const uint64_t* erow, const uint32_t* ecol,
  * edges) writes its kept and undecided candidates (k, edge, edge(i,k),
  * edge(j,k)) with their flags, in order, compacted from its first slot
  * off[256 b] on and their number to bcnt[b]; undecided ones are queued on
- * q1 by position (aux = their edge) */
+ * q1 by position (aux = their edge).  edead[e] (cleared by the caller;
+ * null: not wanted) is set for the alpha edges a rejected candidate shows
+ * covered by one ball: no simplex with such an edge is empty. */
 void launch_tri_enum_filter(const Stage& S, Cnt ne, const uint64_t* erow,
                             const uint32_t* ecol, const uint32_t* eleft,
                             const uint64_t* off, uint32_t* cval,
                             uint32_t* cseg, uint32_t* cea, uint32_t* ceb,
                             uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep,
-                            Queue q1, PipeLaunch L, uint64_t lim = ~0ull);
+                            uint8_t* edead, Queue q1, PipeLaunch L,
+                            uint64_t lim = ~0ull);
 /* after the ladder (bkeep by launch_tet_block_keep over the ne alpha
  * edges, bout its exclusive scan): the kept triangles of each block to
- * (tk, tedge, teik, tejk) in order, the alpha-triangle row start of every
+ * (tk, tedge, teik, tejk) in order (tkd: tk with kDeadBit where one of the
+ * three edges is marked in edead), the alpha-triangle row start of every
  * alpha edge, trow[0 .. ne], and (tpair, if given) each edge's tet slots,
  * L (L - 1) / 2 for its L triangles (each one's row tail) */
 void launch_tri_block_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
                            const uint32_t* cval, const uint32_t* cseg,
                            const uint32_t* cea, const uint32_t* ceb,
                            const uint8_t* flag, const uint64_t* bout,
-                           uint32_t* tk, uint32_t* tedge, uint32_t* teik,
-                           uint32_t* tejk, uint64_t* trow, uint64_t* tpair,
-                           PipeLaunch L, uint64_t ocap = ~0ull);
+                           const uint8_t* edead, uint32_t* tk, uint32_t* tkd,
+                           uint32_t* tedge, uint32_t* teik, uint32_t* tejk,
+                           uint64_t* trow, uint64_t* tpair, PipeLaunch L,
+                           uint64_t ocap = ~0ull);
 /* tet candidates of the alpha triangles, each filtered by the first
  * precision stage in the same kernel; enumeration block b (256 alpha
  * triangles) writes its kept and undecided tets (i, j, k, l) with their
  * flags, in order, compacted from its first slot on (bbase[b]) and their
- * number to bcnt[b]; undecided ones are queued on q1 by position.  Slot
+ * number to bcnt[b]; undecided ones are queued on q1 by position.  Kept
+ * tets one of whose triangles has kDeadBit in tkd are counted (CTR_DROP)
+ * but not written.  Slot
  * offsets per triangle from off[], or (off null) from roff, the exclusive
  * scan of launch_tri_block_copy's tpair (each triangle's slots its row's
  * tail: not for chunk sub-inputs, whose unowned triangles get none) */
 void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
-                            const uint32_t* tk, const uint32_t* tedge,
+                            const uint32_t* tkd, const uint32_t* tedge,
                             const uint32_t* teik, const uint32_t* tejk,
                             const uint32_t* eleft, const uint32_t* ecol,
                             const uint64_t* off, const uint64_t* roff,
@@ -523,10 +534,10 @@ void launch_tet_ac2_exact_sorted(const Stage& S, const uint32_t* item,
 /* kind 0 triangles, 1 edges */
 void launch_low_ac2_hot(const Stage& S, int kind, Cnt nitems,
                         const uint32_t* ecol, const uint32_t* eleft,
-                        const uint32_t* tk, const uint32_t* tedge,
-                        const uint8_t* in_flag, uint8_t* flag, Queue q1,
-                        uint32_t* rest, unsigned* nrest, int budget,
-                        PipeLaunch L);
+                        const uint32_t* tkd, const uint32_t* tedge,
+                        const uint8_t* edead, const uint8_t* in_flag,
+                        uint8_t* flag, Queue q1, uint32_t* rest, unsigned* nrest,
+                        int budget, PipeLaunch L);
 void launch_low_ac2_esc(const Stage& S, int kind, QRef q,
                         const uint32_t* ecol, const uint32_t* eleft,
                         const uint32_t* tk, const uint32_t* tedge,

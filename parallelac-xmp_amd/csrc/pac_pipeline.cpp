@@ -539,6 +539,12 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   Cnt Ecand(0), Ealpha(0);
   DBuf<uint64_t> erow(P, n + 1);
   DBuf<uint32_t> ecol, eleft;
+  /* marks of the alpha edges covered by one ball (k_tri_enum_filter),
+   * whose simplices need no emptiness scan: with the exact cell policy,
+   * whose scans see every ball (the reference's stencil may miss the
+   * covering one), and where tets are tested */
+  const bool prune = opt.cell_policy == PAC_CELL_EXACT && !opt.skip_tet_ac2;
+  DBuf<uint8_t> edead;
   CandCtx C0{nullptr, nullptr, nullptr, nullptr, nullptr};
   if (!no_edges) {
     DBuf<uint64_t> off(P, n + 1);
@@ -578,8 +584,9 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
         RC_EALPHA);
     ecol = DBuf<uint32_t>(P, Ealpha.cap);
     eleft = DBuf<uint32_t>(P, Ealpha.cap);
+    if (prune) edead = DBuf<uint8_t>(P, Ealpha.cap);
     launch_edge_copy(n, off.get(), bcnt.get(), cval.get(), flag.get(),
-                     erow.get(), ecol.get(), eleft.get(), L,
+                     erow.get(), ecol.get(), eleft.get(), edead.get(), L,
                      (uint64_t)Ealpha.cap);
     KCHK();
   } else {
@@ -597,7 +604,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
    * triangles no slots and keep per-triangle offsets */
   const bool tail_slots = !SG.chunk;
   DBuf<uint64_t> tpair(P, tail_slots ? std::max<int64_t>(Ealpha.cap, 1) : 1);
-  DBuf<uint32_t> tk, tedge, teik, tejk;
+  DBuf<uint32_t> tk, tkd, tedge, teik, tejk;
+  uint8_t* const dead = edead.get();
   CandCtx C1{eleft.get(), ecol.get(), nullptr, nullptr, nullptr};
   {
     DBuf<uint64_t> off(P, Ealpha.cap + 1);
@@ -631,7 +639,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           launch_tri_enum_filter(SG, Ealpha, erow.get(), ecol.get(), eleft.get(),
                                  off.get(), cval.get(), cseg.get(), cea.get(),
                                  ceb.get(), flag.get(), bcnt.get(), bkeep.get(),
-                                 qq, L, (uint64_t)Tslots.cap);
+                                 dead, qq, L, (uint64_t)Tslots.cap);
         },
         [&](QRef qr, Queue q2) {
           launch_filter_esc(SG, 2, C1, qr, cval.get(), flag.get(), q2, L);
@@ -647,12 +655,13 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
         },
         RC_TALPHA);
     tk = DBuf<uint32_t>(P, Talpha.cap);
+    tkd = DBuf<uint32_t>(P, Talpha.cap);
     tedge = DBuf<uint32_t>(P, Talpha.cap);
     teik = DBuf<uint32_t>(P, Talpha.cap);
     tejk = DBuf<uint32_t>(P, Talpha.cap);
     launch_tri_block_copy(Ealpha, off.get(), bcnt.get(), cval.get(), cseg.get(),
-                          cea.get(), ceb.get(), flag.get(), bout.get(), tk.get(),
-                          tedge.get(), teik.get(), tejk.get(), trow.get(),
+                          cea.get(), ceb.get(), flag.get(), bout.get(), dead,
+                          tk.get(), tkd.get(), tedge.get(), teik.get(), tejk.get(), trow.get(),
                           tail_slots ? tpair.get() : nullptr, L,
                           (uint64_t)Talpha.cap);
     KCHK();
@@ -703,9 +712,11 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     Kalpha = ladder(
         std::min<int64_t>(Kslots.cap, Kslots.cap / 32 + 65536), KP_TET_FILL, -1,
         [&](Queue qq) {
-          if (runs++ && !rec)
+          if (runs++ && !rec) {
             zero_u64(ctr + (CTR_CAND + 2) * CTR_SLOTS, CTR_SLOTS, s);
-          launch_tet_enum_filter(SG, Talpha, trow.get(), tk.get(), tedge.get(),
+            zero_u64(ctr + CTR_DROP * CTR_SLOTS, CTR_SLOTS, s);
+          }
+          launch_tet_enum_filter(SG, Talpha, trow.get(), tkd.get(), tedge.get(),
                                  teik.get(), tejk.get(), eleft.get(), ecol.get(),
                                  tail_slots ? nullptr : off.get(),
                                  tail_slots ? roff.get() : nullptr, bbase.get(),
@@ -856,8 +867,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       Tf = ladder(
           ac2_cap(Talpha.cap), KP_TRI_AC2, -1,
           [&](Queue q) {
-            launch_low_ac2_hot(SG, 0, Talpha, ecol.get(), eleft.get(), tk.get(),
-                               tedge.get(), tri_skip, tflag.get(), q,
+            launch_low_ac2_hot(SG, 0, Talpha, ecol.get(), eleft.get(), tkd.get(),
+                               tedge.get(), nullptr, tri_skip, tflag.get(), q,
                                rest.get(), nrest, budget, L);
           },
           [&](QRef q, Queue q2) {
@@ -923,7 +934,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           ac2_cap(Ealpha.cap), KP_EDGE_AC2, -1,
           [&](Queue q) {
             launch_low_ac2_hot(SG, 1, Ealpha, ecol.get(), eleft.get(), nullptr,
-                               nullptr, edge_skip, eflag.get(), q,
+                               nullptr, dead, edge_skip, eflag.get(), q,
                                rest.get(), nrest, budget, L);
           },
           [&](QRef q, Queue q2) {

@@ -260,9 +260,13 @@ __global__ __launch_bounds__(kBlock) void k_tet_ac2_quick(
   block_flush(S.ctr, CTR_PAIRS + 0, pairs);
 }
 
+/* What an emptiness kernel walks: every simplex (one per thread), or those
+ * a pass before it listed, up to the phase-one budget; or the ones the
+ * first phase left. */
+enum { PH_ALL = 0, PH_LIST = 1, PH_REST = 2 };
 /* Phase A (budget > 0): at most `budget` pair tests per tet, in scan order;
  * tets not settled within the budget are appended to `rest`.  Phase B
- * (grid-stride over `rest`): the remaining pairs of those tets, skipping the
+ * (persistent, over `rest`): the remaining pairs of those tets, skipping the
  * first `budget` ones.  Splitting keeps lanes of a wave busy with similar
  * amounts of work: most tets are rejected by one of their first few
  * neighbours, while accepted tets must test every ball of their box.
@@ -270,32 +274,32 @@ __global__ __launch_bounds__(kBlock) void k_tet_ac2_quick(
  * (balls in fine-cell order, fid their ids).  A vertex of the simplex lies
  * on its orthosphere, so its certified test is always undecided: the
  * fine scan looks a ball's id up only then, to skip the vertices. */
-template <class R, bool PHASE_B, bool FINE, bool MOL>
+template <class R, int PH, bool FINE, bool MOL>
 __global__ __launch_bounds__(kBlock) void k_tet_ac2_hot(
-    Stage S, Cnt c_nk, const uint32_t* items, const unsigned* nitems,
+    Stage S0, Cnt c_nk, const uint32_t* items, const unsigned* nitems,
     const uint4* tets, uint8_t* flag, Queue q1, uint32_t* rest,
     unsigned* nrest, int budget) {
   unsigned evals = 0, pairs = 0;
   /* phase A: the alpha tets, or the list `items` of them (those the quick
    * pass left); phase B: `rest` */
   __shared__ uint32_t s_pre[LSLOTS + 1];
-  if (PHASE_B) list_table(nrest, S.lcap, s_pre);
-  else if (items) list_table(nitems, S.lcap, s_pre);
+  if (PH != PH_ALL) list_table(PH == PH_REST ? nrest : nitems, S0.lcap, s_pre);
   const int64_t total =
-      PHASE_B || items ? (int64_t)s_pre[LSLOTS] : c_nk.get();
-  uint32_t rest_id = 0xffffffffu; /* phase A: at most one item per thread */
+      PH != PH_ALL ? (int64_t)s_pre[LSLOTS] : c_nk.get();
+  uint32_t rest_id = 0xffffffffu; /* phase A: the item left for phase B */
   auto item = [&](int64_t w) {
+    const Stage& S = fresh_stage();
     const int64_t id =
-        PHASE_B ? (int64_t)list_at(rest, S.lcap, s_pre, (uint32_t)w)
-                : (items ? (int64_t)list_at(items, S.lcap, s_pre, (uint32_t)w)
-                         : w);
+        PH == PH_ALL ? w
+                     : (int64_t)list_at(PH == PH_REST ? rest : items, S.lcap,
+                                        s_pre, (uint32_t)w);
     uint4 t = tets[id];
     Ball v[4] = {S.ball[t.x], S.ball[t.y], S.ball[t.z], S.ball[t.w]};
     const GridP g = FINE ? sgrid_at<MOL>(S, t.x) : grid_at<MOL>(S, t.x);
     PairSS<R> P;
     typename std::conditional<FINE, SphBox, CellBox>::type box;
     if (!tet_setup(g, v, P, box)) {
-      if (!PHASE_B) {
+      if (PH != PH_REST) {
         push_q(q1, (uint32_t)id, 0xffffffffu);
         flag[id] = 2;
       }
@@ -309,7 +313,7 @@ __global__ __launch_bounds__(kBlock) void k_tet_ac2_hot(
     int seen = 0;
     auto visit = [&](uint32_t j, const Ball& E) {
       if (!FINE && (j == t.x || j == t.y || j == t.z || j == t.w)) return false;
-      if (PHASE_B) {
+      if (PH == PH_REST) {
         if (seen < budget) {
           ++seen;
           return false;
@@ -342,7 +346,7 @@ __global__ __launch_bounds__(kBlock) void k_tet_ac2_hot(
      * a group all run; a certain violator among them ends the scan (its
      * ties need no queueing: the tet is rejected). */
     auto group = [&](uint32_t p, uint32_t n) -> bool {
-      if (PHASE_B) {
+      if (PH == PH_REST) {
         if (seen < budget) {
           seen += (int)n;
           return false;
@@ -381,7 +385,7 @@ __global__ __launch_bounds__(kBlock) void k_tet_ac2_hot(
       scan_sph_flat(g, S.fstart, box, group);
     else
       scan_box4(g, S.cstart, S.ball, box, visit);
-    if (PHASE_B) {
+    if (PH == PH_REST) {
       if (stop == 1)
         flag[id] = 0;
       else if (pending)
@@ -391,16 +395,17 @@ __global__ __launch_bounds__(kBlock) void k_tet_ac2_hot(
       if (stop == 2) rest_id = (uint32_t)id;
     }
   };
-  if constexpr (PHASE_B) {
-    for_work(S.bchunk, total, item); /* persistent launch */
+  if constexpr (PH == PH_REST) {
+    for_work(S0.bchunk, total, item); /* persistent launch */
   } else {
+    /* (a list's grid covers all simplices: its length is known only on the
+     * device, and a loop over it costs 30 VGPRs, 7 -> 4 waves per SIMD) */
+    if ((int64_t)blockIdx.x * kBlock >= total) return;
     if (gtid() < total) item(gtid());
-  }
-  if (!PHASE_B) {
-    list_append(rest, nrest, S.lcap, rest_id != 0xffffffffu, rest_id);
+    list_append(rest, nrest, S0.lcap, rest_id != 0xffffffffu, rest_id);
   }
   (void)evals;
-  block_flush(S.ctr, CTR_PAIRS + 0, pairs);
+  block_flush(S0.ctr, CTR_PAIRS + 0, pairs);
 }
 
 /* FP64 then double-double for queued pairs / uncertified tets */
@@ -736,45 +741,108 @@ __device__ __forceinline__ bool low_setup(const GridP& g, const Ball* v,
   return place_box<R>(g, simplex_reach<R>(g, rho_up), c, e, box);
 }
 
-/* KIND 0: triangles (items = alpha triangle ids), 1: edges (alpha edge ids).
- * Simplices already in the closure (in_flag) pass without a test, those
- * with an edge that one ball covers (kDeadBit in tkd, edead) fail without
- * one: a third of the 100k globule's alpha triangles and half of its alpha
- * edges are left to scan.  Same phase A / phase B split as the tet kernel. */
-template <class R, int KIND, bool PHASE_B, bool FINE, bool MOL>
+/* KIND 0: triangles (items = alpha triangle ids), 1: edges (alpha edge
+ * ids).  What is decided without a scan: 1 for a simplex already in the
+ * closure (in_flag), 0 for one with an edge that one ball covers (kDeadBit
+ * in tkd, edead), else -1. */
+template <int KIND>
+__device__ __forceinline__ int low_known(int64_t id, const uint32_t* tkd,
+                                         const uint8_t* edead,
+                                         const uint8_t* in_flag) {
+  if (in_flag[id]) return 1;
+  if (KIND == 0) return (tkd[id] & kDeadBit) ? 0 : -1;
+  return edead && edead[id] ? 0 : -1;
+}
+/* The flags of the simplices decided without a scan, and the list of the
+ * others: on the 100k globule 2.4M of 11.4M triangles and 0.4M of 2.2M
+ * edges.  Scanned in place, the few of each wave keep all of it busy:
+ * triangle phase A 280 us against 33 us for the list and 116 us for its
+ * scans. */
+template <int KIND>
+__global__ __launch_bounds__(kBlock) void k_low_list(
+    Stage S, Cnt c_n, const uint32_t* tkd, const uint8_t* edead,
+    const uint8_t* in_flag, uint8_t* flag, uint32_t* next, unsigned* nnext) {
+  /* kListRun items a thread, 256 apart (coalesced), one append for all */
+  const int64_t n = c_n.get();
+  const int64_t i0 = (int64_t)blockIdx.x * (kBlock * kListRun) + threadIdx.x;
+  int c[kListRun];
+#pragma unroll
+  for (int q = 0; q < kListRun; ++q) {
+    const int64_t id = i0 + q * kBlock;
+    c[q] = id < n ? low_known<KIND>(id, tkd, edead, in_flag) : 0;
+  }
+#pragma unroll
+  for (int q = 0; q < kListRun; ++q) {
+    const int64_t id = i0 + q * kBlock;
+    if (id < n && c[q] >= 0) flag[id] = (uint8_t)c[q];
+  }
+  /* positions: by thread within the wave, then by wave; a wave's items stay
+   * together, neighbours in the list share their surroundings */
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  __shared__ unsigned s_w[kBlock / 64], s_base;
+  unsigned wtot = 0;
+  uint64_t m[kListRun];
+#pragma unroll
+  for (int q = 0; q < kListRun; ++q) {
+    m[q] = __ballot(c[q] < 0);
+    wtot += (unsigned)__popcll(m[q]);
+  }
+  if (lane == 0) s_w[w] = wtot;
+  __syncthreads();
+  const unsigned k = blockIdx.x & (LSLOTS - 1);
+  if (threadIdx.x == 0) {
+    unsigned t = 0;
+    for (int q = 0; q < kBlock / 64; ++q) t += s_w[q];
+    s_base = t ? atomicAdd(nnext + k * kSlotWords, t) : 0u;
+  }
+  __syncthreads();
+  unsigned at = s_base;
+  for (int q = 0; q < w; ++q) at += s_w[q];
+  const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+#pragma unroll
+  for (int q = 0; q < kListRun; ++q) {
+    const unsigned o = at + (unsigned)__popcll(m[q] & lt);
+    if (c[q] < 0 && o < S.lcap)
+      next[(uint64_t)k * S.lcap + o] = (uint32_t)(i0 + q * kBlock);
+    at += (unsigned)__popcll(m[q]);
+  }
+}
+
+/* Same phase A / phase B split as the tet kernel; phase A runs over the
+ * listed simplices (items), or over all, deciding the known ones itself. */
+template <class R, int KIND, int PH, bool FINE, bool MOL>
 __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
-    Stage S, Cnt c_nitems, const uint32_t* ecol, const uint32_t* eleft,
+    Stage S0, Cnt c_nitems, const uint32_t* items, const unsigned* nitems,
+    const uint32_t* ecol, const uint32_t* eleft,
     const uint32_t* tkd, const uint32_t* tedge, const uint8_t* edead,
     const uint8_t* in_flag, uint8_t* flag, Queue q1, uint32_t* rest,
     unsigned* nrest, int budget) {
   unsigned evals = 0, pairs = 0;
   __shared__ uint32_t s_pre[LSLOTS + 1];
-  if (PHASE_B) list_table(nrest, S.lcap, s_pre);
-  const int64_t total = PHASE_B ? (int64_t)s_pre[LSLOTS] : c_nitems.get();
-  uint32_t rest_id = 0xffffffffu; /* phase A: at most one item per thread */
+  if (PH != PH_ALL) list_table(PH == PH_REST ? nrest : nitems, S0.lcap, s_pre);
+  const int64_t total =
+      PH != PH_ALL ? (int64_t)s_pre[LSLOTS] : c_nitems.get();
+  uint32_t rest_id = 0xffffffffu; /* phase A: the item left for phase B */
   auto item = [&](int64_t w) {
+    const Stage& S = fresh_stage();
     const int64_t id =
-        PHASE_B ? (int64_t)list_at(rest, S.lcap, s_pre, (uint32_t)w) : w;
-    if (!PHASE_B && in_flag[id]) {
-      flag[id] = 1;
-      return;
+        PH == PH_ALL ? w
+                     : (int64_t)list_at(PH == PH_REST ? rest : items, S.lcap,
+                                        s_pre, (uint32_t)w);
+    if (PH == PH_ALL) {
+      const int c = low_known<KIND>(id, tkd, edead, in_flag);
+      if (c >= 0) {
+        flag[id] = (uint8_t)c;
+        return;
+      }
     }
     uint32_t vid[3];
     if (KIND == 0) {
       uint32_t e = tedge[id];
-      const uint32_t kd = tkd[id];
-      if (!PHASE_B && (kd & kDeadBit)) { /* an edge of it is covered */
-        flag[id] = 0;
-        return;
-      }
       vid[0] = eleft[e];
       vid[1] = ecol[e];
-      vid[2] = kd & ~kDeadBit;
+      vid[2] = tkd[id] & ~kDeadBit;
     } else {
-      if (!PHASE_B && edead && edead[id]) {
-        flag[id] = 0;
-        return;
-      }
       vid[0] = eleft[id];
       vid[1] = ecol[id];
       vid[2] = vid[1];
@@ -784,7 +852,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     PairSS<R> P;
     typename std::conditional<FINE, SphBox, CellBox>::type box;
     if (!low_setup<R, KIND>(g, v, P, box)) {
-      if (!PHASE_B) {
+      if (PH != PH_REST) {
         push_q(q1, (uint32_t)id, 0xffffffffu);
         flag[id] = 2;
       }
@@ -795,7 +863,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     int seen = 0;
     auto visit = [&](uint32_t j, const Ball& E) {
       if (!FINE && (j == vid[0] || j == vid[1] || j == vid[2])) return false;
-      if (PHASE_B) {
+      if (PH == PH_REST) {
         if (seen < budget) {
           ++seen;
           return false;
@@ -823,7 +891,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     };
     /* fine grid: four balls at a time, as in k_tet_ac2_hot */
     auto group = [&](uint32_t p, uint32_t n) -> bool {
-      if (PHASE_B) {
+      if (PH == PH_REST) {
         if (seen < budget) {
           seen += (int)n;
           return false;
@@ -860,7 +928,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
       scan_sph_flat(g, S.fstart, box, group);
     else
       scan_box4(g, S.cstart, S.ball, box, visit);
-    if (PHASE_B) {
+    if (PH == PH_REST) {
       if (stop == 1)
         flag[id] = 0;
       else if (pending)
@@ -870,16 +938,17 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
       if (stop == 2) rest_id = (uint32_t)id;
     }
   };
-  if constexpr (PHASE_B) {
-    for_work(S.bchunk, total, item); /* persistent launch */
+  if constexpr (PH == PH_REST) {
+    for_work(S0.bchunk, total, item); /* persistent launch */
   } else {
+    /* (a list's grid covers all simplices: its length is known only on the
+     * device, and a loop over it costs 30 VGPRs, 7 -> 4 waves per SIMD) */
+    if ((int64_t)blockIdx.x * kBlock >= total) return;
     if (gtid() < total) item(gtid());
-  }
-  if (!PHASE_B) {
-    list_append(rest, nrest, S.lcap, rest_id != 0xffffffffu, rest_id);
+    list_append(rest, nrest, S0.lcap, rest_id != 0xffffffffu, rest_id);
   }
   (void)evals;
-  block_flush(S.ctr, CTR_PAIRS + 1 + KIND, pairs);
+  block_flush(S0.ctr, CTR_PAIRS + 1 + KIND, pairs);
 }
 
 template <int KIND>
@@ -1131,21 +1200,24 @@ static void tet_hot3(const Stage& S, Cnt nk, const uint4* tets, uint8_t* flag,
   dim3 gr((unsigned)((nk.cap + kBlock - 1) / kBlock)), gb((unsigned)S.bgrid);
   const uint32_t* items = nullptr;
   if (FINE && S.quick) { /* quick pass, then the certified scan of the rest */
-    zero_u32(nnext, LSLOTS, L.s);
     hipLaunchKernelGGL((k_tet_ac2_quick<R, MOL>), gr, dim3(kBlock), 0, L.s, S,
                        nk, tets, flag, next, nnext);
     items = next;
   } else if (S.chunk) {
-    zero_u32(nnext, LSLOTS, L.s);
     hipLaunchKernelGGL(k_tet_need, gr, dim3(kBlock), 0, L.s, S, nk, tets, flag,
                        next, nnext);
     items = next;
   }
-  hipLaunchKernelGGL((k_tet_ac2_hot<R, false, FINE, MOL>), gr, dim3(kBlock), 0,
-                     L.s, S, nk, items, nnext, tets, flag, q1, rest, nrest,
-                     budget);
+  if (items)
+    hipLaunchKernelGGL((k_tet_ac2_hot<R, PH_LIST, FINE, MOL>), gr,
+                       dim3(kBlock), 0, L.s, S, nk, items, nnext, tets, flag,
+                       q1, rest, nrest, budget);
+  else
+    hipLaunchKernelGGL((k_tet_ac2_hot<R, PH_ALL, FINE, MOL>), gr, dim3(kBlock),
+                       0, L.s, S, nk, items, nnext, tets, flag, q1, rest, nrest,
+                       budget);
   if (budget > 0) {
-    hipLaunchKernelGGL((k_tet_ac2_hot<R, true, FINE, MOL>), gb,
+    hipLaunchKernelGGL((k_tet_ac2_hot<R, PH_REST, FINE, MOL>), gb,
                        dim3((unsigned)S.bblock), 0, L.s, S, nk, items, nnext,
                        tets, flag, q1, rest, nrest, budget);
   }
@@ -1243,17 +1315,31 @@ static void low_hot4(const Stage& S, Cnt nitems, const uint32_t* ecol,
                      const uint32_t* eleft, const uint32_t* tkd,
                      const uint32_t* tedge, const uint8_t* edead,
                      const uint8_t* in_flag, uint8_t* flag, Queue q1,
-                     uint32_t* rest, unsigned* nrest, int budget,
-                     PipeLaunch L) {
-  dim3 gr((unsigned)((nitems.cap + kBlock - 1) / kBlock)), gb((unsigned)S.bgrid);
-  hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, false, FINE, MOL>), gr,
-                     dim3(kBlock), 0, L.s, S, nitems, ecol, eleft, tkd, tedge,
-                     edead, in_flag, flag, q1, rest, nrest, budget);
-  if (budget > 0) {
-    hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, true, FINE, MOL>), gb,
-                       dim3((unsigned)S.bblock), 0, L.s, S, nitems, ecol, eleft,
-                       tkd, tedge, edead, in_flag, flag, q1, rest, nrest,
+                     uint32_t* rest, unsigned* nrest, uint32_t* next,
+                     unsigned* nnext, int budget, PipeLaunch L) {
+  const dim3 gr((unsigned)((nitems.cap + kBlock - 1) / kBlock)),
+      gb((unsigned)S.bgrid);
+  if (nitems.cap >= kListItems) {
+    const int64_t per = kBlock * kListRun;
+    hipLaunchKernelGGL(k_low_list<KIND>,
+                       dim3((unsigned)((nitems.cap + per - 1) / per)),
+                       dim3(kBlock), 0, L.s, S, nitems, tkd, edead, in_flag,
+                       flag, next, nnext);
+    hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, PH_LIST, FINE, MOL>), gr,
+                       dim3(kBlock), 0, L.s, S, nitems, next,
+                       nnext, ecol, eleft, tkd, tedge, edead, in_flag, flag, q1,
+                       rest, nrest, budget);
+  } else {
+    hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, PH_ALL, FINE, MOL>), gr,
+                       dim3(kBlock), 0, L.s, S, nitems, next, nnext, ecol,
+                       eleft, tkd, tedge, edead, in_flag, flag, q1, rest, nrest,
                        budget);
+  }
+  if (budget > 0) {
+    hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, PH_REST, FINE, MOL>), gb,
+                       dim3((unsigned)S.bblock), 0, L.s, S, nitems, next, nnext,
+                       ecol, eleft, tkd, tedge, edead, in_flag, flag, q1, rest,
+                       nrest, budget);
   }
 }
 template <class R, int KIND, bool FINE>
@@ -1261,53 +1347,57 @@ static void low_hot3(const Stage& S, Cnt nitems, const uint32_t* ecol,
                      const uint32_t* eleft, const uint32_t* tkd,
                      const uint32_t* tedge, const uint8_t* edead,
                      const uint8_t* in_flag, uint8_t* flag, Queue q1,
-                     uint32_t* rest, unsigned* nrest, int budget,
-                     PipeLaunch L) {
+                     uint32_t* rest, unsigned* nrest, uint32_t* next,
+                     unsigned* nnext, int budget, PipeLaunch L) {
   if (S.mol)
     low_hot4<R, KIND, FINE, true>(S, nitems, ecol, eleft, tkd, tedge, edead,
-                                  in_flag, flag, q1, rest, nrest, budget, L);
+                                  in_flag, flag, q1, rest, nrest, next, nnext,
+                                  budget, L);
   else
     low_hot4<R, KIND, FINE, false>(S, nitems, ecol, eleft, tkd, tedge, edead,
-                                   in_flag, flag, q1, rest, nrest, budget, L);
+                                   in_flag, flag, q1, rest, nrest, next, nnext,
+                                   budget, L);
 }
 template <class R, int KIND>
 static void low_hot2(const Stage& S, Cnt nitems, const uint32_t* ecol,
                      const uint32_t* eleft, const uint32_t* tkd,
                      const uint32_t* tedge, const uint8_t* edead,
                      const uint8_t* in_flag, uint8_t* flag, Queue q1,
-                     uint32_t* rest, unsigned* nrest, int budget,
-                     PipeLaunch L) {
+                     uint32_t* rest, unsigned* nrest, uint32_t* next,
+                     unsigned* nnext, int budget, PipeLaunch L) {
   if (S.fine)
     low_hot3<R, KIND, true>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
-                            flag, q1, rest, nrest, budget, L);
+                            flag, q1, rest, nrest, next, nnext, budget, L);
   else
-    low_hot3<R, KIND, false>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
-                             flag, q1, rest, nrest, budget, L);
+    low_hot3<R, KIND, false>(S, nitems, ecol, eleft, tkd, tedge, edead,
+                             in_flag, flag, q1, rest, nrest, next, nnext,
+                             budget, L);
 }
 void launch_low_ac2_hot(const Stage& S, int kind, Cnt nitems,
                         const uint32_t* ecol, const uint32_t* eleft,
                         const uint32_t* tkd, const uint32_t* tedge,
                         const uint8_t* edead, const uint8_t* in_flag,
                         uint8_t* flag, Queue q1, uint32_t* rest,
-                        unsigned* nrest, int budget, PipeLaunch L) {
+                        unsigned* nrest, uint32_t* next, unsigned* nnext,
+                        int budget, PipeLaunch L) {
   if (nitems.cap <= 0) return;
   if constexpr (!kBallF64) {
     if (S.staged) {
       if (kind == 0)
         low_hot2<float, 0>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
-                           flag, q1, rest, nrest, budget, L);
+                           flag, q1, rest, nrest, next, nnext, budget, L);
       else
         low_hot2<float, 1>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
-                           flag, q1, rest, nrest, budget, L);
+                           flag, q1, rest, nrest, next, nnext, budget, L);
       return;
     }
   }
   if (kind == 0)
     low_hot2<double, 0>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
-                        flag, q1, rest, nrest, budget, L);
+                        flag, q1, rest, nrest, next, nnext, budget, L);
   else
     low_hot2<double, 1>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
-                        flag, q1, rest, nrest, budget, L);
+                        flag, q1, rest, nrest, next, nnext, budget, L);
 }
 void launch_low_ac2_esc(const Stage& S, int kind, QRef q,
                         const uint32_t* ecol, const uint32_t* eleft,

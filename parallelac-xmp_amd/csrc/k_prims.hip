@@ -532,65 +532,89 @@ void radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
  * the capacity (entries were dropped) sets `bit` in *status and the
  * largest counter goes to *fill (fresh: both overwritten and fill[1]
  * cleared, for the ladder's second view; else merged).
- * The counters it read, and *also (if set), are cleared for the next
- * producer, so no separate zeroing launch precedes a ladder. */
-__global__ void k_make_view(const QEntry* q, uint32_t cap, unsigned* cnt,
-                            QView* v, unsigned* status, unsigned bit,
-                            unsigned* fill, unsigned* also, int fresh) {
-  if (threadIdx.x != 0) return;
-  unsigned c[QSLOTS];
-  unsigned mx = 0;
-  for (int k = 0; k < QSLOTS; ++k) {
-    c[k] = cnt[k];
-    cnt[k] = 0;
-    mx = c[k] > mx ? c[k] : mx;
+ * The counters it read, and (lists, the word of the QK_REST counters) the
+ * two lists' counters, are cleared for the next producer, so no separate
+ * zeroing launch precedes a ladder.  One wave, lane k for slot k. */
+__global__ __launch_bounds__(64) void k_make_view(const QEntry* q, uint32_t cap,
+                                                  unsigned* cnt, QView* v,
+                                                  unsigned* status,
+                                                  unsigned bit, unsigned* fill,
+                                                  unsigned* lists, int fresh) {
+  const int k = threadIdx.x;
+  const bool slot = k < QSLOTS;
+  const unsigned c = slot ? cnt[k * kSlotWords] : 0u;
+  if (slot) {
+    cnt[k * kSlotWords] = 0;
+    if (lists) {
+      lists[k * kSlotWords] = 0;
+      lists[k * kSlotWords + QK_NEXT - QK_REST] = 0;
+    }
   }
+  unsigned mx = c;
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1)
+    mx = max(mx, (unsigned)__shfl_xor((int)mx, d, 64));
   /* an eager ladder's first view (fresh) is empty when its queue
    * overflowed: the ladder runs again with a larger queue, and its
    * consumers need not work through the partial one */
-  const bool drop = fresh && mx > cap;
-  uint32_t acc = 0;
-  for (int k = 0; k < QSLOTS; ++k) {
-    v->off[k] = acc;
-    acc += drop ? 0u : (c[k] < cap ? c[k] : cap);
+  const uint32_t n = fresh && mx > cap ? 0u : (c < cap ? c : cap);
+  uint32_t incl = n;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t y = (uint32_t)__shfl_up((int)incl, d, 64);
+    if (k >= d) incl += y;
   }
-  v->off[QSLOTS] = acc;
-  v->q = q;
-  v->cap = cap;
-  if (also)
-    for (int k = 0; k < LSLOTS; ++k) also[k] = 0;
-  const unsigned b = mx > cap ? bit : 0u;
-  if (fresh) { /* first view of a ladder: also resets the second's fill */
-    fill[0] = mx;
-    fill[1] = 0;
-    *status = b;
-  } else {
-    atomicMax(fill, mx);
-    if (b) atomicOr(status, b);
+  if (slot) v->off[k + 1] = incl;
+  if (k == 0) {
+    v->off[0] = 0;
+    v->q = q;
+    v->cap = cap;
+    const unsigned b = mx > cap ? bit : 0u;
+    if (fresh) { /* first view of a ladder: also resets the second's fill */
+      fill[0] = mx;
+      fill[1] = 0;
+      *status = b;
+    } else {
+      atomicMax(fill, mx);
+      if (b) atomicOr(status, b);
+    }
   }
 }
 void launch_make_view(const QEntry* q, uint32_t cap, unsigned* cnt, QView* v,
                       unsigned* status, unsigned bit, unsigned* fill,
-                      unsigned* also, bool fresh, hipStream_t s) {
+                      unsigned* lists, bool fresh, hipStream_t s) {
   hipLaunchKernelGGL(k_make_view, dim3(1), dim3(64), 0, s, q, cap, cnt, v,
-                     status, bit, fill, also, (int)fresh);
+                     status, bit, fill, lists, (int)fresh);
 }
 
 /* An eager ladder's state in one buffer for one read-back: the
- * sub-queue counts of its last queue (then cleared for the next producer)
- * and its count, beside the status and fill its first view left */
-__global__ void k_ladder_state(unsigned* cnt, const uint64_t* count,
-                               unsigned* lad) {
-  const int t = threadIdx.x;
-  if (t < QSLOTS) {
-    lad[kLadCnt + t] = cnt[t];
-    cnt[t] = 0;
+ * sub-queue counts of its last queue and its count, beside the status and
+ * fill its first view left.  The queue's counters and (lists, the word of
+ * the QK_REST counters) the two lists' are cleared for the next ladder. */
+__global__ __launch_bounds__(64) void k_ladder_state(unsigned* cnt,
+                                                     unsigned* lists,
+                                                     const uint64_t* count,
+                                                     unsigned* lad) {
+  const int k = threadIdx.x;
+  if (k < QSLOTS) {
+    lad[kLadCnt + k] = cnt[k * kSlotWords];
+    cnt[k * kSlotWords] = 0;
+    lists[k * kSlotWords] = 0;
+    lists[k * kSlotWords + QK_NEXT - QK_REST] = 0;
   }
-  if (t == 0) *reinterpret_cast<uint64_t*>(lad + kLadCount) = *count;
+  if (k == 0) *reinterpret_cast<uint64_t*>(lad + kLadCount) = *count;
 }
-void launch_ladder_state(unsigned* cnt, const uint64_t* count, unsigned* lad,
-                         hipStream_t s) {
-  hipLaunchKernelGGL(k_ladder_state, dim3(1), dim3(64), 0, s, cnt, count, lad);
+void launch_ladder_state(unsigned* cnt, unsigned* lists, const uint64_t* count,
+                         unsigned* lad, hipStream_t s) {
+  hipLaunchKernelGGL(k_ladder_state, dim3(1), dim3(64), 0, s, cnt, lists, count,
+                     lad);
+}
+
+__global__ void k_zero_counter(unsigned long long* ctr, int idx) {
+  if (threadIdx.x < CTR_SLOTS) ctr[threadIdx.x * CTR_COUNT + idx] = 0;
+}
+void zero_counter(unsigned long long* ctr, int idx, hipStream_t s) {
+  hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, ctr, idx);
 }
 
 __global__ void k_cap_check(const uint64_t* v, uint64_t cap, unsigned* status,

@@ -25,7 +25,7 @@ __device__ __forceinline__ void flush_ctr(unsigned long long* ctr, int idx,
                                           unsigned v) {
   v = wave_sum(v);
   if ((threadIdx.x & 63) == 0 && v)
-    atomicAdd(&ctr[idx * CTR_SLOTS + (blockIdx.x & (CTR_SLOTS - 1))],
+    atomicAdd(&ctr[(blockIdx.x & (CTR_SLOTS - 1)) * CTR_COUNT + idx],
               (unsigned long long)v);
 }
 /* Block-level versions (every thread of the block must call them): one
@@ -42,7 +42,7 @@ __device__ __forceinline__ void block_flush(unsigned long long* ctr, int idx,
     const int waves = (int)(blockDim.x >> 6);
     for (int w = 0; w < waves; ++w) t += s_part[w];
     if (t)
-      atomicAdd(&ctr[idx * CTR_SLOTS + (blockIdx.x & (CTR_SLOTS - 1))],
+      atomicAdd(&ctr[(blockIdx.x & (CTR_SLOTS - 1)) * CTR_COUNT + idx],
                 (unsigned long long)t);
   }
   __syncthreads();
@@ -68,13 +68,13 @@ __device__ __forceinline__ unsigned block_append(unsigned* counter, bool want) {
   return r;
 }
 /* Append v (where want) to the sub-list of this block (LSLOTS sub-lists
- * of lcap entries, counters cnt[LSLOTS]); every thread of the block must
+ * of lcap entries, LSLOTS counters at cnt); every thread of the block must
  * call it. */
 __device__ __forceinline__ void list_append(uint32_t* data, unsigned* cnt,
                                             uint32_t lcap, bool want,
                                             uint32_t v) {
   const unsigned k = blockIdx.x & (LSLOTS - 1);
-  const unsigned at = block_append(cnt + k, want);
+  const unsigned at = block_append(cnt + k * kSlotWords, want);
   if (want && at < lcap) data[(uint64_t)k * lcap + at] = v;
 }
 /* A consumer block's table of the sub-lists' starts in the concatenation:
@@ -84,7 +84,7 @@ __device__ __forceinline__ void list_table(const unsigned* cnt, uint32_t lcap,
                                            uint32_t* s_pre) {
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
-    uint32_t c = lane < LSLOTS ? min(cnt[lane], lcap) : 0u;
+    uint32_t c = lane < LSLOTS ? min(cnt[lane * kSlotWords], lcap) : 0u;
     uint32_t incl = c;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -216,7 +216,7 @@ __device__ __forceinline__ bool same_pos(const Ball& a, const Ball& b) {
 __device__ __forceinline__ void push_q(const Queue& q, uint32_t item,
                                        uint32_t aux) {
   const uint32_t k = blockIdx.x & (QSLOTS - 1);
-  unsigned p = atomicAdd(q.n + k, 1u);
+  unsigned p = atomicAdd(q.n + k * kSlotWords, 1u);
   if (p < q.cap) q.q[(uint64_t)k * q.cap + p] = QEntry{item, aux};
 }
 
@@ -639,6 +639,18 @@ template <bool MOL>
 __device__ __forceinline__ GridP sgrid_at(const Stage& S, uint32_t b) {
   if constexpr (MOL) return S.sgrids[S.mol[b]];
   else return S.sg;
+}
+/* The Stage of a kernel whose first parameter it is, read again from the
+ * kernel's arguments.  An item loop that takes it through here once per
+ * item keeps nothing derived from it in registers between items: hoisted
+ * out of the loop, the grid's FP32 conversions (vector instructions) and
+ * the scalar registers they crowd out raised the emptiness kernels from 67
+ * to 88 - 106 VGPRs, 7 to 4 - 5 waves per SIMD. */
+__device__ __forceinline__ const Stage& fresh_stage() {
+  typedef const __attribute__((address_space(4))) Stage* KPtr;
+  KPtr p = (KPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const Stage*)p;
 }
 
 /* Centre c = p0 + num / (2 den) and per-axis error bounds from certified

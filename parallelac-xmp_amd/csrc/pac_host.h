@@ -370,7 +370,7 @@ inline void stats_from_counters(const unsigned long long* hs, bool staged,
   unsigned long long h[CTR_COUNT];
   for (int c = 0; c < CTR_COUNT; ++c) {
     h[c] = 0;
-    for (int k = 0; k < CTR_SLOTS; ++k) h[c] += hs[c * CTR_SLOTS + k];
+    for (int k = 0; k < CTR_SLOTS; ++k) h[c] += hs[k * CTR_COUNT + c];
   }
   for (int f = 0; f < 6; ++f)
     for (int q = 0; q < 4; ++q)

@@ -80,7 +80,11 @@ enum {
   CTR_DROP = 31,        /* alpha tets with a covered edge (not listed) */
   CTR_COUNT = 32
 };
-constexpr int CTR_SLOTS = 32;   /* copies of each counter (see flush_ctr) */
+/* copies of each counter (see flush_ctr): counter c of copy k is word
+ * k * CTR_COUNT + c, so a copy fills two cache lines of its own and blocks
+ * adding to different copies do not meet in one (device-scope atomics on
+ * one line pass ~6 ns apart, whichever of its words they address) */
+constexpr int CTR_SLOTS = 32;
 enum { FAM_EDGE = 0, FAM_TRI = 1, FAM_TET = 2, FAM_TET_AC2 = 3,
        FAM_TRI_AC2 = 4, FAM_EDGE_AC2 = 5 };
 
@@ -155,19 +159,29 @@ constexpr int QSLOTS = 32;
  * entries [k * lcap, k * lcap + n[k]) with n[k] <= lcap, lcap =
  * list_slot_cap(the producer's blocks).  One counter for the ~10^5 blocks
  * of a launch serialized their device-scope atomics (on the 100k globule,
- * 0.45 ms of a 0.88 ms tet emptiness first phase). */
+ * 0.45 ms of a 0.88 ms tet emptiness first phase), and so did 32 counters
+ * in one 128-byte line: appending 44,600 blocks' items took 262 us, with a
+ * line for each counter 53 us. */
 constexpr int LSLOTS = 32;
+constexpr int kListRun = 8; /* items a thread of a listing pass takes */
 inline uint32_t list_slot_cap(int64_t blocks) {
-  return (uint32_t)((blocks + LSLOTS - 1) / LSLOTS * kBlock);
+  /* blocks of kBlock items, or of kListRun times as many */
+  return (uint32_t)((blocks + LSLOTS * kListRun - 1) / (LSLOTS * kListRun) *
+                    (kBlock * kListRun));
 }
-/* queue counter words of a run: the hot and escalation sub-queue counters
- * (2 QSLOTS), then the counters of the list of simplices left for the
- * second emptiness phase and of the list of tets a quick rejection pass
- * left (2 LSLOTS) */
-constexpr int QN_WORDS = 2 * QSLOTS + 2 * LSLOTS;
+/* queue counters of a run: slot k's line of kSlotWords words holds the
+ * fills of sub-queue k of the hot (QK_HOT) and escalation (QK_ESC) queues
+ * and of sub-list k of the list of simplices left for the second emptiness
+ * phase (QK_REST) and of those a pass before the first one listed
+ * (QK_NEXT).  A queue's or list's counters are passed as the address of its
+ * first one; counter k is kSlotWords * k words on. */
+constexpr int kSlotWords = 32; /* 128 bytes */
+enum { QK_HOT = 0, QK_ESC = 1, QK_REST = 2, QK_NEXT = 3 };
+static_assert(QSLOTS == LSLOTS, "the counters share their lines");
+constexpr int QN_WORDS = QSLOTS * kSlotWords;
 struct Queue {
   QEntry* q;
-  unsigned* n;   /* QSLOTS counters */
+  unsigned* n;   /* QSLOTS counters, kSlotWords apart */
   uint32_t cap;  /* per sub-queue */
 };
 /* consumer view: entry i of the concatenated sub-queues */
@@ -221,14 +235,16 @@ enum { REC_CAP = 0,    /* bits 0..8: a count exceeded its capacity */
        REC_Q1 = 9,     /* hot queue overflow */
        REC_Q2 = 10,    /* escalation queue overflow */
        REC_STALE = 11  /* the input no longer matches the recorded plan */ };
-/* view of QSLOTS sub-queues (counters cleared after reading, and the
- * LSLOTS list counters at also);
+/* set counter idx of every copy to zero */
+void zero_counter(unsigned long long* ctr, int idx, hipStream_t s);
+/* view of QSLOTS sub-queues (counters cleared after reading, and with
+ * lists the counters of both lists beside them);
  * fresh (an eager ladder's first view): status / fill overwritten, and
  * the view left empty when a sub-queue overflowed (the ladder reruns);
  * else status / fill merged and the view clamped to the capacity */
 void launch_make_view(const QEntry* q, uint32_t cap, unsigned* cnt, QView* v,
                       unsigned* status, unsigned bit, unsigned* fill,
-                      unsigned* also, bool fresh, hipStream_t s);
+                      unsigned* lists, bool fresh, hipStream_t s);
 void launch_cap_check(const uint64_t* v, uint64_t cap, unsigned* status,
                       unsigned bit, hipStream_t s);
 /* eager ladder state (u32 words): [kLadStatus] status, [kLadFill] fill of
@@ -236,8 +252,8 @@ void launch_cap_check(const uint64_t* v, uint64_t cap, unsigned* status,
  * last queue's sub-queue counts */
 constexpr int kLadStatus = 0, kLadFill = 1, kLadCount = 4, kLadCnt = 6;
 constexpr int kLadWords = kLadCnt + QSLOTS;
-void launch_ladder_state(unsigned* cnt, const uint64_t* count, unsigned* lad,
-                         hipStream_t s);
+void launch_ladder_state(unsigned* cnt, unsigned* lists, const uint64_t* count,
+                         unsigned* lad, hipStream_t s);
 void launch_plan_check(const Bounds* now, const Bounds* ref, int64_t m,
                        int scale, unsigned* status, unsigned bit,
                        hipStream_t s);
@@ -506,8 +522,15 @@ void launch_filter_exact(const Stage& S, int kind, CandCtx C, QRef q, const uint
 /* ---- emptiness (k_ac2.hip) ---- */
 /* rest / nrest: scratch list of simplices left for phase B (capacity =
  * number of items); budget = phase A pair budget (0: single phase) */
-/* next / nnext: scratch list (capacity = number of tets) of the tets a
- * quick rejection pass leaves for the certified scan (fine scan grid) */
+/* next / nnext: scratch list (capacity = number of items) of the simplices
+ * phase A scans, where a pass before it left only some: the quick
+ * rejection pass (tets, fine scan grid), a chunk sub-input's needed tets,
+ * the triangles / edges neither in the closure nor covered (kListItems).
+ * Both lists' counters come cleared (the ladder's last kernel does it). */
+/* triangles / edges from this many on are listed before their scans: the
+ * dead and closed ones leave most lanes of a wave idle otherwise; below it
+ * the extra launch costs more than the idle lanes do */
+constexpr int64_t kListItems = 1 << 17;
 /* chunk sub-input: in_flag[id] = 1 (pass untested) for the triangles
  * (kind 0) / edges (kind 1) no owned simplex depends on */
 void launch_own_mark(const Stage& S, int kind, Cnt n, const uint32_t* ecol,
@@ -536,7 +559,8 @@ void launch_low_ac2_hot(const Stage& S, int kind, Cnt nitems,
                         const uint32_t* ecol, const uint32_t* eleft,
                         const uint32_t* tkd, const uint32_t* tedge,
                         const uint8_t* edead, const uint8_t* in_flag,
-                        uint8_t* flag, Queue q1, uint32_t* rest, unsigned* nrest,
+                        uint8_t* flag, Queue q1, uint32_t* rest,
+                        unsigned* nrest, uint32_t* next, unsigned* nnext,
                         int budget, PipeLaunch L);
 void launch_low_ac2_esc(const Stage& S, int kind, QRef q,
                         const uint32_t* ecol, const uint32_t* eleft,

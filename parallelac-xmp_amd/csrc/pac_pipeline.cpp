@@ -318,17 +318,16 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     SG.ctr = ctr_own.get();
   }
   unsigned long long* const ctr = SG.ctr;
-  /* [0, QSLOTS) hot queue, [QSLOTS, 2 QSLOTS) escalation queue, then the
-   * LSLOTS counters of the list of simplices left for the second emptiness
-   * phase and those of the list of tets a quick rejection pass left */
+  /* queue and list counters (QK_*) */
   DBuf<unsigned> qn_own;
   if (!rec) {
     qn_own = DBuf<unsigned>(P, QN_WORDS);
-    zero_u32(qn_own.get(), QN_WORDS, s); /* then kept clear by the views */
+    zero_u32(qn_own.get(), QN_WORDS, s); /* then kept clear by the ladders */
   }
   unsigned* const qn = rec ? rec->qn : qn_own.get();
-  unsigned* const nrest = qn + 2 * QSLOTS;
-  unsigned* const nnext = nrest + LSLOTS;
+  unsigned* const nesc = qn + QK_ESC;
+  unsigned* const nrest = qn + QK_REST;
+  unsigned* const nnext = qn + QK_NEXT;
   /* eager ladders: the device view of q1 and the state read back once */
   DBuf<QView> ev_view(P, 1);
   DBuf<unsigned> lad(P, kLadWords);
@@ -428,8 +427,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
                        1u << REC_Q1, rec->fill, nrest, false, s);
       QRef r{QView{}, rec->views, QSLOTS * rec->c1};
       if (staged) {
-        esc(r, Queue{rec->q2, qn + QSLOTS, rec->c2});
-        launch_make_view(rec->q2, rec->c2, qn + QSLOTS, rec->views + 1,
+        esc(r, Queue{rec->q2, nesc, rec->c2});
+        launch_make_view(rec->q2, rec->c2, nesc, rec->views + 1,
                          rec->status, 1u << REC_Q2, rec->fill + 1, nullptr,
                          false, s);
         r = QRef{QView{}, rec->views + 1, QSLOTS * rec->c2};
@@ -448,7 +447,6 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     DBuf<QEntry> q1, q2;
     for (;;) {
       q1 = DBuf<QEntry>(P, (size_t)c1 * QSLOTS);
-      zero_u32(nrest, LSLOTS, s);
       if (kp_hot >= 0) KP.begin(kp_hot);
       hot(Queue{q1.get(), qn, c1});
       if (kp_hot >= 0) KP.end();
@@ -461,14 +459,14 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
         launch_make_view(q1.get(), c1, qn, ev_view.get(), lad.get() + kLadStatus,
                          1u, lad.get() + kLadFill, nullptr, true, s);
         esc(QRef{QView{}, ev_view.get(), QSLOTS * c1},
-            Queue{q2.get(), qn + QSLOTS, c2});
+            Queue{q2.get(), nesc, c2});
         KCHK();
         last = q2.get();
         clast = c2;
-        cnt_last = qn + QSLOTS;
+        cnt_last = nesc;
       }
       tail();
-      launch_ladder_state(cnt_last, dcnt + q, lad.get(), s);
+      launch_ladder_state(cnt_last, nrest, dcnt + q, lad.get(), s);
       KCHK();
       unsigned h[kLadWords];
       HIPCHK(hipMemcpyAsync(E->pinned, lad.get(), sizeof(h),
@@ -635,7 +633,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
         std::min<int64_t>(Tslots.cap, Tslots.cap / 32 + 65536), KP_TRI_FILL, -1,
         [&](Queue qq) {
           if (runs++ && !rec)
-            zero_u64(ctr + (CTR_CAND + 1) * CTR_SLOTS, CTR_SLOTS, s);
+            zero_counter(ctr, CTR_CAND + 1, s);
           launch_tri_enum_filter(SG, Ealpha, erow.get(), ecol.get(), eleft.get(),
                                  off.get(), cval.get(), cseg.get(), cea.get(),
                                  ceb.get(), flag.get(), bcnt.get(), bkeep.get(),
@@ -713,8 +711,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
         std::min<int64_t>(Kslots.cap, Kslots.cap / 32 + 65536), KP_TET_FILL, -1,
         [&](Queue qq) {
           if (runs++ && !rec) {
-            zero_u64(ctr + (CTR_CAND + 2) * CTR_SLOTS, CTR_SLOTS, s);
-            zero_u64(ctr + CTR_DROP * CTR_SLOTS, CTR_SLOTS, s);
+            zero_counter(ctr, CTR_CAND + 2, s);
+            zero_counter(ctr, CTR_DROP, s);
           }
           launch_tet_enum_filter(SG, Talpha, trow.get(), tkd.get(), tedge.get(),
                                  teik.get(), tejk.get(), eleft.get(), ecol.get(),
@@ -743,7 +741,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   T.mark(5);
 
   auto ac2_cap = [](int64_t items) {
-    return (uint32_t)std::min<int64_t>(std::max<int64_t>(1 << 20, items / 8),
+    return (uint32_t)std::min<int64_t>(std::max<int64_t>(1 << 20, items / 2),
                                        (int64_t)UINT32_MAX - 1);
   };
 
@@ -780,7 +778,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       (std::max({Kalpha.cap, Talpha.cap, Ealpha.cap, (int64_t)1}) + kBlock - 1) /
       kBlock);
   DBuf<uint32_t> rest(P, (size_t)LSLOTS * SG.lcap);
-  DBuf<uint32_t> next(P, pl.kf || sub ? (size_t)LSLOTS * SG.lcap : 1);
+  DBuf<uint32_t> next(P, (size_t)LSLOTS * SG.lcap);
   DBuf<uint8_t> kflag(P, Kalpha.cap);
   Cnt Kf(0);
   DBuf<uint4> ftets;
@@ -869,7 +867,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           [&](Queue q) {
             launch_low_ac2_hot(SG, 0, Talpha, ecol.get(), eleft.get(), tkd.get(),
                                tedge.get(), nullptr, tri_skip, tflag.get(), q,
-                               rest.get(), nrest, budget, L);
+                               rest.get(), nrest, next.get(), nnext, budget, L);
           },
           [&](QRef q, Queue q2) {
             launch_low_ac2_esc(SG, 0, q, ecol.get(), eleft.get(), tk.get(),
@@ -935,7 +933,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           [&](Queue q) {
             launch_low_ac2_hot(SG, 1, Ealpha, ecol.get(), eleft.get(), nullptr,
                                nullptr, dead, edge_skip, eflag.get(), q,
-                               rest.get(), nrest, budget, L);
+                               rest.get(), nrest, next.get(), nnext, budget, L);
           },
           [&](QRef q, Queue q2) {
             launch_low_ac2_esc(SG, 1, q, ecol.get(), eleft.get(), nullptr,

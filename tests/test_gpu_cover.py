@@ -1,8 +1,10 @@
 """Emptiness decisions spared by covered edges (tet candidates counted but
 not listed, triangles and edges failing without a scan) against the oracle,
 row for row: balls swallowed by larger ones, alpha below and above zero,
-alpha-edge counts around one enumeration block (256), and the same input as
-a batch, in chunks, recorded and in FP64."""
+alpha-edge counts around one enumeration block (256), alpha triangles on
+either side of the count from which they are listed before their scans
+(131072, between 1300 and 1500 balls), and the same input as a batch, in
+chunks, recorded and in FP64."""
 import numpy as np
 import pytest
 
@@ -28,7 +30,7 @@ def _same(got, want, what):
 @pytest.mark.parametrize("n,spread,s,a", [
     (3, 1.0, 1.4, 0.0), (24, 1.6, 1.4, 0.0), (40, 1.0, 0.4, 0.0),
     (257, 2.2, 1.4, 0.0), (900, 1.8, 1.0, -1.5), (900, 1.5, 0.0, 4.0),
-    (2500, 2.0, 1.4, 0.0)])
+    (1300, 1.0, 1.4, 0.0), (1500, 1.0, 1.4, 0.0), (2500, 2.0, 1.4, 0.0)])
 def test_covered_edges(n, spread, s, a):
     print("case:", n, spread, s, a, flush=True)
     b = _balls(n, 40 + n, spread)

@@ -699,42 +699,42 @@ __device__ __forceinline__ bool low_setup(const GridP& g, const Ball* v,
   const R ax = v[0].x, ay = v[0].y, az = v[0].z;
   R ux = (R)v[1].x - ax, uy = (R)v[1].y - ay, uz = (R)v[1].z - az;
   R wa = (R)v[0].w * (R)v[0].w, w1 = (R)v[1].w * (R)v[1].w;
-  R uu = ux * ux + uy * uy + uz * uz;
-  SS<R> A{(uu + wa) - w1, (uu + wa) + w1};
+  const R uu = dot3(ux, uy, uz, ux, uy, uz);
+  const SS<R> A{(uu + wa) - w1, (uu + wa) + w1};
   FE<R> den;
   V3<FE<R>> num;
   if (KIND == 0) {
     R vx = (R)v[2].x - ax, vy = (R)v[2].y - ay, vz = (R)v[2].z - az;
     R w2 = (R)v[2].w * (R)v[2].w;
-    R vv = vx * vx + vy * vy + vz * vz;
-    SS<R> B{(vv + wa) - w2, (vv + wa) + w2};
+    const R vv = dot3(vx, vy, vz, vx, vy, vz);
+    const SS<R> B{(vv + wa) - w2, (vv + wa) + w2};
     /* permanents bounded by max norms: every component of n = u x v by
      * pn = 2 |u|_inf |v|_inf, of v x n by 2 |v|_inf pn, of u x n by
      * 2 |u|_inf pn */
-    const R mu = fmax(fabs(ux), fmax(fabs(uy), fabs(uz)));
-    const R mv = fmax(fabs(vx), fmax(fabs(vy), fabs(vz)));
+    const R mu = max3(fabs(ux), fabs(uy), fabs(uz));
+    const R mv = max3(fabs(vx), fabs(vy), fabs(vz));
     const R pn = ((R)2 * mu) * mv;
-    const R nx = uy * vz - uz * vy, ny = uz * vx - ux * vz, nz = ux * vy - uy * vx;
-    SS<R> nn{nx * nx + ny * ny + nz * nz, ((R)3 * pn) * pn};
+    const R nx = det2(uy, vz, uz, vy), ny = det2(uz, vx, ux, vz),
+            nz = det2(ux, vy, uy, vx);
+    const SS<R> nn{dot3(nx, ny, nz, nx, ny, nz), ((R)3 * pn) * pn};
     /* X = A (v x n) - B (u x n) */
-    const R vn[3] = {vy * nz - vz * ny, vz * nx - vx * nz, vx * ny - vy * nx};
-    const R un[3] = {uy * nz - uz * ny, uz * nx - ux * nz, ux * ny - uy * nx};
-    const R xp = ((R)2 * pn) * (A.p * mv + B.p * mu);
-    SS<R> X[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q)
-      X[q] = SS<R>{A.v * vn[q] - B.v * un[q], xp};
-    den = ss_fe(nn, 8);
-    num = V3<FE<R>>{ss_fe(X[0], 12), ss_fe(X[1], 12), ss_fe(X[2], 12)};
+    const R vn[3] = {det2(vy, nz, vz, ny), det2(vz, nx, vx, nz),
+                     det2(vx, ny, vy, nx)};
+    const R un[3] = {det2(uy, nz, uz, ny), det2(uz, nx, ux, nz),
+                     det2(ux, ny, uy, nx)};
+    const R xp = ((R)2 * pn) * fmaR(A.p, mv, B.p * mu);
+    den = ss_fe(nn, 11);
+    num.x = ss_fe(SS<R>{det2(A.v, vn[0], B.v, un[0]), xp}, 16);
+    num.y = FE<R>{det2(A.v, vn[1], B.v, un[1]), num.x.e};
+    num.z = FE<R>{det2(A.v, vn[2], B.v, un[2]), num.x.e};
   } else {
-    SS<R> uuS{uu, uu};
-    den = ss_fe(uuS, 4);
-    num = V3<FE<R>>{ss_fe(SS<R>{A.v * ux, A.p * fabs(ux)}, 8),
-                    ss_fe(SS<R>{A.v * uy, A.p * fabs(uy)}, 8),
-                    ss_fe(SS<R>{A.v * uz, A.p * fabs(uz)}, 8)};
+    den = ss_fe(SS<R>{uu, uu}, 5);
+    num = V3<FE<R>>{ss_fe(SS<R>{A.v * ux, A.p * fabs(ux)}, 9),
+                    ss_fe(SS<R>{A.v * uy, A.p * fabs(uy)}, 9),
+                    ss_fe(SS<R>{A.v * uz, A.p * fabs(uz)}, 9)};
   }
   V3<FE<R>> pa{FE<R>{ax, (R)0}, FE<R>{ay, (R)0}, FE<R>{az, (R)0}};
-  FE<R> waf{wa, FEc<R>::u() * wa * FEc<R>::slack()};
+  FE<R> waf{wa, FEc<R>::u() * FEc<R>::slack() * wa};
   if (!pairss_init(P, pa, waf, den, num) || P.sden < 0) return false;
   R c[3], e[3], rho_up;
   if (!centre_err<R>(den, num, v[0], waf, c, e, &rho_up)) return false;

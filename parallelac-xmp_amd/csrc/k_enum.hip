@@ -395,13 +395,14 @@ __device__ int tet_code(const Ball& a, const Ball& b, const Ball& c,
 /* The first stages of the edge and triangle filters, semi-static as
  * tet_dn_ss: each value evaluated once in precision R together with its
  * permanent (the same expression on absolute values, subtractions made
- * additions), the error bound gamma_h times the permanent (ss_fe) for
- * the expression tree's height h, leaves u, v = p - p_a and w = r^2
- * rounded once, alpha exact, products by 2 and 4 exact.
- *   edge: V = 4 |u|^2 (w_a + alpha) - A^2, A = |u|^2 + w_a - w_b; h 8;
- *   triangle: |n|^2 (n = u x v), h 6, and V = 4 |n|^2 (w_a + alpha) -
- *   ((A^2 |v|^2 - 2 A B u.v) + B^2 |u|^2), A = |u|^2 + w_a - w_b,
- *   B = |v|^2 + w_a - w_c; h 11.
+ * additions), its bound the rounding count k times u times the permanent
+ * (ss_fe), leaves u, v = p - p_a and w = r^2 rounded once, alpha exact,
+ * products by 2 and 4 exact.
+ *   edge: V = 4 |u|^2 (w_a + alpha) - A^2, A = |u|^2 + w_a - w_b: A^2 15,
+ *   V 16;
+ *   triangle: |n|^2 (n = u x v) 11, and V = 4 |n|^2 (w_a + alpha) -
+ *   (A^2 |v|^2 - 2 A B u.v + B^2 |u|^2), A = |u|^2 + w_a - w_b,
+ *   B = |v|^2 + w_a - w_c: A^2 |v|^2 21, its sum 23, V 24.
  * The same values as edge_val / tri_val; the bound replaces a running
  * error per operation (~4x the instructions for triangles). */
 template <class R>
@@ -409,11 +410,12 @@ __device__ __forceinline__ int edge_code_ss(const Ball& a, const Ball& b,
                                             Real alpha) {
   const R ux = (R)b.x - (R)a.x, uy = (R)b.y - (R)a.y, uz = (R)b.z - (R)a.z;
   const R wa = (R)a.w * (R)a.w, wb = (R)b.w * (R)b.w, al = (R)alpha;
-  const R uu = (ux * ux + uy * uy) + uz * uz;
+  const R uu = dot3(ux, uy, uz, ux, uy, uz);
   const R A = (uu + wa) - wb, Ap = (uu + wa) + wb;
-  const R V = ((R)4 * uu) * (wa + al) - A * A;
-  const R Vp = ((R)4 * uu) * (wa + fabs(al)) + Ap * Ap;
-  return code_of(fe_sign(ss_fe(SS<R>{V, Vp}, 8)));
+  const R u4 = (R)4 * uu;
+  const R V = fmaR(u4, wa + al, -(A * A));
+  const R Vp = fmaR(u4, wa + fabs(al), Ap * Ap);
+  return code_of(fe_sign(ss_fe(SS<R>{V, Vp}, 16)));
 }
 /* A rejected triangle (a, b, c) also tells which of its edges one ball
  * covers.  The points of equal power to a and b with that power <= alpha
@@ -425,8 +427,9 @@ __device__ __forceinline__ int edge_code_ss(const Ball& a, const Ball& b,
  * simplex with the edge ab has its orthocentre on the disk, where c's
  * power is strictly below the simplex's value, and is not empty.
  * The coordinates (times 2 |n|^2 > 0): b: A |v|^2 - B u.v, c: B |u|^2 -
- * A u.v, a: 2 |n|^2 minus both; at most 18 roundings on any path of the
- * last (14 of the others), bounded by 24 u times the permanent.
+ * A u.v, a: 2 |n|^2 minus both; at most 17 roundings on any path of the
+ * last (A 7, |v|^2 - u.v 6, their product 14 and two sums; 14 of the
+ * others).
  * cover: bit q set when vertex q (a, b, c) certainly covers the opposite
  * edge; set only with the result REJECT. */
 template <class R>
@@ -438,31 +441,35 @@ __device__ __forceinline__ int tri_code_ss(const Ball& a, const Ball& b,
   const R ux = (R)b.x - ax, uy = (R)b.y - ay, uz = (R)b.z - az;
   const R vx = (R)c.x - ax, vy = (R)c.y - ay, vz = (R)c.z - az;
   const R wa = (R)a.w * (R)a.w, wb = (R)b.w * (R)b.w, wc = (R)c.w * (R)c.w;
-  SS<R> n[3];
-  cross_ss(ux, uy, uz, vx, vy, vz, n);
-  const R nn = (n[0].v * n[0].v + n[1].v * n[1].v) + n[2].v * n[2].v;
-  const R nnp = (n[0].p * n[0].p + n[1].p * n[1].p) + n[2].p * n[2].p;
-  if (fe_sign(ss_fe(SS<R>{nn, nnp}, 6)) <= 0) return UNDEC;
-  const R uu = (ux * ux + uy * uy) + uz * uz;
-  const R vv = (vx * vx + vy * vy) + vz * vz;
-  const R uv = (ux * vx + uy * vy) + uz * vz;
-  const R uvp = (fabs(ux) * fabs(vx) + fabs(uy) * fabs(vy)) + fabs(uz) * fabs(vz);
+  const R n0 = det2(uy, vz, uz, vy), n1 = det2(uz, vx, ux, vz),
+          n2 = det2(ux, vy, uy, vx);
+  /* permanents of n by max norms, as in tet_dn_ss: 2 |u|_inf |v|_inf each,
+   * 12 (|u|_inf |v|_inf)^2 for |n|^2 */
+  const R pm = max3(fabs(ux), fabs(uy), fabs(uz)) *
+               max3(fabs(vx), fabs(vy), fabs(vz));
+  const R nn = dot3(n0, n1, n2, n0, n1, n2);
+  const R nnp = ((R)12 * pm) * pm;
+  if (fe_sign(ss_fe(SS<R>{nn, nnp}, 11)) <= 0) return UNDEC;
+  const R uu = dot3(ux, uy, uz, ux, uy, uz);
+  const R vv = dot3(vx, vy, vz, vx, vy, vz);
+  const R uv = dot3(ux, uy, uz, vx, vy, vz);
+  const R uvp = (R)3 * pm;
   const R A = (uu + wa) - wb, Ap = (uu + wa) + wb;
   const R B = (vv + wa) - wc, Bp = (vv + wa) + wc;
-  const R lhs = ((A * A) * vv - (((R)2 * A) * B) * uv) + (B * B) * uu;
-  const R lhsp = ((Ap * Ap) * vv + (((R)2 * Ap) * Bp) * uvp) + (Bp * Bp) * uu;
+  const R lhs = fmaR(A * A, vv, fmaR(B * B, uu, -((((R)2 * A) * B) * uv)));
+  const R lhsp = fmaR(Ap * Ap, vv, fmaR(Bp * Bp, uu, (((R)2 * Ap) * Bp) * uvp));
   const R al = (R)alpha;
-  const R V = ((R)4 * nn) * (wa + al) - lhs;
-  const R Vp = ((R)4 * nnp) * (wa + fabs(al)) + lhsp;
-  const int r = code_of(fe_sign(ss_fe(SS<R>{V, Vp}, 11)));
+  const R V = fmaR((R)4 * nn, wa + al, -lhs);
+  const R Vp = fmaR((R)4 * nnp, wa + fabs(al), lhsp);
+  const int r = code_of(fe_sign(ss_fe(SS<R>{V, Vp}, 24)));
   if (r == REJECT) {
-    const SS<R> lb{A * vv - B * uv, Ap * vv + Bp * uvp};
-    const SS<R> lc{B * uu - A * uv, Bp * uu + Ap * uvp};
-    const SS<R> la{(A * (uv - vv) + B * (uv - uu)) + (R)2 * nn,
-                   (Ap * (uvp + vv) + Bp * (uvp + uu)) + (R)2 * nnp};
-    cover = (fe_sign(ss_fe(la, 22)) < 0 ? 1u : 0u) |
-            (fe_sign(ss_fe(lb, 22)) < 0 ? 2u : 0u) |
-            (fe_sign(ss_fe(lc, 22)) < 0 ? 4u : 0u);
+    const SS<R> lb{det2(A, vv, B, uv), fmaR(Ap, vv, Bp * uvp)};
+    const SS<R> lc{det2(B, uu, A, uv), fmaR(Bp, uu, Ap * uvp)};
+    const SS<R> la{fmaR(A, uv - vv, fmaR(B, uv - uu, (R)2 * nn)),
+                   fmaR(Ap, uvp + vv, fmaR(Bp, uvp + uu, (R)2 * nnp))};
+    cover = (fe_sign(ss_fe(la, 18)) < 0 ? 1u : 0u) |
+            (fe_sign(ss_fe(lb, 18)) < 0 ? 2u : 0u) |
+            (fe_sign(ss_fe(lc, 18)) < 0 ? 4u : 0u);
   }
   return r;
 }
@@ -722,18 +729,26 @@ constexpr int fam_of(int KIND) {
 
 /* Tets of alpha triangle q = (i,j,k): l in T(i,j) after k, T(i,k), T(j,k)
  * (computePossibleTetCount / fillPossibleTets, Parallel:418-543), fused
- * with the tet filter's first stage (markRealTets, :531-591).  A block's
- * candidate slots are one contiguous range, staged in LDS as (i, j, k, l)
- * during the three-list merges; the block then filters the staged slots
- * round robin (uniform work per lane), writes every slot's flag coalesced
- * and the four vertex ids only of the slots that are kept or undecided
- * (the later stages read no others).  Slots past the LDS stage were
- * written to global memory during the merges and are filtered from there.
+ * with the tet filter's first stage (markRealTets, :531-591).
+ * A wave takes kTetSeg = 64 triangles, one a lane, whose candidate slots
+ * are one contiguous range.  The three-list merges leave each triangle's
+ * fourth vertices in LDS from its first slot on; then the wave filters the
+ * candidates themselves, 64 at a time (of the slots, the tails of the
+ * triangles' rows, 59% hold one on a globule: candidate d's triangle is
+ * found in the lanes' prefix counts), and writes the kept and undecided
+ * ones compacted, in slot order, from its first slot on, with their flags.
+ * No barrier: a wave waits for no other until the counters are summed.
+ * Against blocks of 256 triangles filtering every slot from a 16-byte
+ * stage: 523 -> 434 us at 100k balls, 9.6 -> 1.8 ms on 200k balls with a
+ * lattice block (whose blocks overflowed the stage), and 405 us with the
+ * filter on fused multiply-adds.  At 100k the vector memory path (TD 96%
+ * busy, TA 86%: the merges' gathers) and the vector ALU (86%) bound it
+ * together.  Slots past the LDS stage (1,120 a wave; a lattice's waves
+ * average 530, a globule's 230) are kept in the candidates' own array.
  * A candidate with a covered edge (kDeadBit of one of its triangles in
- * tkd, carried through the merge in the slot's first id) is filtered like
- * any other, but an alpha tet among them is only counted (CTR_DROP), not
- * written: it cannot be empty.  On the 100k globule 4.6M of the 19.1M
- * alpha tets are written. */
+ * tkd, carried with the fourth vertex) is filtered like any other, but an
+ * alpha tet among them is only counted (CTR_DROP), not written: it cannot
+ * be empty.  On the 100k globule 4.6M of the 19.1M alpha tets are written. */
 /* First slot of alpha triangle q without a per-triangle offset array:
  * the triangles of edge e occupy rows trow[e] .. trow[e+1]-1 and each has
  * its row's tail after it as slots, so triangle s + k of a row of L = trow
@@ -756,185 +771,187 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
     const uint32_t* eleft, const uint32_t* ecol, const uint64_t* off,
     const uint64_t* roff, uint64_t* bbase, uint4* ctet, uint8_t* flag,
     uint32_t* bcnt, uint32_t* bkeep, Queue q1, uint64_t lim) {
+  static_assert(kTetSeg == 64, "a triangle a lane");
+  constexpr uint32_t CAP = 1120; /* with the tables, 8 blocks per CU */
+  __shared__ uint32_t s_l[kBlock / 64][CAP];
+  __shared__ uint32_t s_end[kBlock / 64][64], s_off[kBlock / 64][64];
   const int64_t nt = c_nt.get();
-  /* 8 blocks per CU fit in LDS with block_flush's 16 B (the kernel's 60
-   * VGPRs allow 8 waves per SIMD); a block of 256 alpha triangles averages
-   * ~600 slots */
-  constexpr int CAP = 1272;
-  __shared__ uint4 s_out[CAP];
-  const int64_t q0 = (int64_t)blockIdx.x * kBlock;
-  if (q0 >= nt) { /* whole block past the (device) count */
-    if (threadIdx.x == 0) {
-      bcnt[blockIdx.x] = bkeep[blockIdx.x] = 0;
-      bbase[blockIdx.x] = 0;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t seg = gtid() >> 6, q = gtid();
+  unsigned found = 0, dropped = 0;
+  if (seg * kTetSeg >= nt) {
+    /* a segment past the (device) count */
+    if (lane == 0 && seg * kTetSeg < c_nt.cap) {
+      bcnt[seg] = bkeep[seg] = 0;
+      bbase[seg] = 0;
     }
-    return;
-  }
-  __shared__ unsigned s_und; /* an undecided candidate written */
-  if (threadIdx.x == 0) s_und = 0;
-  const int64_t q1e = q0 + kBlock < nt ? q0 + kBlock : nt;
-  /* the triangle's slots [o, oe): off[] per triangle, or (roff) the
-   * closed form, a triangle's slots being its row's tail; the block's
-   * range runs from its first triangle's o to its last one's oe */
-  const int64_t q = gtid();
-  uint32_t eij = 0;
-  uint64_t o = 0, oe = 0;
-  if (q < nt) {
-    eij = tedge[q];
-    if (off) {
-      o = off[q];
-      oe = off[q + 1];
-    } else {
-      o = tet_slot_off(roff, trow, eij, (uint32_t)q);
-      oe = o + (trow[eij + 1] - (uint64_t)q - 1);
-    }
-  }
-  __shared__ uint64_t s_span[2];
-  if (q == q0) s_span[0] = o;
-  if (q == q1e - 1) s_span[1] = oe;
-  __syncthreads();
-  if (threadIdx.x == 0) bbase[blockIdx.x] = s_span[0];
-  BlockOut4<CAP> B{s_out, s_span[0], s_span[1] - s_span[0], lim};
-  unsigned found = 0;
-  if (q < nt) {
-    const uint32_t eik = teik[q], ejk = tejk[q];
-    const uint32_t kd = tkd[q], k = kd & ~kDeadBit;
-    const uint32_t i = eleft[eij], j = ecol[eij];
-    if constexpr (BUF) {
-      /* the same merge over byte offsets into tkd (below 4 GiB): no 64-bit
-       * address arithmetic per load.  A triangle's slots are its row's
-       * tail after it, so o < oe holds while a < ae, unless it was given
-       * none (chunk sub-inputs): then the merge is empty. */
-      const BufU32 K{tkd, (uint32_t)(c_nt.cap * 4)};
-      uint32_t a = ((uint32_t)q + 1u) << 2, ae = (uint32_t)trow[eij + 1] << 2;
-      uint32_t b = (uint32_t)trow[eik] << 2, be = (uint32_t)trow[eik + 1] << 2;
-      uint32_t c = (uint32_t)trow[ejk] << 2, ce = (uint32_t)trow[ejk + 1] << 2;
-      if (o == oe) ae = a;
-      /* two merge steps a round: each list's next element is loaded with
-       * its current one (kEnd past the row's end, above every ball id) */
-      constexpr uint32_t kEnd = ~kDeadBit;
-      while (a < ae && b < be && c < ce) {
-        const uint32_t xd0 = K.at(a), yd0 = K.at(b), zd0 = K.at(c);
-        const uint32_t xd1 = a + 4u < ae ? K.at(a + 4u) : kEnd;
-        const uint32_t yd1 = b + 4u < be ? K.at(b + 4u) : kEnd;
-        const uint32_t zd1 = c + 4u < ce ? K.at(c + 4u) : kEnd;
-        const uint32_t x0 = xd0 & kEnd, y0 = yd0 & kEnd, z0 = zd0 & kEnd;
-        const uint32_t m0 = max(x0, max(y0, z0));
-        const bool all0 = x0 == m0 && y0 == m0 && z0 == m0;
-        if (all0) {
-          const uint32_t dead = (kd | xd0 | yd0 | zd0) & kDeadBit;
-          B.put(ctet, o, make_uint4(i | dead, j, k, m0));
-          ++o;
-          ++found;
-        }
-        const bool sa = all0 || x0 < m0, sb = all0 || y0 < m0,
-                   sc = all0 || z0 < m0;
-        const uint32_t xd = sa ? xd1 : xd0, yd = sb ? yd1 : yd0,
-                       zd = sc ? zd1 : zd0;
-        const uint32_t x = xd & kEnd, y = yd & kEnd, z = zd & kEnd;
-        const uint32_t m = max(x, max(y, z));
-        const bool all = x == m && y == m && z == m;
-        if (all && m != kEnd) {
-          const uint32_t dead = (kd | xd | yd | zd) & kDeadBit;
-          B.put(ctet, o, make_uint4(i | dead, j, k, m));
-          ++o;
-          ++found;
-        }
-        a += (sa ? 4u : 0u) + ((all || x < m) ? 4u : 0u);
-        b += (sb ? 4u : 0u) + ((all || y < m) ? 4u : 0u);
-        c += (sc ? 4u : 0u) + ((all || z < m) ? 4u : 0u);
+  } else {
+    /* the triangle's slots [o, oe): off[] per triangle, or (roff) the
+     * closed form, a triangle's slots being its row's tail */
+    uint32_t eij = 0, eik = 0, ejk = 0, i = 0, j = 0, kd = 0;
+    uint64_t o = 0, oe = 0;
+    if (q < nt) {
+      eij = tedge[q];
+      eik = teik[q];
+      ejk = tejk[q];
+      kd = tkd[q];
+      i = eleft[eij];
+      j = ecol[eij];
+      if (off) {
+        o = off[q];
+        oe = off[q + 1];
+      } else {
+        o = tet_slot_off(roff, trow, eij, (uint32_t)q);
+        oe = o + (trow[eij + 1] - (uint64_t)q - 1);
       }
-    } else {
-      /* alpha-triangle ids fit 32 bits (the slot count is checked below
-       * 2^32): 32-bit cursors halve the merge's index arithmetic; the
-       * slots end with T(i,j) (o < oe adds nothing then) unless the
-       * triangle was given none (chunk sub-inputs) */
-      uint32_t a = (uint32_t)q + 1, ae = (uint32_t)trow[eij + 1];
-      uint32_t b = (uint32_t)trow[eik], be = (uint32_t)trow[eik + 1];
-      uint32_t c = (uint32_t)trow[ejk], ce = (uint32_t)trow[ejk + 1];
-      while (a < ae && b < be && c < ce && o < oe) {
-        const uint32_t xd = tkd[a], yd = tkd[b], zd = tkd[c];
-        const uint32_t x = xd & ~kDeadBit, y = yd & ~kDeadBit,
-                       z = zd & ~kDeadBit;
-        const uint32_t m = max(x, max(y, z));
-        if (x == m && y == m && z == m) {
-          const uint32_t dead = (kd | xd | yd | zd) & kDeadBit;
-          B.put(ctet, o, make_uint4(i | dead, j, k, m));
-          ++o;
-          ++found;
-          ++a;
-          ++b;
-          ++c;
+    }
+    const uint32_t k = kd & ~kDeadBit;
+    const uint64_t base = (uint64_t)__shfl((unsigned long long)o, 0, 64);
+    /* the wave's slots, numbered from its first one; [rel, end) this
+     * lane's, cut at the arrays' end */
+    const uint32_t rel = (uint32_t)(o - base);
+    const uint32_t end =
+        o >= lim ? rel : rel + (uint32_t)((oe < lim ? oe : lim) - o);
+    uint32_t* const spill = reinterpret_cast<uint32_t*>(ctet + base);
+    uint32_t at = rel;
+    auto put = [&](uint32_t v) {
+      ++found;
+      if (at < end) {
+        if (at < CAP) s_l[wv][at] = v;
+        else spill[4 * (uint64_t)at] = v;
+        ++at;
+      }
+    };
+    /* two merge steps a round: each list's next element is loaded with its
+     * current one (kEnd past the row's end, above every ball id).  A
+     * triangle without slots (a chunk sub-input's unowned one) merges
+     * nothing. */
+    constexpr uint32_t kEnd = ~kDeadBit;
+    if (o < oe) {
+      if constexpr (BUF) {
+        /* byte offsets into tkd (below 4 GiB): no 64-bit address
+         * arithmetic per load */
+        const BufU32 K{tkd, (uint32_t)(c_nt.cap * 4)};
+        uint32_t a = ((uint32_t)q + 1u) << 2, ae = (uint32_t)trow[eij + 1] << 2;
+        uint32_t b = (uint32_t)trow[eik] << 2, be = (uint32_t)trow[eik + 1] << 2;
+        uint32_t c = (uint32_t)trow[ejk] << 2, ce = (uint32_t)trow[ejk + 1] << 2;
+        while (a < ae && b < be && c < ce) {
+          const uint32_t xd0 = K.at(a), yd0 = K.at(b), zd0 = K.at(c);
+          const uint32_t xd1 = a + 4u < ae ? K.at(a + 4u) : kEnd;
+          const uint32_t yd1 = b + 4u < be ? K.at(b + 4u) : kEnd;
+          const uint32_t zd1 = c + 4u < ce ? K.at(c + 4u) : kEnd;
+          const uint32_t x0 = xd0 & kEnd, y0 = yd0 & kEnd, z0 = zd0 & kEnd;
+          const uint32_t m0 = max(x0, max(y0, z0));
+          const bool all0 = x0 == m0 && y0 == m0 && z0 == m0;
+          if (all0) put(m0 | ((kd | xd0 | yd0 | zd0) & kDeadBit));
+          const bool sa = all0 || x0 < m0, sb = all0 || y0 < m0,
+                     sc = all0 || z0 < m0;
+          const uint32_t xd = sa ? xd1 : xd0, yd = sb ? yd1 : yd0,
+                         zd = sc ? zd1 : zd0;
+          const uint32_t x = xd & kEnd, y = yd & kEnd, z = zd & kEnd;
+          const uint32_t m = max(x, max(y, z));
+          const bool all = x == m && y == m && z == m;
+          if (all && m != kEnd) put(m | ((kd | xd | yd | zd) & kDeadBit));
+          a += (sa ? 4u : 0u) + ((all || x < m) ? 4u : 0u);
+          b += (sb ? 4u : 0u) + ((all || y < m) ? 4u : 0u);
+          c += (sc ? 4u : 0u) + ((all || z < m) ? 4u : 0u);
+        }
+      } else {
+        /* alpha-triangle ids fit 32 bits (the slot count is checked below
+         * 2^32): 32-bit cursors halve the merge's index arithmetic */
+        uint32_t a = (uint32_t)q + 1, ae = (uint32_t)trow[eij + 1];
+        uint32_t b = (uint32_t)trow[eik], be = (uint32_t)trow[eik + 1];
+        uint32_t c = (uint32_t)trow[ejk], ce = (uint32_t)trow[ejk + 1];
+        while (a < ae && b < be && c < ce) {
+          const uint32_t xd = tkd[a], yd = tkd[b], zd = tkd[c];
+          const uint32_t x = xd & kEnd, y = yd & kEnd, z = zd & kEnd;
+          const uint32_t m = max(x, max(y, z));
+          if (x == m && y == m && z == m) {
+            put(m | ((kd | xd | yd | zd) & kDeadBit));
+            ++a;
+            ++b;
+            ++c;
+          } else {
+            a += (x < m);
+            b += (y < m);
+            c += (z < m);
+          }
+        }
+      }
+    }
+    /* candidate d of the wave belongs to the first lane whose inclusive
+     * count exceeds d, and sits at slot d + s_off of that lane */
+    const uint32_t mine = at - rel;
+    uint32_t incl = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t y = (uint32_t)__shfl_up((int)incl, d, 64);
+      if (lane >= d) incl += y;
+    }
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    const bool spilled = __ballot(at > CAP) != 0; /* wave-uniform */
+    s_end[wv][lane] = incl;
+    s_off[wv][lane] = rel - (incl - mine);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    /* First precision stage.  A written position is at most the number of
+     * the candidate it holds, and that at most its slot: an unread spilled
+     * candidate lies past every position written before it. */
+    const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+    uint32_t run = 0; /* kept + undecided written so far (wave-uniform) */
+    bool und = false;
+    for (uint32_t d0 = 0; d0 < total; d0 += 64) {
+      const uint32_t d = d0 + (uint32_t)lane;
+      int t = 0; /* last lane with an inclusive count <= d, plus one */
+#pragma unroll
+      for (int h = 32; h >= 1; h >>= 1)
+        t += s_end[wv][t + h - 1] <= d ? h : 0;
+      t &= 63; /* (d past the last candidate) */
+      const uint32_t ti = (uint32_t)__shfl((int)i, t, 64);
+      const uint32_t tj = (uint32_t)__shfl((int)j, t, 64);
+      const uint32_t tk = (uint32_t)__shfl((int)k, t, 64);
+      uint4 v = make_uint4(ti, tj, tk, 0u);
+      int r = REJECT;
+      if (d < total) {
+        const uint32_t slot = d + s_off[wv][t];
+        /* (two branches: one load through a selected pointer would be a
+         * flat one) */
+        uint32_t ld = 0;
+        if (!spilled) {
+          ld = s_l[wv][slot];
         } else {
-          a += (x < m);
-          b += (y < m);
-          c += (z < m);
+          if (slot < CAP) ld = s_l[wv][slot];
+          if (slot >= CAP) ld = spill[4 * (uint64_t)slot];
         }
-      }
-    }
-    for (; o < oe; ++o) B.put(ctet, o, make_uint4(0xffffffffu, 0u, 0u, 0u));
-  }
-  __syncthreads(); /* LDS stage and the overflow slots written */
-  /* First precision stage over the block's slots, 256 per round; the kept
-   * and undecided ones are written compacted, in slot order, from the
-   * block's first slot on: position base + (kept before them) <= their
-   * own slot, and every slot of this round and the earlier ones was read
-   * before the round's first barrier, so no unread overflow slot is
-   * overwritten. */
-  __shared__ unsigned s_wsum[kBlock / 64];
-  const uint64_t base = B.base;
-  const uint64_t m = base >= lim ? 0 : (B.total < lim - base ? B.total : lim - base);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-  uint32_t run = 0; /* kept + undecided written so far (block-uniform) */
-  unsigned dropped = 0;
-  for (uint64_t r0 = 0; r0 < m; r0 += kBlock) {
-    const uint64_t t = r0 + threadIdx.x;
-    uint4 v = make_uint4(0xffffffffu, 0u, 0u, 0u);
-    int r = REJECT;
-    if (t < m) {
-      v = t < (uint64_t)CAP ? s_out[t] : ctet[base + t];
-      if (v.x != 0xffffffffu) {
-        const bool dead = (v.x & kDeadBit) != 0;
-        v.x &= ~kDeadBit;
+        v.w = ld & kEnd;
         const Ball bv[4] = {S.ball[v.x], S.ball[v.y], S.ball[v.z], S.ball[v.w]};
         /* the weights are first used after the test of D's sign; left
          * alone, the compiler loads them there, a second round trip per
          * round; used here (an empty asm), each ball is one 16-byte load */
 #pragma unroll
-        for (int k = 0; k < 4; ++k) asm volatile("" ::"v"(bv[k].w));
+        for (int z = 0; z < 4; ++z) asm volatile("" ::"v"(bv[z].w));
         r = tet_code_ss<R>(bv, S.alpha);
-        if (dead && r == KEEP) { /* an alpha tet, certainly not empty */
+        if ((ld & kDeadBit) && r == KEEP) { /* alpha, certainly not empty */
           ++dropped;
           r = REJECT;
         }
       }
-    }
-    const uint64_t bm = __ballot(r != REJECT);
-    if (lane == 0) s_wsum[w] = (unsigned)__popcll(bm);
-    __syncthreads();
-    uint32_t pre = run + (uint32_t)__popcll(bm & lt), tot = 0;
-#pragma unroll
-    for (int q = 0; q < kBlock / 64; ++q) {
-      const unsigned c = s_wsum[q];
-      if (q < w) pre += c;
-      tot += c;
-    }
-    if (r != REJECT) {
-      const uint64_t at = base + pre;
-      ctet[at] = v;
-      flag[at] = (uint8_t)r;
-      if (r == UNDEC) {
-        push_q(q1, (uint32_t)at, v.x);
-        s_und = 1;
+      const uint64_t bm = __ballot(r != REJECT);
+      if (r != REJECT) {
+        const uint64_t w = base + run + (uint32_t)__popcll(bm & lt);
+        ctet[w] = v;
+        flag[w] = (uint8_t)r;
+        if (r == UNDEC) push_q(q1, (uint32_t)w, v.x);
       }
+      und |= __ballot(r == UNDEC) != 0;
+      run += (uint32_t)__popcll(bm);
     }
-    run += tot;
-    __syncthreads(); /* s_wsum is rewritten next round */
-  }
-  if (threadIdx.x == 0) {
-    bcnt[blockIdx.x] = run;
-    bkeep[blockIdx.x] = s_und ? kRecount : run;
+    if (lane == 0) {
+      bbase[seg] = base;
+      bcnt[seg] = run;
+      bkeep[seg] = und ? kRecount : run;
+    }
   }
   block_flush(S.ctr, CTR_CAND + 2, found);
   block_flush(S.ctr, CTR_DROP, dropped);
@@ -968,83 +985,87 @@ void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
                      bkeep, q1, lim);
 }
 
-/* After the ladder: the kept tets of each enumeration block (its first
- * bcnt[b] positions from off[256 b] hold its kept and formerly undecided
- * tets), one wave per block. */
-__global__ __launch_bounds__(kBlock) void k_tet_block_keep(
-    Cnt c_nt, const uint64_t* off, int stride, const uint32_t* bcnt,
-    const uint8_t* flag, uint32_t* bkeep) {
-  const int64_t nt = c_nt.get();
-  const int64_t nblk = (c_nt.cap + kBlock - 1) / kBlock;
-  const int64_t b = gtid() >> 6;
-  const int lane = threadIdx.x & 63;
-  if (b >= nblk) return;
-  /* a block that queued no undecided candidate kept all it wrote: its
-   * enumeration left that count here */
-  if (bkeep[b] != kRecount) return;
-  unsigned c = 0;
-  if (b * kBlock < nt) {
-    const uint64_t base = off[b * stride];
-    const uint32_t n = bcnt[b];
-    for (uint32_t t = lane; t < n; t += 64) c += flag[base + t] == KEEP;
-  }
-  c = wave_sum(c);
-  if (lane == 0) bkeep[b] = c;
+/* kSegLanes lanes per enumeration segment in the two kernels below: a tet
+ * segment holds ~26 entries on a globule, and whole waves left most lanes
+ * idle.  A segment's lanes stay together; seg_ballot is their ballot. */
+constexpr int kSegLanes = 16;
+__device__ __forceinline__ unsigned seg_ballot(bool p) {
+  const int first = (threadIdx.x & 63) & ~(kSegLanes - 1);
+  return (unsigned)(__ballot(p) >> first) & ((1u << kSegLanes) - 1u);
 }
-/* the kept tets of block b to tets[bout[b], ...), in order; one wave per
- * block (a block holds ~100 entries: with 256-thread workgroups the copy
- * waits on four times fewer blocks in flight, each a chain of dependent
- * loads).  Grid as k_tet_block_keep's. */
-__global__ __launch_bounds__(kBlock) void k_tet_block_copy(
-    Cnt c_nt, const uint64_t* off, int stride, const uint32_t* bcnt,
-    const uint4* ctet, const uint8_t* flag, const uint64_t* bout, uint4* tets,
-    uint64_t ocap) {
+/* After the ladder: the kept candidates of each enumeration segment of
+ * `seg` items (its first bcnt[b] positions from off[b * stride] hold its
+ * kept and formerly undecided ones). */
+__global__ __launch_bounds__(kBlock) void k_seg_kept(
+    Cnt c_n, int seg, const uint64_t* off, int stride, const uint32_t* bcnt,
+    const uint8_t* flag, uint32_t* bkeep) {
+  const int64_t n = c_n.get();
+  const int64_t nseg = (c_n.cap + seg - 1) / seg;
+  const int64_t b = gtid() / kSegLanes;
+  const uint32_t sub = threadIdx.x & (kSegLanes - 1);
+  /* a segment that queued no undecided candidate kept all it wrote: its
+   * enumeration left that count here */
+  if (b >= nseg || bkeep[b] != kRecount) return;
+  unsigned c = 0;
+  if (b * seg < n) {
+    const uint64_t base = off[b * stride];
+    const uint32_t m = bcnt[b];
+    for (uint32_t r0 = 0; r0 < m; r0 += kSegLanes) {
+      const uint32_t t = r0 + sub;
+      c += (unsigned)__popc(seg_ballot(t < m && flag[base + t] == KEEP));
+    }
+  }
+  if (sub == 0) bkeep[b] = c;
+}
+/* the kept tets of segment b to tets[bout[b], ...), in order */
+__global__ __launch_bounds__(kBlock) void k_tet_seg_copy(
+    Cnt c_nt, const uint64_t* bbase, const uint32_t* bcnt, const uint4* ctet,
+    const uint8_t* flag, const uint64_t* bout, uint4* tets, uint64_t ocap) {
   const int64_t nt = c_nt.get();
-  const int64_t b = gtid() >> 6;
-  const int lane = threadIdx.x & 63;
-  if (b * kBlock >= nt) return; /* wave-uniform */
-  const uint64_t base = off[b * stride];
+  const int64_t b = gtid() / kSegLanes;
+  const uint32_t sub = threadIdx.x & (kSegLanes - 1);
+  if (b * kTetSeg >= nt) return;
+  const uint64_t base = bbase[b];
   const uint32_t n = bcnt[b];
   uint64_t o = bout[b];
   if (bout[b + 1] - o == n) { /* every entry kept: a straight copy */
-    for (uint32_t t = lane; t < n; t += 64)
+    for (uint32_t t = sub; t < n; t += kSegLanes)
       if (o + t < ocap) tets[o + t] = ctet[base + t];
     return;
   }
-  const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-  for (uint32_t r0 = 0; r0 < n; r0 += 64) {
-    const uint32_t t = r0 + lane;
+  for (uint32_t r0 = 0; r0 < n; r0 += kSegLanes) {
+    const uint32_t t = r0 + sub;
     bool keep = false;
     uint4 v = make_uint4(0u, 0u, 0u, 0u);
     if (t < n) { /* both loads in flight together */
       v = ctet[base + t];
       keep = flag[base + t] == KEEP;
     }
-    const uint64_t bm = __ballot(keep);
-    const uint64_t pre = o + (uint64_t)__popcll(bm & lt);
+    const unsigned bm = seg_ballot(keep);
+    const uint64_t pre = o + (unsigned)__popc(bm & ((1u << sub) - 1u));
     if (keep && pre < ocap) tets[pre] = v;
-    o += (uint64_t)__popcll(bm);
+    o += (unsigned)__popc(bm);
   }
 }
-void launch_tet_block_keep(Cnt nt, const uint64_t* off, int stride,
-                           const uint32_t* bcnt, const uint8_t* flag,
-                           uint32_t* bkeep, PipeLaunch L) {
-  if (nt.cap <= 0) return;
-  const int64_t nblk = (nt.cap + kBlock - 1) / kBlock;
-  hipLaunchKernelGGL(k_tet_block_keep,
-                     dim3((unsigned)((nblk * 64 + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, nt, off, stride, bcnt, flag, bkeep);
+void launch_seg_kept(Cnt n, int seg, const uint64_t* off, int stride,
+                     const uint32_t* bcnt, const uint8_t* flag, uint32_t* bkeep,
+                     PipeLaunch L) {
+  if (n.cap <= 0) return;
+  const int64_t nseg = (n.cap + seg - 1) / seg;
+  hipLaunchKernelGGL(k_seg_kept,
+                     dim3((unsigned)((nseg * kSegLanes + kBlock - 1) / kBlock)),
+                     dim3(kBlock), 0, L.s, n, seg, off, stride, bcnt, flag,
+                     bkeep);
 }
-void launch_tet_block_copy(Cnt nt, const uint64_t* off, int stride,
-                           const uint32_t* bcnt, const uint4* ctet,
-                           const uint8_t* flag, const uint64_t* bout,
-                           uint4* tets, PipeLaunch L, uint64_t ocap) {
+void launch_tet_seg_copy(Cnt nt, const uint64_t* bbase, const uint32_t* bcnt,
+                         const uint4* ctet, const uint8_t* flag,
+                         const uint64_t* bout, uint4* tets, PipeLaunch L,
+                         uint64_t ocap) {
   if (nt.cap <= 0) return;
-  const int64_t nblk = (nt.cap + kBlock - 1) / kBlock;
-  hipLaunchKernelGGL(k_tet_block_copy,
-                     dim3((unsigned)((nblk * 64 + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, nt, off, stride, bcnt, ctet, flag,
-                     bout, tets, ocap);
+  const int64_t nseg = (nt.cap + kTetSeg - 1) / kTetSeg;
+  hipLaunchKernelGGL(
+      k_tet_seg_copy,
+      dim3((unsigned)((nseg * kSegLanes + kBlock - 1) / kBlock)), dim3(kBlock), 0, L.s, nt, bbase, bcnt, ctet, flag, bout, tets, ocap);
 }
 
 /* Edge candidates of ball i (j > i in the stencil rows, Parallel:122-201)

@@ -159,27 +159,6 @@ struct BlockOut {
   }
 };
 
-/* the same for one array of uint4 entries */
-template <int CAP>
-struct BlockOut4 {
-  uint4* s; /* LDS, CAP */
-  uint64_t base, total, lim;
-  __device__ __forceinline__ void put(uint4* g, uint64_t o, const uint4& v) {
-    if (o >= lim) return;
-    uint64_t lo = o - base;
-    if (lo < (uint64_t)CAP) s[lo] = v;
-    else g[o] = v;
-  }
-  __device__ __forceinline__ void flush(uint4* g) {
-    __syncthreads();
-    uint64_t m64 = total < (uint64_t)CAP ? total : (uint64_t)CAP;
-    if (base >= lim) m64 = 0;
-    else if (m64 > lim - base) m64 = lim - base;
-    const uint32_t m = (uint32_t)m64;
-    for (uint32_t t = threadIdx.x; t < m; t += blockDim.x) g[base + t] = s[t];
-  }
-};
-
 struct StageCnt {
   unsigned c[4];
   __device__ StageCnt() { c[0] = c[1] = c[2] = c[3] = 0; }
@@ -753,27 +732,36 @@ __device__ __forceinline__ bool pairss_init(PairSS<R>& P, const V3<FE<R>>& pa,
 }
 /* Semi-static setup: D, N (tets) or den, num (triangles, edges) evaluated
  * once in precision R together with the same expressions on absolute
- * values (perm); with leaves y = p - p_a and w = r^2 each rounded once, a
- * tree of height h has |computed - exact| <= gamma_{h} * perm, and
- * gamma_{h} <= (h + 1) u for h u << 1.  Heights used: D 6, N 10 (tets);
- * |n|^2 6, X 10 (triangles); |u|^2 4, A u 8 (edges), rounded up. */
+ * values (perm).  A value whose terms each pass through at most k roundings
+ * has |computed - exact| <= gamma_k * perm, gamma_k <= k u plus what the
+ * slack covers.  Leaves y = p - p_a and w = r^2 are rounded once; a product
+ * has its factors' counts plus one, a sum its larger one plus one, and a
+ * fused multiply-add (dot3, det2) one rounding where a product and a sum
+ * take two: a component of a cross product of leaves 4, |y|^2 5,
+ * A = |y|^2 + w_a - w 7; tets D 8, N 14; triangles |n|^2 11, X 16; edges
+ * A u 9. */
 template <class R>
 struct SS {
   R v, p; /* value, permanent */
 };
+/* the value with its bound k u perm */
 template <class R>
-__device__ __forceinline__ FE<R> ss_fe(const SS<R>& a, int h) {
-  R g = (R)(h + 2) * FEc<R>::u();
-  return FE<R>{a.v, g * a.p * FEc<R>::slack() + (R)64 * FEc<R>::tiny()};
+__device__ __forceinline__ FE<R> ss_fe(const SS<R>& a, int k) {
+  const R g = (R)k * FEc<R>::u() * FEc<R>::slack();
+  return FE<R>{a.v, fmaR(a.p, g, (R)64 * FEc<R>::tiny())};
 }
 template <class R>
-__device__ __forceinline__ void cross_ss(R ax, R ay, R az, R bx, R by, R bz,
-                                         SS<R>* c) {
-  R aX = fabs(ax), aY = fabs(ay), aZ = fabs(az), bX = fabs(bx), bY = fabs(by),
-    bZ = fabs(bz);
-  c[0] = SS<R>{ay * bz - az * by, aY * bZ + aZ * bY};
-  c[1] = SS<R>{az * bx - ax * bz, aZ * bX + aX * bZ};
-  c[2] = SS<R>{ax * by - ay * bx, aX * bY + aY * bX};
+__device__ __forceinline__ R dot3(R ax, R ay, R az, R bx, R by, R bz) {
+  return fmaR(ax, bx, fmaR(ay, by, az * bz));
+}
+/* a b - c d */
+template <class R>
+__device__ __forceinline__ R det2(R a, R b, R c, R d) {
+  return fmaR(a, b, -(c * d));
+}
+template <class R>
+__device__ __forceinline__ R max3(R a, R b, R c) {
+  return fmax(a, fmax(b, c));
 }
 
 /* The pair test's gap g = sign(den) (L den - y . num) for ball e and the
@@ -823,8 +811,9 @@ __device__ __forceinline__ void pairss_masks(const PairSS<R>& P,
 
 /* Orthocentre numerators N and denominator D of a tet at precision R with
  * a-priori (semi-static) error bounds, and w_a = r_a^2 with its rounding
- * bound: the same D, N as tet_DN, each bounded by gamma_h times its
- * permanent instead of a running error per operation. */
+ * bound: the same D, N as tet_DN, each bounded by its rounding count times
+ * its permanent instead of a running error per operation (N's parts share
+ * one bound). */
 template <class R>
 struct TetCert {
   FE<R> D;
@@ -834,66 +823,66 @@ struct TetCert {
 template <class R>
 __device__ __forceinline__ void tet_dn_ss(const Ball v[4], TetCert<R>& T) {
   const R ax = v[0].x, ay = v[0].y, az = v[0].z;
-  R ux = (R)v[1].x - ax, uy = (R)v[1].y - ay, uz = (R)v[1].z - az;
-  R vx = (R)v[2].x - ax, vy = (R)v[2].y - ay, vz = (R)v[2].z - az;
-  R tx = (R)v[3].x - ax, ty = (R)v[3].y - ay, tz = (R)v[3].z - az;
-  R wa = (R)v[0].w * (R)v[0].w;
-  R w1 = (R)v[1].w * (R)v[1].w, w2 = (R)v[2].w * (R)v[2].w,
-    w3 = (R)v[3].w * (R)v[3].w;
+  const R ux = (R)v[1].x - ax, uy = (R)v[1].y - ay, uz = (R)v[1].z - az;
+  const R vx = (R)v[2].x - ax, vy = (R)v[2].y - ay, vz = (R)v[2].z - az;
+  const R tx = (R)v[3].x - ax, ty = (R)v[3].y - ay, tz = (R)v[3].z - az;
+  const R wa = (R)v[0].w * (R)v[0].w;
+  const R w1 = (R)v[1].w * (R)v[1].w, w2 = (R)v[2].w * (R)v[2].w,
+          w3 = (R)v[3].w * (R)v[3].w;
   /* the permanents of the cross products bounded by max norms:
-   * |v_y t_z| + |v_z t_y| <= 2 |v|_inf |t|_inf for every component */
-  const R mu = fmax(fabs(ux), fmax(fabs(uy), fabs(uz)));
-  const R mv = fmax(fabs(vx), fmax(fabs(vy), fabs(vz)));
-  const R mt = fmax(fabs(tx), fmax(fabs(ty), fabs(tz)));
-  const R pvt = ((R)2 * mv) * mt, ptu = ((R)2 * mt) * mu, puv = ((R)2 * mu) * mv;
-  const R vt[3] = {vy * tz - vz * ty, vz * tx - vx * tz, vx * ty - vy * tx};
-  const R tu[3] = {ty * uz - tz * uy, tz * ux - tx * uz, tx * uy - ty * ux};
-  const R uv[3] = {uy * vz - uz * vy, uz * vx - ux * vz, ux * vy - uy * vx};
-  SS<R> D{ux * vt[0] + uy * vt[1] + uz * vt[2],
-          ((fabs(ux) + fabs(uy)) + fabs(uz)) * pvt};
-  R uu = ux * ux + uy * uy + uz * uz, vv = vx * vx + vy * vy + vz * vz,
-    tt = tx * tx + ty * ty + tz * tz;
-  SS<R> A{(uu + wa) - w1, (uu + wa) + w1}, B{(vv + wa) - w2, (vv + wa) + w2},
-      C{(tt + wa) - w3, (tt + wa) + w3};
-  const R np = A.p * pvt + B.p * ptu + C.p * puv;
-  SS<R> N[3];
-#pragma unroll
-  for (int q = 0; q < 3; ++q)
-    N[q] = SS<R>{A.v * vt[q] + B.v * tu[q] + C.v * uv[q], np};
-  T.D = ss_fe(D, 6);
-  T.N = V3<FE<R>>{ss_fe(N[0], 10), ss_fe(N[1], 10), ss_fe(N[2], 10)};
-  T.wa = FE<R>{wa, FEc<R>::u() * wa * FEc<R>::slack()};
+   * |v_y t_z| + |v_z t_y| <= 2 |v|_inf |t|_inf for every component; the
+   * factor 2 is left to the bounds' counts (ss_fe's k) */
+  const R mu = max3(fabs(ux), fabs(uy), fabs(uz));
+  const R mv = max3(fabs(vx), fabs(vy), fabs(vz));
+  const R mt = max3(fabs(tx), fabs(ty), fabs(tz));
+  const R pvt = mv * mt, ptu = mt * mu, puv = mu * mv;
+  const R vt[3] = {det2(vy, tz, vz, ty), det2(vz, tx, vx, tz),
+                   det2(vx, ty, vy, tx)};
+  const R tu[3] = {det2(ty, uz, tz, uy), det2(tz, ux, tx, uz),
+                   det2(tx, uy, ty, ux)};
+  const R uv[3] = {det2(uy, vz, uz, vy), det2(uz, vx, ux, vz),
+                   det2(ux, vy, uy, vx)};
+  const SS<R> D{dot3(ux, uy, uz, vt[0], vt[1], vt[2]),
+                ((fabs(ux) + fabs(uy)) + fabs(uz)) * pvt};
+  const R uu = dot3(ux, uy, uz, ux, uy, uz), vv = dot3(vx, vy, vz, vx, vy, vz),
+          tt = dot3(tx, ty, tz, tx, ty, tz);
+  const SS<R> A{(uu + wa) - w1, (uu + wa) + w1},
+      B{(vv + wa) - w2, (vv + wa) + w2}, C{(tt + wa) - w3, (tt + wa) + w3};
+  const R np = fmaR(A.p, pvt, fmaR(B.p, ptu, C.p * puv));
+  T.D = ss_fe(D, 2 * 8);
+  T.N.x = ss_fe(SS<R>{dot3(A.v, B.v, C.v, vt[0], tu[0], uv[0]), np}, 2 * 14);
+  T.N.y = FE<R>{dot3(A.v, B.v, C.v, vt[1], tu[1], uv[1]), T.N.x.e};
+  T.N.z = FE<R>{dot3(A.v, B.v, C.v, vt[2], tu[2], uv[2]), T.N.x.e};
+  T.wa = FE<R>{wa, FEc<R>::u() * FEc<R>::slack() * wa};
 }
 /* Sign of V = 4 D^2 (w_a + alpha) - |N|^2 (alpha exact) from the
- * certified D, N, w_a: 1 certainly > 0, -1 certainly < 0, 0 undecided.
- * One bound instead of a running error per operation:
+ * certified D, N (one bound e for its three parts, as tet_dn_ss gives), w_a:
+ * 1 certainly > 0, -1 certainly < 0, 0 undecided.  One bound instead of a
+ * running error per operation:
  *  - the inputs' errors: |4 D*^2 (w*+a) - 4 D^2 (w+a)| <=
  *    4 (2|D| eD + eD^2)(|w+a| + ew) + 4 D^2 ew, and
- *    ||N*|^2 - |N|^2| <= sum_q (2|N_q| + eN_q) eN_q;
+ *    ||N*|^2 - |N|^2| <= sum_q (2|N_q| + e) e = (2 sum |N_q| + 3 e) e;
  *  - the evaluation's roundings: 4 D is exact, 4 D^2 (w+a) and |N|^2 each
  *    carry at most three roundings (gamma_3 / (1 - gamma_3) < 4u of their
  *    computed magnitudes), the difference one more (u / (1 - u) < 2u of
- *    the computed V);
+ *    the computed V, at most the magnitudes' sum);
  *  - 64 tiny for products that underflow; the slack covers the rounding
  *    of the bound's own evaluation. */
 template <class R>
 __device__ __forceinline__ int tet_val_ss(const TetCert<R>& T, R alpha) {
-  const R u = FEc<R>::u();
-  const R D = T.D.v, eD = T.D.e;
+  const R u = FEc<R>::u(), sl = FEc<R>::slack();
+  const R D = T.D.v, eD = T.D.e, e = T.N.x.e;
   const R s = T.wa.v + alpha, es = T.wa.e;
   const R t2 = ((R)4 * D) * D;
   const R t3 = t2 * s;
   const R nx = T.N.x.v, ny = T.N.y.v, nz = T.N.z.v;
-  const R n2 = (nx * nx + ny * ny) + nz * nz;
+  const R n2 = dot3(nx, ny, nz, nx, ny, nz);
   const R V = t3 - n2;
-  const R eDD = ((R)2 * fabs(D) + eD) * eD;
-  const R eN = ((R)2 * fabs(nx) + T.N.x.e) * T.N.x.e +
-               ((R)2 * fabs(ny) + T.N.y.e) * T.N.y.e +
-               ((R)2 * fabs(nz) + T.N.z.e) * T.N.z.e;
-  const R ein = (R)4 * eDD * (fabs(s) + es) + t2 * es + eN;
-  const R B = (ein + (R)4 * u * (fabs(t3) + n2) + (R)2 * u * fabs(V) +
-               (R)64 * FEc<R>::tiny()) *
-              FEc<R>::slack();
+  const R eDD = fmaR((R)8, fabs(D), (R)4 * eD) * eD;
+  const R eN = fmaR((R)2, (fabs(nx) + fabs(ny)) + fabs(nz), (R)3 * e) * e;
+  const R ein = fmaR(eDD, fabs(s) + es, fmaR(t2, es, eN));
+  const R B = fmaR(fmaR(fabs(t3) + n2, (R)6 * u, ein), sl,
+                   (R)128 * FEc<R>::tiny());
   return V > B ? 1 : (V < -B ? -1 : 0);
 }
 

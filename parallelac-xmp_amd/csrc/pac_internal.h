@@ -464,7 +464,7 @@ void launch_tri_enum_filter(const Stage& S, Cnt ne, const uint64_t* erow,
                             uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep,
                             uint8_t* edead, Queue q1, PipeLaunch L,
                             uint64_t lim = ~0ull);
-/* after the ladder (bkeep by launch_tet_block_keep over the ne alpha
+/* after the ladder (bkeep by launch_seg_kept over the ne alpha
  * edges, bout its exclusive scan): the kept triangles of each block to
  * (tk, tedge, teik, tejk) in order (tkd: tk with kDeadBit where one of the
  * three edges is marked in edead), the alpha-triangle row start of every
@@ -479,15 +479,16 @@ void launch_tri_block_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
                            uint64_t* trow, uint64_t* tpair, PipeLaunch L,
                            uint64_t ocap = ~0ull);
 /* tet candidates of the alpha triangles, each filtered by the first
- * precision stage in the same kernel; enumeration block b (256 alpha
+ * precision stage in the same kernel; enumeration segment b (kTetSeg alpha
  * triangles) writes its kept and undecided tets (i, j, k, l) with their
  * flags, in order, compacted from its first slot on (bbase[b]) and their
  * number to bcnt[b]; undecided ones are queued on q1 by position.  Kept
  * tets one of whose triangles has kDeadBit in tkd are counted (CTR_DROP)
- * but not written.  Slot
- * offsets per triangle from off[], or (off null) from roff, the exclusive
- * scan of launch_tri_block_copy's tpair (each triangle's slots its row's
- * tail: not for chunk sub-inputs, whose unowned triangles get none) */
+ * but not written.  Slot offsets per triangle from off[], or (off null)
+ * from roff, the exclusive scan of launch_tri_block_copy's tpair (each
+ * triangle's slots its row's tail: not for chunk sub-inputs, whose unowned
+ * triangles get none) */
+constexpr int kTetSeg = 64;
 void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
                             const uint32_t* tkd, const uint32_t* tedge,
                             const uint32_t* teik, const uint32_t* tejk,
@@ -497,21 +498,21 @@ void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
                             uint32_t* bcnt, uint32_t* bkeep, Queue q1,
                             PipeLaunch L, uint64_t lim = ~0ull);
 /* The triangle and tet enumerations also write bkeep[b]: bcnt[b] when the
- * block queued no undecided candidate (the ladder cannot drop any of its
+ * segment queued no undecided candidate (the ladder cannot drop any of its
  * entries), else kRecount. */
 constexpr uint32_t kRecount = 0xffffffffu;
-/* after the ladder: kept tets per enumeration block (ceil(nt.cap / 256)
- * entries; blocks marked kRecount recounted from their flags), then, with
- * bout their exclusive scan, the kept tets in order; block b's entries
- * start at off[b * stride] (per-item offsets: stride 256; per-block
- * bases: 1) */
-void launch_tet_block_keep(Cnt nt, const uint64_t* off, int stride,
-                           const uint32_t* bcnt, const uint8_t* flag,
-                           uint32_t* bkeep, PipeLaunch L);
-void launch_tet_block_copy(Cnt nt, const uint64_t* off, int stride,
-                           const uint32_t* bcnt, const uint4* ctet,
-                           const uint8_t* flag, const uint64_t* bout,
-                           uint4* tets, PipeLaunch L, uint64_t ocap = ~0ull);
+/* after the ladder: kept candidates per enumeration segment of `seg` items
+ * (ceil(n.cap / seg) entries; segments marked kRecount recounted from their
+ * flags), then, with bout their exclusive scan, the kept tets in order;
+ * segment b's entries start at off[b * stride] (per-item offsets: stride
+ * seg; per-segment bases: 1) */
+void launch_seg_kept(Cnt n, int seg, const uint64_t* off, int stride,
+                     const uint32_t* bcnt, const uint8_t* flag, uint32_t* bkeep,
+                     PipeLaunch L);
+void launch_tet_seg_copy(Cnt nt, const uint64_t* bbase, const uint32_t* bcnt,
+                         const uint4* ctet, const uint8_t* flag,
+                         const uint64_t* bout, uint4* tets, PipeLaunch L,
+                         uint64_t ocap = ~0ull);
 /* escalation and exact stages of the filters (the first stages are fused
  * with the enumerations): kind 1 edges, 2 triangles, 3 tets */
 void launch_filter_esc(const Stage& S, int kind, CandCtx C, QRef q, const uint32_t* cval, uint8_t* flag,

@@ -646,8 +646,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           launch_filter_exact(SG, 2, C1, qr, cval.get(), flag.get(), L);
         },
         [&] {
-          launch_tet_block_keep(Ealpha, off.get(), kBlock, bcnt.get(), flag.get(),
-                                bkeep.get(), L);
+          launch_seg_kept(Ealpha, kBlock, off.get(), kBlock, bcnt.get(),
+                          flag.get(), bkeep.get(), L);
           scan_u32_to_u64(bkeep.get(), bout.get(), Cnt(nblk), tmp.get(), 0, s,
                           dcnt + RC_TALPHA);
         },
@@ -696,11 +696,11 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     DBuf<uint4> ctet(P, Kslots.cap);
     DBuf<uint8_t> flag(P, Kslots.cap);
     C2.ctet = ctet.get();
-    /* enumeration and first filter stage in one kernel, each block's kept
-     * and undecided tets compacted in place (its count in bcnt); the
-     * ladder settles the undecided ones; then the kept tets of each block
+    /* enumeration and first filter stage in one kernel, each segment's
+     * kept and undecided tets compacted in place (its count in bcnt); the
+     * ladder settles the undecided ones; then the kept tets of each segment
      * are counted, scanned and copied out in order */
-    const int64_t nblk = (Talpha.cap + kBlock - 1) / kBlock;
+    const int64_t nblk = (Talpha.cap + kTetSeg - 1) / kTetSeg;
     DBuf<uint32_t> bcnt(P, nblk + 1), bkeep(P, nblk + 1);
     DBuf<uint64_t> bout(P, nblk + 1), bbase(P, nblk + 1);
     auto tmp = scan_tmp(nblk);
@@ -726,16 +726,16 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
         },
         [&](QRef qr) { launch_filter_exact(SG, 3, C2, qr, nullptr, flag.get(), L); },
         [&] {
-          launch_tet_block_keep(Talpha, bbase.get(), 1, bcnt.get(), flag.get(),
-                                bkeep.get(), L);
+          launch_seg_kept(Talpha, kTetSeg, bbase.get(), 1, bcnt.get(),
+                          flag.get(), bkeep.get(), L);
           scan_u32_to_u64(bkeep.get(), bout.get(), Cnt(nblk), tmp.get(), 0, s,
                           dcnt + RC_KALPHA);
         },
         RC_KALPHA);
     tets = DBuf<uint4>(P, Kalpha.cap);
-    launch_tet_block_copy(Talpha, bbase.get(), 1, bcnt.get(), ctet.get(),
-                          flag.get(), bout.get(), tets.get(), L,
-                          (uint64_t)Kalpha.cap);
+    launch_tet_seg_copy(Talpha, bbase.get(), bcnt.get(), ctet.get(),
+                        flag.get(), bout.get(), tets.get(), L,
+                        (uint64_t)Kalpha.cap);
     KCHK();
   }
   T.mark(5);

@@ -16,6 +16,8 @@
  * orient3d / insphere_w / orientation4SoS_w, predicates.h:2015, :4250,
  * :4669), checkDanglingTris :807-881, checkDanglingEdges :928-1015.
  */
+#include <algorithm>
+
 #include "pac_dev.h"
 #include "pac_wide.h"
 #include "pac_sos_table.h"
@@ -223,6 +225,7 @@ __global__ __launch_bounds__(kBlock) void k_tet_need(Stage S, Cnt c_nk,
                                                      uint8_t* flag,
                                                      uint32_t* next,
                                                      unsigned* nnext) {
+  stamp(S.ts, 5);
   const int64_t nk = c_nk.get();
   const int64_t id = gtid();
   bool need = false;
@@ -241,6 +244,7 @@ template <class R, bool MOL>
 __global__ __launch_bounds__(kBlock) void k_tet_ac2_quick(
     Stage S, Cnt c_nk, const uint4* tets, uint8_t* flag, uint32_t* next,
     unsigned* nnext) {
+  stamp(S.ts, 5);
   unsigned pairs = 0;
   const int64_t nk = c_nk.get();
   const int64_t id = gtid();
@@ -279,6 +283,7 @@ __global__ __launch_bounds__(kBlock) void k_tet_ac2_hot(
     Stage S0, Cnt c_nk, const uint32_t* items, const unsigned* nitems,
     const uint4* tets, uint8_t* flag, Queue q1, uint32_t* rest,
     unsigned* nrest, int budget) {
+  if (PH == PH_ALL) stamp(S0.ts, 5);
   unsigned evals = 0, pairs = 0;
   /* phase A: the alpha tets, or the list `items` of them (those the quick
    * pass left); phase B: `rest` */
@@ -415,8 +420,10 @@ __device__ __forceinline__ int tet_pair_code_T(const TetQ<T>& t, int sD,
   return tet_pair_code(t, sD, e);
 }
 __global__ __launch_bounds__(kBlock) void k_tet_ac2_esc(
-    Stage S, QRef q, const uint4* tets, uint8_t* flag,
+    Stage S, QRef qr, const uint4* tets, uint8_t* flag,
     Queue q2) {
+  __shared__ uint32_t s_off[QSLOTS + 1];
+  const QTab q = q_table(qr, s_off);
   StageCnt sc;
   for_queue(q, [&](uint32_t t) {
     if (!live_entry(q.at(t), flag)) return;
@@ -600,8 +607,10 @@ __device__ __forceinline__ void tet_exact_entry(const Stage& S,
 }
 
 __global__ __launch_bounds__(kBlock) void k_tet_ac2_exact(
-    Stage S, QRef q, const uint4* tets,
+    Stage S, QRef qr, const uint4* tets,
     const uint32_t* perm, uint8_t* flag) {
+  __shared__ uint32_t s_off[QSLOTS + 1];
+  const QTab q = q_table(qr, s_off);
   unsigned cnt = 0, sos = 0;
   const bool lead = Grp<kTPI>::idx() == 0;
   __shared__ uint32_t s_lift[kBlock / 64][20 * 64]; /* SoS lifted matrices */
@@ -653,7 +662,13 @@ __global__ __launch_bounds__(kBlock) void k_view_split(QView v, uint32_t* item,
                                                        uint32_t* aux) {
   const int64_t i = gtid();
   if (i >= (int64_t)v.size()) return;
-  const QEntry e = v.at((uint32_t)i);
+  int lo = 0, hi = QSLOTS - 1; /* last sub-queue starting at or before i */
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if ((int64_t)v.off[mid] <= i) lo = mid;
+    else hi = mid - 1;
+  }
+  const QEntry e = v.q[(uint64_t)lo * v.cap + ((uint32_t)i - v.off[lo])];
   item[i] = e.item;
   aux[i] = e.aux;
 }
@@ -953,9 +968,11 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
 
 template <int KIND>
 __global__ __launch_bounds__(kBlock) void k_low_ac2_esc(
-    Stage S, QRef q, const uint32_t* ecol,
+    Stage S, QRef qr, const uint32_t* ecol,
     const uint32_t* eleft, const uint32_t* tk, const uint32_t* tedge,
     uint8_t* flag, Queue q2) {
+  __shared__ uint32_t s_off[QSLOTS + 1];
+  const QTab q = q_table(qr, s_off);
   StageCnt sc;
   for_queue(q, [&](uint32_t t) {
     if (!live_entry(q.at(t), flag)) return;
@@ -1147,9 +1164,11 @@ __device__ __forceinline__ void low_exact_entry(const Stage& S,
  * group of kTPI lanes */
 template <int KIND>
 __global__ __launch_bounds__(kBlock) void k_low_ac2_exact(
-    Stage S, QRef q, const uint32_t* ecol,
+    Stage S, QRef qr, const uint32_t* ecol,
     const uint32_t* eleft, const uint32_t* tk, const uint32_t* tedge,
     uint8_t* flag) {
+  __shared__ uint32_t s_off[QSLOTS + 1];
+  const QTab q = q_table(qr, s_off);
   unsigned cnt = 0;
   const bool lead = Grp<kTPI>::idx() == 0;
   for_queue_grp<kTPI>(q, [&](uint32_t t) {
@@ -1193,11 +1212,16 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_exact_sorted(
 }
 
 /* ---------------- launchers ---------------- */
+/* blocks of the persistent second phase: no more than the items fill */
+static unsigned rest_grid(const Stage& S, Cnt n) {
+  const int64_t b = (n.cap + S.bblock - 1) / S.bblock;
+  return (unsigned)std::min<int64_t>(std::max<int64_t>(b, 1), S.bgrid);
+}
 template <class R, bool FINE, bool MOL>
 static void tet_hot3(const Stage& S, Cnt nk, const uint4* tets, uint8_t* flag,
                      Queue q1, uint32_t* rest, unsigned* nrest, uint32_t* next,
                      unsigned* nnext, int budget, PipeLaunch L) {
-  dim3 gr((unsigned)((nk.cap + kBlock - 1) / kBlock)), gb((unsigned)S.bgrid);
+  dim3 gr((unsigned)((nk.cap + kBlock - 1) / kBlock)), gb(rest_grid(S, nk));
   const uint32_t* items = nullptr;
   if (FINE && S.quick) { /* quick pass, then the certified scan of the rest */
     hipLaunchKernelGGL((k_tet_ac2_quick<R, MOL>), gr, dim3(kBlock), 0, L.s, S,
@@ -1318,7 +1342,7 @@ static void low_hot4(const Stage& S, Cnt nitems, const uint32_t* ecol,
                      uint32_t* rest, unsigned* nrest, uint32_t* next,
                      unsigned* nnext, int budget, PipeLaunch L) {
   const dim3 gr((unsigned)((nitems.cap + kBlock - 1) / kBlock)),
-      gb((unsigned)S.bgrid);
+      gb(rest_grid(S, nitems));
   if (nitems.cap >= kListItems) {
     const int64_t per = kBlock * kListRun;
     hipLaunchKernelGGL(k_low_list<KIND>,

@@ -35,7 +35,9 @@ void launch_or_flags(Cnt n, const uint8_t* a, const uint8_t* b, uint8_t* out,
 /* faces of the final tets -> tri_in */
 __global__ __launch_bounds__(kBlock) void k_mark_faces(
     Cnt c_nk, const uint4* ftets, const uint64_t* erow, const uint32_t* ecol,
-    const uint64_t* trow, const uint32_t* tk, uint8_t* tri_in) {
+    const uint64_t* trow, const uint32_t* tk, uint8_t* tri_in,
+    unsigned long long* ts) {
+  stamp(ts, 6);
   const int64_t nk = c_nk.get();
   int64_t id = gtid();
   if (id >= nk) return;
@@ -58,18 +60,21 @@ __global__ __launch_bounds__(kBlock) void k_mark_faces(
 }
 void launch_mark_faces(Cnt nk, const uint4* ftets, const uint64_t* erow,
                        const uint32_t* ecol, const uint64_t* trow,
-                       const uint32_t* tk, uint8_t* tri_in, PipeLaunch L) {
+                       const uint32_t* tk, uint8_t* tri_in,
+                       unsigned long long* ts, PipeLaunch L) {
   if (nk.cap <= 0) return;
   hipLaunchKernelGGL(k_mark_faces, dim3((unsigned)((nk.cap + kBlock - 1) / kBlock)),
                      dim3(kBlock), 0, L.s, nk, ftets, erow, ecol, trow, tk,
-                     tri_in);
+                     tri_in, ts);
 }
 
 /* edges of the final triangles -> edge_in (edge ids recorded at
  * enumeration: (i,j) = tedge, (i,k) = teik, (j,k) = tejk) */
 __global__ __launch_bounds__(kBlock) void k_mark_edges(
     Cnt c_nt, const uint32_t* ftri, const uint32_t* tedge,
-    const uint32_t* teik, const uint32_t* tejk, uint8_t* edge_in) {
+    const uint32_t* teik, const uint32_t* tejk, uint8_t* edge_in,
+    unsigned long long* ts) {
+  stamp(ts, 7);
   const int64_t nt = c_nt.get();
   int64_t id = gtid();
   if (id >= nt) return;
@@ -80,11 +85,11 @@ __global__ __launch_bounds__(kBlock) void k_mark_edges(
 }
 void launch_mark_edges(Cnt nt, const uint32_t* ftri, const uint32_t* tedge,
                        const uint32_t* teik, const uint32_t* tejk,
-                       uint8_t* edge_in, PipeLaunch L) {
+                       uint8_t* edge_in, unsigned long long* ts, PipeLaunch L) {
   if (nt.cap <= 0) return;
   hipLaunchKernelGGL(k_mark_edges, dim3((unsigned)((nt.cap + kBlock - 1) / kBlock)),
                      dim3(kBlock), 0, L.s, nt, ftri, tedge, teik, tejk,
-                     edge_in);
+                     edge_in, ts);
 }
 
 /* ---- emission in original ids ---- */

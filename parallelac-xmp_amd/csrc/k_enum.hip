@@ -122,35 +122,79 @@ __device__ void bred_block(BRed& mine, BRed* sh) {
   mine = sh[0];
 }
 
-__global__ __launch_bounds__(kBlock) void k_bounds_part(const Ball* raw,
-                                                        int64_t n,
-                                                        Real solvent,
-                                                        BRed* part) {
+/* the reduced bounds to `out`, and posted */
+__device__ __forceinline__ void bounds_done(const BRed& b, Bounds* out,
+                                            const Post& post, Bounds* s_b) {
+  if (threadIdx.x == 0) {
+    *s_b = bred_out(b);
+    *out = *s_b;
+  }
+  if (!post.box) return;
+  __syncthreads();
+  constexpr int kW = sizeof(Bounds) / sizeof(unsigned);
+  static_assert(sizeof(Bounds) % sizeof(unsigned) == 0 && kW <= 64, "one wave");
+  if (threadIdx.x < kW)
+    post.box[kBoxData + threadIdx.x] =
+        reinterpret_cast<const unsigned*>(s_b)[threadIdx.x];
+  if (threadIdx.x < 64) {
+    __threadfence_system();
+    if (threadIdx.x == 0)
+      __hip_atomic_store(
+          reinterpret_cast<unsigned long long*>(post.box + kBoxTicket),
+          post.ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+/* Bounds of the balls; a run's first kernel, so it also clears the run's
+ * control words (ctl) and keeps the balls in input order with their final
+ * radii (orig, for alpha values and the adjoint), each where given.  A
+ * single block's partial is the result. */
+__global__ __launch_bounds__(kBlock) void k_bounds_part(
+    const Ball* raw, int64_t n, Real solvent, BRed* part, Bounds* out,
+    double4* orig, unsigned long long* ctl, int ctl_words, Post post) {
   __shared__ BRed sh[kBlock];
+  __shared__ Bounds s_b;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  if (ctl) {
+    for (int64_t i = gtid(); i < ctl_words; i += stride)
+      ctl[i] = i == ctl_words - kStamps + 1 ? wall_clock64() : 0ull;
+  }
   BRed b;
   bred_init(b);
-  for (int64_t i = gtid(); i < n; i += (int64_t)gridDim.x * blockDim.x)
-    bred_ball(b, raw[i], solvent);
+  for (int64_t i = gtid(); i < n; i += stride) {
+    const Ball a = raw[i];
+    bred_ball(b, a, solvent);
+    if (orig)
+      orig[i] = make_double4(a.x, a.y, a.z, (double)add_r(a.w, solvent));
+  }
   bred_block(b, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = b;
+  if (gridDim.x == 1)
+    bounds_done(b, out, post, &s_b);
+  else if (threadIdx.x == 0)
+    part[blockIdx.x] = b;
 }
 __global__ __launch_bounds__(kBlock) void k_bounds_final(const BRed* part,
-                                                         int np, Bounds* out) {
+                                                         int np, Bounds* out,
+                                                         Post post) {
   __shared__ BRed sh[kBlock];
+  __shared__ Bounds s_b;
   BRed b;
   bred_init(b);
   for (int i = threadIdx.x; i < np; i += blockDim.x) bred_merge(b, part[i]);
   bred_block(b, sh);
-  if (threadIdx.x == 0) *out = bred_out(b);
+  bounds_done(b, out, post, &s_b);
 }
 void launch_bounds(const Ball* raw, int64_t n, Real solvent, Bounds* part,
-                   Bounds* out, PipeLaunch L) {
-  int nb = (int)std::min<int64_t>(1024, (n + kBlock - 1) / kBlock);
-  if (nb < 1) nb = 1;
+                   Bounds* out, double4* orig, unsigned long long* ctl,
+                   int ctl_words, Post post, PipeLaunch L) {
+  /* one block up to 2048 balls: a second launch costs more than 8 balls a
+   * thread */
+  int nb = n <= 2048 ? 1
+                     : (int)std::min<int64_t>(1024, (n + kBlock - 1) / kBlock);
   hipLaunchKernelGGL(k_bounds_part, dim3(nb), dim3(kBlock), 0, L.s, raw, n,
-                     solvent, (BRed*)part);
-  hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlock), 0, L.s,
-                     (const BRed*)part, nb, out);
+                     solvent, (BRed*)part, out, orig, ctl, ctl_words, post);
+  if (nb > 1)
+    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlock), 0, L.s,
+                       (const BRed*)part, nb, out, post);
 }
 
 /* Per-molecule bounds of a batch: block m reduces the balls of molecule m
@@ -506,6 +550,7 @@ __device__ __forceinline__ void cell_xyz(uint32_t c, const GridP& g, int& x,
 }
 
 __global__ __launch_bounds__(kBlock) void k_edge_count(Stage S, uint32_t* cnt) {
+  stamp(S.ts, 2);
   int64_t i = gtid();
   if (i >= S.n) return;
   const GridP g = grid_of(S, (uint32_t)i);
@@ -598,7 +643,9 @@ __global__ __launch_bounds__(kBlock) void k_tri_count(Cnt c_ne,
                                                      const uint64_t* erow,
                                                      const uint32_t* ecol,
                                                      const uint32_t* eleft,
-                                                     uint32_t* cnt) {
+                                                     uint32_t* cnt,
+                                                     unsigned long long* ts) {
+  stamp(ts, 3);
   const int64_t ne = c_ne.get();
   int64_t q = gtid();
   if (q >= ne) return;
@@ -637,11 +684,12 @@ __global__ __launch_bounds__(kBlock) void k_tri_count(Cnt c_ne,
   cnt[q] = c;
 }
 void launch_tri_count(Cnt ne, const uint64_t* erow, const uint32_t* ecol,
-                      const uint32_t* eleft, uint32_t* cnt, PipeLaunch L) {
+                      const uint32_t* eleft, uint32_t* cnt,
+                      unsigned long long* ts, PipeLaunch L) {
   if (ne.cap <= 0) return;
   auto kf = ne.cap < ((int64_t)1 << 30) ? k_tri_count<true> : k_tri_count<false>;
   hipLaunchKernelGGL(kf, dim3((unsigned)((ne.cap + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, ne, erow, ecol, eleft, cnt);
+                     dim3(kBlock), 0, L.s, ne, erow, ecol, eleft, cnt, ts);
 }
 
 /* ------------------------------------------------------------------ */
@@ -772,6 +820,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
     const uint64_t* roff, uint64_t* bbase, uint4* ctet, uint8_t* flag,
     uint32_t* bcnt, uint32_t* bkeep, Queue q1, uint64_t lim) {
   static_assert(kTetSeg == 64, "a triangle a lane");
+  stamp(S.ts, 4);
   constexpr uint32_t CAP = 1120; /* with the tables, 8 blocks per CU */
   __shared__ uint32_t s_l[kBlock / 64][CAP];
   __shared__ uint32_t s_end[kBlock / 64][64], s_off[kBlock / 64][64];
@@ -1524,10 +1573,12 @@ void launch_tri_block_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
 
 template <int KIND>
 __global__ __launch_bounds__(kBlock) void k_filter_esc(Stage S, CandCtx C,
-                                                       QRef q,
+                                                       QRef qr,
                                                        const uint32_t* cval,
                                                        uint8_t* flag,
                                                        Queue q2) {
+  __shared__ uint32_t s_off[QSLOTS + 1];
+  const QTab q = q_table(qr, s_off);
   StageCnt sc;
   for_queue(q, [&](uint32_t t) {
     QEntry e = q.at(t);
@@ -1557,9 +1608,11 @@ __global__ __launch_bounds__(kBlock) void k_filter_esc(Stage S, CandCtx C,
  * wavefront-cooperative wide-integer evaluation. */
 template <int KIND>
 __global__ __launch_bounds__(kBlock) void k_filter_exact(Stage S, CandCtx C,
-                                                         QRef q,
+                                                         QRef qr,
                                                          const uint32_t* cval,
                                                          uint8_t* flag) {
+  __shared__ uint32_t s_off[QSLOTS + 1];
+  const QTab q = q_table(qr, s_off);
   __shared__ uint32_t s_pend[kBlock / 64][64];
   unsigned cnt = 0;
   const uint32_t n = q.size();

@@ -41,6 +41,25 @@ __device__ __forceinline__ uint64_t block_excl_scan_u64(uint64_t v,
   return base + inc - v;
 }
 
+/* The post of a stage's last kernel, by one whole wave (pac_internal.h). */
+__device__ __forceinline__ void do_post(const Post& P, uint64_t count) {
+  const int k = threadIdx.x & 63;
+  if (P.qn && k < QSLOTS) {
+    unsigned* const line = P.qn + k * kSlotWords;
+    P.box[kBoxQ1 + k] = line[QK_HOT];
+    P.box[kBoxQ2 + k] = line[QK_ESC];
+    line[QK_HOT] = 0;
+    line[QK_ESC] = 0;
+    line[QK_REST] = 0;
+    line[QK_NEXT] = 0;
+  }
+  if (k == 0) *reinterpret_cast<uint64_t*>(P.box + kBoxCount) = count;
+  __threadfence_system(); /* the wave's stores before the ticket */
+  if (k == 0)
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(P.box + kBoxTicket),
+                       P.ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 template <class TIn, bool kFlag>
 __device__ __forceinline__ uint64_t load_val(const TIn* in, int64_t i,
                                              int64_t n) {
@@ -66,14 +85,54 @@ __global__ __launch_bounds__(kBlock) void k_tile_sums(const TIn* in, Cnt cn,
   if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
 
-template <class TIn, bool kFlag, class TOut>
+/* Sum of in[0, m) by the block, m a multiple of kTile: 16-byte loads,
+ * eight in flight a thread. */
+template <class TIn>
+__device__ __forceinline__ uint64_t sum_before(const TIn* in, int64_t m) {
+  constexpr int kPer = 16 / sizeof(TIn);
+  struct alignas(16) Vec {
+    TIn v[kPer];
+  };
+  const Vec* p = reinterpret_cast<const Vec*>(in);
+  const int64_t nv = m / kPer;
+  uint64_t s = 0;
+  for (int64_t i = threadIdx.x; i < nv; i += 8 * kBlock) {
+    Vec x[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (i + q * kBlock < nv) x[q] = p[i + q * kBlock];
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (i + q * kBlock < nv)
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) s += (uint64_t)x[q].v[k];
+  }
+  uint64_t tot;
+  block_excl_scan_u64(s, &tot);
+  return tot;
+}
+/* FEW: the whole scan in one launch of at most kFewTiles blocks, each
+ * summing all tiles before its own (from L2) instead of reading their
+ * offset: for small arrays two launches fewer (~4 us each) for ~2 us more
+ * of reading. */
+constexpr int64_t kFewTiles = 16;
+template <class TIn, bool kFlag, class TOut, bool FEW>
 __global__ __launch_bounds__(kBlock) void k_tile_scan(const TIn* in, Cnt cn,
                                                       const uint64_t* tile_off,
                                                       TOut* out,
-                                                      uint64_t* total64) {
+                                                      uint64_t* total64,
+                                                      Post post) {
   __shared__ uint64_t tile[kTile];
+  __shared__ uint64_t s_total;
   const int64_t n = cn.get();
   int64_t base = (int64_t)blockIdx.x * kTile;
+  uint64_t before = 0;
+  static_assert(!kFlag, "flags have scans of their own");
+  if constexpr (FEW) {
+    if (base < n) before = sum_before(in, base);
+  } else {
+    before = tile_off ? tile_off[blockIdx.x] : 0;
+  }
 #pragma unroll
   for (int q = 0; q < kScanItems; ++q) {
     int t = q * kBlock + threadIdx.x;
@@ -88,7 +147,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_scan(const TIn* in, Cnt cn,
     s += v[q];
   }
   uint64_t tot;
-  uint64_t ex = block_excl_scan_u64(s, &tot) + (tile_off ? tile_off[blockIdx.x] : 0);
+  uint64_t ex = block_excl_scan_u64(s, &tot) + before;
 #pragma unroll
   for (int q = 0; q < kScanItems; ++q) {
     tile[threadIdx.x * kScanItems + q] = ex;
@@ -104,14 +163,22 @@ __global__ __launch_bounds__(kBlock) void k_tile_scan(const TIn* in, Cnt cn,
    * the grand total at out[n] */
   const bool holds = (n >= base && n < base + kTile) ||
                      (blockIdx.x == gridDim.x - 1 && n == base + kTile);
-  if (holds && threadIdx.x == kBlock - 1) {
-    out[n] = (TOut)ex;
-    if (total64) *total64 = ex;
+  if (holds) { /* block-uniform */
+    if (threadIdx.x == kBlock - 1) {
+      out[n] = (TOut)ex;
+      if (total64) *total64 = ex;
+      s_total = ex;
+    }
+    if (post.box) {
+      __syncthreads();
+      if (threadIdx.x < 64) do_post(post, s_total);
+    }
   }
 }
 
 size_t scan_tmp_bytes(int64_t n) {
-  size_t b = 0;
+  /* (the offsets of up to kFlagFew tiles: see flag_tile_offsets) */
+  size_t b = (size_t)(64 + 1) * sizeof(uint64_t);
   int64_t m = n;
   while (m > kTile) {
     int64_t t = (m + kTile - 1) / kTile;
@@ -121,8 +188,16 @@ size_t scan_tmp_bytes(int64_t n) {
   return b + 256;
 }
 
+/* the scan of nothing: out[0] = 0 */
 template <class TOut>
-__global__ void k_store(TOut* out, TOut v) { *out = v; }
+__global__ __launch_bounds__(64) void k_scan_none(TOut* out, uint64_t* total64,
+                                                  Post post) {
+  if (threadIdx.x == 0) {
+    if (out) *out = 0;
+    if (total64) *total64 = 0;
+  }
+  if (post.box) do_post(post, 0);
+}
 
 /* Exclusive scan of up to kSumsMax tile sums by one block of 1024
  * threads (out[m] = total): each thread sums a run of consecutive values,
@@ -133,8 +208,10 @@ constexpr int64_t kSumsMax = (int64_t)kSumsBlock * 64;
 __global__ __launch_bounds__(kSumsBlock) void k_scan_sums(const uint64_t* in,
                                                           int64_t m,
                                                           uint64_t* out,
-                                                          uint64_t* total64) {
+                                                          uint64_t* total64,
+                                                          Post post) {
   __shared__ uint64_t wsum[kSumsBlock / 64];
+  __shared__ uint64_t s_total;
   const int per = (int)((m + kSumsBlock - 1) / kSumsBlock); /* <= 64 */
   const int64_t b = (int64_t)threadIdx.x * per;
   /* the run in batches of 16 values held in registers: a batch's loads
@@ -171,6 +248,11 @@ __global__ __launch_bounds__(kSumsBlock) void k_scan_sums(const uint64_t* in,
   if (threadIdx.x == kSumsBlock - 1) {
     out[m] = ex;
     if (total64) *total64 = ex;
+    s_total = ex;
+  }
+  if (post.box) {
+    __syncthreads();
+    if (threadIdx.x < 64) do_post(post, s_total);
   }
 }
 
@@ -180,32 +262,35 @@ static void scan_u64_rec(const uint64_t* in, uint64_t* out, int64_t n,
 
 template <class TIn, bool kFlag, class TOut = uint64_t>
 static void scan_impl(const TIn* in, TOut* out, Cnt n, uint64_t* tmp,
-                      hipStream_t s, uint64_t* total64 = nullptr) {
+                      hipStream_t s, uint64_t* total64 = nullptr,
+                      Post post = Post()) {
   if (n.cap <= 0) {
-    hipLaunchKernelGGL(k_store<TOut>, dim3(1), dim3(1), 0, s, out, (TOut)0);
-    if (total64)
-      hipLaunchKernelGGL(k_store<uint64_t>, dim3(1), dim3(1), 0, s, total64,
-                         (uint64_t)0);
+    hipLaunchKernelGGL(k_scan_none<TOut>, dim3(1), dim3(64), 0, s, out, total64,
+                       post);
     return;
   }
   int64_t tiles = (n.cap + kTile - 1) / kTile;
-  if (tiles == 1) {
-    hipLaunchKernelGGL((k_tile_scan<TIn, kFlag, TOut>), dim3(1), dim3(kBlock),
-                       0, s, in, n, (const uint64_t*)nullptr, out, total64);
+  if (tiles <= kFewTiles) {
+    hipLaunchKernelGGL((k_tile_scan<TIn, kFlag, TOut, true>),
+                       dim3((unsigned)tiles), dim3(kBlock), 0, s, in, n,
+                       (const uint64_t*)nullptr, out, total64, post);
     return;
   }
   uint64_t* sums = tmp;
   uint64_t* offs = tmp + (tiles + 1);
   hipLaunchKernelGGL((k_tile_sums<TIn, kFlag>), dim3((unsigned)tiles),
                      dim3(kBlock), 0, s, in, n, sums);
-  if (tiles <= kSumsMax) /* the tile sums in one block: three launches */
+  if (tiles <= kSumsMax) { /* the tile sums in one block: three launches */
     hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kSumsBlock), 0, s,
-                       (const uint64_t*)sums, tiles, offs, (uint64_t*)nullptr);
-  else
+                       (const uint64_t*)sums, tiles, offs, (uint64_t*)nullptr,
+                       post);
+    post = Post(); /* the total is known before the last launch */
+  } else {
     scan_u64_rec(sums, offs, tiles, tmp + 2 * (tiles + 1), s);
-  hipLaunchKernelGGL((k_tile_scan<TIn, kFlag, TOut>), dim3((unsigned)tiles),
-                     dim3(kBlock), 0, s, in, n, (const uint64_t*)offs, out,
-                     total64);
+  }
+  hipLaunchKernelGGL((k_tile_scan<TIn, kFlag, TOut, false>),
+                     dim3((unsigned)tiles), dim3(kBlock), 0, s, in, n,
+                     (const uint64_t*)offs, out, total64, post);
 }
 
 static void scan_u64_rec(const uint64_t* in, uint64_t* out, int64_t n,
@@ -214,12 +299,12 @@ static void scan_u64_rec(const uint64_t* in, uint64_t* out, int64_t n,
 }
 
 void scan_u32_to_u64(const uint32_t* in, uint64_t* out, Cnt n, void* tmp,
-                     size_t, hipStream_t s, uint64_t* total64) {
-  scan_impl<uint32_t, false>(in, out, n, (uint64_t*)tmp, s, total64);
+                     hipStream_t s, uint64_t* total64, Post post) {
+  scan_impl<uint32_t, false>(in, out, n, (uint64_t*)tmp, s, total64, post);
 }
 void scan_u64_to_u64(const uint64_t* in, uint64_t* out, Cnt n, void* tmp,
-                     size_t, hipStream_t s, uint64_t* total64) {
-  scan_impl<uint64_t, false>(in, out, n, (uint64_t*)tmp, s, total64);
+                     hipStream_t s, uint64_t* total64, Post post) {
+  scan_impl<uint64_t, false>(in, out, n, (uint64_t*)tmp, s, total64, post);
 }
 /* Flag scans (u8 flags, nonzero = 1 -> u32 positions), the scan every
  * compaction runs: a thread owns kScanItems (8) consecutive flags, read as
@@ -287,9 +372,10 @@ __global__ __launch_bounds__(kBlock) void k_flag_scan(const uint8_t* in, Cnt cn,
   }
 }
 void scan_u8flag_to_u32(const uint8_t* in, uint32_t* out, Cnt n, void* tmp,
-                        size_t, hipStream_t s, uint64_t* total64) {
+                        hipStream_t s, uint64_t* total64) {
   if (n.cap <= 0) {
-    scan_impl<uint8_t, true, uint32_t>(in, out, n, (uint64_t*)tmp, s, total64);
+    hipLaunchKernelGGL(k_scan_none<uint32_t>, dim3(1), dim3(64), 0, s, out,
+                       total64, Post());
     return;
   }
   const int64_t tiles = (n.cap + kTile - 1) / kTile;
@@ -305,7 +391,8 @@ void scan_u8flag_to_u32(const uint8_t* in, uint32_t* out, Cnt n, void* tmp,
                      n, sums);
   if (tiles <= kSumsMax)
     hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kSumsBlock), 0, s,
-                       (const uint64_t*)sums, tiles, offs, (uint64_t*)nullptr);
+                       (const uint64_t*)sums, tiles, offs, (uint64_t*)nullptr,
+                       Post());
   else
     scan_u64_rec(sums, offs, tiles, t + 2 * (tiles + 1), s);
   hipLaunchKernelGGL(k_flag_scan, dim3((unsigned)tiles), dim3(kBlock), 0, s, in,
@@ -319,15 +406,60 @@ void scan_u8flag_to_u32(const uint8_t* in, uint32_t* out, Cnt n, void* tmp,
  * k_flag_scan and write only the kept entries.  Against a position array
  * (k_flag_scan, then one thread per flag reading flag and position) this
  * writes and reads no 4 bytes per entry and launches 8x fewer waves. */
-__global__ void k_copy_u64(const uint64_t* src, uint64_t* dst) { *dst = *src; }
+__global__ __launch_bounds__(64) void k_copy_total(const uint64_t* src,
+                                                   uint64_t* dst, Post post) {
+  const uint64_t v = *src;
+  if (dst && threadIdx.x == 0) *dst = v;
+  if (post.box) do_post(post, v);
+}
+/* the same for at most kFlagFew tiles in one launch of one block: a wave
+ * sums a tile (32 flags a lane), the first wave scans the sums */
+constexpr int64_t kFlagFew = 64;
+__global__ __launch_bounds__(kSumsBlock) void k_flag_few(const uint8_t* in,
+                                                         Cnt cn, int tiles,
+                                                         uint64_t* offs,
+                                                         uint64_t* total64,
+                                                         Post post) {
+  __shared__ unsigned s_sum[kFlagFew];
+  const int64_t n = cn.get();
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  for (int t = w; t < tiles; t += kSumsBlock / 64) {
+    const int64_t i0 = (int64_t)t * kTile + lane * 8;
+    unsigned c = 0;
+#pragma unroll
+    for (int q = 0; q < kTile / 512; ++q) {
+      const uint2 f = load_flags8(in, i0 + q * 512, n);
+      c += nz_bytes(f.x) + nz_bytes(f.y);
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) c += (unsigned)__shfl_xor((int)c, d, 64);
+    if (lane == 0) s_sum[t] = c;
+  }
+  __syncthreads();
+  if (w != 0) return;
+  const uint64_t v = lane < tiles ? s_sum[lane] : 0u;
+  const uint64_t inc = wave_incl_scan_u64(v);
+  if (lane < tiles) offs[lane] = inc - v;
+  const uint64_t tot = __shfl(inc, 63, 64);
+  if (lane == 0) {
+    offs[tiles] = tot;
+    if (total64) *total64 = tot;
+  }
+  if (post.box) do_post(post, tot);
+}
 const uint64_t* flag_tile_offsets(const uint8_t* in, Cnt n, void* tmp,
-                                  hipStream_t s, uint64_t* total64) {
+                                  hipStream_t s, uint64_t* total64,
+                                  Post post) {
   uint64_t* t = (uint64_t*)tmp;
   const int64_t tiles = (n.cap + kTile - 1) / kTile;
   if (tiles <= 0) {
-    if (total64)
-      hipLaunchKernelGGL(k_store<uint64_t>, dim3(1), dim3(1), 0, s, total64,
-                         (uint64_t)0);
+    hipLaunchKernelGGL(k_scan_none<uint64_t>, dim3(1), dim3(64), 0, s,
+                       (uint64_t*)nullptr, total64, post);
+    return t;
+  }
+  if (tiles <= kFlagFew) {
+    hipLaunchKernelGGL(k_flag_few, dim3(1), dim3(kSumsBlock), 0, s, in, n,
+                       (int)tiles, t, total64, post);
     return t;
   }
   uint64_t* sums = t;
@@ -336,12 +468,11 @@ const uint64_t* flag_tile_offsets(const uint8_t* in, Cnt n, void* tmp,
                      n, sums);
   if (tiles <= kSumsMax) {
     hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kSumsBlock), 0, s,
-                       (const uint64_t*)sums, tiles, offs, total64);
+                       (const uint64_t*)sums, tiles, offs, total64, post);
   } else {
     scan_u64_rec(sums, offs, tiles, t + 2 * (tiles + 1), s);
-    if (total64)
-      hipLaunchKernelGGL(k_copy_u64, dim3(1), dim3(1), 0, s,
-                         (const uint64_t*)(offs + tiles), total64);
+    hipLaunchKernelGGL(k_copy_total, dim3(1), dim3(64), 0, s,
+                       (const uint64_t*)(offs + tiles), total64, post);
   }
   return offs;
 }
@@ -528,86 +659,67 @@ void radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
 /* ------------------------------------------------------------------ */
 /* recorded (fixed-capacity) pipelines                                 */
 /* ------------------------------------------------------------------ */
-/* Consumer view of QSLOTS sub-queues from their counters; a counter past
- * the capacity (entries were dropped) sets `bit` in *status and the
- * largest counter goes to *fill (fresh: both overwritten and fill[1]
- * cleared, for the ladder's second view; else merged).
- * The counters it read, and (lists, the word of the QK_REST counters) the
- * two lists' counters, are cleared for the next producer, so no separate
- * zeroing launch precedes a ladder.  One wave, lane k for slot k. */
-__global__ __launch_bounds__(64) void k_make_view(const QEntry* q, uint32_t cap,
-                                                  unsigned* cnt, QView* v,
-                                                  unsigned* status,
-                                                  unsigned bit, unsigned* fill,
-                                                  unsigned* lists, int fresh) {
+/* The end of a recorded ladder, one wave, lane k for slot k: the largest
+ * fills, overflows (counters past the capacity: entries were dropped) into
+ * the status, every counter cleared for the next ladder. */
+__global__ __launch_bounds__(64) void k_ladder_rec(unsigned* qn, uint32_t c1,
+                                                   uint32_t c2,
+                                                   unsigned* status,
+                                                   unsigned* fill) {
   const int k = threadIdx.x;
-  const bool slot = k < QSLOTS;
-  const unsigned c = slot ? cnt[k * kSlotWords] : 0u;
-  if (slot) {
-    cnt[k * kSlotWords] = 0;
-    if (lists) {
-      lists[k * kSlotWords] = 0;
-      lists[k * kSlotWords + QK_NEXT - QK_REST] = 0;
-    }
+  unsigned f1 = 0, f2 = 0;
+  if (k < QSLOTS) {
+    unsigned* const line = qn + k * kSlotWords;
+    f1 = line[QK_HOT];
+    f2 = line[QK_ESC];
+    line[QK_HOT] = 0;
+    line[QK_ESC] = 0;
+    line[QK_REST] = 0;
+    line[QK_NEXT] = 0;
   }
-  unsigned mx = c;
 #pragma unroll
-  for (int d = 32; d >= 1; d >>= 1)
-    mx = max(mx, (unsigned)__shfl_xor((int)mx, d, 64));
-  /* an eager ladder's first view (fresh) is empty when its queue
-   * overflowed: the ladder runs again with a larger queue, and its
-   * consumers need not work through the partial one */
-  const uint32_t n = fresh && mx > cap ? 0u : (c < cap ? c : cap);
-  uint32_t incl = n;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t y = (uint32_t)__shfl_up((int)incl, d, 64);
-    if (k >= d) incl += y;
+  for (int d = 32; d >= 1; d >>= 1) {
+    f1 = max(f1, (unsigned)__shfl_xor((int)f1, d, 64));
+    f2 = max(f2, (unsigned)__shfl_xor((int)f2, d, 64));
   }
-  if (slot) v->off[k + 1] = incl;
   if (k == 0) {
-    v->off[0] = 0;
-    v->q = q;
-    v->cap = cap;
-    const unsigned b = mx > cap ? bit : 0u;
-    if (fresh) { /* first view of a ladder: also resets the second's fill */
-      fill[0] = mx;
-      fill[1] = 0;
-      *status = b;
-    } else {
-      atomicMax(fill, mx);
-      if (b) atomicOr(status, b);
-    }
+    if (f1 > fill[0]) fill[0] = f1;
+    if (f2 > fill[1]) fill[1] = f2;
+    const unsigned b = (f1 > c1 ? 1u << REC_Q1 : 0u) |
+                       (f2 > c2 ? 1u << REC_Q2 : 0u);
+    if (b) atomicOr(status, b);
   }
 }
-void launch_make_view(const QEntry* q, uint32_t cap, unsigned* cnt, QView* v,
-                      unsigned* status, unsigned bit, unsigned* fill,
-                      unsigned* lists, bool fresh, hipStream_t s) {
-  hipLaunchKernelGGL(k_make_view, dim3(1), dim3(64), 0, s, q, cap, cnt, v,
-                     status, bit, fill, lists, (int)fresh);
+void launch_ladder_rec(unsigned* qn, uint32_t c1, uint32_t c2, unsigned* status,
+                       unsigned* fill, hipStream_t s) {
+  hipLaunchKernelGGL(k_ladder_rec, dim3(1), dim3(64), 0, s, qn, c1, c2, status,
+                     fill);
 }
 
-/* An eager ladder's state in one buffer for one read-back: the
- * sub-queue counts of its last queue and its count, beside the status and
- * fill its first view left.  The queue's counters and (lists, the word of
- * the QK_REST counters) the two lists' are cleared for the next ladder. */
-__global__ __launch_bounds__(64) void k_ladder_state(unsigned* cnt,
-                                                     unsigned* lists,
-                                                     const uint64_t* count,
-                                                     unsigned* lad) {
-  const int k = threadIdx.x;
-  if (k < QSLOTS) {
-    lad[kLadCnt + k] = cnt[k * kSlotWords];
-    cnt[k * kSlotWords] = 0;
-    lists[k * kSlotWords] = 0;
-    lists[k * kSlotWords + QK_NEXT - QK_REST] = 0;
+/* A run's statistics: one block, a thread per counter copy's word. */
+__global__ __launch_bounds__(kSumsBlock) void k_post_stats(
+    const unsigned long long* ctr, const unsigned long long* ts, Post post) {
+  __shared__ unsigned long long s_v[CTR_SLOTS][CTR_COUNT];
+  static_assert(CTR_SLOTS * CTR_COUNT == kSumsBlock, "a thread per word");
+  s_v[threadIdx.x / CTR_COUNT][threadIdx.x % CTR_COUNT] = ctr[threadIdx.x];
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  const int c = threadIdx.x;
+  unsigned long long* const out =
+      reinterpret_cast<unsigned long long*>(post.box + kBoxData);
+  if (c < CTR_COUNT) {
+    unsigned long long v = 0;
+    for (int k = 0; k < CTR_SLOTS; ++k) v += s_v[k][c];
+    out[c] = v;
   }
-  if (k == 0) *reinterpret_cast<uint64_t*>(lad + kLadCount) = *count;
+  if (c < kStamps)
+    out[CTR_COUNT + c] = c == kStamps - 1 ? wall_clock64() : ts[c];
+  do_post(post, 0);
 }
-void launch_ladder_state(unsigned* cnt, unsigned* lists, const uint64_t* count,
-                         unsigned* lad, hipStream_t s) {
-  hipLaunchKernelGGL(k_ladder_state, dim3(1), dim3(64), 0, s, cnt, lists, count,
-                     lad);
+void launch_post_stats(const unsigned long long* ctr,
+                       const unsigned long long* ts, Post post, hipStream_t s) {
+  hipLaunchKernelGGL(k_post_stats, dim3(1), dim3(kSumsBlock), 0, s, ctr, ts,
+                     post);
 }
 
 __global__ void k_zero_counter(unsigned long long* ctr, int idx) {
@@ -615,15 +727,6 @@ __global__ void k_zero_counter(unsigned long long* ctr, int idx) {
 }
 void zero_counter(unsigned long long* ctr, int idx, hipStream_t s) {
   hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, ctr, idx);
-}
-
-__global__ void k_cap_check(const uint64_t* v, uint64_t cap, unsigned* status,
-                            unsigned bit) {
-  if (threadIdx.x == 0 && *v > cap) atomicOr(status, bit);
-}
-void launch_cap_check(const uint64_t* v, uint64_t cap, unsigned* status,
-                      unsigned bit, hipStream_t s) {
-  hipLaunchKernelGGL(k_cap_check, dim3(1), dim3(64), 0, s, v, cap, status, bit);
 }
 
 /* bounds of the current input against those the pipeline was planned for:

@@ -168,6 +168,10 @@ struct StageCnt {
   }
 };
 
+/* a phase's time stamp, by the first thread of its first kernel */
+__device__ __forceinline__ void stamp(unsigned long long* ts, int k) {
+  if (ts && blockIdx.x == 0 && threadIdx.x == 0) ts[k] = wall_clock64();
+}
 __device__ __forceinline__ int64_t gtid() {
   return (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
 }
@@ -208,11 +212,50 @@ __device__ __forceinline__ bool live_entry(const QEntry& e,
   return e.aux == 0xffffffffu || flag[e.item] != 0;
 }
 
+/* A consumer block's view of a queue: the sub-queues end to end, their
+ * starts in LDS (s_off, QSLOTS + 1 words), from the host's view or from the
+ * queue's counters.  Every thread of the block must call q_table. */
+struct QTab {
+  const QEntry* q;
+  uint32_t cap;
+  const uint32_t* off;
+  __device__ uint32_t size() const { return off[QSLOTS]; }
+  __device__ QEntry at(uint32_t i) const {
+    int lo = 0, hi = QSLOTS - 1; /* last k with off[k] <= i */
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (off[mid] <= i) lo = mid;
+      else hi = mid - 1;
+    }
+    return q[(uint64_t)lo * cap + (i - off[lo])];
+  }
+};
+__device__ __forceinline__ QTab q_table(const QRef& r, uint32_t* s_off) {
+  if (threadIdx.x < 64) {
+    const int k = threadIdx.x;
+    if (r.cnt) {
+      const unsigned c = k < QSLOTS ? r.cnt[k * kSlotWords] : 0u;
+      const bool over = __ballot(c > r.v.cap) != 0;
+      uint32_t incl = over && r.drop ? 0u : min(c, r.v.cap);
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)incl, d, 64);
+        if (k >= d) incl += y;
+      }
+      if (k < QSLOTS) s_off[k + 1] = incl;
+      if (k == 0) s_off[0] = 0;
+    } else if (k <= QSLOTS) {
+      s_off[k] = r.v.off[k];
+    }
+  }
+  __syncthreads();
+  return QTab{r.v.q, r.v.cap, s_off};
+}
 /* Entries of a queue for its consumer kernel: thread t takes entry t,
  * then t + grid, ... (a host view's grid covers its entries; a device
- * view's is at most a few hundred blocks). */
+ * queue's is at most a few hundred blocks). */
 template <class F>
-__device__ __forceinline__ void for_queue(const QRef& q, F&& body) {
+__device__ __forceinline__ void for_queue(const QTab& q, F&& body) {
   const uint32_t n = q.size();
   const uint32_t grid = gridDim.x * blockDim.x;
   const uint32_t t0 = (uint32_t)gtid();

@@ -4,9 +4,9 @@
  *
  * Replaces the reference's main() phase sequence (AlphaComplexParallel.cu:
  * 1126-1806): one HIP stream per call, device-resident intermediates taken
- * from a caching pool (no hipMalloc in steady state), counts read back
- * between stages only where a buffer must be sized, hipEvents around the
- * reference's eight phases.  Errors are returned as status codes, never
+ * from a caching pool (no hipMalloc in steady state), counts posted by the
+ * kernels between stages only where a buffer must be sized, time stamps by
+ * the first kernel of each of the reference's eight phases.  Errors are returned as status codes, never
  * printed (the reference prints and continues: :55-61).
  */
 #include <hip/hip_runtime.h>
@@ -55,7 +55,13 @@ Engine* engine_for(int dev) {
   Engine* e = new Engine();
   e->device = dev;
   HIPCHK(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
-  HIPCHK(hipHostMalloc(&e->pinned, 4096, hipHostMallocDefault));
+  HIPCHK(hipHostMalloc((void**)&e->box, kBoxWords * sizeof(unsigned),
+                       hipHostMallocMapped | hipHostMallocCoherent));
+  std::memset(e->box, 0, kBoxWords * sizeof(unsigned));
+  int khz = 0;
+  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) ==
+          hipSuccess && khz > 0)
+    e->clock_khz = khz;
   g_engines[dev] = e;
   return e;
 }
@@ -89,41 +95,27 @@ void zero_u64(unsigned long long* p, int64_t n, hipStream_t s) {
 }  // namespace pac
 
 
-/* copy raw input with solvent-added radii, original order (kept for rho /
- * adjoint queries) */
-__device__ __forceinline__ double add_r_orig(float a, float s) {
-  return (double)__fadd_rn(a, s);
-}
-__device__ __forceinline__ double add_r_orig(double a, double s) { return a + s; }
-template <class B, class R>
-__global__ void k_balls_orig(const B* raw, int64_t n, R solvent, double4* out) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  B a = raw[i];
-  out[i] = make_double4(a.x, a.y, a.z, add_r_orig(a.w, solvent));
-}
-
 static void run_variant(Engine* E, const float4* raw, int64_t n, float solvent,
                         float alpha, const pac_options& opt, pac_result* R,
-                        hipStream_t s, Timer& T, KProf& KP) {
-  vf32::run_pipeline(E, raw, n, solvent, alpha, opt, R, s, T, KP);
+                        hipStream_t s, KProf& KP) {
+  vf32::run_pipeline(E, raw, n, solvent, alpha, opt, R, s, KP);
 }
 static void run_variant(Engine* E, const double4* raw, int64_t n,
                         double solvent, double alpha, const pac_options& opt,
-                        pac_result* R, hipStream_t s, Timer& T, KProf& KP) {
-  vf64::run_pipeline(E, raw, n, solvent, alpha, opt, R, s, T, KP);
+                        pac_result* R, hipStream_t s, KProf& KP) {
+  vf64::run_pipeline(E, raw, n, solvent, alpha, opt, R, s, KP);
 }
 static void run_chunked_variant(Engine* E, const float4* raw, int64_t n,
                                 float solvent, float alpha,
                                 const pac_options& opt, pac_result* R,
-                                hipStream_t s, Timer& T, KProf& KP) {
-  vf32::run_chunked(E, raw, n, solvent, alpha, opt, R, s, T, KP);
+                                hipStream_t s, KProf& KP) {
+  vf32::run_chunked(E, raw, n, solvent, alpha, opt, R, s, KP);
 }
 static void run_chunked_variant(Engine* E, const double4* raw, int64_t n,
                                 double solvent, double alpha,
                                 const pac_options& opt, pac_result* R,
-                                hipStream_t s, Timer& T, KProf& KP) {
-  vf64::run_chunked(E, raw, n, solvent, alpha, opt, R, s, T, KP);
+                                hipStream_t s, KProf& KP) {
+  vf64::run_chunked(E, raw, n, solvent, alpha, opt, R, s, KP);
 }
 
 /* canonical order: vertices of each row by original id, rows lexicographic */
@@ -145,8 +137,16 @@ static void canonicalize(Engine* E, pac_result* R, int64_t n, hipStream_t s) {
   }
 }
 
-static void fill_phase_ms(Timer& T, pac_stats& st) {
-  for (int q = 0; q < 8; ++q) st.phase_ms[q] = T.ms(q, q + 1);
+/* runs f; should it throw, waits for the kernels it left in flight before
+ * anyone can take their buffers (the caller holds the engine's lock) */
+template <class F>
+static void drained(hipStream_t s, F&& f) {
+  try {
+    f();
+  } catch (...) {
+    (void)hipStreamSynchronize(s);
+    throw;
+  }
 }
 
 /* one molecule; F is float (FP32 balls, the reference's input) or double
@@ -177,12 +177,14 @@ static void compute_one(const F* xyzr, int64_t n, F solvent, F alpha,
   R->filt = opt.filtration != 0;
   std::memset(&R->st, 0, sizeof(R->st));
   R->counts[0] = n;
-  Timer T(s);
   KProf KP;
   KP.on = opt.profile != 0;
   KP.s = s;
-  T.mark(0);
-  auto t_host0 = std::chrono::steady_clock::now();
+  using clk = std::chrono::steady_clock;
+  auto since = [](clk::time_point t) {
+    return std::chrono::duration<double, std::milli>(clk::now() - t).count();
+  };
+  const auto t_host0 = clk::now();
   DBuf<B> raw_own;
   const B* raw = (const B*)xyzr;
   if (n > 0 && !opt.device_inputs) {
@@ -191,27 +193,23 @@ static void compute_one(const F* xyzr, int64_t n, F solvent, F alpha,
                           hipMemcpyHostToDevice, s));
     raw = raw_own.get();
   }
-  T.mark(1);
+  const double t_in = since(t_host0);
   if (n > 0) {
+    /* filled by the run's first kernel, or here for a chunked one */
     R->balls = DBuf<double4>(&E->pool, n);
-    hipLaunchKernelGGL((k_balls_orig<B, F>), dim3((unsigned)((n + 255) / 256)),
-                       dim3(256), 0, s, raw, n, solvent, R->balls.get());
-    KCHK();
-    if (opt.chunk_balls > 0)
-      run_chunked_variant(E, raw, n, solvent, alpha, opt, R.get(), s, T, KP);
-    else
-      run_variant(E, raw, n, solvent, alpha, opt, R.get(), s, T, KP);
-    if (opt.order == PAC_ORDER_CANONICAL) canonicalize(E, R.get(), n, s);
-  } else {
-    for (int i = 2; i <= 8; ++i) T.mark(i);
+    drained(s, [&] {
+      if (opt.chunk_balls > 0)
+        run_chunked_variant(E, raw, n, solvent, alpha, opt, R.get(), s, KP);
+      else
+        run_variant(E, raw, n, solvent, alpha, opt, R.get(), s, KP);
+      if (opt.order == PAC_ORDER_CANONICAL) canonicalize(E, R.get(), n, s);
+    });
   }
   HIPCHK(hipStreamSynchronize(s));
-  auto t_host1 = std::chrono::steady_clock::now();
   pac_stats& st = R->st;
-  fill_phase_ms(T, st);
   for (int q = 0; q < 8; ++q) st.phase_ms[q] += R->phase_add[q];
-  st.total_ms =
-      std::chrono::duration<double, std::milli>(t_host1 - t_host0).count();
+  st.phase_ms[0] += t_in;
+  st.total_ms = since(t_host0);
   KP.collect(st.kernel_ms);
   *out = R.release();
 }
@@ -372,19 +370,15 @@ void pac::compute_batch(const float* xyzr, const int64_t* offsets,
     R->alpha = alpha;
     std::memset(&R->st, 0, sizeof(R->st));
     R->counts[0] = gn;
-    Timer T(s);
     KProf KP;
     KP.on = opt.profile != 0;
     KP.s = s;
-    T.mark(0);
-    T.mark(1);
-    if (gn > 0) {
-      vf32::run_pipeline(E, raw + b0, gn, solvent, alpha, opt, R.get(), s, T, KP,
-                   rel.data(), gm);
-      if (opt.order == PAC_ORDER_CANONICAL) canonicalize(E, R.get(), gn, s);
-    } else {
-      for (int i = 2; i <= 8; ++i) T.mark(i);
-    }
+    if (gn > 0)
+      drained(s, [&] {
+        vf32::run_pipeline(E, raw + b0, gn, solvent, alpha, opt, R.get(), s, KP,
+                           rel.data(), gm);
+        if (opt.order == PAC_ORDER_CANONICAL) canonicalize(E, R.get(), gn, s);
+      });
     /* per-molecule row ranges of the group's lists */
     if (gm == 1) {
       for (int d = 1; d <= 3; ++d) B->row0[d - 1][m0] = 0;
@@ -416,7 +410,6 @@ void pac::compute_batch(const float* xyzr, const int64_t* offsets,
       B->mol_group[m0 + q] = (int32_t)B->groups.size();
     }
     HIPCHK(hipStreamSynchronize(s));
-    fill_phase_ms(T, R->st);
     KP.collect(R->st.kernel_ms);
     add_stats(B->st, R->st);
     B->group_first.push_back(m0);
@@ -617,7 +610,6 @@ static void compute_noalloc(const float* xyzr, int64_t n, float solvent,
   R.alpha = alpha;
   std::memset(&R.st, 0, sizeof(R.st));
   R.counts[0] = n;
-  Timer T(s, false);
   KProf KP;
   DBuf<float4> raw_own;
   const float4* raw = (const float4*)xyzr;
@@ -627,7 +619,7 @@ static void compute_noalloc(const float* xyzr, int64_t n, float solvent,
                           hipMemcpyHostToDevice, s));
     raw = raw_own.get();
   }
-  run_variant(E, raw, n, solvent, alpha, opt, &R, s, T, KP);
+  run_variant(E, raw, n, solvent, alpha, opt, &R, s, KP);
   if (opt.order == PAC_ORDER_CANONICAL) canonicalize(E, &R, n, s);
   bool over = false;
   for (int d = 1; d <= 3; ++d) {

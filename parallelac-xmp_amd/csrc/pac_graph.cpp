@@ -64,7 +64,6 @@ struct pac_graph {
   DBuf<unsigned> status;         /* [0] REC_* bits, [1..2] largest fills */
   DBuf<unsigned long long> ctr;
   DBuf<unsigned> qn;
-  DBuf<QView> views;
   DBuf<QEntry> q1, q2;
   uint32_t c1 = 0, c2 = 0;
   hipGraph_t graph = nullptr;
@@ -85,7 +84,6 @@ struct pac_graph {
     status.release();
     ctr.release();
     qn.release();
-    views.release();
     q1.release();
     q2.release();
     pool.trim();
@@ -106,10 +104,8 @@ int64_t with_headroom(int64_t v, double h) {
 void record_all(pac_graph* G) {
   hipStream_t s = G->s;
   zero_u32(G->status.get(), 4, s);
-  zero_u32(G->qn.get(), QN_WORDS, s); /* then kept clear by the views */
+  zero_u32(G->qn.get(), QN_WORDS, s); /* then kept clear by the ladders */
   zero_u64(G->ctr.get(), CTR_COUNT * CTR_SLOTS, s);
-  Timer T(s);
-  T.on = false;
   KProf KP;
   for (auto& pp : G->passes) {
     GPass& p = *pp;
@@ -130,13 +126,12 @@ void record_all(pac_graph* G) {
     rec.fill = G->status.get() + 1;
     rec.ctr = G->ctr.get();
     rec.qn = G->qn.get();
-    rec.views = G->views.get();
     rec.q1 = G->q1.get();
     rec.q2 = G->q2.get();
     rec.c1 = G->c1;
     rec.c2 = G->c2;
     vf32::run_pipeline(G->E, G->raw + p.b0, p.gn, G->solvent, G->alpha,
-                       G->opt, p.R.get(), s, T, KP, p.rel.data(), p.gm, &rec);
+                       G->opt, p.R.get(), s, KP, p.rel.data(), p.gm, &rec);
     static const int fin[3] = {RC_EF, RC_TF, RC_KF};
     for (int d = 1; d <= 3; ++d)
       launch_mol_rows(p.R->lists[d - 1].get(),
@@ -162,14 +157,17 @@ void check_status(pac_graph* G, const char* when) {
     fail(PAC_ERR_OVERFLOW, w + "escalation queue overflow (" +
                                std::to_string(h[2]) + " of " +
                                std::to_string(G->c2) + "); record again");
+}
+
+/* a pass's counts against its capacities (an excess entry was dropped) */
+void check_counts(const GPass& p, const uint64_t* h, const char* when) {
   static const char* names[RC_COUNT] = {
       "edge candidates", "alpha edges", "triangle slots", "alpha triangles",
       "tet slots", "alpha tets", "final tets", "final triangles", "final edges"};
   for (int q = 0; q < RC_COUNT; ++q)
-    if (h[0] & (1u << (REC_CAP + q)))
-      fail(PAC_ERR_OVERFLOW, w + std::string(names[q]) +
+    if ((int64_t)h[q] > p.cap[q])
+      fail(PAC_ERR_OVERFLOW, std::string(when) + ": " + names[q] +
                                  " exceed the recorded capacity; record again");
-  fail(PAC_ERR_OVERFLOW, w + "recorded capacity exceeded");
 }
 
 void graph_create(const float* xyzr, const int64_t* offsets, int64_t nmol,
@@ -277,7 +275,6 @@ void graph_create(const float* xyzr, const int64_t* offsets, int64_t nmol,
   G->status = DBuf<unsigned>(&G->pool, 4);
   G->ctr = DBuf<unsigned long long>(&G->pool, CTR_COUNT * CTR_SLOTS);
   G->qn = DBuf<unsigned>(&G->pool, QN_WORDS);
-  G->views = DBuf<QView>(&G->pool, 2);
   G->q1 = DBuf<QEntry>(&G->pool, (size_t)G->c1 * QSLOTS);
   G->q2 = DBuf<QEntry>(&G->pool, (size_t)G->c2 * QSLOTS);
 
@@ -291,6 +288,7 @@ void graph_create(const float* xyzr, const int64_t* offsets, int64_t nmol,
     if (p.gn == 0) continue;
     uint64_t h[RC_COUNT];
     HIPCHK(hipMemcpy(h, p.dcnt.get(), sizeof(h), hipMemcpyDeviceToHost));
+    check_counts(p, h, "recorded run");
     for (int q = 0; q < RC_COUNT; ++q)
       if ((int64_t)h[q] != p.probe[q])
         fail(PAC_ERR_DEVICE, "recorded run count " + std::to_string(q) + " = " +
@@ -373,6 +371,7 @@ void graph_result(pac_graph* G, pac_batch_result** out) {
     if (p.gn > 0) {
       uint64_t h[RC_COUNT];
       HIPCHK(hipMemcpy(h, p.dcnt.get(), sizeof(h), hipMemcpyDeviceToHost));
+      check_counts(p, h, "graph launch");
       HIPCHK(hipMemcpy(hr.data(), p.rows.get(), hr.size() * sizeof(uint64_t),
                        hipMemcpyDeviceToHost));
       static const int fin[3] = {RC_EF, RC_TF, RC_KF};
@@ -419,6 +418,8 @@ void graph_result(pac_graph* G, pac_batch_result** out) {
   HIPCHK(hipMemcpyAsync(hs.data(), G->ctr.get(), hs.size() * sizeof(hs[0]),
                         hipMemcpyDeviceToHost, G->s));
   HIPCHK(hipStreamSynchronize(G->s));
+  for (int k = 1; k < CTR_SLOTS; ++k) /* the copies' sums, in the first */
+    for (int c = 0; c < CTR_COUNT; ++c) hs[c] += hs[k * CTR_COUNT + c];
   stats_from_counters(hs.data(), G->opt.precision == PAC_PREC_STAGED, ecand,
                       B->st);
   float ms = 0;

@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -165,7 +166,34 @@ struct Engine {
   hipStream_t stream = nullptr;
   Pool pool;
   std::mutex run_mu;
-  void* pinned = nullptr; /* small pinned staging for scalar read-backs */
+  /* pinned, host-coherent words that kernels post small results to, and the
+   * last ticket given out (Post; one run at a time, under run_mu) */
+  unsigned* box = nullptr;
+  unsigned long long ticket = 0;
+  double clock_khz = 1e5; /* rate of the device's wall clock (time stamps) */
+  Post post(unsigned* qn = nullptr) { return Post{box, ++ticket, qn}; }
+  /* waits for the post: spins on its ticket (a few microseconds, while the
+   * kernels before it run), then, should it take long, in the runtime, which
+   * also reports a failed stream */
+  void wait(const Post& p, hipStream_t s) const {
+    const unsigned long long* t = (const unsigned long long*)(box + kBoxTicket);
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int k = 0;; ++k) {
+      if (__atomic_load_n(t, __ATOMIC_ACQUIRE) == p.ticket) return;
+      if ((k & 255) == 255 &&
+          std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2))
+        break;
+      __builtin_ia32_pause();
+    }
+    HIPCHK(hipStreamSynchronize(s));
+    if (__atomic_load_n(t, __ATOMIC_ACQUIRE) != p.ticket)
+      fail(PAC_ERR_DEVICE, "internal: a post is missing");
+  }
+  uint64_t posted_count() const {
+    uint64_t v;
+    std::memcpy(&v, box + kBoxCount, sizeof(v));
+    return v;
+  }
   /* the allocation-free entry point: the device's scratch array (its
    * address on this device) as an arena, and the pool a run takes its
    * buffers from while it holds run_mu (NULL: `pool`) */
@@ -286,28 +314,18 @@ inline int neg_lsb_exp_host(double v) {
   return lsb < 0 ? -lsb : 0;
 }
 
+/* hipEvents around the parts of a chunk outside its pipeline run */
 struct Timer {
-  hipEvent_t ev[10];
-  int used = 0;
+  hipEvent_t ev[4];
   hipStream_t s;
-  bool on = true; /* off: marks are skipped (recorded pipelines) */
-  bool made = true;
-  /* events = false: no events are created, marks are skipped and every
-   * phase reads 0 (the allocation-free entry point) */
-  explicit Timer(hipStream_t st, bool events = true)
-      : s(st), on(events), made(events) {
-    if (on)
-      for (auto& e : ev) HIPCHK(hipEventCreate(&e));
+  explicit Timer(hipStream_t st) : s(st) {
+    for (auto& e : ev) HIPCHK(hipEventCreate(&e));
   }
   ~Timer() {
-    if (made)
-      for (auto& e : ev) (void)hipEventDestroy(e);
+    for (auto& e : ev) (void)hipEventDestroy(e);
   }
-  void mark(int i) {
-    if (on) HIPCHK(hipEventRecord(ev[i], s));
-  }
+  void mark(int i) { HIPCHK(hipEventRecord(ev[i], s)); }
   double ms(int a, int b) {
-    if (!made) return 0.0;
     float t = 0;
     HIPCHK(hipEventElapsedTime(&t, ev[a], ev[b]));
     return t;
@@ -351,27 +369,11 @@ struct KProf {
 enum { KP_EDGE_FILL, KP_TRI_FILL, KP_TET_FILL, KP_TET_AC2, KP_TRI_AC2,
        KP_EDGE_AC2, KP_SORT, KP_TET_AC2_EXACT };
 
-template <class T>
-inline T readback(Engine* E, hipStream_t s, const T* dptr) {
-  HIPCHK(hipMemcpyAsync(E->pinned, dptr, sizeof(T), hipMemcpyDeviceToHost, s));
-  HIPCHK(hipStreamSynchronize(s));
-  T v;
-  std::memcpy(&v, E->pinned, sizeof(T));
-  return v;
-}
-
-/* Statistics from the device counters (CTR_*, CTR_SLOTS copies each):
- * evaluations per precision stage of each family, SoS calls, emptiness
- * pairs.  Hot-stage evaluations of the filters are one per candidate (the
- * edge candidates are counted on the host, the others on the device);
- * those of the emptiness scans one per (simplex, ball) pair.  Adds to st. */
-inline void stats_from_counters(const unsigned long long* hs, bool staged,
+/* Statistics from the counters' sums (CTR_*): stage evaluations, candidate
+ * counts (`edge_candidates`: the hot edge filter's evaluations, booked on
+ * the host), alpha tets not listed, pair counts, SoS calls; added to `st`. */
+inline void stats_from_counters(const unsigned long long* h, bool staged,
                                 int64_t edge_candidates, pac_stats& st) {
-  unsigned long long h[CTR_COUNT];
-  for (int c = 0; c < CTR_COUNT; ++c) {
-    h[c] = 0;
-    for (int k = 0; k < CTR_SLOTS; ++k) h[c] += hs[k * CTR_COUNT + c];
-  }
   for (int f = 0; f < 6; ++f)
     for (int q = 0; q < 4; ++q)
       st.stage_evals[f][q] += (int64_t)h[CTR_STAGE + 4 * f + q];
@@ -391,7 +393,8 @@ inline void stats_from_counters(const unsigned long long* hs, bool staged,
 
 
 /* One pipeline pass recorded with fixed capacities (for capture into a
- * graph): nothing is read back, every count stays on the device, and
+ * graph): nothing is read back, every count stays on the device (whoever
+ * launches compares them with the capacities afterwards), and queue
  * overflows or a stale plan set status bits (REC_*). */
 enum { RC_ECAND, RC_EALPHA, RC_TSLOTS, RC_TALPHA, RC_KSLOTS, RC_KALPHA,
        RC_KF, RC_TF, RC_EF, RC_COUNT };
@@ -406,7 +409,6 @@ struct PassRec {
   unsigned* fill;          /* device [2]: largest sub-queue fills */
   unsigned long long* ctr; /* device counters (shared by the passes) */
   unsigned* qn;            /* device [QN_WORDS] queue counters */
-  QView* views;            /* device [2] */
   QEntry *q1, *q2;         /* hot / escalation queues */
   uint32_t c1, c2;         /* their sub-queue capacities */
 };
@@ -417,6 +419,14 @@ struct PassRec {
 struct SubInput {
   Bounds grid;
   uint32_t own_lo, own_hi;
+};
+
+/* what a run's first kernel does beside the bounds: the control words it
+ * clears and (one molecule) the balls it keeps for the result */
+struct RunCtl {
+  unsigned long long* p = nullptr;
+  int words = 0;
+  double4* orig = nullptr;
 };
 
 namespace PAC_V {
@@ -439,31 +449,32 @@ struct PassPlan {
 void plan_pass(Engine* E, const Ball* raw, int64_t n, Real solvent,
                Real alpha, const pac_options& opt, hipStream_t s,
                const int64_t* moff, int64_t nmol, PassPlan& pl,
-               const Bounds* gridb = nullptr);
+               const Bounds* gridb = nullptr,
+               const RunCtl* ctl = nullptr);
 }  // namespace PAC_V
 namespace vf32 {
 void run_pipeline(Engine* E, const float4* raw, int64_t n, float solvent,
                   float alpha, const pac_options& opt, pac_result* R,
-                  hipStream_t s, Timer& T, KProf& KP,
+                  hipStream_t s, KProf& KP,
                   const int64_t* moff = nullptr, int64_t nmol = 1,
                   const PassRec* rec = nullptr,
                   const SubInput* sub = nullptr);
 /* the chunked (LD) driver over opt.chunk_balls */
 void run_chunked(Engine* E, const float4* raw, int64_t n, float solvent,
                  float alpha, const pac_options& opt, pac_result* R,
-                 hipStream_t s, Timer& T, KProf& KP);
+                 hipStream_t s, KProf& KP);
 }
 namespace vf64 {
 void run_pipeline(Engine* E, const double4* raw, int64_t n, double solvent,
                   double alpha, const pac_options& opt, pac_result* R,
-                  hipStream_t s, Timer& T, KProf& KP,
+                  hipStream_t s, KProf& KP,
                   const int64_t* moff = nullptr, int64_t nmol = 1,
                   const PassRec* rec = nullptr,
                   const SubInput* sub = nullptr);
 /* the chunked (LD) driver over opt.chunk_balls */
 void run_chunked(Engine* E, const double4* raw, int64_t n, double solvent,
                  double alpha, const pac_options& opt, pac_result* R,
-                 hipStream_t s, Timer& T, KProf& KP);
+                 hipStream_t s, KProf& KP);
 }
 
 }  // namespace pac

@@ -88,24 +88,43 @@ constexpr int CTR_SLOTS = 32;
 enum { FAM_EDGE = 0, FAM_TRI = 1, FAM_TET = 2, FAM_TET_AC2 = 3,
        FAM_TRI_AC2 = 4, FAM_EDGE_AC2 = 5 };
 
+/* ---- posts: small results to the host without a copy ----
+ * The last kernel of a stage writes what the host needs next straight into
+ * the engine's pinned, host-coherent box and then, released to the system,
+ * its ticket; the host spins on the ticket (Engine::wait).  A read-back
+ * through a copy and a stream synchronisation left the GPU idle for ~20 us
+ * (copy kernel, completion signal, wake-up), a post for ~8.
+ * Box words: the ticket (u64), the count (u64), the sub-queue fills of the
+ * hot and of the escalation queue (QSLOTS each), then kBoxData words of
+ * data (bounds, statistics). */
+struct Post {
+  unsigned* box = nullptr; /* null: nothing is posted */
+  unsigned long long ticket = 0;
+  unsigned* qn = nullptr; /* a ladder's last post: its queue counters, which
+                             are read, then cleared for the next ladder */
+};
+constexpr int kBoxTicket = 0, kBoxCount = 2, kBoxQ1 = 4, kBoxQ2 = 36,
+              kBoxData = 128, kBoxWords = 2048;
+
 /* ---- primitives (k_prims.hip) ---- */
 /* exclusive scan; out has n+1 entries, out[n] = total */
-/* total64 (optional, device): also receives the total */
+/* total64 (optional, device): also receives the total; post: the total is
+ * posted as the count */
 void scan_u32_to_u64(const uint32_t* in, uint64_t* out, Cnt n, void* tmp,
-                     size_t tmp_bytes, hipStream_t s,
-                     uint64_t* total64 = nullptr);
+                     hipStream_t s, uint64_t* total64 = nullptr,
+                     Post post = Post());
 void scan_u64_to_u64(const uint64_t* in, uint64_t* out, Cnt n, void* tmp,
-                     size_t tmp_bytes, hipStream_t s,
-                     uint64_t* total64 = nullptr);
+                     hipStream_t s, uint64_t* total64 = nullptr,
+                     Post post = Post());
 /* flags (nonzero = 1) -> u32 positions; n < 2^32 */
 void scan_u8flag_to_u32(const uint8_t* in, uint32_t* out, Cnt n, void* tmp,
-                        size_t tmp_bytes, hipStream_t s,
-                        uint64_t* total64 = nullptr);
+                        hipStream_t s, uint64_t* total64 = nullptr);
 size_t scan_tmp_bytes(int64_t n);
 /* tile offsets of flags (nonzero = 1) for the compactions below, inside
  * tmp (scan_tmp_bytes(n)); the count of nonzero flags at *total64 */
 const uint64_t* flag_tile_offsets(const uint8_t* in, Cnt n, void* tmp,
-                                  hipStream_t s, uint64_t* total64);
+                                  hipStream_t s, uint64_t* total64,
+                                  Post post = Post());
 /* stable LSD radix sort of (key, val) by the low `bits` bits of key */
 void radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
                       uint32_t* vals_alt, int64_t n, int bits, void* tmp,
@@ -184,33 +203,31 @@ struct Queue {
   unsigned* n;   /* QSLOTS counters, kSlotWords apart */
   uint32_t cap;  /* per sub-queue */
 };
-/* consumer view: entry i of the concatenated sub-queues */
+/* entries of a queue's sub-queues end to end, its counts known on the host */
 struct QView {
   const QEntry* q;
   uint32_t cap;
   uint32_t off[QSLOTS + 1]; /* exclusive prefix of the sub-queue counts */
   __host__ __device__ uint32_t size() const { return off[QSLOTS]; }
-  __device__ QEntry at(uint32_t i) const {
-    int lo = 0, hi = QSLOTS - 1; /* last k with off[k] <= i */
-    while (lo < hi) {
-      int mid = (lo + hi + 1) >> 1;
-      if (off[mid] <= i) lo = mid;
-      else hi = mid - 1;
-    }
-    return q[(uint64_t)lo * cap + (i - off[lo])];
-  }
 };
-/* what a consumer kernel gets: the view by value (built on the host), or a
- * pointer to one built on the device (graph-captured pipelines) and the
- * number of items its grid covers */
+/* what a consumer kernel gets: a host-built view, or (cnt set) the queue
+ * itself, whose counters each block reads (q_table), and the number of
+ * items its grid covers.  drop: an overflown queue is empty to its
+ * consumers (an eager ladder then runs again with a larger one), otherwise
+ * cut at its capacity. */
 struct QRef {
   QView v;
-  const QView* dv;
+  const unsigned* cnt;
   uint32_t bound;
-  __device__ uint32_t size() const { return dv ? dv->size() : v.size(); }
-  __device__ QEntry at(uint32_t i) const { return dv ? dv->at(i) : v.at(i); }
-  uint32_t launch_items() const { return dv ? bound : v.size(); }
+  int drop;
+  uint32_t launch_items() const { return cnt ? bound : v.size(); }
 };
+inline QRef queue_ref(const Queue& q, bool drop) {
+  QRef r{QView{}, q.n, QSLOTS * q.cap, (int)drop};
+  r.v.q = q.q;
+  r.v.cap = q.cap;
+  return r;
+}
 /* grid of a queue consumer: host views (size known) one entry per
  * thread; device views (size known only on the device) at most maxb
  * blocks striding over the entries, so that a queue sized for many
@@ -218,42 +235,35 @@ struct QRef {
 constexpr unsigned kEscBlocks = 1024, kExactBlocks = 512;
 inline dim3 qgrid(const QRef& q, unsigned maxb) {
   const unsigned b = (q.launch_items() + kBlock - 1) / kBlock;
-  if (!q.dv) return dim3(b ? b : 1); /* host view: one entry per thread */
+  if (!q.cnt) return dim3(b ? b : 1); /* host view: one entry per thread */
   return dim3(b < maxb ? (b ? b : 1) : maxb);
 }
 /* the same for consumers that take one entry per group of tpi lanes */
 inline dim3 qgrid_grp(const QRef& q, unsigned maxb, unsigned tpi) {
   const uint64_t b = ((uint64_t)q.launch_items() * tpi + kBlock - 1) / kBlock;
-  if (!q.dv) return dim3(b ? (unsigned)b : 1u);
+  if (!q.cnt) return dim3(b ? (unsigned)b : 1u);
   return dim3(b < maxb ? (b ? (unsigned)b : 1u) : maxb);
 }
 
 /* ---- recorded pipelines (k_prims.hip) ----
- * Fixed-capacity runs keep every count on the device; overflows and a
- * stale plan are reported through status bits. */
-enum { REC_CAP = 0,    /* bits 0..8: a count exceeded its capacity */
-       REC_Q1 = 9,     /* hot queue overflow */
+ * Fixed-capacity runs keep every count on the device; queue overflows and a
+ * stale plan are reported through status bits (a count past its capacity
+ * the host sees by itself, after the run). */
+enum { REC_Q1 = 9,     /* hot queue overflow */
        REC_Q2 = 10,    /* escalation queue overflow */
        REC_STALE = 11  /* the input no longer matches the recorded plan */ };
 /* set counter idx of every copy to zero */
 void zero_counter(unsigned long long* ctr, int idx, hipStream_t s);
-/* view of QSLOTS sub-queues (counters cleared after reading, and with
- * lists the counters of both lists beside them);
- * fresh (an eager ladder's first view): status / fill overwritten, and
- * the view left empty when a sub-queue overflowed (the ladder reruns);
- * else status / fill merged and the view clamped to the capacity */
-void launch_make_view(const QEntry* q, uint32_t cap, unsigned* cnt, QView* v,
-                      unsigned* status, unsigned bit, unsigned* fill,
-                      unsigned* lists, bool fresh, hipStream_t s);
-void launch_cap_check(const uint64_t* v, uint64_t cap, unsigned* status,
-                      unsigned bit, hipStream_t s);
-/* eager ladder state (u32 words): [kLadStatus] status, [kLadFill] fill of
- * the first view, [kLadCount] the count (u64), [kLadCnt, + QSLOTS) the
- * last queue's sub-queue counts */
-constexpr int kLadStatus = 0, kLadFill = 1, kLadCount = 4, kLadCnt = 6;
-constexpr int kLadWords = kLadCnt + QSLOTS;
-void launch_ladder_state(unsigned* cnt, unsigned* lists, const uint64_t* count,
-                         unsigned* lad, hipStream_t s);
+/* the end of a recorded ladder: the largest fills of its queues (capacity
+ * c1, c2 per sub-queue) into fill[0..1], overflows into *status, and the
+ * queue and list counters cleared for the next ladder */
+void launch_ladder_rec(unsigned* qn, uint32_t c1, uint32_t c2, unsigned* status,
+                       unsigned* fill, hipStream_t s);
+/* a run's statistics: the counters summed over their copies (CTR_COUNT
+ * u64) and the time stamps (kStamps u64) to the box's data words */
+constexpr int kStamps = 9;
+void launch_post_stats(const unsigned long long* ctr,
+                       const unsigned long long* ts, Post post, hipStream_t s);
 void launch_plan_check(const Bounds* now, const Bounds* ref, int64_t m,
                        int scale, unsigned* status, unsigned bit,
                        hipStream_t s);
@@ -285,10 +295,11 @@ void launch_or_flags(Cnt n, const uint8_t* a, const uint8_t* b, uint8_t* out,
                      PipeLaunch L);
 void launch_mark_faces(Cnt nk, const uint4* ftets, const uint64_t* erow,
                        const uint32_t* ecol, const uint64_t* trow,
-                       const uint32_t* tk, uint8_t* tri_in, PipeLaunch L);
+                       const uint32_t* tk, uint8_t* tri_in,
+                       unsigned long long* ts, PipeLaunch L);
 void launch_mark_edges(Cnt nt, const uint32_t* ftri, const uint32_t* tedge,
                        const uint32_t* teik, const uint32_t* tejk,
-                       uint8_t* edge_in, PipeLaunch L);
+                       uint8_t* edge_in, unsigned long long* ts, PipeLaunch L);
 void launch_emit_tets(Cnt nk, const uint4* ftets, const uint32_t* perm,
                       int32_t* out, PipeLaunch L);
 void launch_emit_tris(Cnt nt, const uint32_t* ftri, const uint32_t* ecol,
@@ -347,8 +358,10 @@ namespace pac {
 namespace PAC_V {
 /* ---- binning (k_enum.hip) ---- */
 
+/* (post: the bounds are posted, in the box's data words) */
 void launch_bounds(const Ball* raw, int64_t n, Real solvent, Bounds* part,
-                   Bounds* out, PipeLaunch L);
+                   Bounds* out, double4* orig, unsigned long long* ctl,
+                   int ctl_words, Post post, PipeLaunch L);
 /* per-molecule bounds of a batch: one block per molecule, moff[nmol+1] */
 void launch_bounds_mol(const Ball* raw, const uint32_t* moff, int64_t nmol,
                        Real solvent, Bounds* out, PipeLaunch L);
@@ -384,6 +397,10 @@ struct Stage {
   Real alpha;
   ExactScale ex;
   unsigned long long* ctr;
+  /* time stamps (kStamps), set by the first kernel of each phase: 1 bounds,
+   * 2 edges, 3 triangles, 4 tets, 5 - 7 the emptiness tests, 8 the end
+   * (null: none) */
+  unsigned long long* ts;
   int staged;
   /* second emptiness phase: a persistent launch of bgrid blocks of bblock
    * threads whose waves take bchunk entries of the left-over list at a
@@ -448,7 +465,8 @@ void launch_tet_caps(const Stage& S, Cnt m, const uint64_t* trow,
                      PipeLaunch L);
 /* exact triangle count per alpha edge */
 void launch_tri_count(Cnt ne, const uint64_t* erow, const uint32_t* ecol,
-                      const uint32_t* eleft, uint32_t* cnt, PipeLaunch L);
+                      const uint32_t* eleft, uint32_t* cnt,
+                      unsigned long long* ts, PipeLaunch L);
 /* triangle candidates of the alpha edges, each filtered by the first
  * precision stage in the same kernel: enumeration block b (256 alpha
  * edges) writes its kept and undecided candidates (k, edge, edge(i,k),

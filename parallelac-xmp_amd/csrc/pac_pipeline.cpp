@@ -116,16 +116,20 @@ static GridPlan plan_grid(const Bounds& B, Real alpha, int policy) {
 void plan_pass(Engine* E, const Ball* raw, int64_t n, Real solvent,
                Real alpha, const pac_options& opt, hipStream_t s,
                const int64_t* moff, int64_t nmol, PassPlan& pl,
-               const Bounds* gridb) {
+               const Bounds* gridb, const RunCtl* ctl) {
   Pool* P = pool_of(E);
   PipeLaunch L{s, kBlock};
   const bool batch = nmol > 1;
   std::vector<Bounds> hb(std::max<int64_t>(nmol, 1));
   if (!batch) {
     DBuf<Bounds> bpart(P, 1024 * 2 + 4), bout(P, 1);
-    launch_bounds(raw, n, solvent, bpart.get(), bout.get(), L);
+    const Post post = E->post();
+    launch_bounds(raw, n, solvent, bpart.get(), bout.get(),
+                  ctl ? ctl->orig : nullptr, ctl ? ctl->p : nullptr,
+                  ctl ? ctl->words : 0, post, L);
     KCHK();
-    hb[0] = readback(E, s, bout.get());
+    E->wait(post, s);
+    std::memcpy(&hb[0], E->box + kBoxData, sizeof(Bounds));
   } else {
     std::vector<uint32_t> mo(nmol + 1);
     for (int64_t m = 0; m <= nmol; ++m) mo[m] = (uint32_t)moff[m];
@@ -133,6 +137,7 @@ void plan_pass(Engine* E, const Ball* raw, int64_t n, Real solvent,
     HIPCHK(hipMemcpyAsync(pl.dmoff.get(), mo.data(), (nmol + 1) * sizeof(uint32_t),
                           hipMemcpyHostToDevice, s));
     DBuf<Bounds> bout(P, nmol);
+    if (ctl) zero_u64(ctl->p, ctl->words, s);
     launch_bounds_mol(raw, pl.dmoff.get(), nmol, solvent, bout.get(), L);
     KCHK();
     HIPCHK(hipMemcpyAsync(hb.data(), bout.get(), nmol * sizeof(Bounds),
@@ -243,7 +248,7 @@ void plan_pass(Engine* E, const Ball* raw, int64_t n, Real solvent,
  * queues of fixed size, overflows setting status bits. */
 void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
                   Real alpha, const pac_options& opt, pac_result* R,
-                  hipStream_t s, Timer& T, KProf& KP, const int64_t* moff,
+                  hipStream_t s, KProf& KP, const int64_t* moff,
                   int64_t nmol, const PassRec* rec, const SubInput* sub) {
   Pool* P = rec ? rec->pool : pool_of(E);
   PipeLaunch L{s, kBlock};
@@ -253,10 +258,22 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   if (n > (int64_t)INT32_MAX) fail(PAC_ERR_OVERFLOW, "too many balls");
 
   /* ---- bounds, grids (AlphaComplexParallel.cu:1089-1124) ---- */
+  /* control words: the statistics counters, the queue and list counters
+   * (QK_*, kept clear by the ladders), the time stamps; cleared by the
+   * run's first kernel */
   PassPlan own;
-  if (!rec)
+  RunCtl ctl;
+  DBuf<unsigned long long> ctl_own;
+  unsigned long long* ts = nullptr;
+  if (!rec) {
+    ctl.words = CTR_COUNT * CTR_SLOTS + QN_WORDS / 2 + kStamps;
+    ctl_own = DBuf<unsigned long long>(P, ctl.words);
+    ctl.p = ctl_own.get();
+    ctl.orig = sub || nmol > 1 ? nullptr : R->balls.get();
+    ts = ctl.p + ctl.words - kStamps;
     plan_pass(E, raw, n, solvent, alpha, opt, s, moff, nmol, own,
-              sub ? &sub->grid : nullptr);
+              sub ? &sub->grid : nullptr, &ctl);
+  }
   const PassPlan& pl = rec ? *(const PassPlan*)rec->plan : own;
   /* counts left on the device by the scans (RC_*) */
   DBuf<uint64_t> dcnt_own;
@@ -272,7 +289,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       launch_bounds_mol(raw, pl.dmoff.get(), nmol, solvent, rec->bnow, L);
     } else {
       DBuf<Bounds> bpart(P, 1024 * 2 + 4);
-      launch_bounds(raw, n, solvent, bpart.get(), rec->bnow, L);
+      launch_bounds(raw, n, solvent, bpart.get(), rec->bnow, nullptr, nullptr, 0,
+                    Post(), L);
     }
     launch_plan_check(rec->bnow, rec->bref, (int64_t)pl.bounds.size(), pl.S,
                       rec->status, 1u << REC_STALE, s);
@@ -309,28 +327,14 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     SG.own_lo = sub->own_lo;
     SG.own_hi = sub->own_hi;
   }
-  DBuf<unsigned long long> ctr_own;
-  if (rec) {
-    SG.ctr = rec->ctr;
-  } else {
-    ctr_own = DBuf<unsigned long long>(P, CTR_COUNT * CTR_SLOTS);
-    zero_u64(ctr_own.get(), CTR_COUNT * CTR_SLOTS, s);
-    SG.ctr = ctr_own.get();
-  }
+  SG.ctr = rec ? rec->ctr : ctl.p;
+  SG.ts = ts;
   unsigned long long* const ctr = SG.ctr;
-  /* queue and list counters (QK_*) */
-  DBuf<unsigned> qn_own;
-  if (!rec) {
-    qn_own = DBuf<unsigned>(P, QN_WORDS);
-    zero_u32(qn_own.get(), QN_WORDS, s); /* then kept clear by the ladders */
-  }
-  unsigned* const qn = rec ? rec->qn : qn_own.get();
+  unsigned* const qn =
+      rec ? rec->qn : (unsigned*)(ctl.p + CTR_COUNT * CTR_SLOTS);
   unsigned* const nesc = qn + QK_ESC;
   unsigned* const nrest = qn + QK_REST;
   unsigned* const nnext = qn + QK_NEXT;
-  /* eager ladders: the device view of q1 and the state read back once */
-  DBuf<QView> ev_view(P, 1);
-  DBuf<unsigned> lad(P, kLadWords);
 
   /* ---- binning: key, stable radix sort, gather, cell starts ---- */
   DBuf<uint32_t> key(P, n), idx(P, n), key2(P, n), idx2(P, n);
@@ -382,33 +386,33 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     SG.fid = fid.get();
     SG.fstart = fstart.get();
   }
-  T.mark(2);
 
   auto scan_tmp = [&](int64_t m) { return DBuf<uint8_t>(P, scan_tmp_bytes(m) + 64); };
   const bool staged = SG.staged != 0;
 
-  /* the count a scan left at dcnt[q]: read back, or (recorded) kept on the
-   * device under its capacity, an excess setting status bit q */
-  auto settle = [&](int q) -> Cnt {
-    if (!rec) return Cnt((int64_t)readback(E, s, dcnt + q));
-    launch_cap_check(dcnt + q, (uint64_t)rec->cap[q], rec->status,
-                     1u << (REC_CAP + q), s);
-    return Cnt(rec->cap[q], dcnt + q);
+  /* the count a scan posted and left at dcnt[q]: waited for, or (recorded)
+   * kept on the device under its capacity */
+  auto settle = [&](int q, const Post& post) -> Cnt {
+    if (rec) return Cnt(rec->cap[q], dcnt + q);
+    E->wait(post, s);
+    return Cnt((int64_t)E->posted_count());
+  };
+  auto new_post = [&](bool ladder_end) {
+    return rec ? Post() : E->post(ladder_end ? qn : nullptr);
   };
 
   /* Precision ladder: hot kernel (q1) -> [staged: escalation kernel FP64 ->
    * double-double (q1 -> q2)] -> exact wide-integer kernel, then `tail`,
    * the scan that leaves the ladder's count at dcnt[q].
-   * Eager: the escalation reads q1 through a view built on the device, and
-   * the tail runs before the exact stage on the chance that the last queue
-   * (q2; q1 without escalation) is empty, which it almost always is; one
-   * read-back then brings that queue's counts, the count and the overflow
-   * status.  Only when the last queue holds entries are they read into a
-   * host view (for the exact stage, sorted when long), and the tail run
-   * again after it.  An overflow reruns the ladder with larger queues (the
-   * stages are idempotent).
-   * Recorded: views built on the device, queues of fixed size, overflows
-   * reported through the status word. */
+   * Eager: the tail runs before the exact stage on the chance that the last
+   * queue (q2; q1 without escalation) is empty, which it almost always is;
+   * its last kernel posts the queues' counts and the count.  Only when the
+   * last queue holds entries are they read through a host view (for the
+   * exact stage, sorted when long), and the tail run again after it.  An
+   * overflow reruns the ladder with larger queues (the stages are
+   * idempotent).
+   * Recorded: queues of fixed size, overflows reported through the status
+   * word. */
   const int64_t qmax = (int64_t)(UINT32_MAX / QSLOTS) - 1;
   /* sub-queue capacity for up to `total` entries spread over the slots;
    * a one-item-per-thread producer of n items never exceeds n/QSLOTS + 512
@@ -421,23 +425,16 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   };
   auto ladder = [&](int64_t cap1_total, int kp_hot, int kp_exact, auto&& hot,
                     auto&& esc, auto&& exact, auto&& tail, int q) -> Cnt {
-    if (rec) { /* once, over the recorded queues; views built on the device */
-      hot(Queue{rec->q1, qn, rec->c1});
-      launch_make_view(rec->q1, rec->c1, qn, rec->views, rec->status,
-                       1u << REC_Q1, rec->fill, nrest, false, s);
-      QRef r{QView{}, rec->views, QSLOTS * rec->c1};
-      if (staged) {
-        esc(r, Queue{rec->q2, nesc, rec->c2});
-        launch_make_view(rec->q2, rec->c2, nesc, rec->views + 1,
-                         rec->status, 1u << REC_Q2, rec->fill + 1, nullptr,
-                         false, s);
-        r = QRef{QView{}, rec->views + 1, QSLOTS * rec->c2};
-      }
-      exact(r);
+    if (rec) { /* once, over the recorded queues */
+      const Queue h{rec->q1, qn, rec->c1}, e{rec->q2, nesc, rec->c2};
+      hot(h);
+      if (staged) esc(queue_ref(h, false), e);
+      exact(queue_ref(staged ? e : h, false));
       KCHK();
-      tail();
+      tail(Post());
+      launch_ladder_rec(qn, rec->c1, rec->c2, rec->status, rec->fill, s);
       KCHK();
-      return settle(q);
+      return settle(q, Post());
     }
     uint32_t c1 = slot_cap(cap1_total);
     /* q2 as large as q1: an escalated pair queues at most itself; a
@@ -447,44 +444,36 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     DBuf<QEntry> q1, q2;
     for (;;) {
       q1 = DBuf<QEntry>(P, (size_t)c1 * QSLOTS);
+      const Queue h{q1.get(), qn, c1};
       if (kp_hot >= 0) KP.begin(kp_hot);
-      hot(Queue{q1.get(), qn, c1});
+      hot(h);
       if (kp_hot >= 0) KP.end();
       KCHK();
-      const QEntry* last = q1.get();
-      uint32_t clast = c1;
-      unsigned* cnt_last = qn;
+      Queue last = h;
       if (staged) {
         q2 = DBuf<QEntry>(P, (size_t)c2 * QSLOTS);
-        launch_make_view(q1.get(), c1, qn, ev_view.get(), lad.get() + kLadStatus,
-                         1u, lad.get() + kLadFill, nullptr, true, s);
-        esc(QRef{QView{}, ev_view.get(), QSLOTS * c1},
-            Queue{q2.get(), nesc, c2});
+        last = Queue{q2.get(), nesc, c2};
+        esc(queue_ref(h, true), last);
         KCHK();
-        last = q2.get();
-        clast = c2;
-        cnt_last = nesc;
       }
-      tail();
-      launch_ladder_state(cnt_last, nrest, dcnt + q, lad.get(), s);
+      const Post post = new_post(true);
+      tail(post);
       KCHK();
-      unsigned h[kLadWords];
-      HIPCHK(hipMemcpyAsync(E->pinned, lad.get(), sizeof(h),
-                            hipMemcpyDeviceToHost, s));
-      HIPCHK(hipStreamSynchronize(s));
-      std::memcpy(h, E->pinned, sizeof(h));
+      E->wait(post, s);
+      const unsigned* const f1 = E->box + kBoxQ1;
+      const unsigned* const fl = E->box + (staged ? kBoxQ2 : kBoxQ1);
       QView vx;
-      vx.q = last;
-      vx.cap = clast;
+      vx.q = last.q;
+      vx.cap = last.cap;
       uint64_t acc = 0;
-      unsigned mx = 0;
+      unsigned fill1 = 0, mx = 0;
       for (int k = 0; k < QSLOTS; ++k) {
         vx.off[k] = (uint32_t)acc;
-        acc += std::min(h[kLadCnt + k], clast);
-        mx = std::max(mx, h[kLadCnt + k]);
+        acc += std::min(fl[k], last.cap);
+        mx = std::max(mx, fl[k]);
+        fill1 = std::max(fill1, f1[k]);
       }
       vx.off[QSLOTS] = (uint32_t)acc;
-      const unsigned fill1 = staged ? h[kLadFill] : mx;
       R->sizes[9] = std::max<int64_t>(R->sizes[9], fill1);
       if (staged) R->sizes[10] = std::max<int64_t>(R->sizes[10], mx);
       if (fill1 > c1) { /* q1 overflowed: everything again, larger */
@@ -492,22 +481,19 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
         if (staged) c2 = std::max(c2, slot_cap((int64_t)c1 * QSLOTS + 4096));
         continue;
       }
-      if (mx > clast) { /* q2 overflowed */
+      if (mx > last.cap) { /* q2 overflowed */
         c2 = grow(mx);
         continue;
       }
-      if (!vx.size()) {
-        uint64_t cnt;
-        std::memcpy(&cnt, h + kLadCount, sizeof(cnt));
-        return Cnt((int64_t)cnt);
-      }
+      if (!vx.size()) return Cnt((int64_t)E->posted_count());
       if (kp_exact >= 0) KP.begin(kp_exact);
-      exact(QRef{vx, nullptr, 0});
+      exact(QRef{vx, nullptr, 0, 0});
       if (kp_exact >= 0) KP.end();
       KCHK();
-      tail();
+      const Post again = new_post(true);
+      tail(again);
       KCHK();
-      return settle(q);
+      return settle(q, again);
     }
   };
 
@@ -518,12 +504,13 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   int64_t host_evals[6] = {0, 0, 0, 0, 0, 0};
   auto count_scan = [&](const uint32_t* cnt, Cnt nseg, uint64_t* off, int q,
                         const char* what) -> Cnt {
+    const Post post = new_post(false);
     {
       auto tmp = scan_tmp(nseg.cap);
-      scan_u32_to_u64(cnt, off, nseg, tmp.get(), 0, s, dcnt + q);
+      scan_u32_to_u64(cnt, off, nseg, tmp.get(), s, dcnt + q, post);
     }
     KCHK();
-    Cnt tot = settle(q);
+    Cnt tot = settle(q, post);
     if (tot.cap >= ((int64_t)1 << 32))
       fail(PAC_ERR_OVERFLOW, std::string(what) + " candidates exceed 2^32");
     return tot;
@@ -574,10 +561,10 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
         [&](QRef qr) {
           launch_filter_exact(SG, 1, C0, qr, cval.get(), flag.get(), L);
         },
-        [&] {
+        [&](Post post) {
           launch_seg_keep(n, off.get(), bcnt.get(), flag.get(), keep.get(), L);
-          scan_u32_to_u64(keep.get(), erow.get(), Cnt(n), tmp.get(), 0, s,
-                          dcnt + RC_EALPHA);
+          scan_u32_to_u64(keep.get(), erow.get(), Cnt(n), tmp.get(), s,
+                          dcnt + RC_EALPHA, post);
         },
         RC_EALPHA);
     ecol = DBuf<uint32_t>(P, Ealpha.cap);
@@ -592,7 +579,6 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     ecol = DBuf<uint32_t>(P, 1);
     eleft = DBuf<uint32_t>(P, 1);
   }
-  T.mark(3);
 
   /* ---- triangles (AlphaComplexParallel.cu:1279-1371) ---- */
   Cnt Tslots(0), Talpha(0);
@@ -611,7 +597,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       /* exact counts: a triangle's third vertex must be in both rows, and
        * the merge that counts it is cheap next to filtering empty slots */
       DBuf<uint32_t> cnt(P, Ealpha.cap);
-      launch_tri_count(Ealpha, erow.get(), ecol.get(), eleft.get(), cnt.get(), L);
+      launch_tri_count(Ealpha, erow.get(), ecol.get(), eleft.get(), cnt.get(), ts,
+                       L);
       Tslots = count_scan(cnt.get(), Ealpha, off.get(), RC_TSLOTS, "triangle");
     }
     DBuf<uint32_t> cval(P, Tslots.cap), cseg(P, Tslots.cap),
@@ -645,11 +632,11 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
         [&](QRef qr) {
           launch_filter_exact(SG, 2, C1, qr, cval.get(), flag.get(), L);
         },
-        [&] {
+        [&](Post post) {
           launch_seg_kept(Ealpha, kBlock, off.get(), kBlock, bcnt.get(),
                           flag.get(), bkeep.get(), L);
-          scan_u32_to_u64(bkeep.get(), bout.get(), Cnt(nblk), tmp.get(), 0, s,
-                          dcnt + RC_TALPHA);
+          scan_u32_to_u64(bkeep.get(), bout.get(), Cnt(nblk), tmp.get(), s,
+                          dcnt + RC_TALPHA, post);
         },
         RC_TALPHA);
     tk = DBuf<uint32_t>(P, Talpha.cap);
@@ -664,7 +651,6 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
                           (uint64_t)Talpha.cap);
     KCHK();
   }
-  T.mark(4);
 
   /* ---- tets (AlphaComplexParallel.cu:1381-1442) ---- */
   Cnt Kslots(0), Kalpha(0);
@@ -676,13 +662,14 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     DBuf<uint64_t> off, roff;
     if (tail_slots) {
       roff = DBuf<uint64_t>(P, Ealpha.cap + 1);
+      const Post post = new_post(false);
       {
         auto tmp = scan_tmp(Ealpha.cap);
-        scan_u64_to_u64(tpair.get(), roff.get(), Ealpha, tmp.get(), 0, s,
-                        dcnt + RC_KSLOTS);
+        scan_u64_to_u64(tpair.get(), roff.get(), Ealpha, tmp.get(), s,
+                        dcnt + RC_KSLOTS, post);
       }
       KCHK();
-      Kslots = settle(RC_KSLOTS);
+      Kslots = settle(RC_KSLOTS, post);
       if (Kslots.cap >= ((int64_t)1 << 32))
         fail(PAC_ERR_OVERFLOW, "tet candidates exceed 2^32");
     } else {
@@ -725,11 +712,11 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           launch_filter_esc(SG, 3, C2, qr, nullptr, flag.get(), q2, L);
         },
         [&](QRef qr) { launch_filter_exact(SG, 3, C2, qr, nullptr, flag.get(), L); },
-        [&] {
+        [&](Post post) {
           launch_seg_kept(Talpha, kTetSeg, bbase.get(), 1, bcnt.get(),
                           flag.get(), bkeep.get(), L);
-          scan_u32_to_u64(bkeep.get(), bout.get(), Cnt(nblk), tmp.get(), 0, s,
-                          dcnt + RC_KALPHA);
+          scan_u32_to_u64(bkeep.get(), bout.get(), Cnt(nblk), tmp.get(), s,
+                          dcnt + RC_KALPHA, post);
         },
         RC_KALPHA);
     tets = DBuf<uint4>(P, Kalpha.cap);
@@ -738,7 +725,6 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
                         (uint64_t)Kalpha.cap);
     KCHK();
   }
-  T.mark(5);
 
   auto ac2_cap = [](int64_t items) {
     return (uint32_t)std::min<int64_t>(std::max<int64_t>(1 << 20, items / 2),
@@ -748,11 +734,11 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   /* A long host view of exact pairs (degenerate inputs) as (item, aux)
    * arrays sorted by item, so that an item's pairs share its exact
    * per-simplex terms; false (nothing done) below 65536 entries or for a
-   * device-built view.  items < nitems. */
+   * device queue.  items < nitems. */
   auto sorted_view = [&](const QRef& q, int64_t nitems, DBuf<uint32_t>& k1,
                          DBuf<uint32_t>& v1, DBuf<uint32_t>& k2,
                          DBuf<uint32_t>& v2, bool& alt) -> uint32_t {
-    const uint32_t ne = q.dv ? 0u : q.v.size();
+    const uint32_t ne = q.cnt ? 0u : q.v.size();
     if (ne < (1u << 16)) return 0;
     k1 = DBuf<uint32_t>(P, ne);
     v1 = DBuf<uint32_t>(P, ne);
@@ -770,8 +756,17 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   };
 
   /* ---- tet emptiness ---- */
-  /* phase-one budget: 0 = the default (4), < 0 = no second phase */
-  int budget = opt.ac2_budget > 0 ? opt.ac2_budget : (opt.ac2_budget < 0 ? 0 : 4);
+  /* phase-one budget: 0 = the default, < 0 = no second phase.  The default
+   * is 4 where the items fill the chip many times over, and one phase below
+   * kOnePhase items: then no wave waits for a slot, the run is as long as
+   * its longest scan either way, and the second phase's launch comes on top
+   * (262 balls, 8,000 tets: 11 us in one phase, 11 + 21 in two). */
+  constexpr int64_t kOnePhase = 1 << 16;
+  auto budget = [&](Cnt items) {
+    return opt.ac2_budget > 0
+               ? opt.ac2_budget
+               : (opt.ac2_budget < 0 || items.cap < kOnePhase ? 0 : 4);
+  };
   /* the left-over and quick-pass lists: LSLOTS sub-lists sized for the
    * largest first-phase grid */
   SG.lcap = list_slot_cap(
@@ -785,21 +780,23 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   {
     auto tmp = scan_tmp(Kalpha.cap);
     const uint64_t* koffs = nullptr; /* tile offsets of kflag, in tmp */
-    auto tail = [&] {
-      koffs = flag_tile_offsets(kflag.get(), Kalpha, tmp.get(), s, dcnt + RC_KF);
+    auto tail = [&](Post post) {
+      koffs = flag_tile_offsets(kflag.get(), Kalpha, tmp.get(), s,
+                                dcnt + RC_KF, post);
     };
     if (opt.skip_tet_ac2 || !Kalpha.cap) {
       fill_u8(kflag.get(), Kalpha.cap, 1, s);
-      tail();
+      const Post post = new_post(false);
+      tail(post);
       KCHK();
-      Kf = settle(RC_KF);
+      Kf = settle(RC_KF, post);
     } else {
       Kf = ladder(
           ac2_cap(Kalpha.cap), KP_TET_AC2, KP_TET_AC2_EXACT,
           [&](Queue q) {
             launch_tet_ac2_hot(SG, Kalpha, tets.get(), kflag.get(), q,
                                rest.get(), nrest, next.get(), nnext,
-                               budget, L);
+                               budget(Kalpha), L);
           },
           [&](QRef q, Queue q2) {
             launch_tet_ac2_esc(SG, q, tets.get(), kflag.get(), q2, L);
@@ -826,7 +823,6 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     KCHK();
   }
   tets.release();
-  T.mark(6);
 
   /* ---- triangle closure + dangling emptiness ---- */
   /* filtration: every final triangle and edge gets its emptiness test (an
@@ -836,7 +832,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   DBuf<uint8_t> tri_in(P, Talpha.cap), tflag(P, Talpha.cap);
   fill_u8(tri_in.get(), Talpha.cap, 0, s);
   launch_mark_faces(Kf, ftets.get(), erow.get(), ecol.get(), trow.get(),
-                    tk.get(), tri_in.get(), L);
+                    tk.get(), tri_in.get(), ts, L);
   DBuf<uint8_t> tri_skip_own, tfin;
   uint8_t* tri_skip = tri_in.get(); /* passes without a test */
   if (filt) {
@@ -853,21 +849,24 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   {
     auto tmp = scan_tmp(Talpha.cap);
     const uint64_t* toffs = nullptr; /* tile offsets of tfinal, in tmp */
-    auto tail = [&] {
+    auto tail = [&](Post post) {
       if (filt) launch_or_flags(Talpha, tflag.get(), tri_in.get(), tfin.get(), L);
-      toffs = flag_tile_offsets(tfinal, Talpha, tmp.get(), s, dcnt + RC_TF);
+      toffs = flag_tile_offsets(tfinal, Talpha, tmp.get(), s,
+                                dcnt + RC_TF, post);
     };
     if (!Talpha.cap) {
-      tail();
+      const Post post = new_post(false);
+      tail(post);
       KCHK();
-      Tf = settle(RC_TF);
+      Tf = settle(RC_TF, post);
     } else {
       Tf = ladder(
           ac2_cap(Talpha.cap), KP_TRI_AC2, -1,
           [&](Queue q) {
             launch_low_ac2_hot(SG, 0, Talpha, ecol.get(), eleft.get(), tkd.get(),
                                tedge.get(), nullptr, tri_skip, tflag.get(), q,
-                               rest.get(), nrest, next.get(), nnext, budget, L);
+                               rest.get(), nrest, next.get(), nnext,
+                               budget(Talpha), L);
           },
           [&](QRef q, Queue q2) {
             launch_low_ac2_esc(SG, 0, q, ecol.get(), eleft.get(), tk.get(),
@@ -897,13 +896,12 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     }
     KCHK();
   }
-  T.mark(7);
 
   /* ---- edge closure + dangling emptiness ---- */
   DBuf<uint8_t> edge_in(P, Ealpha.cap), eflag(P, Ealpha.cap);
   fill_u8(edge_in.get(), Ealpha.cap, 0, s);
   launch_mark_edges(Tf, ftri.get(), tedge.get(), teik.get(), tejk.get(),
-                    edge_in.get(), L);
+                    edge_in.get(), ts, L);
   DBuf<uint8_t> edge_skip_own, efin;
   uint8_t* edge_skip = edge_in.get();
   if (filt) {
@@ -919,21 +917,24 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   auto etmp = scan_tmp(Ealpha.cap);
   const uint64_t* eoffs = nullptr; /* tile offsets of efinal, in etmp */
   {
-    auto tail = [&] {
+    auto tail = [&](Post post) {
       if (filt) launch_or_flags(Ealpha, eflag.get(), edge_in.get(), efin.get(), L);
-      eoffs = flag_tile_offsets(efinal, Ealpha, etmp.get(), s, dcnt + RC_EF);
+      eoffs = flag_tile_offsets(efinal, Ealpha, etmp.get(), s,
+                                dcnt + RC_EF, post);
     };
     if (!Ealpha.cap) {
-      tail();
+      const Post post = new_post(false);
+      tail(post);
       KCHK();
-      Ef = settle(RC_EF);
+      Ef = settle(RC_EF, post);
     } else {
       Ef = ladder(
           ac2_cap(Ealpha.cap), KP_EDGE_AC2, -1,
           [&](Queue q) {
             launch_low_ac2_hot(SG, 1, Ealpha, ecol.get(), eleft.get(), nullptr,
                                nullptr, dead, edge_skip, eflag.get(), q,
-                               rest.get(), nrest, next.get(), nnext, budget, L);
+                               rest.get(), nrest, next.get(), nnext,
+                               budget(Ealpha), L);
           },
           [&](QRef q, Queue q2) {
             launch_low_ac2_esc(SG, 1, q, ecol.get(), eleft.get(), nullptr,
@@ -990,12 +991,20 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   st.edges_final = Ef.cap;
   st.tris_final = Tf.cap;
   st.tets_final = Kf.cap;
-  T.mark(8);
 
-  unsigned long long hs[CTR_COUNT * CTR_SLOTS];
-  HIPCHK(hipMemcpyAsync(hs, ctr, sizeof(hs), hipMemcpyDeviceToHost, s));
-  HIPCHK(hipStreamSynchronize(s));
+  const Post post = E->post();
+  launch_post_stats(ctr, ts, post, s);
+  KCHK();
+  E->wait(post, s);
+  unsigned long long hs[CTR_COUNT + kStamps];
+  std::memcpy(hs, E->box + kBoxData, sizeof(hs));
   stats_from_counters(hs, SG.staged != 0, host_evals[0], st);
+  /* a phase without work left no stamp: it takes no time */
+  unsigned long long* const t = hs + CTR_COUNT;
+  for (int q = kStamps - 2; q >= 1; --q)
+    if (!t[q]) t[q] = t[q + 1];
+  for (int q = 1; q < kStamps - 1; ++q)
+    st.phase_ms[q] = (double)(t[q + 1] - t[q]) / E->clock_khz;
 }
 
 /* The LD driver (AlphaComplexLargeData.cu:1227-1992).  The cell-sorted
@@ -1023,11 +1032,11 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
  * halo's repeated enumeration. */
 void run_chunked(Engine* E, const Ball* raw, int64_t n, Real solvent,
                  Real alpha, const pac_options& opt, pac_result* R,
-                 hipStream_t s, Timer& T, KProf& KP) {
+                 hipStream_t s, KProf& KP) {
   int64_t C = 512;
   while (C < (int64_t)opt.chunk_balls) C *= 2;
   if (n <= C) {
-    run_pipeline(E, raw, n, solvent, alpha, opt, R, s, T, KP);
+    run_pipeline(E, raw, n, solvent, alpha, opt, R, s, KP);
     return;
   }
   if (n > (int64_t)INT32_MAX) fail(PAC_ERR_OVERFLOW, "too many balls");
@@ -1036,7 +1045,9 @@ void run_chunked(Engine* E, const Ball* raw, int64_t n, Real solvent,
 
   /* the whole input's grid and cell-sorted order */
   PassPlan gp;
-  plan_pass(E, raw, n, solvent, alpha, opt, s, nullptr, 1, gp);
+  RunCtl keep;
+  keep.orig = R->balls.get();
+  plan_pass(E, raw, n, solvent, alpha, opt, s, nullptr, 1, gp, nullptr, &keep);
   const GridP g = gp.grids[0];
   const Bounds gb = gp.bounds[0];
   DBuf<uint32_t> rank(P, n);
@@ -1060,8 +1071,6 @@ void run_chunked(Engine* E, const Ball* raw, int64_t n, Real solvent,
                           s));
     HIPCHK(hipStreamSynchronize(s));
   }
-  for (int q = 2; q <= 8; ++q) T.mark(q);
-
   const uint64_t exy = (uint64_t)g.ex * (uint64_t)g.ey;
   const double reach2 = (double)gb.max_r * (double)gb.max_r + (double)alpha;
   const double D = reach2 > 0 ? 2 * std::sqrt(reach2) : 0.0;
@@ -1098,7 +1107,7 @@ void run_chunked(Engine* E, const Ball* raw, int64_t n, Real solvent,
     Timer Tc(s);
     Tc.mark(0);
     launch_rank_flag(rank.get(), n, (uint32_t)slo, (uint32_t)shi, flag.get(), s);
-    scan_u8flag_to_u32(flag.get(), pos.get(), Cnt(n), stmp.get(), 0, s);
+    scan_u8flag_to_u32(flag.get(), pos.get(), Cnt(n), stmp.get(), s);
     DBuf<Ball> sraw(P, m);
     DBuf<uint32_t> sid(P, m);
     launch_select_balls(raw, flag.get(), pos.get(), n, m, sraw.get(), sid.get(), s);
@@ -1112,8 +1121,9 @@ void run_chunked(Engine* E, const Ball* raw, int64_t n, Real solvent,
     sub.grid = gb;
     sub.own_lo = (uint32_t)(lo - slo);
     sub.own_hi = (uint32_t)(hi - slo);
-    run_pipeline(E, sraw.get(), m, solvent, alpha, opt, &Rs, s, Tc, KP,
+    run_pipeline(E, sraw.get(), m, solvent, alpha, opt, &Rs, s, KP,
                  nullptr, 1, nullptr, &sub);
+    Tc.mark(2);
     for (int d = 1; d <= 3; ++d)
       launch_row_bounds(Rs.lists[d - 1].get(), Rs.counts[d], d + 1, sid.get(),
                         rank.get(), (uint32_t)lo, (uint32_t)hi,
@@ -1138,11 +1148,10 @@ void run_chunked(Engine* E, const Ball* raw, int64_t n, Real solvent,
       }
     }
     KCHK();
-    Tc.mark(9);
+    Tc.mark(3);
     HIPCHK(hipStreamSynchronize(s));
-    for (int q = 2; q < 8; ++q) Rs.st.phase_ms[q] = Tc.ms(q, q + 1);
-    Rs.st.phase_ms[1] = Tc.ms(0, 2);  /* selection + binning */
-    Rs.st.phase_ms[0] = Tc.ms(8, 9);  /* owned rows out */
+    Rs.st.phase_ms[1] += Tc.ms(0, 1); /* selection beside the binning */
+    Rs.st.phase_ms[0] = Tc.ms(2, 3);  /* owned rows out */
     add_stats(acc, Rs.st);
   }
 

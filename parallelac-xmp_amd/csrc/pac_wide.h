@@ -230,7 +230,7 @@ __device__ __forceinline__ CW<TPI> cw_of(const WI& a) {
  * g, then g + groups, ...  Every lane of a group calls body(t) with the
  * same t. */
 template <int TPI, class F>
-__device__ __forceinline__ void for_queue_grp(const QRef& q, F&& body) {
+__device__ __forceinline__ void for_queue_grp(const QTab& q, F&& body) {
   const uint32_t n = q.size();
   const uint32_t groups = (gridDim.x * blockDim.x) / TPI;
   const uint32_t g0 = (uint32_t)(gtid() / TPI);

@@ -14,6 +14,55 @@
 #include "pac_dev.h"
 
 namespace pac {
+/* Device words to pinned host memory in segments of 16 KiB; a segment posts
+ * its ticket when its stores are out, and the host moves it on while the
+ * later ones still cross the bus.  So few blocks that the segments arrive one
+ * after the other: with a block per segment they share the bus and all
+ * arrive last.  288 lists of 0.47 MB on average to the caller's memory: 9.0
+ * ms with 8 or 16 blocks, 9.9 with 32, 11.0 with a block per segment, 11.8
+ * with segments of 64 KiB, 13.3 with the runtime's copy. */
+__global__ __launch_bounds__(kBlock) void k_copy_out(
+    const uint32_t* src, int64_t words, int32_t base, unsigned char* ring,
+    unsigned long long* ring_ticket, int slot0, unsigned long long ticket) {
+  constexpr int kW = kSegBytes / 4;
+  const uint32_t b = (uint32_t)base;
+  for (int64_t k = blockIdx.x; k * kW < words; k += gridDim.x) {
+    const int slot = slot0 + (int)k;
+    const uint32_t* const in = src + k * kW;
+    const int n = words - k * kW < kW ? (int)(words - k * kW) : kW;
+    uint32_t* const out =
+        reinterpret_cast<uint32_t*>(ring + (size_t)slot * kSegBytes);
+    int t0 = 0;
+    if (((uintptr_t)in & 15) == 0) { /* rows of a list may start at any word */
+      const uint4* const iv = reinterpret_cast<const uint4*>(in);
+      uint4* const ov = reinterpret_cast<uint4*>(out);
+      const int nv = n / 4;
+      for (int t = threadIdx.x; t < nv; t += kBlock) {
+        const uint4 v = iv[t];
+        ov[t] = make_uint4(v.x - b, v.y - b, v.z - b, v.w - b);
+      }
+      t0 = nv * 4;
+    }
+    for (int t = t0 + threadIdx.x; t < n; t += kBlock) out[t] = in[t] - b;
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0)
+      __hip_atomic_store(ring_ticket + slot, ticket, __ATOMIC_RELEASE,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+void launch_copy_out(const uint32_t* src, int64_t words, int32_t base,
+                     unsigned char* ring, unsigned long long* ring_ticket,
+                     int slot0, unsigned long long ticket, hipStream_t s) {
+  if (words <= 0) return;
+  constexpr int64_t kW = kSegBytes / 4;
+  const int64_t nseg = (words + kW - 1) / kW;
+  hipLaunchKernelGGL(k_copy_out,
+                     dim3((unsigned)(nseg < kCopyBlocks ? nseg : kCopyBlocks)),
+                     dim3(kBlock), 0, s, src, words, base, ring, ring_ticket,
+                     slot0, ticket);
+}
+
 using namespace PAC_V; /* type-independent device helpers */
 
 /* Orthocentre of a simplex relative to its first vertex, x = c - p_0, and

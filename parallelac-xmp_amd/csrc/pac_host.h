@@ -171,6 +171,13 @@ struct Engine {
   unsigned* box = nullptr;
   unsigned long long ticket = 0;
   double clock_khz = 1e5; /* rate of the device's wall clock (time stamps) */
+  /* copies to host memory (to_host): a ring of pinned segments with a
+   * ticket each, a stream of their own, one copy at a time */
+  std::mutex copy_mu;
+  hipStream_t cstream = nullptr;
+  unsigned char* ring = nullptr;
+  unsigned long long* ring_ticket = nullptr;
+  unsigned long long copy_ticket = 0;
   Post post(unsigned* qn = nullptr) { return Post{box, ++ticket, qn}; }
   /* waits for the post: spins on its ticket (a few microseconds, while the
    * kernels before it run), then, should it take long, in the runtime, which

@@ -308,6 +308,13 @@ void launch_emit_tris(Cnt nt, const uint32_t* ftri, const uint32_t* ecol,
                       int32_t* out, PipeLaunch L);
 
 /* ---- outputs (k_output.hip) ---- */
+/* words of src (4-byte units, minus base; at most half a ring) to the pinned
+ * ring: segment k of kSegBytes to slot0 + k, whose ticket then becomes
+ * `ticket` */
+constexpr int kSegBytes = 1 << 14, kRingSegs = 256, kCopyBlocks = 16;
+void launch_copy_out(const uint32_t* src, int64_t words, int32_t base,
+                     unsigned char* ring, unsigned long long* ring_ticket,
+                     int slot0, unsigned long long ticket, hipStream_t s);
 /* Filtration keys of all simplices, key[0, n + E + T + K) (balls, edges,
  * triangles, tets; order-preserving 64-bit images of the values): lists in
  * reference order, gab[0..1] the own-value flags of edges / triangles,

@@ -779,20 +779,22 @@ constexpr int fam_of(int KIND) {
  * (computePossibleTetCount / fillPossibleTets, Parallel:418-543), fused
  * with the tet filter's first stage (markRealTets, :531-591).
  * A wave takes kTetSeg = 64 triangles, one a lane, whose candidate slots
- * are one contiguous range.  The three-list merges leave each triangle's
- * fourth vertices in LDS from its first slot on; then the wave filters the
- * candidates themselves, 64 at a time (of the slots, the tails of the
- * triangles' rows, 59% hold one on a globule: candidate d's triangle is
- * found in the lanes' prefix counts), and writes the kept and undecided
- * ones compacted, in slot order, from its first slot on, with their flags.
+ * are one contiguous range.  The masks that k_tri_block_copy left per alpha
+ * edge give each triangle the l in both T(i,j) after k and T(i,k) as the set
+ * bits of one 64-bit word; the wave lists them in LDS and takes them 64 at a
+ * time, whatever triangle they belong to: is (j,k,l) a triangle (a bit of
+ * the third mask), then the filter.  The kept and undecided ones are written
+ * compacted, in order, from the wave's first slot on, with their flags.
  * No barrier: a wave waits for no other until the counters are summed.
- * Against blocks of 256 triangles filtering every slot from a 16-byte
- * stage: 523 -> 434 us at 100k balls, 9.6 -> 1.8 ms on 200k balls with a
- * lattice block (whose blocks overflowed the stage), and 405 us with the
- * filter on fused multiply-adds.  At 100k the vector memory path (TD 96%
- * busy, TA 86%: the merges' gathers) and the vector ALU (86%) bound it
- * together.  Slots past the LDS stage (1,120 a wave; a lattice's waves
- * average 530, a globule's 230) are kept in the candidates' own array.
+ * A wave with a triangle whose row is cut off in a mask (a third vertex 63
+ * or more edges on: dense inputs) merges the three rows instead, each lane
+ * its own, into fourth vertices in LDS (928 of them, the rest in the
+ * candidates' own array).
+ * At 100k balls 277 us; 395 with all waves merging, whose rounds last as
+ * long as their longest rows; 523 with blocks of 256 triangles filtering
+ * every slot.  200k balls with a lattice block: 1.39 ms against 1.70 and
+ * 9.6.  The vector ALU bounds it, the filter's 114 instructions being half
+ * of a round.
  * A candidate with a covered edge (kDeadBit of one of its triangles in
  * tkd, carried with the fourth vertex) is filtered like any other, but an
  * alpha tet among them is only counted (CTR_DROP), not written: it cannot
@@ -816,14 +818,16 @@ __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_filter(
     Stage S, Cnt c_nt, const uint64_t* trow, const uint32_t* tkd,
     const uint32_t* tedge, const uint32_t* teik, const uint32_t* tejk,
-    const uint32_t* eleft, const uint32_t* ecol, const uint64_t* off,
-    const uint64_t* roff, uint64_t* bbase, uint4* ctet, uint8_t* flag,
-    uint32_t* bcnt, uint32_t* bkeep, Queue q1, uint64_t lim) {
+    const uint32_t* eleft, const uint32_t* ecol, const ulonglong2* emask,
+    const uint64_t* off, const uint64_t* roff, uint64_t* bbase, uint4* ctet,
+    uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep, Queue q1, uint64_t lim) {
   static_assert(kTetSeg == 64, "a triangle a lane");
   stamp(S.ts, 4);
-  constexpr uint32_t CAP = 1120; /* with the tables, 8 blocks per CU */
-  __shared__ uint32_t s_l[kBlock / 64][CAP];
-  __shared__ uint32_t s_end[kBlock / 64][64], s_off[kBlock / 64][64];
+  /* LDS of a wave, 4,992 bytes (8 blocks per CU): by masks, three rows of
+   * 16 bytes a triangle and the listed bits; by merges, the stage of fourth
+   * vertices and the lanes' prefix counts */
+  constexpr uint32_t RAW = 312, LIST = (RAW - 192) * 8, CAP = 928;
+  __shared__ uint4 s_raw[kBlock / 64][RAW];
   const int64_t nt = c_nt.get();
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int64_t seg = gtid() >> 6, q = gtid();
@@ -835,10 +839,9 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
       bbase[seg] = 0;
     }
   } else {
-    /* the triangle's slots [o, oe): off[] per triangle, or (roff) the
-     * closed form, a triangle's slots being its row's tail */
+    constexpr uint32_t kEnd = ~kDeadBit;
     uint32_t eij = 0, eik = 0, ejk = 0, i = 0, j = 0, kd = 0;
-    uint64_t o = 0, oe = 0;
+    ulonglong2 mij = make_ulonglong2(0, 0), mik = mij, mjk = mij;
     if (q < nt) {
       eij = tedge[q];
       eik = teik[q];
@@ -846,155 +849,249 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
       kd = tkd[q];
       i = eleft[eij];
       j = ecol[eij];
-      if (off) {
-        o = off[q];
-        oe = off[q + 1];
-      } else {
-        o = tet_slot_off(roff, trow, eij, (uint32_t)q);
-        oe = o + (trow[eij + 1] - (uint64_t)q - 1);
-      }
+      mij = emask[eij];
+      mik = emask[eik];
+      mjk = emask[ejk];
     }
-    const uint32_t k = kd & ~kDeadBit;
-    const uint64_t base = (uint64_t)__shfl((unsigned long long)o, 0, 64);
-    /* the wave's slots, numbered from its first one; [rel, end) this
-     * lane's, cut at the arrays' end */
-    const uint32_t rel = (uint32_t)(o - base);
-    const uint32_t end =
-        o >= lim ? rel : rel + (uint32_t)((oe < lim ? oe : lim) - o);
-    uint32_t* const spill = reinterpret_cast<uint32_t*>(ctet + base);
-    uint32_t at = rel;
-    auto put = [&](uint32_t v) {
-      ++found;
-      if (at < end) {
-        if (at < CAP) s_l[wv][at] = v;
-        else spill[4 * (uint64_t)at] = v;
-        ++at;
-      }
-    };
-    /* two merge steps a round: each list's next element is loaded with its
-     * current one (kEnd past the row's end, above every ball id).  A
-     * triangle without slots (a chunk sub-input's unowned one) merges
-     * nothing. */
-    constexpr uint32_t kEnd = ~kDeadBit;
-    if (o < oe) {
-      if constexpr (BUF) {
-        /* byte offsets into tkd (below 4 GiB): no 64-bit address
-         * arithmetic per load */
-        const BufU32 K{tkd, (uint32_t)(c_nt.cap * 4)};
-        uint32_t a = ((uint32_t)q + 1u) << 2, ae = (uint32_t)trow[eij + 1] << 2;
-        uint32_t b = (uint32_t)trow[eik] << 2, be = (uint32_t)trow[eik + 1] << 2;
-        uint32_t c = (uint32_t)trow[ejk] << 2, ce = (uint32_t)trow[ejk + 1] << 2;
-        while (a < ae && b < be && c < ce) {
-          const uint32_t xd0 = K.at(a), yd0 = K.at(b), zd0 = K.at(c);
-          const uint32_t xd1 = a + 4u < ae ? K.at(a + 4u) : kEnd;
-          const uint32_t yd1 = b + 4u < be ? K.at(b + 4u) : kEnd;
-          const uint32_t zd1 = c + 4u < ce ? K.at(c + 4u) : kEnd;
-          const uint32_t x0 = xd0 & kEnd, y0 = yd0 & kEnd, z0 = zd0 & kEnd;
-          const uint32_t m0 = max(x0, max(y0, z0));
-          const bool all0 = x0 == m0 && y0 == m0 && z0 == m0;
-          if (all0) put(m0 | ((kd | xd0 | yd0 | zd0) & kDeadBit));
-          const bool sa = all0 || x0 < m0, sb = all0 || y0 < m0,
-                     sc = all0 || z0 < m0;
-          const uint32_t xd = sa ? xd1 : xd0, yd = sb ? yd1 : yd0,
-                         zd = sc ? zd1 : zd0;
-          const uint32_t x = xd & kEnd, y = yd & kEnd, z = zd & kEnd;
-          const uint32_t m = max(x, max(y, z));
-          const bool all = x == m && y == m && z == m;
-          if (all && m != kEnd) put(m | ((kd | xd | yd | zd) & kDeadBit));
-          a += (sa ? 4u : 0u) + ((all || x < m) ? 4u : 0u);
-          b += (sb ? 4u : 0u) + ((all || y < m) ? 4u : 0u);
-          c += (sc ? 4u : 0u) + ((all || z < m) ? 4u : 0u);
-        }
-      } else {
-        /* alpha-triangle ids fit 32 bits (the slot count is checked below
-         * 2^32): 32-bit cursors halve the merge's index arithmetic */
-        uint32_t a = (uint32_t)q + 1, ae = (uint32_t)trow[eij + 1];
-        uint32_t b = (uint32_t)trow[eik], be = (uint32_t)trow[eik + 1];
-        uint32_t c = (uint32_t)trow[ejk], ce = (uint32_t)trow[ejk + 1];
-        while (a < ae && b < be && c < ce) {
-          const uint32_t xd = tkd[a], yd = tkd[b], zd = tkd[c];
-          const uint32_t x = xd & kEnd, y = yd & kEnd, z = zd & kEnd;
-          const uint32_t m = max(x, max(y, z));
-          if (x == m && y == m && z == m) {
-            put(m | ((kd | xd | yd | zd) & kDeadBit));
-            ++a;
-            ++b;
-            ++c;
-          } else {
-            a += (x < m);
-            b += (y < m);
-            c += (z < m);
-          }
-        }
-      }
-    }
-    /* candidate d of the wave belongs to the first lane whose inclusive
-     * count exceeds d, and sits at slot d + s_off of that lane */
-    const uint32_t mine = at - rel;
-    uint32_t incl = mine;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const uint32_t y = (uint32_t)__shfl_up((int)incl, d, 64);
-      if (lane >= d) incl += y;
-    }
-    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-    const bool spilled = __ballot(at > CAP) != 0; /* wave-uniform */
-    s_end[wv][lane] = incl;
-    s_off[wv][lane] = rel - (incl - mine);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    /* First precision stage.  A written position is at most the number of
-     * the candidate it holds, and that at most its slot: an unread spilled
-     * candidate lies past every position written before it. */
+    const uint32_t k = kd & kEnd;
+    /* the wave's first slot */
+    const uint32_t q0 = __builtin_amdgcn_readfirstlane((uint32_t)q);
+    const uint32_t e0 = __builtin_amdgcn_readfirstlane(eij);
+    const uint64_t base = off ? off[q0] : tet_slot_off(roff, trow, e0, q0);
     const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
     uint32_t run = 0; /* kept + undecided written so far (wave-uniform) */
     bool und = false;
-    for (uint32_t d0 = 0; d0 < total; d0 += 64) {
-      const uint32_t d = d0 + (uint32_t)lane;
-      int t = 0; /* last lane with an inclusive count <= d, plus one */
+    auto wave_sync = [] {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
+    auto prefix = [&](uint32_t x) {
 #pragma unroll
-      for (int h = 32; h >= 1; h >>= 1)
-        t += s_end[wv][t + h - 1] <= d ? h : 0;
-      t &= 63; /* (d past the last candidate) */
-      const uint32_t ti = (uint32_t)__shfl((int)i, t, 64);
-      const uint32_t tj = (uint32_t)__shfl((int)j, t, 64);
-      const uint32_t tk = (uint32_t)__shfl((int)k, t, 64);
-      uint4 v = make_uint4(ti, tj, tk, 0u);
-      int r = REJECT;
-      if (d < total) {
-        const uint32_t slot = d + s_off[wv][t];
-        /* (two branches: one load through a selected pointer would be a
-         * flat one) */
-        uint32_t ld = 0;
-        if (!spilled) {
-          ld = s_l[wv][slot];
+      for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)x, d, 64);
+        if (lane >= d) x += y;
+      }
+      return x;
+    };
+    /* candidates 0 .. total - 1 of the wave, `step` at a time */
+    const bool masks = __ballot((mij.x | mik.x | mjk.x) >> 63) == 0;
+    uint4* const tab = s_raw[wv];
+    uint16_t* const list = reinterpret_cast<uint16_t*>(s_raw[wv] + 192);
+    uint32_t* const s_l = reinterpret_cast<uint32_t*>(s_raw[wv]);
+    uint32_t* const s_end = s_l + CAP;
+    uint32_t* const s_off = s_end + 64;
+    uint32_t* const spill = reinterpret_cast<uint32_t*>(ctet + base);
+    uint32_t total, step, at = 0, lo = 0, hi = 0;
+    bool spilled = false;
+    if (masks) {
+      /* By masks: l in T(i,j) after k and in T(i,k) are the common bits of
+       * the two edges' masks, both over the edges (i,.) that follow (i,k);
+       * l is the next triangle of T(i,j) but as many as `after` has bits
+       * before it, and the edge (j,l) recorded there has its bit in the
+       * mask of (j,k) if (j,k,l) is a triangle.  A triangle without slots
+       * (a chunk sub-input's unowned one) has no candidates. */
+      const uint32_t d = (eik - eij) & 63u; /* 1 .. 63 */
+      const uint64_t after = mij.x >> d;
+      const uint64_t dead = (mij.y >> d) | mik.y | ((kd & kDeadBit) ? ~0ull : 0ull);
+      uint64_t both = after & mik.x;
+      if (off && q < nt && off[q] == off[q + 1]) both = 0;
+      tab[3 * lane] = make_uint4((uint32_t)after, (uint32_t)(after >> 32),
+                                 (uint32_t)dead, (uint32_t)(dead >> 32));
+      tab[3 * lane + 1] =
+          make_uint4((uint32_t)mjk.x, (uint32_t)(mjk.x >> 32),
+                     (uint32_t)mjk.y, (uint32_t)(mjk.y >> 32));
+      tab[3 * lane + 2] = make_uint4(i, j, k, ejk + 1u);
+      const uint32_t incl = prefix((uint32_t)__popcll(both));
+      at = incl - (uint32_t)__popcll(both);
+      total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+      step = LIST;
+      lo = (uint32_t)both;
+      hi = (uint32_t)(both >> 32);
+    } else {
+      /* By merges, where a row is too long for some mask: the three rows
+       * are merged by each lane into a stage of fourth vertices from its
+       * triangle's first slot on.
+       * the triangle's slots [o, oe): off[] per triangle, or (roff) the
+       * closed form, a triangle's slots being its row's tail */
+      uint64_t o = 0, oe = 0;
+      if (q < nt) {
+        if (off) {
+          o = off[q];
+          oe = off[q + 1];
         } else {
-          if (slot < CAP) ld = s_l[wv][slot];
-          if (slot >= CAP) ld = spill[4 * (uint64_t)slot];
+          o = tet_slot_off(roff, trow, eij, (uint32_t)q);
+          oe = o + (trow[eij + 1] - (uint64_t)q - 1);
         }
-        v.w = ld & kEnd;
-        const Ball bv[4] = {S.ball[v.x], S.ball[v.y], S.ball[v.z], S.ball[v.w]};
-        /* the weights are first used after the test of D's sign; left
-         * alone, the compiler loads them there, a second round trip per
-         * round; used here (an empty asm), each ball is one 16-byte load */
+      }
+      /* the wave's slots, numbered from its first one; [rel, end) this
+       * lane's, cut at the arrays' end */
+      const uint32_t rel = (uint32_t)(o - base);
+      const uint32_t end =
+          o >= lim ? rel : rel + (uint32_t)((oe < lim ? oe : lim) - o);
+      at = rel;
+      auto put = [&](uint32_t v) {
+        ++found;
+        if (at < end) {
+          if (at < CAP) s_l[at] = v;
+          else spill[4 * (uint64_t)at] = v;
+          ++at;
+        }
+      };
+      /* two merge steps a round: each list's next element is loaded with
+       * its current one (kEnd past the row's end, above every ball id) */
+      if (o < oe) {
+        if constexpr (BUF) {
+          /* byte offsets into tkd (below 4 GiB): no 64-bit address
+           * arithmetic per load */
+          const BufU32 K{tkd, (uint32_t)(c_nt.cap * 4)};
+          uint32_t a = ((uint32_t)q + 1u) << 2, ae = (uint32_t)trow[eij + 1] << 2;
+          uint32_t b = (uint32_t)trow[eik] << 2, be = (uint32_t)trow[eik + 1] << 2;
+          uint32_t c = (uint32_t)trow[ejk] << 2, ce = (uint32_t)trow[ejk + 1] << 2;
+          while (a < ae && b < be && c < ce) {
+            const uint32_t xd0 = K.at(a), yd0 = K.at(b), zd0 = K.at(c);
+            const uint32_t xd1 = a + 4u < ae ? K.at(a + 4u) : kEnd;
+            const uint32_t yd1 = b + 4u < be ? K.at(b + 4u) : kEnd;
+            const uint32_t zd1 = c + 4u < ce ? K.at(c + 4u) : kEnd;
+            const uint32_t x0 = xd0 & kEnd, y0 = yd0 & kEnd, z0 = zd0 & kEnd;
+            const uint32_t m0 = max(x0, max(y0, z0));
+            const bool all0 = x0 == m0 && y0 == m0 && z0 == m0;
+            if (all0) put(m0 | ((kd | xd0 | yd0 | zd0) & kDeadBit));
+            const bool sa = all0 || x0 < m0, sb = all0 || y0 < m0,
+                       sc = all0 || z0 < m0;
+            const uint32_t xd = sa ? xd1 : xd0, yd = sb ? yd1 : yd0,
+                           zd = sc ? zd1 : zd0;
+            const uint32_t x = xd & kEnd, y = yd & kEnd, z = zd & kEnd;
+            const uint32_t m = max(x, max(y, z));
+            const bool all = x == m && y == m && z == m;
+            if (all && m != kEnd) put(m | ((kd | xd | yd | zd) & kDeadBit));
+            a += (sa ? 4u : 0u) + ((all || x < m) ? 4u : 0u);
+            b += (sb ? 4u : 0u) + ((all || y < m) ? 4u : 0u);
+            c += (sc ? 4u : 0u) + ((all || z < m) ? 4u : 0u);
+          }
+        } else {
+          /* alpha-triangle ids fit 32 bits (the slot count is checked below
+           * 2^32): 32-bit cursors halve the merge's index arithmetic */
+          uint32_t a = (uint32_t)q + 1, ae = (uint32_t)trow[eij + 1];
+          uint32_t b = (uint32_t)trow[eik], be = (uint32_t)trow[eik + 1];
+          uint32_t c = (uint32_t)trow[ejk], ce = (uint32_t)trow[ejk + 1];
+          while (a < ae && b < be && c < ce) {
+            const uint32_t xd = tkd[a], yd = tkd[b], zd = tkd[c];
+            const uint32_t x = xd & kEnd, y = yd & kEnd, z = zd & kEnd;
+            const uint32_t m = max(x, max(y, z));
+            if (x == m && y == m && z == m) {
+              put(m | ((kd | xd | yd | zd) & kDeadBit));
+              ++a;
+              ++b;
+              ++c;
+            } else {
+              a += (x < m);
+              b += (y < m);
+              c += (z < m);
+            }
+          }
+        }
+      }
+      const uint32_t mine = at - rel;
+      const uint32_t incl = prefix(mine);
+      total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+      step = total;
+      spilled = __ballot(at > CAP) != 0; /* wave-uniform */
+      s_end[lane] = incl;
+      s_off[lane] = rel - (incl - mine);
+      s_off[64 + lane] = i;
+      s_off[128 + lane] = j;
+      s_off[192 + lane] = k;
+    }
+    /* A written position is at most the number of the candidate it holds,
+     * and that at most its slot: an unread spilled candidate lies past
+     * every position written before it. */
+    for (uint32_t w0 = 0; w0 < total; w0 += step) {
+      const uint32_t wn = min(total - w0, step), we = w0 + wn;
+      if (masks) { /* list the bits of this pass: (triangle, bit) */
+        while (lo && at < we) {
+          list[at - w0] = (uint16_t)(lane << 6 | __builtin_ctz(lo));
+          lo &= lo - 1;
+          ++at;
+        }
+        while (!lo && hi && at < we) {
+          list[at - w0] = (uint16_t)(lane << 6 | 32 | __builtin_ctz(hi));
+          hi &= hi - 1;
+          ++at;
+        }
+      }
+      wave_sync();
+      for (uint32_t d0 = 0; d0 < wn; d0 += 64) {
+        const uint32_t d = d0 + (uint32_t)lane;
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        bool have = d < wn, dead = false;
+        if (masks) {
+          if (have) {
+            const uint32_t e = list[d], t = e >> 6, b = e & 63u;
+            const uint4 x = tab[3 * t], y = tab[3 * t + 1], z = tab[3 * t + 2];
+            const uint64_t ax = (uint64_t)x.y << 32 | x.x;
+            /* (bit b of `after` is set: the count includes it) */
+            const uint32_t tl = q0 + t + (uint32_t)__popcll(ax << (63u - b));
+            const uint32_t p = tejk[tl] - z.w, ld = tkd[tl];
+            const uint32_t mm = p & 32u ? y.y : y.x, md = p & 32u ? y.w : y.z;
+            have = p < 63u && ((mm >> (p & 31u)) & 1u);
+            dead = (((b & 32u ? x.w : x.z) >> (b & 31u)) | (md >> (p & 31u))) & 1u;
+            v = make_uint4(z.x, z.y, z.z, ld & kEnd);
+            found += have;
+          }
+        } else {
+          /* of the first lane whose inclusive count exceeds d, at slot
+           * d + s_off of that lane */
+          int t = 0; /* last lane with an inclusive count <= d, plus one */
 #pragma unroll
-        for (int z = 0; z < 4; ++z) asm volatile("" ::"v"(bv[z].w));
-        r = tet_code_ss<R>(bv, S.alpha);
-        if ((ld & kDeadBit) && r == KEEP) { /* alpha, certainly not empty */
-          ++dropped;
-          r = REJECT;
+          for (int h = 32; h >= 1; h >>= 1)
+            t += s_end[t + h - 1] <= d ? h : 0;
+          t &= 63; /* (d past the last candidate) */
+          if (have) {
+            const uint32_t slot = d + s_off[t];
+            uint32_t ld = 0;
+            /* (two branches: one load through a selected pointer would be a
+             * flat one) */
+            if (!spilled) {
+              ld = s_l[slot];
+            } else {
+              if (slot < CAP) ld = s_l[slot];
+              if (slot >= CAP) ld = spill[4 * (uint64_t)slot];
+            }
+            dead = (ld & kDeadBit) != 0;
+            v = make_uint4(s_off[64 + t], s_off[128 + t], s_off[192 + t],
+                           ld & kEnd);
+          }
         }
+        /* the first precision stage */
+        int r = REJECT;
+        if (have) {
+          const Ball bv[4] = {S.ball[v.x], S.ball[v.y], S.ball[v.z],
+                              S.ball[v.w]};
+          /* the weights are first used after the test of D's sign; left
+           * alone, the compiler loads them there, a second round trip per
+           * round; used here (an empty asm), each ball is one 16-byte load */
+#pragma unroll
+          for (int z = 0; z < 4; ++z) asm volatile("" ::"v"(bv[z].w));
+          r = tet_code_ss<R>(bv, S.alpha);
+          if (dead && r == KEEP) { /* alpha, certainly not empty */
+            ++dropped;
+            r = REJECT;
+          }
+        }
+        const uint64_t bm = __ballot(r != REJECT);
+        if (r != REJECT) {
+          const uint64_t w = base + run + (uint32_t)__popcll(bm & lt);
+          if (w < lim) {
+            ctet[w] = v;
+            flag[w] = (uint8_t)r;
+            if (r == UNDEC) push_q(q1, (uint32_t)w, v.x);
+          }
+        }
+        und |= __ballot(r == UNDEC) != 0;
+        run += (uint32_t)__popcll(bm);
       }
-      const uint64_t bm = __ballot(r != REJECT);
-      if (r != REJECT) {
-        const uint64_t w = base + run + (uint32_t)__popcll(bm & lt);
-        ctet[w] = v;
-        flag[w] = (uint8_t)r;
-        if (r == UNDEC) push_q(q1, (uint32_t)w, v.x);
-      }
-      und |= __ballot(r == UNDEC) != 0;
-      run += (uint32_t)__popcll(bm);
+      wave_sync(); /* the next pass rewrites the list */
     }
     if (lane == 0) {
       bbase[seg] = base;
@@ -1009,8 +1106,8 @@ void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
                             const uint32_t* tkd, const uint32_t* tedge,
                             const uint32_t* teik, const uint32_t* tejk,
                             const uint32_t* eleft, const uint32_t* ecol,
-                            const uint64_t* off, const uint64_t* roff,
-                            uint64_t* bbase, uint4* ctet, uint8_t* flag,
+                            const ulonglong2* emask, const uint64_t* off,
+                            const uint64_t* roff, uint64_t* bbase, uint4* ctet, uint8_t* flag,
                             uint32_t* bcnt, uint32_t* bkeep, Queue q1,
                             PipeLaunch L, uint64_t lim) {
   if (nt.cap <= 0) return;
@@ -1022,16 +1119,16 @@ void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
       auto kf = buf ? k_tet_enum_filter<float, true>
                     : k_tet_enum_filter<float, false>;
       hipLaunchKernelGGL(kf, gr, dim3(kBlock), 0, L.s, S, nt, trow, tkd, tedge,
-                         teik, tejk, eleft, ecol, off, roff, bbase, ctet, flag,
-                         bcnt, bkeep, q1, lim);
+                         teik, tejk, eleft, ecol, emask, off, roff, bbase, ctet,
+                         flag, bcnt, bkeep, q1, lim);
       return;
     }
   }
   auto kd = buf ? k_tet_enum_filter<double, true>
                 : k_tet_enum_filter<double, false>;
   hipLaunchKernelGGL(kd, gr, dim3(kBlock), 0, L.s, S, nt, trow, tkd, tedge, teik,
-                     tejk, eleft, ecol, off, roff, bbase, ctet, flag, bcnt,
-                     bkeep, q1, lim);
+                     tejk, eleft, ecol, emask, off, roff, bbase, ctet, flag,
+                     bcnt, bkeep, q1, lim);
 }
 
 /* kSegLanes lanes per enumeration segment in the two kernels below: a tet
@@ -1445,14 +1542,17 @@ void launch_tri_enum_filter(const Stage& S, Cnt ne, const uint64_t* erow,
  * holding index ne) = bout[b] + the block's kept triangles of edges
  * before e (counted per edge in LDS, then scanned).  tkd: tk with
  * kDeadBit set where one of the triangle's edges is marked in edead (null:
- * none).  Grid: nblk + 1 blocks, nblk = ceil(ne.cap / 256); bout has
+ * none).  emask[e], e = (i,j): x has bit r if (i, j, k) is a triangle and
+ * (i, k) the (r + 1)th edge after e, y the bits of those with kDeadBit; bit
+ * 63 is set if some r is 63 or more.  Grid: nblk + 1 blocks, nblk = ceil(ne.cap / 256); bout has
  * nblk + 1 entries. */
 __global__ __launch_bounds__(kBlock) void k_tri_block_copy(
     Cnt c_ne, const uint64_t* off, const uint32_t* bcnt, const uint32_t* cval,
     const uint32_t* cseg, const uint32_t* cea, const uint32_t* ceb,
     const uint8_t* flag, const uint64_t* bout, const uint8_t* edead,
     uint32_t* tk, uint32_t* tkd, uint32_t* tedge, uint32_t* teik,
-    uint32_t* tejk, uint64_t* trow, uint64_t* tpair, uint64_t ocap) {
+    uint32_t* tejk, uint64_t* trow, uint64_t* tpair, ulonglong2* emask,
+    uint64_t ocap) {
   const int64_t ne = c_ne.get();
   const int64_t b = blockIdx.x;
   const int64_t q0 = b * kBlock;
@@ -1461,8 +1561,16 @@ __global__ __launch_bounds__(kBlock) void k_tri_block_copy(
    * rewritten two rounds later, after the next round's barrier */
   __shared__ unsigned s_wsum[2][kBlock / 64];
   __shared__ uint32_t s_cnt[kBlock];
+  __shared__ unsigned long long s_mask[2][kBlock];
   s_cnt[threadIdx.x] = 0;
+  s_mask[0][threadIdx.x] = s_mask[1][threadIdx.x] = 0;
   __syncthreads();
+  auto mark = [&](uint32_t e, uint32_t eik, uint32_t xd) {
+    const uint32_t r = eik - e - 1u;
+    const unsigned long long bit = 1ull << (r < 63u ? r : 63u);
+    atomicOr(&s_mask[0][e - (uint32_t)q0], bit);
+    if (xd & kDeadBit) atomicOr(&s_mask[1][e - (uint32_t)q0], bit);
+  };
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
   const uint64_t o0 = bout[b];
@@ -1509,6 +1617,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_block_copy(
           tedge[at] = seg;
           teik[at] = av;
           tejk[at] = bv;
+          mark(seg, av, xd);
         }
         o += min((uint32_t)kBlock, n - r0);
         continue;
@@ -1529,11 +1638,12 @@ __global__ __launch_bounds__(kBlock) void k_tri_block_copy(
         tedge[pre] = seg;
         teik[pre] = av;
         tejk[pre] = bv;
+        mark(seg, av, xd);
       }
       o += tot;
     }
   }
-  __syncthreads(); /* the per-edge counts complete */
+  __syncthreads(); /* the per-edge counts and masks complete */
   /* exclusive scan of the per-edge counts (one wave per 64 edges, then
    * the wave totals) */
   const uint32_t c = s_cnt[threadIdx.x];
@@ -1554,6 +1664,8 @@ __global__ __launch_bounds__(kBlock) void k_tri_block_copy(
     const uint64_t v = before + incl - c;
     trow[e] = v < ocap ? v : ocap;
   }
+  if (e < ne)
+    emask[e] = make_ulonglong2(s_mask[0][threadIdx.x], s_mask[1][threadIdx.x]);
   /* the tet slots of the edge's triangles (each one's row tail) */
   if (tpair && e < ne) tpair[e] = c ? (uint64_t)c * (c - 1) / 2 : 0;
 }
@@ -1563,12 +1675,12 @@ void launch_tri_block_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
                            const uint8_t* flag, const uint64_t* bout,
                            const uint8_t* edead, uint32_t* tk, uint32_t* tkd,
                            uint32_t* tedge, uint32_t* teik, uint32_t* tejk,
-                           uint64_t* trow, uint64_t* tpair, PipeLaunch L,
-                           uint64_t ocap) {
+                           uint64_t* trow, uint64_t* tpair, ulonglong2* emask,
+                           PipeLaunch L, uint64_t ocap) {
   const int64_t nblk = (std::max<int64_t>(ne.cap, 0) + kBlock - 1) / kBlock;
   hipLaunchKernelGGL(k_tri_block_copy, dim3((unsigned)(nblk + 1)), dim3(kBlock),
                      0, L.s, ne, off, bcnt, cval, cseg, cea, ceb, flag, bout,
-                     edead, tk, tkd, tedge, teik, tejk, trow, tpair, ocap);
+                     edead, tk, tkd, tedge, teik, tejk, trow, tpair, emask, ocap);
 }
 
 template <int KIND>

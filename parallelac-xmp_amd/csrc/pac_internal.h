@@ -501,8 +501,8 @@ void launch_tri_block_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
                            const uint8_t* flag, const uint64_t* bout,
                            const uint8_t* edead, uint32_t* tk, uint32_t* tkd,
                            uint32_t* tedge, uint32_t* teik, uint32_t* tejk,
-                           uint64_t* trow, uint64_t* tpair, PipeLaunch L,
-                           uint64_t ocap = ~0ull);
+                           uint64_t* trow, uint64_t* tpair, ulonglong2* emask,
+                           PipeLaunch L, uint64_t ocap = ~0ull);
 /* tet candidates of the alpha triangles, each filtered by the first
  * precision stage in the same kernel; enumeration segment b (kTetSeg alpha
  * triangles) writes its kept and undecided tets (i, j, k, l) with their
@@ -518,10 +518,10 @@ void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
                             const uint32_t* tkd, const uint32_t* tedge,
                             const uint32_t* teik, const uint32_t* tejk,
                             const uint32_t* eleft, const uint32_t* ecol,
-                            const uint64_t* off, const uint64_t* roff,
-                            uint64_t* bbase, uint4* ctet, uint8_t* flag,
-                            uint32_t* bcnt, uint32_t* bkeep, Queue q1,
-                            PipeLaunch L, uint64_t lim = ~0ull);
+                            const ulonglong2* emask, const uint64_t* off,
+                            const uint64_t* roff, uint64_t* bbase, uint4* ctet,
+                            uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep,
+                            Queue q1, PipeLaunch L, uint64_t lim = ~0ull);
 /* The triangle and tet enumerations also write bkeep[b]: bcnt[b] when the
  * segment queued no undecided candidate (the ladder cannot drop any of its
  * entries), else kRecount. */

@@ -589,6 +589,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   const bool tail_slots = !SG.chunk;
   DBuf<uint64_t> tpair(P, tail_slots ? std::max<int64_t>(Ealpha.cap, 1) : 1);
   DBuf<uint32_t> tk, tkd, tedge, teik, tejk;
+  DBuf<ulonglong2> emask(P, std::max<int64_t>(Ealpha.cap, 1));
   uint8_t* const dead = edead.get();
   CandCtx C1{eleft.get(), ecol.get(), nullptr, nullptr, nullptr};
   {
@@ -647,7 +648,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     launch_tri_block_copy(Ealpha, off.get(), bcnt.get(), cval.get(), cseg.get(),
                           cea.get(), ceb.get(), flag.get(), bout.get(), dead,
                           tk.get(), tkd.get(), tedge.get(), teik.get(), tejk.get(), trow.get(),
-                          tail_slots ? tpair.get() : nullptr, L,
+                          tail_slots ? tpair.get() : nullptr, emask.get(), L,
                           (uint64_t)Talpha.cap);
     KCHK();
   }
@@ -703,7 +704,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           }
           launch_tet_enum_filter(SG, Talpha, trow.get(), tkd.get(), tedge.get(),
                                  teik.get(), tejk.get(), eleft.get(), ecol.get(),
-                                 tail_slots ? nullptr : off.get(),
+                                 emask.get(), tail_slots ? nullptr : off.get(),
                                  tail_slots ? roff.get() : nullptr, bbase.get(),
                                  ctet.get(), flag.get(), bcnt.get(), bkeep.get(),
                                  qq, L, (uint64_t)Kslots.cap);

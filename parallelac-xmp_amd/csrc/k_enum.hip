@@ -1,20 +1,20 @@
 /*
  * k_enum.hip -- binning, candidate enumeration and the alpha filters.
  *
- * One thread per ball / alpha edge / alpha triangle enumerates its
- * candidates (cells of the stencil, sorted-row intersections, three-way
- * merges), classifies each with one precision stage (FP32 on the staged
- * path, FP64 on the plain path) and appends undecided candidates to a
+ * Waves enumerate the candidates of a ball or of 64 alpha edges or
+ * triangles (cells of the stencil, rows in each other by bitmaps and masks),
+ * 64 at a time whatever item they belong to, classify each with one precision stage (FP32 on the staged
+ * path, FP64 on the plain path) and append undecided candidates to a
  * queue.  The escalation kernel re-decides them in FP64 then double-double;
  * what is still undecided goes to the wide-integer kernel.
  *
  * Reference kernels restated (AlphaComplexLargeData.cu unless noted):
  *   k_cell_key           computeCellIndex :65-78
- *   k_edge_count/fill    computePossibleEdgeCount / fillPotentialEdges
+ *   k_edge_count, k_edge_enum_filter  computePossibleEdgeCount / fillPotentialEdges
  *                        :80-165 + markRealEdges :167-190 (fused)
- *   k_tri_count/fill     computePossibleTriangleCount / fillPossibleTriangles
+ *   k_tri_hits, k_tri_enum_filter  computePossibleTriangleCount / fillPossibleTriangles
  *                        :192-296 + markRealTriangles :298-348 (fused)
- *   k_tet_count/fill     computePossibleTetCount / fillPossibleTets :350-529
+ *   k_tet_enum_filter    computePossibleTetCount / fillPossibleTets :350-529
  *                        + markRealTets :531-591 (fused)
  */
 #include "pac_dev.h"
@@ -636,60 +636,141 @@ void launch_tet_caps(const Stage& S, Cnt m, const uint64_t* trow,
                      cap);
 }
 
-/* number of triangles of alpha edge q = (i,j): the size of row(i) after j
- * intersected with row(j) (computePossibleTriangleCount, Parallel:232-266) */
-template <bool BUF>
-__global__ __launch_bounds__(kBlock) void k_tri_count(Cnt c_ne,
-                                                     const uint64_t* erow,
-                                                     const uint32_t* ecol,
-                                                     const uint32_t* eleft,
-                                                     uint32_t* cnt,
-                                                     unsigned long long* ts) {
-  stamp(ts, 3);
-  const int64_t ne = c_ne.get();
-  int64_t q = gtid();
-  if (q >= ne) return;
-  uint32_t i = eleft[q], j = ecol[q];
-  uint32_t c = 0;
-  if constexpr (BUF) {
-    /* byte offsets into ecol (below 4 GiB): no 64-bit address
-     * arithmetic per load */
-    const BufU32 E{ecol, (uint32_t)(c_ne.cap * 4)};
-    uint32_t a = ((uint32_t)q + 1u) << 2, ae = (uint32_t)erow[i + 1] << 2;
-    uint32_t b = (uint32_t)erow[j] << 2, be = (uint32_t)erow[j + 1] << 2;
-    /* two merge steps a round: each list's next element is loaded with
-     * its current one (~0u past the row's end, above every ball id) */
-    while (a < ae && b < be) {
-      const uint32_t x0 = E.at(a), y0 = E.at(b);
-      const uint32_t x1 = a + 4u < ae ? E.at(a + 4u) : ~0u;
-      const uint32_t y1 = b + 4u < be ? E.at(b + 4u) : ~0u;
-      const bool sa = x0 <= y0, sb = y0 <= x0;
-      const uint32_t x = sa ? x1 : x0, y = sb ? y1 : y0;
-      c += (x0 == y0) + (x == y && x != ~0u);
-      a += (sa ? 4u : 0u) + (x <= y ? 4u : 0u);
-      b += (sb ? 4u : 0u) + (y <= x ? 4u : 0u);
-    }
-  } else {
-    /* alpha-edge ids fit 32 bits (the candidate count is checked below
-     * 2^32), and 32-bit cursors halve the merge's index arithmetic */
-    uint32_t a = (uint32_t)q + 1, ae = (uint32_t)erow[i + 1];
-    uint32_t b = (uint32_t)erow[j], be = (uint32_t)erow[j + 1];
-    while (a < ae && b < be) {
-      const uint32_t x = ecol[a], y = ecol[b];
-      c += (x == y);
-      a += (x <= y);
-      b += (y <= x);
-    }
-  }
-  cnt[q] = c;
+/* orders a wave's LDS and global accesses before those after it */
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
-void launch_tri_count(Cnt ne, const uint64_t* erow, const uint32_t* ecol,
-                      const uint32_t* eleft, uint32_t* cnt,
-                      unsigned long long* ts, PipeLaunch L) {
+/* inclusive sum over the lanes */
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t x) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t y = (uint32_t)__shfl_up((int)x, d, 64);
+    if (lane >= d) x += y;
+  }
+  return x;
+}
+/* of n entries from base on, those below lim (the arrays' end, which only a
+ * recorded pass over its capacity reaches) */
+__device__ __forceinline__ uint32_t cut_at(uint32_t n, uint64_t base,
+                                           uint64_t lim) {
+  const uint64_t room = base < lim ? lim - base : 0;
+  return n < room ? n : (uint32_t)room;
+}
+/* the third vertices of alpha edge (i, j) are row(i) after j, from a on,
+ * merged with row(j): hit(k, a, b) for each */
+template <class F>
+__device__ __forceinline__ void merge_rows(const uint32_t* ecol, uint32_t a,
+                                           uint32_t ae, uint32_t b,
+                                           uint32_t be, F&& hit) {
+  while (a < ae && b < be) {
+    const uint32_t x = ecol[a], y = ecol[b];
+    if (x == y) hit(x, a, b);
+    a += (x <= y);
+    b += (y <= x);
+  }
+}
+struct __attribute__((packed, aligned(4))) U4a4 { /* 16 bytes at any word */
+  uint32_t x, y, z, w;
+};
+/* Triangle candidates of the alpha edges (computePossibleTriangleCount,
+ * Parallel:232-266), a wave per kTriSeg = 64 edges, an edge q = (i, j) a
+ * lane: bit t of hits[q] is set if the t-th of row(j) may be in row(i), and
+ * cnt[seg] is the wave's number of such bits.
+ * The rows of a wave's few i are contiguous in ecol: each goes into an LDS
+ * bitmap over the ids modulo its size (512 words shared by the wave's i, so
+ * usually 4,096 bits for the ~20 ids of a row), and a lane tests its row(j),
+ * four ids a load, instead of merging it with row(i).  The few false hits
+ * are dropped by the enumeration; they cost a slot each.
+ * A wave with a row(j) of more than 128 ids counts by merges and leaves no
+ * bits.  39 us at 100k balls (10.6 at 16068), 85 (20) with every lane
+ * merging its rows; the loads of the rows and the LDS reads bound it.  ecol is readable up to kEcolPad words past its end. */
+__global__ __launch_bounds__(kBlock) void k_tri_hits(
+    Cnt c_ne, const uint64_t* erow, const uint32_t* ecol,
+    const uint32_t* eleft, ulonglong2* hits, uint32_t* cnt,
+    unsigned long long* ts) {
+  static_assert(kTriSeg == 64, "an edge a lane");
+  stamp(ts, 3);
+  constexpr int W = 512; /* words of a wave's bitmaps */
+  __shared__ uint4 s_raw[kBlock / 64][W / 4];
+  const int64_t ne = c_ne.get();
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t seg = gtid() >> 6, q = gtid();
+  if (seg * kTriSeg >= ne) { /* a segment past the (device) count */
+    if (lane == 0 && seg * kTriSeg < c_ne.cap) cnt[seg] = 0;
+    return;
+  }
+  const bool act = q < ne;
+  uint32_t i = ~0u, j = 0, b = 0, len = 0;
+  if (act) {
+    i = eleft[q];
+    j = ecol[q];
+    b = (uint32_t)erow[j];
+    len = (uint32_t)erow[j + 1] - b;
+  }
+  uint32_t n = 0;
+  if (__ballot(len > 128u) != 0) {
+    if (act)
+      merge_rows(ecol, (uint32_t)q + 1u, (uint32_t)erow[i + 1], b, b + len,
+                 [&](uint32_t, uint32_t, uint32_t) { ++n; });
+  } else {
+    /* the wave's different i: this lane's is number `rank` of them */
+    const uint32_t pi = (uint32_t)__shfl_up((int)i, 1, 64);
+    const uint64_t heads = __ballot(act && (lane == 0 || i != pi));
+    const int nd = __popcll(heads);
+    const int rank = __popcll(heads & (~0ull >> (63 - lane))) - 1;
+    const int sh = nd > 1 ? 9 - (32 - __builtin_clz((unsigned)nd - 1u)) : 9;
+    const uint32_t wm = (1u << sh) - 1u;
+    uint32_t* const bm = reinterpret_cast<uint32_t*>(s_raw[wv]);
+    s_raw[wv][lane] = s_raw[wv][64 + lane] = make_uint4(0u, 0u, 0u, 0u);
+    wave_sync();
+    if (act) atomicOr(&bm[(rank << sh) + ((j >> 5) & wm)], 1u << (j & 31u));
+    if (seg * kTriSeg + 64 < ne) { /* the rest of the last row */
+      const uint32_t il = (uint32_t)__builtin_amdgcn_readlane((int)i, 63);
+      const uint32_t ae = (uint32_t)erow[il + 1];
+      for (uint32_t a = (uint32_t)(seg * kTriSeg) + 64u + (uint32_t)lane; a < ae;
+           a += 64) {
+        const uint32_t y = ecol[a];
+        atomicOr(&bm[((nd - 1) << sh) + ((y >> 5) & wm)], 1u << (y & 31u));
+      }
+    }
+    wave_sync();
+    const uint32_t* const mine = bm + (act ? rank << sh : 0);
+    uint32_t h[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      if (__ballot(len > 32u * w) == 0) break;
+      uint32_t x = 0;
+      for (uint32_t t = 0; t < 32 && __ballot(len > 32u * w + t) != 0; t += 4) {
+        U4a4 y = {0u, 0u, 0u, 0u};
+        if (32u * w + t < len)
+          y = *reinterpret_cast<const U4a4*>(ecol + b + 32u * w + t);
+        x |= (((mine[(y.x >> 5) & wm] >> (y.x & 31u)) & 1u) |
+              ((mine[(y.y >> 5) & wm] >> (y.y & 31u)) & 1u) << 1 |
+              ((mine[(y.z >> 5) & wm] >> (y.z & 31u)) & 1u) << 2 |
+              ((mine[(y.w >> 5) & wm] >> (y.w & 31u)) & 1u) << 3)
+             << t;
+      }
+      /* (the ids past the row's end) */
+      const uint32_t left = len > 32u * w ? len - 32u * w : 0u;
+      h[w] = left >= 32u ? x : x & ((1u << left) - 1u);
+      n += (uint32_t)__popc(h[w]);
+    }
+    if (act)
+      hits[q] = make_ulonglong2((uint64_t)h[1] << 32 | h[0],
+                                (uint64_t)h[3] << 32 | h[2]);
+  }
+  n = wave_prefix(n);
+  if (lane == 63) cnt[seg] = n;
+}
+void launch_tri_hits(Cnt ne, const uint64_t* erow, const uint32_t* ecol,
+                     const uint32_t* eleft, ulonglong2* hits, uint32_t* cnt,
+                     unsigned long long* ts, PipeLaunch L) {
   if (ne.cap <= 0) return;
-  auto kf = ne.cap < ((int64_t)1 << 30) ? k_tri_count<true> : k_tri_count<false>;
-  hipLaunchKernelGGL(kf, dim3((unsigned)((ne.cap + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, ne, erow, ecol, eleft, cnt, ts);
+  hipLaunchKernelGGL(k_tri_hits, dim3((unsigned)((ne.cap + kBlock - 1) / kBlock)),
+                     dim3(kBlock), 0, L.s, ne, erow, ecol, eleft, hits, cnt, ts);
 }
 
 /* ------------------------------------------------------------------ */
@@ -779,7 +860,7 @@ constexpr int fam_of(int KIND) {
  * (computePossibleTetCount / fillPossibleTets, Parallel:418-543), fused
  * with the tet filter's first stage (markRealTets, :531-591).
  * A wave takes kTetSeg = 64 triangles, one a lane, whose candidate slots
- * are one contiguous range.  The masks that k_tri_block_copy left per alpha
+ * are one contiguous range.  The masks that k_tri_seg_copy left per alpha
  * edge give each triangle the l in both T(i,j) after k and T(i,k) as the set
  * bits of one 64-bit word; the wave lists them in LDS and takes them 64 at a
  * time, whatever triangle they belong to: is (j,k,l) a triangle (a bit of
@@ -790,7 +871,7 @@ constexpr int fam_of(int KIND) {
  * or more edges on: dense inputs) merges the three rows instead, each lane
  * its own, into fourth vertices in LDS (928 of them, the rest in the
  * candidates' own array).
- * At 100k balls 277 us; 395 with all waves merging, whose rounds last as
+ * At 100k balls 271 us; 395 with all waves merging, whose rounds last as
  * long as their longest rows; 523 with blocks of 256 triangles filtering
  * every slot.  200k balls with a lattice block: 1.39 ms against 1.70 and
  * 9.6.  The vector ALU bounds it, the filter's 114 instructions being half
@@ -803,13 +884,14 @@ constexpr int fam_of(int KIND) {
  * the triangles of edge e occupy rows trow[e] .. trow[e+1]-1 and each has
  * its row's tail after it as slots, so triangle s + k of a row of L = trow
  * [e+1] - s triangles starts k (L - 1) - k (k - 1) / 2 slots into the
- * edge's range, which begins at roff[e] (the exclusive scan over edges of
- * L (L - 1) / 2). */
+ * edge's range, which begins at the sum of L (L - 1) / 2 over the edges
+ * before: roff[] of the segment of kTriSeg edges plus epre[e] within it. */
 __device__ __forceinline__ uint64_t tet_slot_off(const uint64_t* roff,
+                                                 const uint32_t* epre,
                                                  const uint64_t* trow,
                                                  uint32_t e, uint32_t q) {
   const uint64_t s = trow[e], L = trow[e + 1] - s, k = (uint64_t)q - s;
-  return roff[e] + k * (L - 1) - k * (k - 1) / 2;
+  return roff[e / kTriSeg] + epre[e] + k * (L - 1) - k * (k - 1) / 2;
 }
 /* FP32 first stage: 8 waves per SIMD (at most 64 VGPRs, no spills; the
  * LDS stage admits 8 blocks per CU); FP64: the compiler's choice */
@@ -819,8 +901,8 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
     Stage S, Cnt c_nt, const uint64_t* trow, const uint32_t* tkd,
     const uint32_t* tedge, const uint32_t* teik, const uint32_t* tejk,
     const uint32_t* eleft, const uint32_t* ecol, const ulonglong2* emask,
-    const uint64_t* off, const uint64_t* roff, uint64_t* bbase, uint4* ctet,
-    uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep, Queue q1, uint64_t lim) {
+    const uint64_t* off, const uint64_t* roff, const uint32_t* epre,
+    uint64_t* bbase, uint4* ctet, uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep, Queue q1, uint64_t lim) {
   static_assert(kTetSeg == 64, "a triangle a lane");
   stamp(S.ts, 4);
   /* LDS of a wave, 4,992 bytes (8 blocks per CU): by masks, three rows of
@@ -857,23 +939,10 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
     /* the wave's first slot */
     const uint32_t q0 = __builtin_amdgcn_readfirstlane((uint32_t)q);
     const uint32_t e0 = __builtin_amdgcn_readfirstlane(eij);
-    const uint64_t base = off ? off[q0] : tet_slot_off(roff, trow, e0, q0);
+    const uint64_t base = off ? off[q0] : tet_slot_off(roff, epre, trow, e0, q0);
     const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
     uint32_t run = 0; /* kept + undecided written so far (wave-uniform) */
     bool und = false;
-    auto wave_sync = [] {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    };
-    auto prefix = [&](uint32_t x) {
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)x, d, 64);
-        if (lane >= d) x += y;
-      }
-      return x;
-    };
     /* candidates 0 .. total - 1 of the wave, `step` at a time */
     const bool masks = __ballot((mij.x | mik.x | mjk.x) >> 63) == 0;
     uint4* const tab = s_raw[wv];
@@ -902,7 +971,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
           make_uint4((uint32_t)mjk.x, (uint32_t)(mjk.x >> 32),
                      (uint32_t)mjk.y, (uint32_t)(mjk.y >> 32));
       tab[3 * lane + 2] = make_uint4(i, j, k, ejk + 1u);
-      const uint32_t incl = prefix((uint32_t)__popcll(both));
+      const uint32_t incl = wave_prefix((uint32_t)__popcll(both));
       at = incl - (uint32_t)__popcll(both);
       total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
       step = LIST;
@@ -920,7 +989,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
           o = off[q];
           oe = off[q + 1];
         } else {
-          o = tet_slot_off(roff, trow, eij, (uint32_t)q);
+          o = tet_slot_off(roff, epre, trow, eij, (uint32_t)q);
           oe = o + (trow[eij + 1] - (uint64_t)q - 1);
         }
       }
@@ -993,7 +1062,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
         }
       }
       const uint32_t mine = at - rel;
-      const uint32_t incl = prefix(mine);
+      const uint32_t incl = wave_prefix(mine);
       total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
       step = total;
       spilled = __ballot(at > CAP) != 0; /* wave-uniform */
@@ -1093,6 +1162,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
       }
       wave_sync(); /* the next pass rewrites the list */
     }
+    run = cut_at(run, base, lim);
     if (lane == 0) {
       bbase[seg] = base;
       bcnt[seg] = run;
@@ -1107,7 +1177,8 @@ void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
                             const uint32_t* teik, const uint32_t* tejk,
                             const uint32_t* eleft, const uint32_t* ecol,
                             const ulonglong2* emask, const uint64_t* off,
-                            const uint64_t* roff, uint64_t* bbase, uint4* ctet, uint8_t* flag,
+                            const uint64_t* roff, const uint32_t* epre,
+                            uint64_t* bbase, uint4* ctet, uint8_t* flag,
                             uint32_t* bcnt, uint32_t* bkeep, Queue q1,
                             PipeLaunch L, uint64_t lim) {
   if (nt.cap <= 0) return;
@@ -1119,7 +1190,7 @@ void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
       auto kf = buf ? k_tet_enum_filter<float, true>
                     : k_tet_enum_filter<float, false>;
       hipLaunchKernelGGL(kf, gr, dim3(kBlock), 0, L.s, S, nt, trow, tkd, tedge,
-                         teik, tejk, eleft, ecol, emask, off, roff, bbase, ctet,
+                         teik, tejk, eleft, ecol, emask, off, roff, epre, bbase, ctet,
                          flag, bcnt, bkeep, q1, lim);
       return;
     }
@@ -1127,7 +1198,7 @@ void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
   auto kd = buf ? k_tet_enum_filter<double, true>
                 : k_tet_enum_filter<double, false>;
   hipLaunchKernelGGL(kd, gr, dim3(kBlock), 0, L.s, S, nt, trow, tkd, tedge, teik,
-                     tejk, eleft, ecol, emask, off, roff, bbase, ctet, flag,
+                     tejk, eleft, ecol, emask, off, roff, epre, bbase, ctet, flag,
                      bcnt, bkeep, q1, lim);
 }
 
@@ -1140,10 +1211,10 @@ __device__ __forceinline__ unsigned seg_ballot(bool p) {
   return (unsigned)(__ballot(p) >> first) & ((1u << kSegLanes) - 1u);
 }
 /* After the ladder: the kept candidates of each enumeration segment of
- * `seg` items (its first bcnt[b] positions from off[b * stride] hold its
+ * `seg` items (its first bcnt[b] positions from off[b] on hold its
  * kept and formerly undecided ones). */
 __global__ __launch_bounds__(kBlock) void k_seg_kept(
-    Cnt c_n, int seg, const uint64_t* off, int stride, const uint32_t* bcnt,
+    Cnt c_n, int seg, const uint64_t* off, const uint32_t* bcnt,
     const uint8_t* flag, uint32_t* bkeep) {
   const int64_t n = c_n.get();
   const int64_t nseg = (c_n.cap + seg - 1) / seg;
@@ -1154,7 +1225,7 @@ __global__ __launch_bounds__(kBlock) void k_seg_kept(
   if (b >= nseg || bkeep[b] != kRecount) return;
   unsigned c = 0;
   if (b * seg < n) {
-    const uint64_t base = off[b * stride];
+    const uint64_t base = off[b];
     const uint32_t m = bcnt[b];
     for (uint32_t r0 = 0; r0 < m; r0 += kSegLanes) {
       const uint32_t t = r0 + sub;
@@ -1193,15 +1264,13 @@ __global__ __launch_bounds__(kBlock) void k_tet_seg_copy(
     o += (unsigned)__popc(bm);
   }
 }
-void launch_seg_kept(Cnt n, int seg, const uint64_t* off, int stride,
-                     const uint32_t* bcnt, const uint8_t* flag, uint32_t* bkeep,
-                     PipeLaunch L) {
+void launch_seg_kept(Cnt n, int seg, const uint64_t* off, const uint32_t* bcnt,
+                     const uint8_t* flag, uint32_t* bkeep, PipeLaunch L) {
   if (n.cap <= 0) return;
   const int64_t nseg = (n.cap + seg - 1) / seg;
   hipLaunchKernelGGL(k_seg_kept,
                      dim3((unsigned)((nseg * kSegLanes + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, n, seg, off, stride, bcnt, flag,
-                     bkeep);
+                     dim3(kBlock), 0, L.s, n, seg, off, bcnt, flag, bkeep);
 }
 void launch_tet_seg_copy(Cnt nt, const uint64_t* bbase, const uint32_t* bcnt,
                          const uint4* ctet, const uint8_t* flag,
@@ -1302,7 +1371,7 @@ __global__ __launch_bounds__(kBlock) void k_edge_enum_filter(
     /* the next pass rewrites the tables */
     __builtin_amdgcn_wave_barrier();
   }
-  if (lane == 0) bcnt[i] = (uint32_t)(o - o0);
+  if (lane == 0) bcnt[i] = cut_at((uint32_t)(o - o0), o0, lim);
 }
 void launch_edge_enum_filter(const Stage& S, const uint64_t* off,
                              uint32_t* cval, uint32_t* cseg, uint8_t* flag,
@@ -1338,10 +1407,11 @@ void launch_seg_keep(int64_t n, const uint64_t* off, const uint32_t* bcnt,
                      dim3(kBlock), 0, L.s, n, off, bcnt, flag, keep);
 }
 /* ball i's kept edges (one wave per ball) to (ecol, eleft)[erow[i], ...),
- * their marks in edead (if given) cleared for the triangle stage */
+ * their marks in edead (if given) cleared for the triangle stage; erow cut
+ * at the arrays' end */
 __global__ __launch_bounds__(kBlock) void k_edge_copy(
     int64_t n, const uint64_t* off, const uint32_t* bcnt, const uint32_t* cval,
-    const uint8_t* flag, const uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
+    const uint8_t* flag, uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
     uint8_t* edead, uint64_t ocap) {
   const int64_t iw = (int64_t)blockIdx.x * kEdgeBallsPerBlock + (threadIdx.x >> 6);
   if (iw >= n) return;
@@ -1351,6 +1421,9 @@ __global__ __launch_bounds__(kBlock) void k_edge_copy(
   const uint64_t base = off[i];
   const uint32_t m = bcnt[i];
   uint64_t o = erow[i];
+  /* (a recorded pass over its capacity: rows end at the arrays' end) */
+  if (lane == 0 && o > ocap) erow[i] = ocap;
+  if (lane == 0 && i + 1 == n && erow[n] > ocap) erow[n] = ocap;
   for (uint32_t t0 = 0; t0 < m; t0 += 64) {
     const uint32_t t = t0 + lane;
     const bool keep = t < m && flag[base + t] == KEEP;
@@ -1368,7 +1441,7 @@ __global__ __launch_bounds__(kBlock) void k_edge_copy(
 }
 void launch_edge_copy(int64_t n, const uint64_t* off, const uint32_t* bcnt,
                       const uint32_t* cval, const uint8_t* flag,
-                      const uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
+                      uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
                       uint8_t* edead, PipeLaunch L, uint64_t ocap) {
   if (n <= 0) return;
   hipLaunchKernelGGL(
@@ -1381,306 +1454,330 @@ void launch_edge_copy(int64_t n, const uint64_t* off, const uint32_t* bcnt,
 /* Triangles of alpha edge q = (i, j) -- k in row(i) after j and in row(j),
  * the positions of k in the two rows being the alpha-edge ids of (i, k)
  * and (j, k), recorded for the tet stage and the closure -- fused with the
- * triangle filter's first stage (markRealTriangles, Parallel:1294-1340):
- * the block's candidate slots are staged in LDS during the row merges,
- * filtered round robin (uniform work per lane) and the kept and undecided
- * ones written compacted, in slot order, from the block's first slot on
- * (as in k_tet_enum_filter), four arrays and the flag; the filter never
- * reads an array the enumeration wrote for every slot.
+ * triangle filter's first stage (markRealTriangles, Parallel:1294-1340).
+ * A wave takes the kTriSeg edges and hits of k_tri_hits: it lists the hits
+ * (edge, position in row(j)) in LDS and takes them 64 at a time: k's
+ * position in row(i) by a binary search in the wave's part of ecol, which is
+ * in LDS (none: a false hit), then the filter; the kept and undecided ones
+ * are written compacted, in order, from the wave's first slot on, four
+ * arrays and the flag.
+ * 121 us at 100k balls (30 at 16068), 211 (48) for blocks of 256 edges that
+ * merged the rows into LDS and filtered them from there, waiting for their
+ * longest rows and at two barriers a round.
+ * A wave with a row too long for the hits or the LDS merges its rows into
+ * the slots themselves and filters them from there: each round's 64 are read
+ * before any is written, to positions not past them.
  * edead (alpha edges, cleared; may be null): set for the edges a rejected
  * candidate shows covered by one ball (tri_code_ss): no simplex with such
  * an edge is empty. */
-template <class R, bool BUF>
+template <class R>
 __global__ __launch_bounds__(kBlock) void k_tri_enum_filter(
     Stage S, Cnt c_ne, const uint64_t* erow, const uint32_t* ecol,
-    const uint32_t* eleft, const uint64_t* off, uint32_t* cval,
-    uint32_t* cseg, uint32_t* cea, uint32_t* ceb, uint8_t* flag,
-    uint32_t* bcnt, uint32_t* bkeep, uint8_t* edead, Queue q1, uint64_t lim) {
+    const uint32_t* eleft, const ulonglong2* hits, const uint64_t* off,
+    uint32_t* cval, uint32_t* cseg, uint32_t* cea, uint32_t* ceb,
+    uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep, uint8_t* edead, Queue q1,
+    uint64_t lim) {
+  /* with the tables 4,096 bytes of LDS a wave: 8 blocks per CU */
+  constexpr uint32_t LIST = 1152, COLS = 192;
+  __shared__ uint4 s_tab[kBlock / 64][64];
+  __shared__ uint32_t s_col[kBlock / 64][COLS];
+  __shared__ uint16_t s_list[kBlock / 64][LIST];
   const int64_t ne = c_ne.get();
-  /* 6 blocks per CU fit in LDS with the edge table and block_flush's 16 B
-   * (a block averages ~1,800 slots on the 100k globule; the rest go to
-   * global memory: measured 6 > 5 > 8 blocks per CU) */
-  constexpr int CAP = 1570;
-  __shared__ uint32_t s_out[4 * CAP];
-  __shared__ uint2 s_ij[kBlock]; /* the block's edges (i, j) */
-  const int64_t q0 = (int64_t)blockIdx.x * kBlock;
-  if (q0 >= ne) { /* whole block past the (device) count */
-    if (threadIdx.x == 0) bcnt[blockIdx.x] = bkeep[blockIdx.x] = 0;
-    return;
-  }
-  __shared__ unsigned s_und; /* an undecided candidate written */
-  if (threadIdx.x == 0) s_und = 0;
-  const int64_t q1e = q0 + kBlock < ne ? q0 + kBlock : ne;
-  BlockOut<4, CAP> B{s_out, off[q0], off[q1e] - off[q0], lim};
-  uint32_t* const g[4] = {cval, cseg, cea, ceb};
-  const int64_t q = gtid();
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t seg = gtid() >> 6, q = gtid();
   unsigned found = 0;
-  if (q < ne) {
-    const uint32_t i = eleft[q], j = ecol[q];
-    s_ij[threadIdx.x] = make_uint2(i, j);
-    uint64_t o = off[q];
-    if constexpr (BUF) { /* byte offsets into ecol, as in k_tri_count */
-      const BufU32 E{ecol, (uint32_t)(c_ne.cap * 4)};
-      uint32_t a = ((uint32_t)q + 1u) << 2, ae = (uint32_t)erow[i + 1] << 2;
-      uint32_t b = (uint32_t)erow[j] << 2, be = (uint32_t)erow[j + 1] << 2;
-      /* two merge steps a round, as in k_tri_count */
-      while (a < ae && b < be) {
-        const uint32_t x0 = E.at(a), y0 = E.at(b);
-        const uint32_t x1 = a + 4u < ae ? E.at(a + 4u) : ~0u;
-        const uint32_t y1 = b + 4u < be ? E.at(b + 4u) : ~0u;
-        if (x0 == y0) {
-          const uint32_t v[4] = {x0, (uint32_t)q, a >> 2, b >> 2};
-          B.put(g, o, v);
-          ++o;
-          ++found;
-        }
-        const bool sa = x0 <= y0, sb = y0 <= x0;
-        a += sa ? 4u : 0u;
-        b += sb ? 4u : 0u;
-        const uint32_t x = sa ? x1 : x0, y = sb ? y1 : y0;
-        if (x == y && x != ~0u) {
-          const uint32_t v[4] = {x, (uint32_t)q, a >> 2, b >> 2};
-          B.put(g, o, v);
-          ++o;
-          ++found;
-        }
-        a += x <= y ? 4u : 0u;
-        b += y <= x ? 4u : 0u;
-      }
+  if (seg * kTriSeg >= ne) { /* a segment past the (device) count */
+    if (lane == 0 && seg * kTriSeg < c_ne.cap) bcnt[seg] = bkeep[seg] = 0;
+  } else {
+    const uint32_t q0 = __builtin_amdgcn_readfirstlane((uint32_t)q);
+    const uint64_t base = off[seg];
+    uint32_t i = 0, j = 0, b = 0, len = 0, ae = 0;
+    ulonglong2 h = make_ulonglong2(0, 0);
+    if (q < ne) {
+      i = eleft[q];
+      j = ecol[q];
+      b = (uint32_t)erow[j];
+      len = (uint32_t)erow[j + 1] - b;
+      ae = (uint32_t)erow[i + 1];
+      h = hits[q];
+    }
+    const bool listed = __ballot(len > 128u || (q < ne && ae - q0 > COLS)) == 0;
+    const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+    uint32_t w4[4] = {0u, 0u, 0u, 0u};
+    uint32_t total, step, at = 0;
+    if (listed) {
+      w4[0] = (uint32_t)h.x;
+      w4[1] = (uint32_t)(h.x >> 32);
+      w4[2] = (uint32_t)h.y;
+      w4[3] = (uint32_t)(h.y >> 32);
+      const uint32_t n = (uint32_t)(__popcll(h.x) + __popcll(h.y));
+      const uint32_t incl = wave_prefix(n);
+      at = incl - n;
+      total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+      step = LIST;
+      s_tab[wv][lane] = make_uint4(i, j, ae - q0, b);
+      s_col[wv][lane] = j;
+      /* the rest of the last row */
+      const int last = ne - q0 < 64 ? (int)(ne - q0) - 1 : 63;
+      const uint32_t end = (uint32_t)__builtin_amdgcn_readlane((int)ae, last);
+      for (uint32_t t = 64u + (uint32_t)lane; q0 + t < end; t += 64)
+        s_col[wv][t] = ecol[q0 + t];
     } else {
-      uint32_t a = (uint32_t)q + 1, ae = (uint32_t)erow[i + 1];
-      uint32_t b = (uint32_t)erow[j], be = (uint32_t)erow[j + 1];
-      while (a < ae && b < be) {
-        const uint32_t x = ecol[a], y = ecol[b];
-        if (x == y) {
-          const uint32_t v[4] = {x, (uint32_t)q, (uint32_t)a, (uint32_t)b};
-          B.put(g, o, v);
-          ++o;
-          ++found;
+      uint32_t n = 0;
+      if (q < ne)
+        merge_rows(ecol, (uint32_t)q + 1u, ae, b, b + len,
+                   [&](uint32_t, uint32_t, uint32_t) { ++n; });
+      const uint32_t incl = wave_prefix(n);
+      total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+      uint64_t o = base + (incl - n);
+      if (q < ne)
+        merge_rows(ecol, (uint32_t)q + 1u, ae, b, b + len,
+                   [&](uint32_t k, uint32_t a, uint32_t bb) {
+                     if (o < lim) {
+                       cval[o] = k;
+                       cseg[o] = (uint32_t)q;
+                       cea[o] = a;
+                       ceb[o] = bb;
+                     }
+                     ++o;
+                   });
+      total = cut_at(total, base, lim);
+      step = total;
+    }
+    uint32_t run = 0; /* kept + undecided written so far (wave-uniform) */
+    bool und = false;
+    for (uint32_t w0 = 0; w0 < total; w0 += step) {
+      const uint32_t wn = min(total - w0, step), we = w0 + wn;
+      if (listed) { /* list the hits of this pass */
+        bool open = true; /* (all bits of the words before are listed) */
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          while (open && w4[w] && at < we) {
+            s_list[wv][at - w0] =
+                (uint16_t)(lane << 7 | w << 5 | __builtin_ctz(w4[w]));
+            w4[w] &= w4[w] - 1;
+            ++at;
+          }
+          open = open && !w4[w];
         }
-        a += (x <= y);
-        b += (y <= x);
       }
-    }
-  }
-  __syncthreads(); /* LDS stage, edge table and overflow slots written */
-  __shared__ unsigned s_wsum[kBlock / 64];
-  const uint64_t base = B.base;
-  const uint64_t m = base >= lim ? 0 : (B.total < lim - base ? B.total : lim - base);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-  uint32_t run = 0; /* kept + undecided written so far (block-uniform) */
-  for (uint64_t r0 = 0; r0 < m; r0 += kBlock) {
-    const uint64_t t = r0 + threadIdx.x;
-    uint32_t v[4] = {0u, 0u, 0u, 0u};
-    int r = REJECT;
-    if (t < m) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        v[k] = t < (uint64_t)CAP ? s_out[k * CAP + t] : g[k][base + t];
-      const uint2 ij = s_ij[v[1] - (uint32_t)q0];
-      const Ball b0 = S.ball[ij.x], b1 = S.ball[ij.y], b2 = S.ball[v[0]];
-      /* weights used here: one 16-byte load per ball (as for tets) */
-      asm volatile("" ::"v"(b0.w), "v"(b1.w), "v"(b2.w));
-      unsigned cover;
-      r = tri_code_ss<R>(b0, b1, b2, S.alpha, cover);
-      if (cover && edead) { /* opposite edges: (j, k), (i, k), (i, j) */
-        if (cover & 1u) edead[v[3]] = 1;
-        if (cover & 2u) edead[v[2]] = 1;
-        if (cover & 4u) edead[v[1]] = 1;
+      wave_sync();
+      for (uint32_t d0 = 0; d0 < wn; d0 += 64) {
+        const uint32_t d = d0 + (uint32_t)lane;
+        bool have = d < wn;
+        uint32_t vi = 0, vj = 0, k = 0, e = 0, ea = 0, eb = 0;
+        if (listed) {
+          if (have) {
+            const uint32_t x = s_list[wv][d], t = x >> 7;
+            const uint4 T = s_tab[wv][t];
+            eb = T.w + (x & 127u);
+            k = ecol[eb];
+            /* k among the ids after (i, j) in row(i) */
+            uint32_t lo = t + 1u, hi = T.z;
+            while (lo < hi) {
+              const uint32_t m = (lo + hi) >> 1;
+              const bool c = s_col[wv][m] < k;
+              lo = c ? m + 1u : lo;
+              hi = c ? hi : m;
+            }
+            have = lo < T.z && s_col[wv][lo] == k;
+            vi = T.x;
+            vj = T.y;
+            e = q0 + t;
+            ea = q0 + lo;
+          }
+        } else if (have) {
+          k = cval[base + d];
+          e = cseg[base + d];
+          ea = cea[base + d];
+          eb = ceb[base + d];
+          vi = eleft[e];
+          vj = ecol[e];
+        }
+        int r = REJECT;
+        if (have) {
+          ++found;
+          const Ball b0 = S.ball[vi], b1 = S.ball[vj], b2 = S.ball[k];
+          /* weights used here: one 16-byte load per ball (as for tets) */
+          asm volatile("" ::"v"(b0.w), "v"(b1.w), "v"(b2.w));
+          unsigned cover;
+          r = tri_code_ss<R>(b0, b1, b2, S.alpha, cover);
+          if (cover && edead) { /* opposite edges: (j, k), (i, k), (i, j) */
+            if (cover & 1u) edead[eb] = 1;
+            if (cover & 2u) edead[ea] = 1;
+            if (cover & 4u) edead[e] = 1;
+          }
+        }
+        const uint64_t bm = __ballot(r != REJECT);
+        if (r != REJECT) {
+          const uint64_t o = base + run + (uint32_t)__popcll(bm & lt);
+          if (o < lim) {
+            cval[o] = k;
+            cseg[o] = e;
+            cea[o] = ea;
+            ceb[o] = eb;
+            flag[o] = (uint8_t)r;
+            if (r == UNDEC) push_q(q1, (uint32_t)o, e);
+          }
+        }
+        und |= __ballot(r == UNDEC) != 0;
+        run += (uint32_t)__popcll(bm);
       }
+      wave_sync(); /* the next pass rewrites the list */
     }
-    const uint64_t bm = __ballot(r != REJECT);
-    if (lane == 0) s_wsum[w] = (unsigned)__popcll(bm);
-    __syncthreads();
-    uint32_t pre = run + (uint32_t)__popcll(bm & lt), tot = 0;
-#pragma unroll
-    for (int k = 0; k < kBlock / 64; ++k) {
-      const unsigned c = s_wsum[k];
-      if (k < w) pre += c;
-      tot += c;
+    run = cut_at(run, base, lim);
+    if (lane == 0) {
+      bcnt[seg] = run;
+      bkeep[seg] = und ? kRecount : run;
     }
-    if (r != REJECT) {
-      const uint64_t at = base + pre;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) g[k][at] = v[k];
-      flag[at] = (uint8_t)r;
-      if (r == UNDEC) {
-        push_q(q1, (uint32_t)at, v[1]);
-        s_und = 1;
-      }
-    }
-    run += tot;
-    __syncthreads(); /* s_wsum is rewritten next round */
-  }
-  if (threadIdx.x == 0) {
-    bcnt[blockIdx.x] = run;
-    bkeep[blockIdx.x] = s_und ? kRecount : run;
   }
   block_flush(S.ctr, CTR_CAND + 1, found);
 }
 void launch_tri_enum_filter(const Stage& S, Cnt ne, const uint64_t* erow,
                             const uint32_t* ecol, const uint32_t* eleft,
-                            const uint64_t* off, uint32_t* cval,
-                            uint32_t* cseg, uint32_t* cea, uint32_t* ceb,
-                            uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep,
-                            uint8_t* edead, Queue q1, PipeLaunch L,
-                            uint64_t lim) {
+                            const ulonglong2* hits, const uint64_t* off,
+                            uint32_t* cval, uint32_t* cseg, uint32_t* cea,
+                            uint32_t* ceb, uint8_t* flag, uint32_t* bcnt,
+                            uint32_t* bkeep, uint8_t* edead, Queue q1,
+                            PipeLaunch L, uint64_t lim) {
   if (ne.cap <= 0) return;
   dim3 gr((unsigned)((ne.cap + kBlock - 1) / kBlock));
-  /* byte offsets into ecol while it stays below 4 GiB */
-  const bool buf = ne.cap < ((int64_t)1 << 30);
-  auto kf = S.staged ? (buf ? k_tri_enum_filter<float, true>
-                            : k_tri_enum_filter<float, false>)
-                     : (buf ? k_tri_enum_filter<double, true>
-                            : k_tri_enum_filter<double, false>);
-  hipLaunchKernelGGL(kf, gr, dim3(kBlock), 0, L.s, S, ne, erow, ecol, eleft, off,
-                     cval, cseg, cea, ceb, flag, bcnt, bkeep, edead, q1, lim);
+  auto kf = S.staged ? k_tri_enum_filter<float> : k_tri_enum_filter<double>;
+  hipLaunchKernelGGL(kf, gr, dim3(kBlock), 0, L.s, S, ne, erow, ecol, eleft,
+                     hits, off, cval, cseg, cea, ceb, flag, bcnt, bkeep, edead,
+                     q1, lim);
 }
-/* the kept triangles of block b to (tk, tedge, teik, tejk)[bout[b], ...)
- * in order; trow[e] for the block's edges e (and trow[ne], by the block
- * holding index ne) = bout[b] + the block's kept triangles of edges
- * before e (counted per edge in LDS, then scanned).  tkd: tk with
- * kDeadBit set where one of the triangle's edges is marked in edead (null:
- * none).  emask[e], e = (i,j): x has bit r if (i, j, k) is a triangle and
- * (i, k) the (r + 1)th edge after e, y the bits of those with kDeadBit; bit
- * 63 is set if some r is 63 or more.  Grid: nblk + 1 blocks, nblk = ceil(ne.cap / 256); bout has
- * nblk + 1 entries. */
-__global__ __launch_bounds__(kBlock) void k_tri_block_copy(
+/* the kept triangles of segment b to (tk, tedge, teik, tejk)[bout[b], ...)
+ * in order, a wave each; trow[e] for its edges e (and trow[ne], by the wave
+ * holding index ne) = bout[b] + the kept triangles of its edges before e.
+ * tkd (if given): tk with kDeadBit set where one of the triangle's edges is
+ * marked in edead.  emask[e], e = (i,j): x has bit r if (i, j, k) is a
+ * triangle and (i, k) the (r + 1)th edge after e, y the bits of those with
+ * kDeadBit; bit 63 is set if some r is 63 or more.  spair, epre (if given):
+ * the tet slots of the segment's triangles (each one's row tail), and of
+ * those of its edges before e.  Grid: a wave per segment and one more; bout
+ * has one entry more than segments. */
+__global__ __launch_bounds__(kBlock) void k_tri_seg_copy(
     Cnt c_ne, const uint64_t* off, const uint32_t* bcnt, const uint32_t* cval,
     const uint32_t* cseg, const uint32_t* cea, const uint32_t* ceb,
     const uint8_t* flag, const uint64_t* bout, const uint8_t* edead,
     uint32_t* tk, uint32_t* tkd, uint32_t* tedge, uint32_t* teik,
-    uint32_t* tejk, uint64_t* trow, uint64_t* tpair, ulonglong2* emask,
-    uint64_t ocap) {
+    uint32_t* tejk, uint64_t* trow, uint64_t* spair, uint32_t* epre,
+    ulonglong2* emask, uint64_t ocap) {
+  __shared__ uint32_t s_cnt[kBlock / 64][64];
+  __shared__ unsigned long long s_mask[2][kBlock / 64][64];
   const int64_t ne = c_ne.get();
-  const int64_t b = blockIdx.x;
-  const int64_t q0 = b * kBlock;
-  if (q0 > ne) return;
-  /* wave sums double-buffered by round parity: a round's sums are
-   * rewritten two rounds later, after the next round's barrier */
-  __shared__ unsigned s_wsum[2][kBlock / 64];
-  __shared__ uint32_t s_cnt[kBlock];
-  __shared__ unsigned long long s_mask[2][kBlock];
-  s_cnt[threadIdx.x] = 0;
-  s_mask[0][threadIdx.x] = s_mask[1][threadIdx.x] = 0;
-  __syncthreads();
-  auto mark = [&](uint32_t e, uint32_t eik, uint32_t xd) {
-    const uint32_t r = eik - e - 1u;
-    const unsigned long long bit = 1ull << (r < 63u ? r : 63u);
-    atomicOr(&s_mask[0][e - (uint32_t)q0], bit);
-    if (xd & kDeadBit) atomicOr(&s_mask[1][e - (uint32_t)q0], bit);
-  };
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t b = gtid() >> 6, q0 = b * kTriSeg;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  if (q0 > ne) { /* a segment past the (device) count */
+    if (spair && lane == 0 && q0 < c_ne.cap) spair[b] = 0;
+    return;
+  }
+  s_cnt[wv][lane] = 0;
+  s_mask[0][wv][lane] = s_mask[1][wv][lane] = 0;
+  wave_sync();
   const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
   const uint64_t o0 = bout[b];
   if (q0 < ne) {
-    const uint64_t base = off[q0];
+    const uint64_t base = off[b];
     const uint32_t n = bcnt[b];
-    /* every entry kept (bout's step equals the written count): positions
-     * follow without ranking, and no flag is read */
+    /* every entry kept (bout's step equals the written count): no flag is
+     * read */
     const bool all = bout[b + 1] - o0 == n;
     uint64_t o = o0;
-    int par = 0;
-    for (uint32_t r0 = 0; r0 < n; r0 += kBlock, par ^= 1) {
-      const uint32_t t = r0 + threadIdx.x;
-      /* every load of the round in flight together: an entry's arrays are
-       * read whether or not it is kept (all were written) */
-      uint32_t fv = KEEP, sv = 0xffffffffu, xv = 0u, av = 0u, bv = 0u;
-      if (t < n) {
-        if (!all) fv = flag[base + t];
-        sv = cseg[base + t];
-        xv = cval[base + t];
-        av = cea[base + t];
-        bv = ceb[base + t];
-      }
-      const bool keep = t < n && fv == KEEP;
-      const uint32_t seg = keep ? sv : 0xffffffffu;
-      uint32_t xd = xv;
-      if (edead && keep && (edead[sv] | edead[av] | edead[bv])) xd |= kDeadBit;
-      /* entries come in edge order: one LDS add per run of lanes with
-       * the same edge (its first lane adds the run's length) instead of
-       * one per lane on the same counter */
-      const uint32_t prev = (uint32_t)__shfl_up((int)seg, 1, 64);
-      const uint64_t heads = __ballot(lane == 0 || prev != seg);
-      if (keep && ((heads >> lane) & 1ull)) {
-        const uint64_t later = lane == 63 ? 0ull : heads >> (lane + 1);
-        const unsigned len = later ? (unsigned)__builtin_ctzll(later) + 1u
-                                   : 64u - (unsigned)lane;
-        atomicAdd(&s_cnt[seg - (uint32_t)q0], len);
-      }
-      if (all) {
-        if (keep && o + t - r0 < ocap) {
-          const uint64_t at = o + t - r0;
-          tk[at] = xv;
-          tkd[at] = xd;
-          tedge[at] = seg;
-          teik[at] = av;
-          tejk[at] = bv;
-          mark(seg, av, xd);
-        }
-        o += min((uint32_t)kBlock, n - r0);
-        continue;
-      }
-      const uint64_t bm = __ballot(keep);
-      if (lane == 0) s_wsum[par][w] = (unsigned)__popcll(bm);
-      __syncthreads();
-      uint64_t pre = o + (uint64_t)__popcll(bm & lt), tot = 0;
+    /* kU entries a lane in flight together: the rounds' chains of loads are
+     * what the kernel waits for (139 us at 100k balls one by one, 122 by
+     * two, 115 by four; the bytes moved take 55) */
+    constexpr int kU = 4;
+    for (uint32_t r0 = 0; r0 < n; r0 += 64 * kU) {
+      /* an entry's arrays are read whether or not it is kept (all were
+       * written) */
+      uint32_t fv[kU], sv[kU], xv[kU], av[kU], bv[kU];
+      bool dead[kU];
 #pragma unroll
-      for (int k = 0; k < kBlock / 64; ++k) {
-        const unsigned c = s_wsum[par][k];
-        if (k < w) pre += c;
-        tot += c;
+      for (int u = 0; u < kU; ++u) {
+        const uint32_t t = r0 + 64u * u + (uint32_t)lane;
+        const uint64_t at = base + (t < n ? t : n - 1);
+        fv[u] = all ? (uint32_t)KEEP : flag[at];
+        sv[u] = cseg[at];
+        xv[u] = cval[at];
+        av[u] = cea[at];
+        bv[u] = ceb[at];
+        if (t >= n) fv[u] = REJECT;
       }
-      if (keep && pre < ocap) {
-        tk[pre] = xv;
-        tkd[pre] = xd;
-        tedge[pre] = seg;
-        teik[pre] = av;
-        tejk[pre] = bv;
-        mark(seg, av, xd);
+#pragma unroll
+      for (int u = 0; u < kU; ++u)
+        dead[u] = edead && (edead[sv[u]] | edead[av[u]] | edead[bv[u]]);
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        if (r0 + 64u * u >= n) break;
+        const bool keep = fv[u] == KEEP;
+        const uint32_t seg = keep ? sv[u] : 0xffffffffu;
+        /* entries come in edge order: one LDS add per run of lanes with
+         * the same edge (its first lane adds the run's length) instead of
+         * one per lane on the same counter */
+        const uint32_t prev = (uint32_t)__shfl_up((int)seg, 1, 64);
+        const uint64_t heads = __ballot(lane == 0 || prev != seg);
+        const uint64_t bm = __ballot(keep);
+        if (keep) {
+          const uint32_t e = seg - (uint32_t)q0;
+          if ((heads >> lane) & 1ull) {
+            const uint64_t later = lane == 63 ? 0ull : heads >> (lane + 1);
+            const unsigned len = later ? (unsigned)__builtin_ctzll(later) + 1u
+                                       : 64u - (unsigned)lane;
+            atomicAdd(&s_cnt[wv][e], len);
+          }
+          const uint64_t w = o + (uint64_t)__popcll(bm & lt);
+          if (w < ocap) {
+            tk[w] = xv[u];
+            if (tkd) tkd[w] = xv[u] | (dead[u] ? kDeadBit : 0u);
+            tedge[w] = seg;
+            teik[w] = av[u];
+            tejk[w] = bv[u];
+            const uint32_t r = av[u] - seg - 1u;
+            const unsigned long long bit = 1ull << (r < 63u ? r : 63u);
+            atomicOr(&s_mask[0][wv][e], bit);
+            if (dead[u]) atomicOr(&s_mask[1][wv][e], bit);
+          }
+        }
+        o += (uint64_t)__popcll(bm);
       }
-      o += tot;
     }
   }
-  __syncthreads(); /* the per-edge counts and masks complete */
-  /* exclusive scan of the per-edge counts (one wave per 64 edges, then
-   * the wave totals) */
-  const uint32_t c = s_cnt[threadIdx.x];
-  uint32_t incl = c;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t y = (uint32_t)__shfl_up((int)incl, d, 64);
-    if (lane >= d) incl += y;
-  }
-  if (lane == 63) s_wsum[0][w] = incl;
-  __syncthreads();
-  uint64_t before = o0;
-#pragma unroll
-  for (int k = 0; k < kBlock / 64; ++k)
-    if (k < w) before += s_wsum[0][k];
-  const int64_t e = q0 + threadIdx.x;
-  if (e <= ne) {
-    const uint64_t v = before + incl - c;
-    trow[e] = v < ocap ? v : ocap;
-  }
+  wave_sync(); /* the per-edge counts and masks complete */
+  const uint32_t c = s_cnt[wv][lane];
+  const int64_t e = q0 + lane;
+  const uint64_t v = o0 + (wave_prefix(c) - c);
+  if (e <= ne) trow[e] = v < ocap ? v : ocap;
   if (e < ne)
-    emask[e] = make_ulonglong2(s_mask[0][threadIdx.x], s_mask[1][threadIdx.x]);
-  /* the tet slots of the edge's triangles (each one's row tail) */
-  if (tpair && e < ne) tpair[e] = c ? (uint64_t)c * (c - 1) / 2 : 0;
+    emask[e] = make_ulonglong2(s_mask[0][wv][lane], s_mask[1][wv][lane]);
+  if (spair) {
+    const uint64_t m = c ? (uint64_t)c * (c - 1) / 2 : 0;
+    uint64_t x = m;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint64_t y = (uint64_t)__shfl_up((unsigned long long)x, d, 64);
+      if (lane >= d) x += y;
+    }
+    /* (2^32 slots or more end the run after their scan) */
+    if (e < ne) epre[e] = (uint32_t)(x - m);
+    if (lane == 63 && q0 < c_ne.cap) spair[b] = x;
+  }
 }
-void launch_tri_block_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
-                           const uint32_t* cval, const uint32_t* cseg,
-                           const uint32_t* cea, const uint32_t* ceb,
-                           const uint8_t* flag, const uint64_t* bout,
-                           const uint8_t* edead, uint32_t* tk, uint32_t* tkd,
-                           uint32_t* tedge, uint32_t* teik, uint32_t* tejk,
-                           uint64_t* trow, uint64_t* tpair, ulonglong2* emask,
-                           PipeLaunch L, uint64_t ocap) {
-  const int64_t nblk = (std::max<int64_t>(ne.cap, 0) + kBlock - 1) / kBlock;
-  hipLaunchKernelGGL(k_tri_block_copy, dim3((unsigned)(nblk + 1)), dim3(kBlock),
-                     0, L.s, ne, off, bcnt, cval, cseg, cea, ceb, flag, bout,
-                     edead, tk, tkd, tedge, teik, tejk, trow, tpair, emask, ocap);
+void launch_tri_seg_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
+                         const uint32_t* cval, const uint32_t* cseg,
+                         const uint32_t* cea, const uint32_t* ceb,
+                         const uint8_t* flag, const uint64_t* bout,
+                         const uint8_t* edead, uint32_t* tk, uint32_t* tkd,
+                         uint32_t* tedge, uint32_t* teik, uint32_t* tejk,
+                         uint64_t* trow, uint64_t* spair, uint32_t* epre,
+                         ulonglong2* emask, PipeLaunch L, uint64_t ocap) {
+  const int64_t nseg = (std::max<int64_t>(ne.cap, 0) + kTriSeg - 1) / kTriSeg;
+  hipLaunchKernelGGL(k_tri_seg_copy,
+                     dim3((unsigned)((nseg + kBlock / 64) / (kBlock / 64))),
+                     dim3(kBlock), 0, L.s, ne, off, bcnt, cval, cseg, cea, ceb,
+                     flag, bout, edead, tk, tkd, tedge, teik, tejk, trow, spair,
+                     epre, emask, ocap);
 }
 
 template <int KIND>

@@ -123,42 +123,6 @@ struct BufU32 {
   }
 };
 
-/* Block-staged output of a one-thread-per-segment enumeration.  The
- * segments of a block own the contiguous output range [base, base+total)
- * (their exclusive-scan offsets); each thread's entries go to LDS at their
- * offset within that range and the block writes the range out coalesced,
- * instead of 64 lanes each streaming into its own region.  Entries past
- * the LDS capacity CAP are stored directly. */
-template <int NARR, int CAP>
-struct BlockOut {
-  uint32_t* s; /* LDS, NARR x CAP */
-  uint64_t base, total;
-  uint64_t lim; /* capacity of the output arrays: entries at or past it are dropped */
-  __device__ __forceinline__ void put(uint32_t* const g[NARR], uint64_t o,
-                                      const uint32_t v[NARR]) {
-    if (o >= lim) return;
-    uint64_t lo = o - base;
-    if (lo < (uint64_t)CAP) {
-#pragma unroll
-      for (int a = 0; a < NARR; ++a) s[a * CAP + lo] = v[a];
-    } else {
-#pragma unroll
-      for (int a = 0; a < NARR; ++a) g[a][o] = v[a];
-    }
-  }
-  /* every thread of the block calls this once, after its last put */
-  __device__ __forceinline__ void flush(uint32_t* const g[NARR]) {
-    __syncthreads();
-    uint64_t m64 = total < (uint64_t)CAP ? total : (uint64_t)CAP;
-    if (base >= lim) m64 = 0;
-    else if (m64 > lim - base) m64 = lim - base;
-    const uint32_t m = (uint32_t)m64;
-    for (uint32_t t = threadIdx.x; t < m; t += blockDim.x)
-#pragma unroll
-      for (int a = 0; a < NARR; ++a) g[a][base + t] = s[a * CAP + t];
-  }
-};
-
 struct StageCnt {
   unsigned c[4];
   __device__ StageCnt() { c[0] = c[1] = c[2] = c[3] = 0; }

@@ -459,7 +459,7 @@ void launch_seg_keep(int64_t n, const uint64_t* off, const uint32_t* bcnt,
                      const uint8_t* flag, uint32_t* keep, PipeLaunch L);
 void launch_edge_copy(int64_t n, const uint64_t* off, const uint32_t* bcnt,
                       const uint32_t* cval, const uint8_t* flag,
-                      const uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
+                      uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
                       uint8_t* edead, PipeLaunch L, uint64_t ocap = ~0ull);
 /* slot capacity of item q = row[owner[q] + 1] - q - 1 */
 void launch_tail_caps(Cnt m, const uint64_t* row, const uint32_t* owner,
@@ -470,39 +470,44 @@ void launch_tet_caps(const Stage& S, Cnt m, const uint64_t* trow,
                      const uint32_t* tedge, const uint32_t* eleft,
                      const uint32_t* ecol, const uint32_t* tk, uint32_t* cap,
                      PipeLaunch L);
-/* exact triangle count per alpha edge */
-void launch_tri_count(Cnt ne, const uint64_t* erow, const uint32_t* ecol,
-                      const uint32_t* eleft, uint32_t* cnt,
-                      unsigned long long* ts, PipeLaunch L);
+/* the triangle candidates of each segment of kTriSeg alpha edges, or a few
+ * more (cnt), and per edge the positions of its own in row(j) (hits);
+ * ecol has kEcolPad readable words past its edges */
+constexpr int kTriSeg = 64, kEcolPad = 3;
+void launch_tri_hits(Cnt ne, const uint64_t* erow, const uint32_t* ecol,
+                     const uint32_t* eleft, ulonglong2* hits, uint32_t* cnt,
+                     unsigned long long* ts, PipeLaunch L);
 /* triangle candidates of the alpha edges, each filtered by the first
- * precision stage in the same kernel: enumeration block b (256 alpha
+ * precision stage in the same kernel: enumeration segment b (kTriSeg alpha
  * edges) writes its kept and undecided candidates (k, edge, edge(i,k),
  * edge(j,k)) with their flags, in order, compacted from its first slot
- * off[256 b] on and their number to bcnt[b]; undecided ones are queued on
+ * off[b] (the exclusive scan of launch_tri_hits's counts) on and their number to bcnt[b]; undecided ones are queued on
  * q1 by position (aux = their edge).  edead[e] (cleared by the caller;
  * null: not wanted) is set for the alpha edges a rejected candidate shows
  * covered by one ball: no simplex with such an edge is empty. */
 void launch_tri_enum_filter(const Stage& S, Cnt ne, const uint64_t* erow,
                             const uint32_t* ecol, const uint32_t* eleft,
-                            const uint64_t* off, uint32_t* cval,
-                            uint32_t* cseg, uint32_t* cea, uint32_t* ceb,
-                            uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep,
-                            uint8_t* edead, Queue q1, PipeLaunch L,
-                            uint64_t lim = ~0ull);
+                            const ulonglong2* hits, const uint64_t* off,
+                            uint32_t* cval, uint32_t* cseg, uint32_t* cea,
+                            uint32_t* ceb, uint8_t* flag, uint32_t* bcnt,
+                            uint32_t* bkeep, uint8_t* edead, Queue q1,
+                            PipeLaunch L, uint64_t lim = ~0ull);
 /* after the ladder (bkeep by launch_seg_kept over the ne alpha
- * edges, bout its exclusive scan): the kept triangles of each block to
- * (tk, tedge, teik, tejk) in order (tkd: tk with kDeadBit where one of the
- * three edges is marked in edead), the alpha-triangle row start of every
- * alpha edge, trow[0 .. ne], and (tpair, if given) each edge's tet slots,
- * L (L - 1) / 2 for its L triangles (each one's row tail) */
-void launch_tri_block_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
-                           const uint32_t* cval, const uint32_t* cseg,
-                           const uint32_t* cea, const uint32_t* ceb,
-                           const uint8_t* flag, const uint64_t* bout,
-                           const uint8_t* edead, uint32_t* tk, uint32_t* tkd,
-                           uint32_t* tedge, uint32_t* teik, uint32_t* tejk,
-                           uint64_t* trow, uint64_t* tpair, ulonglong2* emask,
-                           PipeLaunch L, uint64_t ocap = ~0ull);
+ * edges, bout its exclusive scan): the kept triangles of each segment to
+ * (tk, tedge, teik, tejk) in order (tkd, if given: tk with kDeadBit where one
+ * of the three edges is marked in edead), the alpha-triangle row start of
+ * every alpha edge, trow[0 .. ne], its third vertices as a mask (emask), and
+ * (spair, if given) the segment's tet slots, L (L - 1) / 2 for an edge of L
+ * triangles (each one's row tail), with epre[e] those before edge e in it */
+void launch_tri_seg_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
+                         const uint32_t* cval, const uint32_t* cseg,
+                         const uint32_t* cea, const uint32_t* ceb,
+                         const uint8_t* flag, const uint64_t* bout,
+                         const uint8_t* edead, uint32_t* tk, uint32_t* tkd,
+                         uint32_t* tedge, uint32_t* teik, uint32_t* tejk,
+                         uint64_t* trow, uint64_t* spair, uint32_t* epre,
+                         ulonglong2* emask, PipeLaunch L,
+                         uint64_t ocap = ~0ull);
 /* tet candidates of the alpha triangles, each filtered by the first
  * precision stage in the same kernel; enumeration segment b (kTetSeg alpha
  * triangles) writes its kept and undecided tets (i, j, k, l) with their
@@ -510,16 +515,17 @@ void launch_tri_block_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
  * number to bcnt[b]; undecided ones are queued on q1 by position.  Kept
  * tets one of whose triangles has kDeadBit in tkd are counted (CTR_DROP)
  * but not written.  Slot offsets per triangle from off[], or (off null)
- * from roff, the exclusive scan of launch_tri_block_copy's tpair (each
- * triangle's slots its row's tail: not for chunk sub-inputs, whose unowned
- * triangles get none) */
+ * from roff, the exclusive scan of launch_tri_seg_copy's spair, and epre
+ * (each triangle's slots its row's tail: not for chunk sub-inputs, whose
+ * unowned triangles get none) */
 constexpr int kTetSeg = 64;
 void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
                             const uint32_t* tkd, const uint32_t* tedge,
                             const uint32_t* teik, const uint32_t* tejk,
                             const uint32_t* eleft, const uint32_t* ecol,
                             const ulonglong2* emask, const uint64_t* off,
-                            const uint64_t* roff, uint64_t* bbase, uint4* ctet,
+                            const uint64_t* roff, const uint32_t* epre,
+                            uint64_t* bbase, uint4* ctet,
                             uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep,
                             Queue q1, PipeLaunch L, uint64_t lim = ~0ull);
 /* The triangle and tet enumerations also write bkeep[b]: bcnt[b] when the
@@ -529,10 +535,9 @@ constexpr uint32_t kRecount = 0xffffffffu;
 /* after the ladder: kept candidates per enumeration segment of `seg` items
  * (ceil(n.cap / seg) entries; segments marked kRecount recounted from their
  * flags), then, with bout their exclusive scan, the kept tets in order;
- * segment b's entries start at off[b * stride] (per-item offsets: stride
- * seg; per-segment bases: 1) */
-void launch_seg_kept(Cnt n, int seg, const uint64_t* off, int stride,
-                     const uint32_t* bcnt, const uint8_t* flag, uint32_t* bkeep,
+ * segment b's entries start at off[b] */
+void launch_seg_kept(Cnt n, int seg, const uint64_t* off, const uint32_t* bcnt,
+                     const uint8_t* flag, uint32_t* bkeep,
                      PipeLaunch L);
 void launch_tet_seg_copy(Cnt nt, const uint64_t* bbase, const uint32_t* bcnt,
                          const uint4* ctet, const uint8_t* flag,

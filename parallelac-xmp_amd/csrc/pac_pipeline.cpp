@@ -567,7 +567,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
                           dcnt + RC_EALPHA, post);
         },
         RC_EALPHA);
-    ecol = DBuf<uint32_t>(P, Ealpha.cap);
+    ecol = DBuf<uint32_t>(P, Ealpha.cap + kEcolPad);
     eleft = DBuf<uint32_t>(P, Ealpha.cap);
     if (prune) edead = DBuf<uint8_t>(P, Ealpha.cap);
     launch_edge_copy(n, off.get(), bcnt.get(), cval.get(), flag.get(),
@@ -576,44 +576,46 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     KCHK();
   } else {
     zero_u64((unsigned long long*)erow.get(), n + 1, s);
-    ecol = DBuf<uint32_t>(P, 1);
+    ecol = DBuf<uint32_t>(P, 1 + kEcolPad);
     eleft = DBuf<uint32_t>(P, 1);
   }
 
   /* ---- triangles (AlphaComplexParallel.cu:1279-1371) ---- */
   Cnt Tslots(0), Talpha(0);
   DBuf<uint64_t> trow(P, Ealpha.cap + 1);
-  /* the tet slots of each alpha edge's triangles (their row tails), for
+  const int64_t neseg = (Ealpha.cap + kTriSeg - 1) / kTriSeg;
+  /* the tet slots of the alpha edges' triangles (their row tails), for
    * the tets' slot offsets in closed form; chunk sub-inputs give unowned
    * triangles no slots and keep per-triangle offsets */
   const bool tail_slots = !SG.chunk;
-  DBuf<uint64_t> tpair(P, tail_slots ? std::max<int64_t>(Ealpha.cap, 1) : 1);
+  DBuf<uint64_t> spair(P, tail_slots ? std::max<int64_t>(neseg, 1) : 1);
+  DBuf<uint32_t> epre(P, tail_slots ? std::max<int64_t>(Ealpha.cap, 1) : 1);
   DBuf<uint32_t> tk, tkd, tedge, teik, tejk;
+  /* per alpha edge 128 bits: first its hits, then its mask of third
+   * vertices */
   DBuf<ulonglong2> emask(P, std::max<int64_t>(Ealpha.cap, 1));
   uint8_t* const dead = edead.get();
   CandCtx C1{eleft.get(), ecol.get(), nullptr, nullptr, nullptr};
   {
-    DBuf<uint64_t> off(P, Ealpha.cap + 1);
+    DBuf<uint64_t> off(P, neseg + 1);
     {
-      /* exact counts: a triangle's third vertex must be in both rows, and
-       * the merge that counts it is cheap next to filtering empty slots */
-      DBuf<uint32_t> cnt(P, Ealpha.cap);
-      launch_tri_count(Ealpha, erow.get(), ecol.get(), eleft.get(), cnt.get(), ts,
-                       L);
-      Tslots = count_scan(cnt.get(), Ealpha, off.get(), RC_TSLOTS, "triangle");
+      DBuf<uint32_t> cnt(P, std::max<int64_t>(neseg, 1));
+      launch_tri_hits(Ealpha, erow.get(), ecol.get(), eleft.get(), emask.get(),
+                      cnt.get(), ts, L);
+      Tslots = count_scan(cnt.get(), Cnt(neseg), off.get(), RC_TSLOTS,
+                          "triangle");
     }
     DBuf<uint32_t> cval(P, Tslots.cap), cseg(P, Tslots.cap),
         cea(P, Tslots.cap), ceb(P, Tslots.cap);
     DBuf<uint8_t> flag(P, Tslots.cap);
-    /* enumeration and first filter stage in one kernel, each block's kept
+    /* enumeration and first filter stage in one kernel, each segment's kept
      * and undecided candidates compacted in place (their count in bcnt);
      * the ladder settles the undecided ones; then the kept triangles of
-     * each block are counted, scanned and copied out in order with the
+     * each segment are counted, scanned and copied out in order with the
      * row starts (as for tets) */
-    const int64_t nblk = (Ealpha.cap + kBlock - 1) / kBlock;
-    DBuf<uint32_t> bcnt(P, nblk + 1), bkeep(P, nblk + 1);
-    DBuf<uint64_t> bout(P, nblk + 1);
-    auto tmp = scan_tmp(nblk);
+    DBuf<uint32_t> bcnt(P, neseg + 1), bkeep(P, neseg + 1);
+    DBuf<uint64_t> bout(P, neseg + 1);
+    auto tmp = scan_tmp(neseg);
     /* a rerun (queue overflow, eager only) recounts the candidates from
      * zero */
     int runs = 0;
@@ -623,9 +625,10 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           if (runs++ && !rec)
             zero_counter(ctr, CTR_CAND + 1, s);
           launch_tri_enum_filter(SG, Ealpha, erow.get(), ecol.get(), eleft.get(),
-                                 off.get(), cval.get(), cseg.get(), cea.get(),
-                                 ceb.get(), flag.get(), bcnt.get(), bkeep.get(),
-                                 dead, qq, L, (uint64_t)Tslots.cap);
+                                 emask.get(), off.get(), cval.get(), cseg.get(),
+                                 cea.get(), ceb.get(), flag.get(), bcnt.get(),
+                                 bkeep.get(), dead, qq, L,
+                                 (uint64_t)Tslots.cap);
         },
         [&](QRef qr, Queue q2) {
           launch_filter_esc(SG, 2, C1, qr, cval.get(), flag.get(), q2, L);
@@ -634,39 +637,43 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           launch_filter_exact(SG, 2, C1, qr, cval.get(), flag.get(), L);
         },
         [&](Post post) {
-          launch_seg_kept(Ealpha, kBlock, off.get(), kBlock, bcnt.get(),
-                          flag.get(), bkeep.get(), L);
-          scan_u32_to_u64(bkeep.get(), bout.get(), Cnt(nblk), tmp.get(), s,
+          launch_seg_kept(Ealpha, kTriSeg, off.get(), bcnt.get(), flag.get(),
+                          bkeep.get(), L);
+          scan_u32_to_u64(bkeep.get(), bout.get(), Cnt(neseg), tmp.get(), s,
                           dcnt + RC_TALPHA, post);
         },
         RC_TALPHA);
     tk = DBuf<uint32_t>(P, Talpha.cap);
-    tkd = DBuf<uint32_t>(P, Talpha.cap);
+    if (prune) tkd = DBuf<uint32_t>(P, Talpha.cap);
     tedge = DBuf<uint32_t>(P, Talpha.cap);
     teik = DBuf<uint32_t>(P, Talpha.cap);
     tejk = DBuf<uint32_t>(P, Talpha.cap);
-    launch_tri_block_copy(Ealpha, off.get(), bcnt.get(), cval.get(), cseg.get(),
-                          cea.get(), ceb.get(), flag.get(), bout.get(), dead,
-                          tk.get(), tkd.get(), tedge.get(), teik.get(), tejk.get(), trow.get(),
-                          tail_slots ? tpair.get() : nullptr, emask.get(), L,
-                          (uint64_t)Talpha.cap);
+    launch_tri_seg_copy(Ealpha, off.get(), bcnt.get(), cval.get(), cseg.get(),
+                        cea.get(), ceb.get(), flag.get(), bout.get(), dead,
+                        tk.get(), tkd.get(), tedge.get(), teik.get(),
+                        tejk.get(), trow.get(),
+                        tail_slots ? spair.get() : nullptr, epre.get(),
+                        emask.get(), L, (uint64_t)Talpha.cap);
     KCHK();
   }
+
+  /* the third vertices, marked with kDeadBit where edges are */
+  const uint32_t* const tkm = prune ? tkd.get() : tk.get();
 
   /* ---- tets (AlphaComplexParallel.cu:1381-1442) ---- */
   Cnt Kslots(0), Kalpha(0);
   DBuf<uint4> tets;
   CandCtx C2{eleft.get(), ecol.get(), tk.get(), tedge.get(), nullptr};
   {
-    /* slot offsets: per alpha edge in closed form (roff), or per alpha
-     * triangle from its cap (off, chunk sub-inputs) */
+    /* slot offsets: per segment of alpha edges in closed form (roff), or
+     * per alpha triangle from its cap (off, chunk sub-inputs) */
     DBuf<uint64_t> off, roff;
     if (tail_slots) {
-      roff = DBuf<uint64_t>(P, Ealpha.cap + 1);
+      roff = DBuf<uint64_t>(P, neseg + 1);
       const Post post = new_post(false);
       {
-        auto tmp = scan_tmp(Ealpha.cap);
-        scan_u64_to_u64(tpair.get(), roff.get(), Ealpha, tmp.get(), s,
+        auto tmp = scan_tmp(neseg);
+        scan_u64_to_u64(spair.get(), roff.get(), Cnt(neseg), tmp.get(), s,
                         dcnt + RC_KSLOTS, post);
       }
       KCHK();
@@ -680,7 +687,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
                       ecol.get(), tk.get(), cap.get(), L);
       Kslots = count_scan(cap.get(), Talpha, off.get(), RC_KSLOTS, "tet");
     }
-    tpair.release();
+    spair.release();
     DBuf<uint4> ctet(P, Kslots.cap);
     DBuf<uint8_t> flag(P, Kslots.cap);
     C2.ctet = ctet.get();
@@ -702,19 +709,20 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
             zero_counter(ctr, CTR_CAND + 2, s);
             zero_counter(ctr, CTR_DROP, s);
           }
-          launch_tet_enum_filter(SG, Talpha, trow.get(), tkd.get(), tedge.get(),
+          launch_tet_enum_filter(SG, Talpha, trow.get(), tkm, tedge.get(),
                                  teik.get(), tejk.get(), eleft.get(), ecol.get(),
                                  emask.get(), tail_slots ? nullptr : off.get(),
-                                 tail_slots ? roff.get() : nullptr, bbase.get(),
-                                 ctet.get(), flag.get(), bcnt.get(), bkeep.get(),
-                                 qq, L, (uint64_t)Kslots.cap);
+                                 tail_slots ? roff.get() : nullptr, epre.get(),
+                                 bbase.get(), ctet.get(), flag.get(),
+                                 bcnt.get(), bkeep.get(), qq, L,
+                                 (uint64_t)Kslots.cap);
         },
         [&](QRef qr, Queue q2) {
           launch_filter_esc(SG, 3, C2, qr, nullptr, flag.get(), q2, L);
         },
         [&](QRef qr) { launch_filter_exact(SG, 3, C2, qr, nullptr, flag.get(), L); },
         [&](Post post) {
-          launch_seg_kept(Talpha, kTetSeg, bbase.get(), 1, bcnt.get(),
+          launch_seg_kept(Talpha, kTetSeg, bbase.get(), bcnt.get(),
                           flag.get(), bkeep.get(), L);
           scan_u32_to_u64(bkeep.get(), bout.get(), Cnt(nblk), tmp.get(), s,
                           dcnt + RC_KALPHA, post);
@@ -864,7 +872,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       Tf = ladder(
           ac2_cap(Talpha.cap), KP_TRI_AC2, -1,
           [&](Queue q) {
-            launch_low_ac2_hot(SG, 0, Talpha, ecol.get(), eleft.get(), tkd.get(),
+            launch_low_ac2_hot(SG, 0, Talpha, ecol.get(), eleft.get(), tkm,
                                tedge.get(), nullptr, tri_skip, tflag.get(), q,
                                rest.get(), nrest, next.get(), nnext,
                                budget(Talpha), L);

@@ -12,6 +12,7 @@
  * in the reference's lexicographic order with no sort or merge.
  */
 #include "pac_dev.h"
+#include "pac_tiles.h"
 
 namespace pac {
 using namespace PAC_V; /* type-independent device helpers */
@@ -31,107 +32,91 @@ void launch_or_flags(Cnt n, const uint8_t* a, const uint8_t* b, uint8_t* out,
   hipLaunchKernelGGL(k_or_flags, dim3((unsigned)((n.cap + kBlock - 1) / kBlock)),
                      dim3(kBlock), 0, L.s, n, a, b, out);
 }
-/* out[pos[i]] = val[i] != 0 for the flagged i */
-/* faces of the final tets -> tri_in */
-__global__ __launch_bounds__(kBlock) void k_mark_faces(
-    Cnt c_nk, const uint4* ftets, const uint64_t* erow, const uint32_t* ecol,
-    const uint64_t* trow, const uint32_t* tk, uint8_t* tri_in,
+/* The final tets out of the alpha tets' flags, a tile of flags a block: each
+ * kept tet in original ids to out, and its faces marked in tri_in (cleared).
+ * t = (i, j, k, l), i < j < k < l: one pass over row i finds the edges ij, ik
+ * and il; the faces ijk and ijl are in the triangle row of ij, ikl in that of
+ * ik, jkl in that of jk, each at the number of bits before its own in the
+ * edge's mask (emask), and the edges jk and jl are recorded with the first
+ * two.  A row that its mask cuts off is searched instead. */
+__global__ __launch_bounds__(kBlock) void k_tile_tets(
+    Cnt c_nk, const uint4* tets, const uint8_t* flag, const uint64_t* offs,
+    const uint64_t* erow, const uint32_t* ecol, const ulonglong2* emask,
+    const uint64_t* trow, const uint32_t* tk, const uint32_t* tejk,
+    const uint32_t* perm, uint8_t* tri_in, int4* out, uint64_t ocap,
     unsigned long long* ts) {
   stamp(ts, 6);
-  const int64_t nk = c_nk.get();
-  int64_t id = gtid();
-  if (id >= nk) return;
-  /* t = (i, j, k, l), i < j < k < l: faces ijk and ijl in the row of
-   * edge ij, ikl in that of ik, jkl in that of jk; edges ij and ik are in
-   * row i, so two row scans find the three edges */
-  const uint4 t = ftets[id];
-  int64_t eij, eik, f, g;
-  find_row2(ecol, erow[t.x], erow[t.x + 1], t.y, t.z, eij, eik);
-  const int64_t ejk = find_row(ecol, erow[t.y], erow[t.y + 1], t.z);
-  if (eij >= 0) {
-    find_row2(tk, trow[eij], trow[eij + 1], t.z, t.w, f, g);
+  /* the triangle of edge e whose third vertex is v, e2 = (i, v) for e =
+   * (i, .); -1 if there is none (a recorded pass over its capacities) */
+  auto face = [&](uint32_t e, uint32_t e2, uint32_t v) -> int64_t {
+    const uint64_t m = emask[e].x, r0 = trow[e];
+    if (m >> 63) return find_row(tk, r0, trow[e + 1], v);
+    const uint32_t r = e2 - e - 1u;
+    if (r >= 63u || !((m >> r) & 1)) return -1;
+    return (int64_t)(r0 + (uint64_t)__popcll(m & ((1ull << r) - 1)));
+  };
+  tile_each(flag, c_nk.get(), offs, [&](int64_t id, uint64_t p) {
+    if (p >= ocap) return;
+    const uint4 t = tets[id];
+    out[p] = make_int4((int)perm[t.x], (int)perm[t.y], (int)perm[t.z],
+                       (int)perm[t.w]);
+    int64_t eij, eik, eil;
+    find_row3(ecol, erow[t.x], erow[t.x + 1], t.y, t.z, t.w, eij, eik, eil);
+    if (eij < 0 || eik < 0 || eil < 0) return;
+    const int64_t f = face((uint32_t)eij, (uint32_t)eik, t.z);
+    const int64_t g = face((uint32_t)eij, (uint32_t)eil, t.w);
+    const int64_t h = face((uint32_t)eik, (uint32_t)eil, t.w);
     if (f >= 0) tri_in[f] = 1;
     if (g >= 0) tri_in[g] = 1;
-  }
-  if (eik >= 0 && (f = find_row(tk, trow[eik], trow[eik + 1], t.w)) >= 0)
-    tri_in[f] = 1;
-  if (ejk >= 0 && (f = find_row(tk, trow[ejk], trow[ejk + 1], t.w)) >= 0)
-    tri_in[f] = 1;
+    if (h >= 0) tri_in[h] = 1;
+    if (f < 0 || g < 0) return;
+    const int64_t q = face(tejk[f], tejk[g], t.w);
+    if (q >= 0) tri_in[q] = 1;
+  });
 }
-void launch_mark_faces(Cnt nk, const uint4* ftets, const uint64_t* erow,
-                       const uint32_t* ecol, const uint64_t* trow,
-                       const uint32_t* tk, uint8_t* tri_in,
-                       unsigned long long* ts, PipeLaunch L) {
+void launch_tile_tets(Cnt nk, const uint4* tets, const uint8_t* flag,
+                      const uint64_t* offs, const uint64_t* erow,
+                      const uint32_t* ecol, const ulonglong2* emask,
+                      const uint64_t* trow, const uint32_t* tk,
+                      const uint32_t* tejk, const uint32_t* perm,
+                      uint8_t* tri_in, int32_t* out, unsigned long long* ts,
+                      PipeLaunch L, uint64_t ocap) {
   if (nk.cap <= 0) return;
-  hipLaunchKernelGGL(k_mark_faces, dim3((unsigned)((nk.cap + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, nk, ftets, erow, ecol, trow, tk,
-                     tri_in, ts);
+  hipLaunchKernelGGL(k_tile_tets, tiles_of(nk), dim3(kBlock), 0, L.s, nk, tets,
+                     flag, offs, erow, ecol, emask, trow, tk, tejk, perm,
+                     tri_in, (int4*)out, ocap, ts);
 }
 
-/* edges of the final triangles -> edge_in (edge ids recorded at
- * enumeration: (i,j) = tedge, (i,k) = teik, (j,k) = tejk) */
-__global__ __launch_bounds__(kBlock) void k_mark_edges(
-    Cnt c_nt, const uint32_t* ftri, const uint32_t* tedge,
-    const uint32_t* teik, const uint32_t* tejk, uint8_t* edge_in,
-    unsigned long long* ts) {
-  stamp(ts, 7);
-  const int64_t nt = c_nt.get();
-  int64_t id = gtid();
-  if (id >= nt) return;
-  uint32_t t = ftri[id];
-  edge_in[tedge[t]] = 1;
-  edge_in[teik[t]] = 1;
-  edge_in[tejk[t]] = 1;
-}
-void launch_mark_edges(Cnt nt, const uint32_t* ftri, const uint32_t* tedge,
-                       const uint32_t* teik, const uint32_t* tejk,
-                       uint8_t* edge_in, unsigned long long* ts, PipeLaunch L) {
-  if (nt.cap <= 0) return;
-  hipLaunchKernelGGL(k_mark_edges, dim3((unsigned)((nt.cap + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, nt, ftri, tedge, teik, tejk,
-                     edge_in, ts);
-}
-
-/* ---- emission in original ids ---- */
-__global__ __launch_bounds__(kBlock) void k_emit_tets(Cnt c_nk,
-                                                      const uint4* ftets,
-                                                      const uint32_t* perm,
-                                                      int4* out) {
-  const int64_t nk = c_nk.get();
-  int64_t id = gtid();
-  if (id >= nk) return;
-  uint4 t = ftets[id];
-  out[id] = make_int4((int)perm[t.x], (int)perm[t.y], (int)perm[t.z],
-                      (int)perm[t.w]);
-}
-void launch_emit_tets(Cnt nk, const uint4* ftets, const uint32_t* perm,
-                      int32_t* out, PipeLaunch L) {
-  if (nk.cap <= 0) return;
-  hipLaunchKernelGGL(k_emit_tets, dim3((unsigned)((nk.cap + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, nk, ftets, perm, (int4*)out);
-}
-__global__ __launch_bounds__(kBlock) void k_emit_tris(
-    Cnt c_nt, const uint32_t* ftri, const uint32_t* ecol,
+/* the same for the final triangles, which mark their edges in edge_in
+ * (edge ids recorded at enumeration: (i,j) = tedge, (i,k) = teik, (j,k) =
+ * tejk) */
+__global__ __launch_bounds__(kBlock) void k_tile_tris(
+    Cnt c_nt, const uint8_t* flag, const uint64_t* offs, const uint32_t* ecol,
     const uint32_t* eleft, const uint32_t* tk, const uint32_t* tedge,
-    const uint32_t* perm, int32_t* out) {
-  const int64_t nt = c_nt.get();
-  int64_t id = gtid();
-  if (id >= nt) return;
-  uint32_t t = ftri[id];
-  uint32_t e = tedge[t];
-  uint64_t w = (uint64_t)id * 3;
-  out[w] = (int32_t)perm[eleft[e]];
-  out[w + 1] = (int32_t)perm[ecol[e]];
-  out[w + 2] = (int32_t)perm[tk[t]];
+    const uint32_t* teik, const uint32_t* tejk, const uint32_t* perm,
+    uint8_t* edge_in, int32_t* out, uint64_t ocap, unsigned long long* ts) {
+  stamp(ts, 7);
+  tile_each(flag, c_nt.get(), offs, [&](int64_t t, uint64_t p) {
+    if (p >= ocap) return;
+    const uint32_t e = tedge[t];
+    edge_in[e] = 1;
+    edge_in[teik[t]] = 1;
+    edge_in[tejk[t]] = 1;
+    out[3 * p] = (int32_t)perm[eleft[e]];
+    out[3 * p + 1] = (int32_t)perm[ecol[e]];
+    out[3 * p + 2] = (int32_t)perm[tk[t]];
+  });
 }
-void launch_emit_tris(Cnt nt, const uint32_t* ftri, const uint32_t* ecol,
-                      const uint32_t* eleft, const uint32_t* tk,
-                      const uint32_t* tedge, const uint32_t* perm,
-                      int32_t* out, PipeLaunch L) {
+void launch_tile_tris(Cnt nt, const uint8_t* flag, const uint64_t* offs,
+                      const uint32_t* ecol, const uint32_t* eleft,
+                      const uint32_t* tk, const uint32_t* tedge,
+                      const uint32_t* teik, const uint32_t* tejk,
+                      const uint32_t* perm, uint8_t* edge_in, int32_t* out,
+                      unsigned long long* ts, PipeLaunch L, uint64_t ocap) {
   if (nt.cap <= 0) return;
-  hipLaunchKernelGGL(k_emit_tris, dim3((unsigned)((nt.cap + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, nt, ftri, ecol, eleft, tk, tedge,
-                     perm, out);
+  hipLaunchKernelGGL(k_tile_tris, tiles_of(nt), dim3(kBlock), 0, L.s, nt, flag,
+                     offs, ecol, eleft, tk, tedge, teik, tejk, perm, edge_in,
+                     out, ocap, ts);
 }
 
 }  // namespace pac

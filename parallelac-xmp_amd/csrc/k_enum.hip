@@ -1407,12 +1407,12 @@ void launch_seg_keep(int64_t n, const uint64_t* off, const uint32_t* bcnt,
                      dim3(kBlock), 0, L.s, n, off, bcnt, flag, keep);
 }
 /* ball i's kept edges (one wave per ball) to (ecol, eleft)[erow[i], ...),
- * their marks in edead (if given) cleared for the triangle stage; erow cut
- * at the arrays' end */
+ * their marks in edead (if given; for the triangle stage) and edge_in (the
+ * closure) cleared; erow cut at the arrays' end */
 __global__ __launch_bounds__(kBlock) void k_edge_copy(
     int64_t n, const uint64_t* off, const uint32_t* bcnt, const uint32_t* cval,
     const uint8_t* flag, uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
-    uint8_t* edead, uint64_t ocap) {
+    uint8_t* edead, uint8_t* edge_in, uint64_t ocap) {
   const int64_t iw = (int64_t)blockIdx.x * kEdgeBallsPerBlock + (threadIdx.x >> 6);
   if (iw >= n) return;
   const uint32_t i = __builtin_amdgcn_readfirstlane((uint32_t)iw);
@@ -1434,6 +1434,7 @@ __global__ __launch_bounds__(kBlock) void k_edge_copy(
         ecol[w] = cval[base + t];
         eleft[w] = i;
         if (edead) edead[w] = 0;
+        edge_in[w] = 0;
       }
     }
     o += (uint64_t)__popcll(bm);
@@ -1442,13 +1443,14 @@ __global__ __launch_bounds__(kBlock) void k_edge_copy(
 void launch_edge_copy(int64_t n, const uint64_t* off, const uint32_t* bcnt,
                       const uint32_t* cval, const uint8_t* flag,
                       uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
-                      uint8_t* edead, PipeLaunch L, uint64_t ocap) {
+                      uint8_t* edead, uint8_t* edge_in, PipeLaunch L,
+                      uint64_t ocap) {
   if (n <= 0) return;
   hipLaunchKernelGGL(
       k_edge_copy,
       dim3((unsigned)((n + kEdgeBallsPerBlock - 1) / kEdgeBallsPerBlock)),
       dim3(kBlock), 0, L.s, n, off, bcnt, cval, flag, erow, ecol, eleft, edead,
-      ocap);
+      edge_in, ocap);
 }
 
 /* Triangles of alpha edge q = (i, j) -- k in row(i) after j and in row(j),
@@ -1651,7 +1653,7 @@ void launch_tri_enum_filter(const Stage& S, Cnt ne, const uint64_t* erow,
  * in order, a wave each; trow[e] for its edges e (and trow[ne], by the wave
  * holding index ne) = bout[b] + the kept triangles of its edges before e.
  * tkd (if given): tk with kDeadBit set where one of the triangle's edges is
- * marked in edead.  emask[e], e = (i,j): x has bit r if (i, j, k) is a
+ * marked in edead; tri_in (the closure's marks) cleared.  emask[e], e = (i,j): x has bit r if (i, j, k) is a
  * triangle and (i, k) the (r + 1)th edge after e, y the bits of those with
  * kDeadBit; bit 63 is set if some r is 63 or more.  spair, epre (if given):
  * the tet slots of the segment's triangles (each one's row tail), and of
@@ -1663,7 +1665,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_seg_copy(
     const uint8_t* flag, const uint64_t* bout, const uint8_t* edead,
     uint32_t* tk, uint32_t* tkd, uint32_t* tedge, uint32_t* teik,
     uint32_t* tejk, uint64_t* trow, uint64_t* spair, uint32_t* epre,
-    ulonglong2* emask, uint64_t ocap) {
+    ulonglong2* emask, uint8_t* tri_in, uint64_t ocap) {
   __shared__ uint32_t s_cnt[kBlock / 64][64];
   __shared__ unsigned long long s_mask[2][kBlock / 64][64];
   const int64_t ne = c_ne.get();
@@ -1734,6 +1736,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_seg_copy(
             tedge[w] = seg;
             teik[w] = av[u];
             tejk[w] = bv[u];
+            tri_in[w] = 0;
             const uint32_t r = av[u] - seg - 1u;
             const unsigned long long bit = 1ull << (r < 63u ? r : 63u);
             atomicOr(&s_mask[0][wv][e], bit);
@@ -1771,13 +1774,14 @@ void launch_tri_seg_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
                          const uint8_t* edead, uint32_t* tk, uint32_t* tkd,
                          uint32_t* tedge, uint32_t* teik, uint32_t* tejk,
                          uint64_t* trow, uint64_t* spair, uint32_t* epre,
-                         ulonglong2* emask, PipeLaunch L, uint64_t ocap) {
+                         ulonglong2* emask, uint8_t* tri_in, PipeLaunch L,
+                         uint64_t ocap) {
   const int64_t nseg = (std::max<int64_t>(ne.cap, 0) + kTriSeg - 1) / kTriSeg;
   hipLaunchKernelGGL(k_tri_seg_copy,
                      dim3((unsigned)((nseg + kBlock / 64) / (kBlock / 64))),
                      dim3(kBlock), 0, L.s, ne, off, bcnt, cval, cseg, cea, ceb,
                      flag, bout, edead, tk, tkd, tedge, teik, tejk, trow, spair,
-                     epre, emask, ocap);
+                     epre, emask, tri_in, ocap);
 }
 
 template <int KIND>

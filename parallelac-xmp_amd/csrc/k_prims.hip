@@ -9,37 +9,9 @@
  *     thrust::sort_by_key of the cell keys (AlphaComplexParallel.cu:1157).
  */
 #include "pac_internal.h"
+#include "pac_tiles.h"
 
 namespace pac {
-
-__device__ __forceinline__ uint64_t wave_incl_scan_u64(uint64_t v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    uint64_t o = __shfl_up(v, d, 64);
-    if (lane >= d) v += o;
-  }
-  return v;
-}
-
-/* block-wide exclusive scan of one value per thread; returns block total */
-__device__ __forceinline__ uint64_t block_excl_scan_u64(uint64_t v,
-                                                        uint64_t* total) {
-  __shared__ uint64_t wsum[kBlock / 64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  uint64_t inc = wave_incl_scan_u64(v);
-  if (lane == 63) wsum[w] = inc;
-  __syncthreads();
-  uint64_t base = 0, tot = 0;
-#pragma unroll
-  for (int q = 0; q < kBlock / 64; ++q) {
-    if (q < w) base += wsum[q];
-    tot += wsum[q];
-  }
-  __syncthreads();
-  *total = tot;
-  return base + inc - v;
-}
 
 /* The post of a stage's last kernel, by one whole wave (pac_internal.h). */
 __device__ __forceinline__ void do_post(const Post& P, uint64_t count) {
@@ -313,19 +285,6 @@ void scan_u64_to_u64(const uint64_t* in, uint64_t* out, Cnt n, void* tmp,
  * as the generic scan (flag arrays and positions are pool buffers, aligned
  * far beyond 16 bytes, and a tile starts at a multiple of kTile items). */
 static_assert(kScanItems == 8, "a thread reads its flags as one 8-byte word");
-__device__ __forceinline__ unsigned nz_bytes(uint32_t x) {
-  /* high bit of each byte set iff the byte is nonzero */
-  const uint32_t y = ((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x;
-  return (unsigned)__popc(y & 0x80808080u);
-}
-__device__ __forceinline__ uint2 load_flags8(const uint8_t* in, int64_t i0,
-                                             int64_t n) {
-  if (i0 + 8 <= n) return *reinterpret_cast<const uint2*>(in + i0);
-  uint32_t w[2] = {0u, 0u};
-  for (int q = 0; q < 8; ++q)
-    if (i0 + q < n) w[q >> 2] |= (uint32_t)in[i0 + q] << (8 * (q & 3));
-  return make_uint2(w[0], w[1]);
-}
 __global__ __launch_bounds__(kBlock) void k_flag_sums(const uint8_t* in,
                                                       Cnt cn, uint64_t* sums) {
   const int64_t n = cn.get();
@@ -476,61 +435,19 @@ const uint64_t* flag_tile_offsets(const uint8_t* in, Cnt n, void* tmp,
   }
   return offs;
 }
-/* the kept entries of this block's tile, in order: emit(i, p), p = the
- * entry's rank among all kept entries */
-template <class F>
-__device__ __forceinline__ void tile_kept(const uint8_t* flag, int64_t n,
-                                          const uint64_t* offs, F&& emit) {
-  const int64_t i0 = (int64_t)blockIdx.x * kTile + (int64_t)threadIdx.x * 8;
-  const uint2 f = load_flags8(flag, i0, n);
-  uint64_t tot;
-  uint64_t p = block_excl_scan_u64(nz_bytes(f.x) + nz_bytes(f.y), &tot) +
-               offs[blockIdx.x];
-#pragma unroll
-  for (int q = 0; q < 8; ++q)
-    if ((((q < 4 ? f.x : f.y) >> (8 * (q & 3))) & 0xffu) != 0) emit(i0 + q, p++);
-}
-__global__ __launch_bounds__(kBlock) void k_tile_compact_u4(
-    Cnt cn, const uint4* in, const uint8_t* flag, const uint64_t* offs,
-    uint4* out, uint64_t ocap) {
-  tile_kept(flag, cn.get(), offs, [&](int64_t i, uint64_t p) {
-    if (p < ocap) out[p] = in[i];
-  });
-}
-__global__ __launch_bounds__(kBlock) void k_tile_compact_ids(
-    Cnt cn, const uint8_t* flag, const uint64_t* offs, uint32_t* out,
-    uint64_t ocap) {
-  tile_kept(flag, cn.get(), offs, [&](int64_t i, uint64_t p) {
-    if (p < ocap) out[p] = (uint32_t)i;
-  });
-}
 __global__ __launch_bounds__(kBlock) void k_tile_compact_u8(
     Cnt cn, const uint8_t* flag, const uint64_t* offs, const uint8_t* val,
     uint8_t* out, uint64_t ocap) {
-  tile_kept(flag, cn.get(), offs, [&](int64_t i, uint64_t p) {
+  tile_each(flag, cn.get(), offs, [&](int64_t i, uint64_t p) {
     if (p < ocap) out[p] = val[i] != 0;
   });
 }
 __global__ __launch_bounds__(kBlock) void k_tile_emit_edges(
     Cnt cn, const uint32_t* ecol, const uint32_t* eleft, const uint8_t* flag,
     const uint64_t* offs, const uint32_t* perm, int2* out, uint64_t ocap) {
-  tile_kept(flag, cn.get(), offs, [&](int64_t i, uint64_t p) {
+  tile_each(flag, cn.get(), offs, [&](int64_t i, uint64_t p) {
     if (p < ocap) out[p] = make_int2((int)perm[eleft[i]], (int)perm[ecol[i]]);
   });
-}
-static dim3 tiles_of(Cnt n) { return dim3((unsigned)((n.cap + kTile - 1) / kTile)); }
-void launch_compact_tets(Cnt n, const uint4* in, const uint8_t* flag,
-                         const uint64_t* offs, uint4* out, PipeLaunch L,
-                         uint64_t ocap) {
-  if (n.cap <= 0) return;
-  hipLaunchKernelGGL(k_tile_compact_u4, tiles_of(n), dim3(kBlock), 0, L.s, n,
-                     in, flag, offs, out, ocap);
-}
-void launch_compact_ids(Cnt n, const uint8_t* flag, const uint64_t* offs,
-                        uint32_t* out, PipeLaunch L, uint64_t ocap) {
-  if (n.cap <= 0) return;
-  hipLaunchKernelGGL(k_tile_compact_ids, tiles_of(n), dim3(kBlock), 0, L.s, n,
-                     flag, offs, out, ocap);
 }
 void launch_compact_u8(Cnt n, const uint8_t* flag, const uint64_t* offs,
                        const uint8_t* val, uint8_t* out, PipeLaunch L,

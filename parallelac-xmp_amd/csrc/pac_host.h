@@ -66,9 +66,9 @@ struct Pool {
     return (b + step - 1) / step * step;
   }
   /* Arena mode (set_arena): blocks are carved from one fixed device range
-   * instead of hipMalloc, 256-byte aligned, top of stack first; a block
-   * freed while it is the topmost is popped with any freed blocks below
-   * it.  Exhausting the range fails with PAC_ERR_NOMEM. */
+   * instead of hipMalloc, 256-byte aligned, from the first hole that
+   * fits or the top of the stack; a block freed while it is the topmost is
+   * popped with any freed blocks below it.  Exhausting the range fails with PAC_ERR_NOMEM. */
   char* abase = nullptr;
   size_t acap = 0, atop = 0, ahigh = 0;
   std::vector<std::pair<size_t, size_t>> ablk; /* (offset, 1 = freed) */
@@ -86,6 +86,23 @@ struct Pool {
     if (abase) {
       std::lock_guard<std::mutex> g(m);
       const size_t b = ((bytes ? bytes : 1) + 255) & ~(size_t)255;
+      /* the first run of freed blocks that holds it (the caller's stream
+       * orders their reuse), else the top */
+      for (size_t k = 0; k < ablk.size(); ++k) {
+        if (!ablk[k].second) continue;
+        size_t e = k + 1;
+        while (e < ablk.size() && ablk[e].second) ++e;
+        const size_t off = ablk[k].first;
+        const size_t room = (e < ablk.size() ? ablk[e].first : atop) - off;
+        if (room < b) {
+          k = e;
+          continue;
+        }
+        ablk.erase(ablk.begin() + k + 1, ablk.begin() + e);
+        ablk[k].second = 0;
+        if (room > b) ablk.insert(ablk.begin() + k + 1, {off + b, 1});
+        return abase + off;
+      }
       if (b > acap - atop)
         fail(PAC_ERR_NOMEM, "device scratch of " + std::to_string(acap) +
                                 " bytes exhausted (" + std::to_string(atop) +

@@ -222,8 +222,13 @@ struct QRef {
   int drop;
   uint32_t launch_items() const { return cnt ? bound : v.size(); }
 };
-inline QRef queue_ref(const Queue& q, bool drop) {
-  QRef r{QView{}, q.n, QSLOTS * q.cap, (int)drop};
+/* a queue whose length is on the device, for a grid fit for `entries` */
+inline QRef queue_ref(const Queue& q, bool drop, int64_t entries) {
+  const int64_t least = 64 * kBlock;
+  QRef r{QView{}, q.n,
+         (uint32_t)std::min<int64_t>((int64_t)QSLOTS * q.cap,
+                                     std::max(entries, least)),
+         (int)drop};
   r.v.q = q.q;
   r.v.cap = q.cap;
   return r;
@@ -276,11 +281,6 @@ struct CandCtx {
 /* ---- compactions by flags over tile offsets (k_prims.hip) ----
  * offs from flag_tile_offsets of the same flags; ocap: capacity of the
  * output (entries past it are dropped) */
-void launch_compact_tets(Cnt n, const uint4* in, const uint8_t* flag,
-                         const uint64_t* offs, uint4* out, PipeLaunch L,
-                         uint64_t ocap = ~0ull);
-void launch_compact_ids(Cnt n, const uint8_t* flag, const uint64_t* offs,
-                        uint32_t* out, PipeLaunch L, uint64_t ocap = ~0ull);
 void launch_compact_u8(Cnt n, const uint8_t* flag, const uint64_t* offs,
                        const uint8_t* val, uint8_t* out, PipeLaunch L,
                        uint64_t ocap = ~0ull);
@@ -293,19 +293,22 @@ void launch_emit_edges(Cnt ne, const uint32_t* ecol, const uint32_t* eleft,
 /* ---- closure + emission (k_closure.hip) ---- */
 void launch_or_flags(Cnt n, const uint8_t* a, const uint8_t* b, uint8_t* out,
                      PipeLaunch L);
-void launch_mark_faces(Cnt nk, const uint4* ftets, const uint64_t* erow,
-                       const uint32_t* ecol, const uint64_t* trow,
-                       const uint32_t* tk, uint8_t* tri_in,
-                       unsigned long long* ts, PipeLaunch L);
-void launch_mark_edges(Cnt nt, const uint32_t* ftri, const uint32_t* tedge,
-                       const uint32_t* teik, const uint32_t* tejk,
-                       uint8_t* edge_in, unsigned long long* ts, PipeLaunch L);
-void launch_emit_tets(Cnt nk, const uint4* ftets, const uint32_t* perm,
-                      int32_t* out, PipeLaunch L);
-void launch_emit_tris(Cnt nt, const uint32_t* ftri, const uint32_t* ecol,
-                      const uint32_t* eleft, const uint32_t* tk,
-                      const uint32_t* tedge, const uint32_t* perm,
-                      int32_t* out, PipeLaunch L);
+/* the final tets / triangles by flags over tile offsets: their rows in
+ * original ids (ocap of them at most), and their faces / edges marked */
+void launch_tile_tets(Cnt nk, const uint4* tets, const uint8_t* flag,
+                      const uint64_t* offs, const uint64_t* erow,
+                      const uint32_t* ecol, const ulonglong2* emask,
+                      const uint64_t* trow, const uint32_t* tk,
+                      const uint32_t* tejk, const uint32_t* perm,
+                      uint8_t* tri_in, int32_t* out, unsigned long long* ts,
+                      PipeLaunch L, uint64_t ocap = ~0ull);
+void launch_tile_tris(Cnt nt, const uint8_t* flag, const uint64_t* offs,
+                      const uint32_t* ecol, const uint32_t* eleft,
+                      const uint32_t* tk, const uint32_t* tedge,
+                      const uint32_t* teik, const uint32_t* tejk,
+                      const uint32_t* perm, uint8_t* edge_in, int32_t* out,
+                      unsigned long long* ts, PipeLaunch L,
+                      uint64_t ocap = ~0ull);
 
 /* ---- outputs (k_output.hip) ---- */
 /* words of src (4-byte units, minus base; at most half a ring) to the pinned
@@ -460,7 +463,8 @@ void launch_seg_keep(int64_t n, const uint64_t* off, const uint32_t* bcnt,
 void launch_edge_copy(int64_t n, const uint64_t* off, const uint32_t* bcnt,
                       const uint32_t* cval, const uint8_t* flag,
                       uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
-                      uint8_t* edead, PipeLaunch L, uint64_t ocap = ~0ull);
+                      uint8_t* edead, uint8_t* edge_in, PipeLaunch L,
+                      uint64_t ocap = ~0ull);
 /* slot capacity of item q = row[owner[q] + 1] - q - 1 */
 void launch_tail_caps(Cnt m, const uint64_t* row, const uint32_t* owner,
                       uint32_t* cap, PipeLaunch L);
@@ -506,7 +510,7 @@ void launch_tri_seg_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
                          const uint8_t* edead, uint32_t* tk, uint32_t* tkd,
                          uint32_t* tedge, uint32_t* teik, uint32_t* tejk,
                          uint64_t* trow, uint64_t* spair, uint32_t* epre,
-                         ulonglong2* emask, PipeLaunch L,
+                         ulonglong2* emask, uint8_t* tri_in, PipeLaunch L,
                          uint64_t ocap = ~0ull);
 /* tet candidates of the alpha triangles, each filtered by the first
  * precision stage in the same kernel; enumeration segment b (kTetSeg alpha

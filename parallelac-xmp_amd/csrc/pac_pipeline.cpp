@@ -423,13 +423,13 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   auto grow = [&](uint32_t need) {
     return (uint32_t)std::min<int64_t>((int64_t)need + need / 4 + 256, qmax);
   };
-  auto ladder = [&](int64_t cap1_total, int kp_hot, int kp_exact, auto&& hot,
+  auto ladder = [&](int64_t cap1_total, int64_t esc_items, int kp_hot, int kp_exact, auto&& hot,
                     auto&& esc, auto&& exact, auto&& tail, int q) -> Cnt {
     if (rec) { /* once, over the recorded queues */
       const Queue h{rec->q1, qn, rec->c1}, e{rec->q2, nesc, rec->c2};
       hot(h);
-      if (staged) esc(queue_ref(h, false), e);
-      exact(queue_ref(staged ? e : h, false));
+      if (staged) esc(queue_ref(h, false, esc_items), e);
+      exact(queue_ref(staged ? e : h, false, esc_items));
       KCHK();
       tail(Post());
       launch_ladder_rec(qn, rec->c1, rec->c2, rec->status, rec->fill, s);
@@ -453,7 +453,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       if (staged) {
         q2 = DBuf<QEntry>(P, (size_t)c2 * QSLOTS);
         last = Queue{q2.get(), nesc, c2};
-        esc(queue_ref(h, true), last);
+        esc(queue_ref(h, true, esc_items), last);
         KCHK();
       }
       const Post post = new_post(true);
@@ -529,7 +529,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
    * whose scans see every ball (the reference's stencil may miss the
    * covering one), and where tets are tested */
   const bool prune = opt.cell_policy == PAC_CELL_EXACT && !opt.skip_tet_ac2;
-  DBuf<uint8_t> edead;
+  DBuf<uint8_t> edead, edge_in; /* edge_in, tri_in: the closure's marks */
   CandCtx C0{nullptr, nullptr, nullptr, nullptr, nullptr};
   if (!no_edges) {
     DBuf<uint64_t> off(P, n + 1);
@@ -549,7 +549,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     auto tmp = scan_tmp(n);
     host_evals[0] += Ecand.cap;
     Ealpha = ladder(
-        std::min<int64_t>(Ecand.cap, Ecand.cap / 32 + 65536), KP_EDGE_FILL, -1,
+        std::min<int64_t>(Ecand.cap, Ecand.cap / 32 + 65536), Ecand.cap / 64, KP_EDGE_FILL, -1,
         [&](Queue qq) {
           launch_edge_enum_filter(SG, off.get(), cval.get(), cseg.get(),
                                   flag.get(), bcnt.get(), qq, L,
@@ -570,14 +570,16 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     ecol = DBuf<uint32_t>(P, Ealpha.cap + kEcolPad);
     eleft = DBuf<uint32_t>(P, Ealpha.cap);
     if (prune) edead = DBuf<uint8_t>(P, Ealpha.cap);
+    edge_in = DBuf<uint8_t>(P, Ealpha.cap);
     launch_edge_copy(n, off.get(), bcnt.get(), cval.get(), flag.get(),
-                     erow.get(), ecol.get(), eleft.get(), edead.get(), L,
-                     (uint64_t)Ealpha.cap);
+                     erow.get(), ecol.get(), eleft.get(), edead.get(),
+                     edge_in.get(), L, (uint64_t)Ealpha.cap);
     KCHK();
   } else {
     zero_u64((unsigned long long*)erow.get(), n + 1, s);
     ecol = DBuf<uint32_t>(P, 1 + kEcolPad);
     eleft = DBuf<uint32_t>(P, 1);
+    edge_in = DBuf<uint8_t>(P, 1);
   }
 
   /* ---- triangles (AlphaComplexParallel.cu:1279-1371) ---- */
@@ -591,6 +593,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   DBuf<uint64_t> spair(P, tail_slots ? std::max<int64_t>(neseg, 1) : 1);
   DBuf<uint32_t> epre(P, tail_slots ? std::max<int64_t>(Ealpha.cap, 1) : 1);
   DBuf<uint32_t> tk, tkd, tedge, teik, tejk;
+  DBuf<uint8_t> tri_in;
   /* per alpha edge 128 bits: first its hits, then its mask of third
    * vertices */
   DBuf<ulonglong2> emask(P, std::max<int64_t>(Ealpha.cap, 1));
@@ -620,7 +623,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
      * zero */
     int runs = 0;
     Talpha = ladder(
-        std::min<int64_t>(Tslots.cap, Tslots.cap / 32 + 65536), KP_TRI_FILL, -1,
+        std::min<int64_t>(Tslots.cap, Tslots.cap / 32 + 65536), Tslots.cap / 64, KP_TRI_FILL, -1,
         [&](Queue qq) {
           if (runs++ && !rec)
             zero_counter(ctr, CTR_CAND + 1, s);
@@ -648,12 +651,13 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     tedge = DBuf<uint32_t>(P, Talpha.cap);
     teik = DBuf<uint32_t>(P, Talpha.cap);
     tejk = DBuf<uint32_t>(P, Talpha.cap);
+    tri_in = DBuf<uint8_t>(P, Talpha.cap);
     launch_tri_seg_copy(Ealpha, off.get(), bcnt.get(), cval.get(), cseg.get(),
                         cea.get(), ceb.get(), flag.get(), bout.get(), dead,
                         tk.get(), tkd.get(), tedge.get(), teik.get(),
                         tejk.get(), trow.get(),
                         tail_slots ? spair.get() : nullptr, epre.get(),
-                        emask.get(), L, (uint64_t)Talpha.cap);
+                        emask.get(), tri_in.get(), L, (uint64_t)Talpha.cap);
     KCHK();
   }
 
@@ -703,7 +707,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
      * zero */
     int runs = 0;
     Kalpha = ladder(
-        std::min<int64_t>(Kslots.cap, Kslots.cap / 32 + 65536), KP_TET_FILL, -1,
+        std::min<int64_t>(Kslots.cap, Kslots.cap / 32 + 65536), Kslots.cap / 64, KP_TET_FILL, -1,
         [&](Queue qq) {
           if (runs++ && !rec) {
             zero_counter(ctr, CTR_CAND + 2, s);
@@ -735,8 +739,9 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     KCHK();
   }
 
-  auto ac2_cap = [](int64_t items) {
-    return (uint32_t)std::min<int64_t>(std::max<int64_t>(1 << 20, items / 2),
+  /* (with the covered ones gone, the items left are likelier to queue) */
+  auto ac2_cap = [&](int64_t items) {
+    return (uint32_t)std::min<int64_t>(std::max<int64_t>(1 << 20, items / (prune ? 2 : 8)),
                                        (int64_t)UINT32_MAX - 1);
   };
 
@@ -785,7 +790,6 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   DBuf<uint32_t> next(P, (size_t)LSLOTS * SG.lcap);
   DBuf<uint8_t> kflag(P, Kalpha.cap);
   Cnt Kf(0);
-  DBuf<uint4> ftets;
   {
     auto tmp = scan_tmp(Kalpha.cap);
     const uint64_t* koffs = nullptr; /* tile offsets of kflag, in tmp */
@@ -801,7 +805,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       Kf = settle(RC_KF, post);
     } else {
       Kf = ladder(
-          ac2_cap(Kalpha.cap), KP_TET_AC2, KP_TET_AC2_EXACT,
+          ac2_cap(Kalpha.cap), Kalpha.cap / 4, KP_TET_AC2, KP_TET_AC2_EXACT,
           [&](Queue q) {
             launch_tet_ac2_hot(SG, Kalpha, tets.get(), kflag.get(), q,
                                rest.get(), nrest, next.get(), nnext,
@@ -826,9 +830,11 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           },
           tail, RC_KF);
     }
-    ftets = DBuf<uint4>(P, Kf.cap);
-    launch_compact_tets(Kalpha, tets.get(), kflag.get(), koffs, ftets.get(), L,
-                        (uint64_t)Kf.cap);
+    R->lists[2] = DBuf<int32_t>(P, 4 * Kf.cap);
+    launch_tile_tets(Kalpha, tets.get(), kflag.get(), koffs, erow.get(),
+                     ecol.get(), emask.get(), trow.get(), tk.get(), tejk.get(),
+                     perm.get(), tri_in.get(), R->lists[2].get(), ts, L,
+                     (uint64_t)Kf.cap);
     KCHK();
   }
   tets.release();
@@ -838,10 +844,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
    * empty smallest orthosphere: the simplex enters at its own rho), and
    * the closure marks join the final flags only after the test */
   const bool filt = opt.filtration != 0 && !rec;
-  DBuf<uint8_t> tri_in(P, Talpha.cap), tflag(P, Talpha.cap);
-  fill_u8(tri_in.get(), Talpha.cap, 0, s);
-  launch_mark_faces(Kf, ftets.get(), erow.get(), ecol.get(), trow.get(),
-                    tk.get(), tri_in.get(), ts, L);
+  DBuf<uint8_t> tflag(P, Talpha.cap);
   DBuf<uint8_t> tri_skip_own, tfin;
   uint8_t* tri_skip = tri_in.get(); /* passes without a test */
   if (filt) {
@@ -854,7 +857,6 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
                   tri_skip, L);
   const uint8_t* tfinal = filt ? tfin.get() : tflag.get();
   Cnt Tf(0);
-  DBuf<uint32_t> ftri;
   {
     auto tmp = scan_tmp(Talpha.cap);
     const uint64_t* toffs = nullptr; /* tile offsets of tfinal, in tmp */
@@ -870,7 +872,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       Tf = settle(RC_TF, post);
     } else {
       Tf = ladder(
-          ac2_cap(Talpha.cap), KP_TRI_AC2, -1,
+          ac2_cap(Talpha.cap), Talpha.cap / 4, KP_TRI_AC2, -1,
           [&](Queue q) {
             launch_low_ac2_hot(SG, 0, Talpha, ecol.get(), eleft.get(), tkm,
                                tedge.get(), nullptr, tri_skip, tflag.get(), q,
@@ -896,8 +898,11 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           },
           tail, RC_TF);
     }
-    ftri = DBuf<uint32_t>(P, Tf.cap);
-    launch_compact_ids(Talpha, tfinal, toffs, ftri.get(), L, (uint64_t)Tf.cap);
+    R->lists[1] = DBuf<int32_t>(P, 3 * Tf.cap);
+    launch_tile_tris(Talpha, tfinal, toffs, ecol.get(), eleft.get(), tk.get(),
+                     tedge.get(), teik.get(), tejk.get(), perm.get(),
+                     edge_in.get(), R->lists[1].get(), ts, L,
+                     (uint64_t)Tf.cap);
     if (filt) {
       R->gab[1] = DBuf<uint8_t>(P, Tf.cap);
       launch_compact_u8(Talpha, tfinal, toffs, tflag.get(), R->gab[1].get(), L,
@@ -907,10 +912,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   }
 
   /* ---- edge closure + dangling emptiness ---- */
-  DBuf<uint8_t> edge_in(P, Ealpha.cap), eflag(P, Ealpha.cap);
-  fill_u8(edge_in.get(), Ealpha.cap, 0, s);
-  launch_mark_edges(Tf, ftri.get(), tedge.get(), teik.get(), tejk.get(),
-                    edge_in.get(), ts, L);
+  DBuf<uint8_t> eflag(P, Ealpha.cap);
   DBuf<uint8_t> edge_skip_own, efin;
   uint8_t* edge_skip = edge_in.get();
   if (filt) {
@@ -938,7 +940,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       Ef = settle(RC_EF, post);
     } else {
       Ef = ladder(
-          ac2_cap(Ealpha.cap), KP_EDGE_AC2, -1,
+          ac2_cap(Ealpha.cap), Ealpha.cap / 4, KP_EDGE_AC2, -1,
           [&](Queue q) {
             launch_low_ac2_hot(SG, 1, Ealpha, ecol.get(), eleft.get(), nullptr,
                                nullptr, dead, edge_skip, eflag.get(), q,
@@ -968,8 +970,6 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
 
   /* ---- emit final lists (original ids, reference order) ---- */
   R->lists[0] = DBuf<int32_t>(P, 2 * Ef.cap);
-  R->lists[1] = DBuf<int32_t>(P, 3 * Tf.cap);
-  R->lists[2] = DBuf<int32_t>(P, 4 * Kf.cap);
   launch_emit_edges(Ealpha, ecol.get(), eleft.get(), efinal, eoffs, perm.get(),
                     R->lists[0].get(), L, (uint64_t)Ef.cap);
   if (filt) {
@@ -979,9 +979,6 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     R->rank = DBuf<uint32_t>(P, n);
     launch_rank_of(perm.get(), n, R->rank.get(), s);
   }
-  launch_emit_tris(Tf, ftri.get(), ecol.get(), eleft.get(), tk.get(),
-                   tedge.get(), perm.get(), R->lists[1].get(), L);
-  launch_emit_tets(Kf, ftets.get(), perm.get(), R->lists[2].get(), L);
   KCHK();
   if (rec) return; /* counts and statistics are read after the graph runs */
   R->counts[1] = Ef.cap;

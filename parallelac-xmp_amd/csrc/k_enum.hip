@@ -241,13 +241,16 @@ void launch_mol_ids(const uint32_t* moff, int64_t nmol, int64_t n,
 }
 
 /* computeCellIndex (LD:65-78): FP32 subtract, IEEE divide, truncate; in a
- * batch the molecule's first global cell id is added. */
+ * batch the molecule's first global cell id is added.  idx: the ball, or
+ * with the cells' counts (cleared) its place among the balls of its cell, in
+ * the order they arrive. */
 __global__ __launch_bounds__(kBlock) void k_cell_key(const Ball* raw,
                                                      int64_t n, GridP g1,
                                                      const GridP* grids,
                                                      const uint32_t* mol,
                                                      uint32_t* key,
-                                                     uint32_t* idx) {
+                                                     uint32_t* idx,
+                                                     uint32_t* cnt) {
   int64_t i = gtid();
   if (i >= n) return;
   const GridP g = mol ? grids[mol[i]] : g1;
@@ -264,15 +267,55 @@ __global__ __launch_bounds__(kBlock) void k_cell_key(const Ball* raw,
   cx = min(max(cx, 0), g.ex - 1);
   cy = min(max(cy, 0), g.ey - 1);
   cz = min(max(cz, 0), g.ez - 1);
-  key[i] = g.cbase + (uint32_t)(cx + g.ex * cy + g.ex * g.ey * cz);
-  idx[i] = (uint32_t)i;
+  const uint32_t c = g.cbase + (uint32_t)(cx + g.ex * cy + g.ex * g.ey * cz);
+  key[i] = c;
+  idx[i] = cnt ? atomicAdd(cnt + c, 1u) : (uint32_t)i;
 }
 void launch_cell_key(const Ball* raw, int64_t n, GridP g,
                      const GridP* grids, const uint32_t* mol, uint32_t* key,
-                     uint32_t* idx, PipeLaunch L) {
+                     uint32_t* idx, uint32_t* cnt, PipeLaunch L) {
   if (n <= 0) return;
   hipLaunchKernelGGL(k_cell_key, dim3((unsigned)((n + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, raw, n, g, grids, mol, key, idx);
+                     dim3(kBlock), 0, L.s, raw, n, g, grids, mol, key, idx, cnt);
+}
+
+/* the balls by cell, in each cell as they arrived */
+__global__ __launch_bounds__(kBlock) void k_cell_put(int64_t n,
+                                                     const uint32_t* key,
+                                                     const uint32_t* place,
+                                                     const uint32_t* cstart,
+                                                     uint32_t* sidx) {
+  const int64_t i = gtid();
+  if (i < n) sidx[cstart[key[i]] + place[i]] = (uint32_t)i;
+}
+/* Each ball to its place by cell and id: as many after its cell's start as
+ * the cell holds smaller ids (the enumeration tests all pairs of a cell, so
+ * a full cell costs no more here). */
+__global__ __launch_bounds__(kBlock) void k_cell_order(
+    const Ball* raw, int64_t n, const uint32_t* sidx, const uint32_t* key,
+    const uint32_t* cstart, Real solvent, Ball* ball, uint32_t* perm,
+    uint32_t* cellk) {
+  const int64_t s = gtid();
+  if (s >= n) return;
+  const uint32_t o = sidx[s];
+  const Ball a = raw[o];
+  const uint32_t c = key[o], b = cstart[c], e = cstart[c + 1];
+  uint32_t at = b;
+  for (uint32_t t = b; t < e; ++t) at += sidx[t] < o;
+  ball[at] = Ball{a.x, a.y, a.z, add_r(a.w, solvent)};
+  perm[at] = o;
+  cellk[at] = c;
+}
+void launch_cell_order(const Ball* raw, int64_t n, const uint32_t* key,
+                       const uint32_t* place, const uint32_t* cstart,
+                       uint32_t* sidx, Real solvent, Ball* ball, uint32_t* perm,
+                       uint32_t* cellk, PipeLaunch L) {
+  if (n <= 0) return;
+  const dim3 gr((unsigned)((n + kBlock - 1) / kBlock));
+  hipLaunchKernelGGL(k_cell_put, gr, dim3(kBlock), 0, L.s, n, key, place,
+                     cstart, sidx);
+  hipLaunchKernelGGL(k_cell_order, gr, dim3(kBlock), 0, L.s, raw, n, sidx, key,
+                     cstart, solvent, ball, perm, cellk);
 }
 
 __global__ __launch_bounds__(kBlock) void k_gather(const Ball* raw,

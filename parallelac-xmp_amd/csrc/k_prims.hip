@@ -274,6 +274,10 @@ void scan_u32_to_u64(const uint32_t* in, uint64_t* out, Cnt n, void* tmp,
                      hipStream_t s, uint64_t* total64, Post post) {
   scan_impl<uint32_t, false>(in, out, n, (uint64_t*)tmp, s, total64, post);
 }
+void scan_u32(const uint32_t* in, uint32_t* out, Cnt n, void* tmp,
+              hipStream_t s) {
+  scan_impl<uint32_t, false>(in, out, n, (uint64_t*)tmp, s);
+}
 void scan_u64_to_u64(const uint64_t* in, uint64_t* out, Cnt n, void* tmp,
                      hipStream_t s, uint64_t* total64, Post post) {
   scan_impl<uint64_t, false>(in, out, n, (uint64_t*)tmp, s, total64, post);

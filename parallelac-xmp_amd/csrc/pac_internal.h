@@ -113,6 +113,8 @@ constexpr int kBoxTicket = 0, kBoxCount = 2, kBoxQ1 = 4, kBoxQ2 = 36,
 void scan_u32_to_u64(const uint32_t* in, uint64_t* out, Cnt n, void* tmp,
                      hipStream_t s, uint64_t* total64 = nullptr,
                      Post post = Post());
+void scan_u32(const uint32_t* in, uint32_t* out, Cnt n, void* tmp,
+              hipStream_t s);
 void scan_u64_to_u64(const uint64_t* in, uint64_t* out, Cnt n, void* tmp,
                      hipStream_t s, uint64_t* total64 = nullptr,
                      Post post = Post());
@@ -381,7 +383,11 @@ void launch_mol_ids(const uint32_t* moff, int64_t nmol, int64_t n,
 /* global cell key; grids/mol == nullptr: the single grid g */
 void launch_cell_key(const Ball* raw, int64_t n, GridP g,
                      const GridP* grids, const uint32_t* mol, uint32_t* key,
-                     uint32_t* idx, PipeLaunch L);
+                     uint32_t* idx, uint32_t* cnt, PipeLaunch L);
+void launch_cell_order(const Ball* raw, int64_t n, const uint32_t* key,
+                       const uint32_t* place, const uint32_t* cstart,
+                       uint32_t* sidx, Real solvent, Ball* ball, uint32_t* perm,
+                       uint32_t* cellk, PipeLaunch L);
 void launch_gather(const Ball* raw, const uint32_t* sidx,
                    const uint32_t* skey, int64_t n, Real solvent,
                    Ball* ball, uint32_t* perm, uint32_t* cellk,

@@ -1255,27 +1255,31 @@ __device__ __forceinline__ unsigned seg_ballot(bool p) {
 }
 /* After the ladder: the kept candidates of each enumeration segment of
  * `seg` items (its first bcnt[b] positions from off[b] on hold its
- * kept and formerly undecided ones). */
+ * kept and formerly undecided ones) to kept[b].  The marks in bkeep stay: the
+ * ladder may decide more of them and count again. */
 __global__ __launch_bounds__(kBlock) void k_seg_kept(
     Cnt c_n, int seg, const uint64_t* off, const uint32_t* bcnt,
-    const uint8_t* flag, uint32_t* bkeep) {
+    const uint8_t* flag, const uint32_t* bkeep, uint32_t* kept) {
   const int64_t n = c_n.get();
   const int64_t nseg = (c_n.cap + seg - 1) / seg;
   const int64_t b = gtid() / kSegLanes;
   const uint32_t sub = threadIdx.x & (kSegLanes - 1);
+  if (b >= nseg) return;
   /* a segment that queued no undecided candidate kept all it wrote: its
-   * enumeration left that count here */
-  if (b >= nseg || bkeep[b] != kRecount) return;
-  unsigned c = 0;
-  if (b * seg < n) {
-    const uint64_t base = off[b];
-    const uint32_t m = bcnt[b];
-    for (uint32_t r0 = 0; r0 < m; r0 += kSegLanes) {
-      const uint32_t t = r0 + sub;
-      c += (unsigned)__popc(seg_ballot(t < m && flag[base + t] == KEEP));
+   * enumeration left that count */
+  unsigned c = bkeep[b];
+  if (c == kRecount) {
+    c = 0;
+    if (b * seg < n) {
+      const uint64_t base = off[b];
+      const uint32_t m = bcnt[b];
+      for (uint32_t r0 = 0; r0 < m; r0 += kSegLanes) {
+        const uint32_t t = r0 + sub;
+        c += (unsigned)__popc(seg_ballot(t < m && flag[base + t] == KEEP));
+      }
     }
   }
-  if (sub == 0) bkeep[b] = c;
+  if (sub == 0) kept[b] = c;
 }
 /* the kept tets of segment b to tets[bout[b], ...), in order */
 __global__ __launch_bounds__(kBlock) void k_tet_seg_copy(
@@ -1308,12 +1312,14 @@ __global__ __launch_bounds__(kBlock) void k_tet_seg_copy(
   }
 }
 void launch_seg_kept(Cnt n, int seg, const uint64_t* off, const uint32_t* bcnt,
-                     const uint8_t* flag, uint32_t* bkeep, PipeLaunch L) {
+                     const uint8_t* flag, const uint32_t* bkeep, uint32_t* kept,
+                     PipeLaunch L) {
   if (n.cap <= 0) return;
   const int64_t nseg = (n.cap + seg - 1) / seg;
   hipLaunchKernelGGL(k_seg_kept,
                      dim3((unsigned)((nseg * kSegLanes + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, n, seg, off, bcnt, flag, bkeep);
+                     dim3(kBlock), 0, L.s, n, seg, off, bcnt, flag, bkeep,
+                     kept);
 }
 void launch_tet_seg_copy(Cnt nt, const uint64_t* bbase, const uint32_t* bcnt,
                          const uint4* ctet, const uint8_t* flag,

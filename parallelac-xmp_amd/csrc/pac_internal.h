@@ -547,7 +547,7 @@ constexpr uint32_t kRecount = 0xffffffffu;
  * flags), then, with bout their exclusive scan, the kept tets in order;
  * segment b's entries start at off[b] */
 void launch_seg_kept(Cnt n, int seg, const uint64_t* off, const uint32_t* bcnt,
-                     const uint8_t* flag, uint32_t* bkeep,
+                     const uint8_t* flag, const uint32_t* bkeep, uint32_t* kept,
                      PipeLaunch L);
 void launch_tet_seg_copy(Cnt nt, const uint64_t* bbase, const uint32_t* bcnt,
                          const uint4* ctet, const uint8_t* flag,

@@ -625,7 +625,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
      * the ladder settles the undecided ones; then the kept triangles of
      * each segment are counted, scanned and copied out in order with the
      * row starts (as for tets) */
-    DBuf<uint32_t> bcnt(P, neseg + 1), bkeep(P, neseg + 1);
+    DBuf<uint32_t> bcnt(P, neseg + 1), bkeep(P, neseg + 1), kept(P, neseg + 1);
     DBuf<uint64_t> bout(P, neseg + 1);
     auto tmp = scan_tmp(neseg);
     /* a rerun (queue overflow, eager only) recounts the candidates from
@@ -650,8 +650,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
         },
         [&](Post post) {
           launch_seg_kept(Ealpha, kTriSeg, off.get(), bcnt.get(), flag.get(),
-                          bkeep.get(), L);
-          scan_u32_to_u64(bkeep.get(), bout.get(), Cnt(neseg), tmp.get(), s,
+                          bkeep.get(), kept.get(), L);
+          scan_u32_to_u64(kept.get(), bout.get(), Cnt(neseg), tmp.get(), s,
                           dcnt + RC_TALPHA, post);
         },
         RC_TALPHA);
@@ -709,7 +709,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
      * ladder settles the undecided ones; then the kept tets of each segment
      * are counted, scanned and copied out in order */
     const int64_t nblk = (Talpha.cap + kTetSeg - 1) / kTetSeg;
-    DBuf<uint32_t> bcnt(P, nblk + 1), bkeep(P, nblk + 1);
+    DBuf<uint32_t> bcnt(P, nblk + 1), bkeep(P, nblk + 1), kept(P, nblk + 1);
     DBuf<uint64_t> bout(P, nblk + 1), bbase(P, nblk + 1);
     auto tmp = scan_tmp(nblk);
     /* a rerun (queue overflow, eager only) recounts the candidates from
@@ -736,8 +736,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
         [&](QRef qr) { launch_filter_exact(SG, 3, C2, qr, nullptr, flag.get(), L); },
         [&](Post post) {
           launch_seg_kept(Talpha, kTetSeg, bbase.get(), bcnt.get(),
-                          flag.get(), bkeep.get(), L);
-          scan_u32_to_u64(bkeep.get(), bout.get(), Cnt(nblk), tmp.get(), s,
+                          flag.get(), bkeep.get(), kept.get(), L);
+          scan_u32_to_u64(kept.get(), bout.get(), Cnt(nblk), tmp.get(), s,
                           dcnt + RC_KALPHA, post);
         },
         RC_KALPHA);

@@ -1260,26 +1260,47 @@ __device__ __forceinline__ unsigned seg_ballot(bool p) {
 __global__ __launch_bounds__(kBlock) void k_seg_kept(
     Cnt c_n, int seg, const uint64_t* off, const uint32_t* bcnt,
     const uint8_t* flag, const uint32_t* bkeep, uint32_t* kept) {
+  __shared__ uint8_t s_list[kBlock / 64][64];
   const int64_t n = c_n.get();
   const int64_t nseg = (c_n.cap + seg - 1) / seg;
-  const int64_t b = gtid() / kSegLanes;
-  const uint32_t sub = threadIdx.x & (kSegLanes - 1);
-  if (b >= nseg) return;
+  const int64_t b = gtid(), b0 = b & ~(int64_t)63;
+  if (b0 >= nseg) return; /* a whole wave */
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   /* a segment that queued no undecided candidate kept all it wrote: its
-   * enumeration left that count */
-  unsigned c = bkeep[b];
-  if (c == kRecount) {
-    c = 0;
-    if (b * seg < n) {
-      const uint64_t base = off[b];
-      const uint32_t m = bcnt[b];
-      for (uint32_t r0 = 0; r0 < m; r0 += kSegLanes) {
-        const uint32_t t = r0 + sub;
-        c += (unsigned)__popc(seg_ballot(t < m && flag[base + t] == KEEP));
+   * enumeration left that count.  The wave's others are listed and counted
+   * by kSegLanes lanes each. */
+  const uint32_t c = b < nseg ? bkeep[b] : 0u;
+  const bool count = c == kRecount && b * seg < n;
+  if (b < nseg && !count) kept[b] = c == kRecount ? 0u : c;
+  const uint64_t todo = __ballot(count);
+  if (!todo) return;
+  const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+  if (count) s_list[wv][__popcll(todo & lt)] = (uint8_t)lane;
+  wave_sync();
+  const int m = __popcll(todo);
+  const uint32_t sub = lane & (kSegLanes - 1);
+  for (int k0 = 0; k0 < m; k0 += 64 / kSegLanes) {
+    const int k = k0 + lane / kSegLanes;
+    const int64_t q = b0 + (k < m ? s_list[wv][k] : 0);
+    const uint64_t base = k < m ? off[q] : 0;
+    const uint32_t cnt = k < m ? bcnt[q] : 0;
+    unsigned sum = 0;
+    for (uint32_t t = sub; t < cnt; t += 8 * kSegLanes) {
+      uint8_t f[8]; /* in flight together */
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const uint32_t x = t + u * kSegLanes;
+        f[u] = flag[base + (x < cnt ? x : sub)];
       }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        sum += t + u * kSegLanes < cnt && f[u] == KEEP;
     }
+#pragma unroll
+    for (int d = 1; d < kSegLanes; d <<= 1)
+      sum += (unsigned)__shfl_xor((int)sum, d, 64);
+    if (k < m && sub == 0) kept[q] = sum;
   }
-  if (sub == 0) kept[b] = c;
 }
 /* the kept tets of segment b to tets[bout[b], ...), in order */
 __global__ __launch_bounds__(kBlock) void k_tet_seg_copy(
@@ -1317,7 +1338,7 @@ void launch_seg_kept(Cnt n, int seg, const uint64_t* off, const uint32_t* bcnt,
   if (n.cap <= 0) return;
   const int64_t nseg = (n.cap + seg - 1) / seg;
   hipLaunchKernelGGL(k_seg_kept,
-                     dim3((unsigned)((nseg * kSegLanes + kBlock - 1) / kBlock)),
+                     dim3((unsigned)((nseg + kBlock - 1) / kBlock)),
                      dim3(kBlock), 0, L.s, n, seg, off, bcnt, flag, bkeep,
                      kept);
 }
@@ -1345,7 +1366,7 @@ constexpr int kEdgeBallsPerBlock = kBlock / 64;
 template <class R>
 __global__ __launch_bounds__(kBlock) void k_edge_enum_filter(
     Stage S, const uint64_t* off, uint32_t* cval, uint32_t* cseg,
-    uint8_t* flag, uint32_t* bcnt, Queue q1, uint64_t lim) {
+    uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep, Queue q1, uint64_t lim) {
   const int64_t iw = (int64_t)blockIdx.x * kEdgeBallsPerBlock + (threadIdx.x >> 6);
   if (iw >= S.n) return; /* a whole wave */
   const uint32_t i = __builtin_amdgcn_readfirstlane((uint32_t)iw);
@@ -1362,6 +1383,7 @@ __global__ __launch_bounds__(kBlock) void k_edge_enum_filter(
   const Ball bi = S.ball[i];
   const uint64_t o0 = off[i];
   uint64_t o = o0; /* next compacted position */
+  bool und = false;
   __shared__ uint32_t s_end[kEdgeBallsPerBlock][64], s_beg[kEdgeBallsPerBlock][64];
   const int wv = threadIdx.x >> 6;
   for (int r0 = 0; r0 < ny * nz; r0 += 64) {
@@ -1406,6 +1428,7 @@ __global__ __launch_bounds__(kBlock) void k_edge_enum_filter(
         code = same_pos(bi, bj) ? REJECT : edge_code_ss<R>(bi, bj, S.alpha);
       }
       const uint64_t m = __ballot(code != REJECT);
+      und |= __ballot(code == UNDEC) != 0;
       if (code != REJECT) {
         const uint64_t w = o + (uint64_t)__popcll(m & lt);
         if (w < lim) {
@@ -1420,40 +1443,24 @@ __global__ __launch_bounds__(kBlock) void k_edge_enum_filter(
     /* the next pass rewrites the tables */
     __builtin_amdgcn_wave_barrier();
   }
-  if (lane == 0) bcnt[i] = cut_at((uint32_t)(o - o0), o0, lim);
+  if (lane == 0) {
+    const uint32_t c = cut_at((uint32_t)(o - o0), o0, lim);
+    bcnt[i] = c;
+    bkeep[i] = und ? kRecount : c;
+  }
 }
 void launch_edge_enum_filter(const Stage& S, const uint64_t* off,
                              uint32_t* cval, uint32_t* cseg, uint8_t* flag,
-                             uint32_t* bcnt, Queue q1, PipeLaunch L,
-                             uint64_t lim) {
+                             uint32_t* bcnt, uint32_t* bkeep, Queue q1,
+                             PipeLaunch L, uint64_t lim) {
   if (S.n <= 0) return;
   dim3 gr((unsigned)((S.n + kEdgeBallsPerBlock - 1) / kEdgeBallsPerBlock));
   if (S.staged)
     hipLaunchKernelGGL(k_edge_enum_filter<float>, gr, dim3(kBlock), 0, L.s, S,
-                       off, cval, cseg, flag, bcnt, q1, lim);
+                       off, cval, cseg, flag, bcnt, bkeep, q1, lim);
   else
     hipLaunchKernelGGL(k_edge_enum_filter<double>, gr, dim3(kBlock), 0, L.s, S,
-                       off, cval, cseg, flag, bcnt, q1, lim);
-}
-/* kept candidates of segment i among its bcnt[i] compacted ones */
-__global__ __launch_bounds__(kBlock) void k_seg_keep(int64_t n,
-                                                     const uint64_t* off,
-                                                     const uint32_t* bcnt,
-                                                     const uint8_t* flag,
-                                                     uint32_t* keep) {
-  const int64_t i = gtid();
-  if (i >= n) return;
-  const uint64_t base = off[i];
-  const uint32_t m = bcnt[i];
-  uint32_t c = 0;
-  for (uint32_t t = 0; t < m; ++t) c += flag[base + t] == KEEP;
-  keep[i] = c;
-}
-void launch_seg_keep(int64_t n, const uint64_t* off, const uint32_t* bcnt,
-                     const uint8_t* flag, uint32_t* keep, PipeLaunch L) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_seg_keep, dim3((unsigned)((n + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, n, off, bcnt, flag, keep);
+                       off, cval, cseg, flag, bcnt, bkeep, q1, lim);
 }
 /* ball i's kept edges (one wave per ball) to (ecol, eleft)[erow[i], ...),
  * their marks in edead (if given; for the triangle stage) and edge_in (the

@@ -459,13 +459,8 @@ void launch_edge_count(const Stage& S, uint32_t* cnt, PipeLaunch L);
  * i) */
 void launch_edge_enum_filter(const Stage& S, const uint64_t* off,
                              uint32_t* cval, uint32_t* cseg, uint8_t* flag,
-                             uint32_t* bcnt, Queue q1, PipeLaunch L,
+                             uint32_t* bcnt, uint32_t* bkeep, Queue q1, PipeLaunch L,
                              uint64_t lim = ~0ull);
-/* after the ladder: keep[i] = kept candidates of ball i; then, with erow
- * their exclusive scan (the alpha-edge CSR rows), the kept edges to
- * (ecol, eleft) in order */
-void launch_seg_keep(int64_t n, const uint64_t* off, const uint32_t* bcnt,
-                     const uint8_t* flag, uint32_t* keep, PipeLaunch L);
 void launch_edge_copy(int64_t n, const uint64_t* off, const uint32_t* bcnt,
                       const uint32_t* cval, const uint8_t* flag,
                       uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
@@ -538,7 +533,7 @@ void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
                             uint64_t* bbase, uint4* ctet,
                             uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep,
                             Queue q1, PipeLaunch L, uint64_t lim = ~0ull);
-/* The triangle and tet enumerations also write bkeep[b]: bcnt[b] when the
+/* The enumerations also write bkeep[b]: bcnt[b] when the
  * segment queued no undecided candidate (the ladder cannot drop any of its
  * entries), else kRecount. */
 constexpr uint32_t kRecount = 0xffffffffu;

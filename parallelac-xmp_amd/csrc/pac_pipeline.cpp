@@ -554,14 +554,14 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
      * in bcnt); the ladder settles the undecided ones; the kept counts'
      * scan is the alpha-edge CSR (erow) and the kept edges are copied out
      * in order */
-    DBuf<uint32_t> bcnt(P, n), keep(P, n);
+    DBuf<uint32_t> bcnt(P, n), bkeep(P, n), kept(P, n);
     auto tmp = scan_tmp(n);
     host_evals[0] += Ecand.cap;
     Ealpha = ladder(
         std::min<int64_t>(Ecand.cap, Ecand.cap / 32 + 65536), Ecand.cap / 64, KP_EDGE_FILL, -1,
         [&](Queue qq) {
           launch_edge_enum_filter(SG, off.get(), cval.get(), cseg.get(),
-                                  flag.get(), bcnt.get(), qq, L,
+                                  flag.get(), bcnt.get(), bkeep.get(), qq, L,
                                   (uint64_t)Ecand.cap);
         },
         [&](QRef qr, Queue q2) {
@@ -571,8 +571,9 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           launch_filter_exact(SG, 1, C0, qr, cval.get(), flag.get(), L);
         },
         [&](Post post) {
-          launch_seg_keep(n, off.get(), bcnt.get(), flag.get(), keep.get(), L);
-          scan_u32_to_u64(keep.get(), erow.get(), Cnt(n), tmp.get(), s,
+          launch_seg_kept(Cnt(n), 1, off.get(), bcnt.get(), flag.get(),
+                          bkeep.get(), kept.get(), L);
+          scan_u32_to_u64(kept.get(), erow.get(), Cnt(n), tmp.get(), s,
                           dcnt + RC_EALPHA, post);
         },
         RC_EALPHA);

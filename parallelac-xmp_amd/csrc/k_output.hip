@@ -347,10 +347,27 @@ void filtration_order(int64_t m, const uint64_t* key, const int64_t counts[4],
  * so d rho / d p_q = 2 lam_q (p_q - c) and d rho / d r_q = -2 lam_q r_q.
  * Contributions are written per (simplex, vertex) slot and summed per ball
  * in slot order after a stable sort by ball: the result is deterministic. */
+/* this lane's place among those counted so far for v: one atomic for a run
+ * of lanes with the same v (rows come by their first vertex), by its first
+ * lane (the lanes at work are the wave's first ones) */
+__device__ __forceinline__ uint32_t count_run(uint32_t* cnt, uint32_t v) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t prev = (uint32_t)__shfl_up((int)v, 1, 64);
+  const uint64_t act = __ballot(true);
+  const uint64_t heads = __ballot(lane == 0 || prev != v);
+  const uint64_t upto = ~0ull >> (63 - lane);
+  const int head = 63 - __builtin_clzll(heads & upto);
+  const uint64_t later = lane == 63 ? 0ull : heads >> (lane + 1);
+  const int end = later ? lane + 1 + __builtin_ctzll(later) : __popcll(act);
+  uint32_t base = 0;
+  if (head == lane) base = atomicAdd(cnt + v, (uint32_t)(end - lane));
+  return (uint32_t)__shfl((int)base, head, 64) + (uint32_t)(lane - head);
+}
 template <int DIM>
 __global__ __launch_bounds__(kBlock) void k_adj_contrib(
     int64_t m, const int32_t* rows, const double4* balls, const double* g,
-    int64_t slot0, uint32_t* key, uint32_t* val, double4* contrib) {
+    int64_t slot0, uint32_t* key, uint32_t* place, uint32_t* cnt,
+    double4* contrib) {
   int64_t id = gtid();
   if (id >= m) return;
   const int32_t* r = rows + (int64_t)(DIM + 1) * id;
@@ -367,49 +384,93 @@ __global__ __launch_bounds__(kBlock) void k_adj_contrib(
     int64_t sl = slot0 + (int64_t)(DIM + 1) * id + q;
     contrib[sl] = make_double4(k * dx, k * dy, k * dz, -k * p.w);
     key[sl] = (uint32_t)r[q];
-    val[sl] = (uint32_t)sl;
+    place[sl] = count_run(cnt, (uint32_t)r[q]);
   }
 }
-__global__ __launch_bounds__(kBlock) void k_adj_gather(
-    int64_t n, const uint32_t* vstart, const uint32_t* sval,
-    const double4* contrib, double* dxyz, double* dr) {
-  int64_t i = gtid();
-  if (i >= n) return;
-  double sx = 0, sy = 0, sz = 0, sr = 0;
-  for (uint32_t q = vstart[i], e = vstart[i + 1]; q < e; ++q) {
-    double4 c = contrib[sval[q]];
-    sx += c.x;
-    sy += c.y;
-    sz += c.z;
-    sr += c.w;
+/* the slots by ball, as they arrived, then in each ball's part by slot (as
+ * many after its start as it holds smaller slots): the sums do not depend on
+ * the order of arrival */
+__global__ __launch_bounds__(kBlock) void k_adj_put(
+    int64_t m, const uint32_t* key, const uint32_t* place,
+    const uint32_t* vstart, uint32_t* slot) {
+  const int64_t i = gtid();
+  if (i < m) slot[vstart[key[i]] + place[i]] = (uint32_t)i;
+}
+__global__ __launch_bounds__(kBlock) void k_adj_order(
+    int64_t m, const uint32_t* key, const uint32_t* vstart,
+    const uint32_t* slot, uint32_t* sorted) {
+  const int64_t i = gtid();
+  if (i >= m) return;
+  const uint32_t o = slot[i], v = key[o], b = vstart[v], e = vstart[v + 1];
+  uint32_t at = b;
+  for (uint32_t t = b; t < e; t += 8) { /* eight loads in flight together */
+    uint32_t x[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) x[k] = slot[t + k < e ? t + k : b];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) at += t + k < e && x[k] < o;
   }
-  dxyz[3 * i] = sx;
-  dxyz[3 * i + 1] = sy;
-  dxyz[3 * i + 2] = sz;
-  dr[i] = sr;
+  sorted[at] = o;
+}
+/* kAdjLanes lanes a ball, each every kAdjLanes-th of its contributions, then
+ * their sums pairwise */
+constexpr int kAdjLanes = 8;
+__global__ __launch_bounds__(kBlock) void k_adj_gather(
+    int64_t n, const uint32_t* vstart, const uint32_t* sorted,
+    const double4* contrib, double* dxyz, double* dr) {
+  const int64_t i = gtid() / kAdjLanes;
+  if (i >= n) return;
+  const uint32_t sub = threadIdx.x & (kAdjLanes - 1);
+  double v[4] = {0, 0, 0, 0};
+  for (uint32_t q = vstart[i] + sub, e = vstart[i + 1]; q < e; q += kAdjLanes) {
+    const double4 c = contrib[sorted[q]];
+    v[0] += c.x;
+    v[1] += c.y;
+    v[2] += c.z;
+    v[3] += c.w;
+  }
+#pragma unroll
+  for (int d = 1; d < kAdjLanes; d <<= 1)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] += __shfl_xor(v[k], d, 64);
+  if (sub == 0) {
+    dxyz[3 * i] = v[0];
+    dxyz[3 * i + 1] = v[1];
+    dxyz[3 * i + 2] = v[2];
+    dr[i] = v[3];
+  }
 }
 void launch_adj_contrib(int dim, int64_t m, const int32_t* rows,
                         const double4* balls, const double* g, int64_t slot0,
-                        uint32_t* key, uint32_t* val, double4* contrib,
-                        hipStream_t s) {
+                        uint32_t* key, uint32_t* place, uint32_t* cnt,
+                        double4* contrib, hipStream_t s) {
   if (m <= 0) return;
   dim3 gr((unsigned)((m + kBlock - 1) / kBlock));
   if (dim == 1)
     hipLaunchKernelGGL(k_adj_contrib<1>, gr, dim3(kBlock), 0, s, m, rows, balls,
-                       g, slot0, key, val, contrib);
+                       g, slot0, key, place, cnt, contrib);
   else if (dim == 2)
     hipLaunchKernelGGL(k_adj_contrib<2>, gr, dim3(kBlock), 0, s, m, rows, balls,
-                       g, slot0, key, val, contrib);
+                       g, slot0, key, place, cnt, contrib);
   else
     hipLaunchKernelGGL(k_adj_contrib<3>, gr, dim3(kBlock), 0, s, m, rows, balls,
-                       g, slot0, key, val, contrib);
+                       g, slot0, key, place, cnt, contrib);
 }
-void launch_adj_gather(int64_t n, const uint32_t* vstart, const uint32_t* sval,
-                       const double4* contrib, double* dxyz, double* dr,
-                       hipStream_t s) {
+void launch_adj_gather(int64_t n, int64_t m, const uint32_t* key,
+                       const uint32_t* place, const uint32_t* vstart,
+                       uint32_t* slot, uint32_t* sorted, const double4* contrib,
+                       double* dxyz, double* dr, hipStream_t s) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_adj_gather, dim3((unsigned)((n + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, s, n, vstart, sval, contrib, dxyz, dr);
+  if (m > 0) {
+    const dim3 gm((unsigned)((m + kBlock - 1) / kBlock));
+    hipLaunchKernelGGL(k_adj_put, gm, dim3(kBlock), 0, s, m, key, place, vstart,
+                       slot);
+    hipLaunchKernelGGL(k_adj_order, gm, dim3(kBlock), 0, s, m, key, vstart,
+                       slot, sorted);
+  }
+  hipLaunchKernelGGL(k_adj_gather,
+                     dim3((unsigned)((n * kAdjLanes + kBlock - 1) / kBlock)),
+                     dim3(kBlock), 0, s, n, vstart, sorted, contrib, dxyz, dr);
 }
 
 /* sort the vertices of each row ascending (rows of k = DIM+1 ids) */

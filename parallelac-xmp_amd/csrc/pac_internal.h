@@ -345,11 +345,12 @@ void launch_rho(int dim, int64_t m, const int32_t* rows, const double4* balls,
  * the slots sorted by vertex */
 void launch_adj_contrib(int dim, int64_t m, const int32_t* rows,
                         const double4* balls, const double* g, int64_t slot0,
-                        uint32_t* key, uint32_t* val, double4* contrib,
+                        uint32_t* key, uint32_t* place, uint32_t* cnt, double4* contrib,
                         hipStream_t s);
-void launch_adj_gather(int64_t n, const uint32_t* vstart, const uint32_t* sval,
-                       const double4* contrib, double* dxyz, double* dr,
-                       hipStream_t s);
+void launch_adj_gather(int64_t n, int64_t m, const uint32_t* key,
+                       const uint32_t* place, const uint32_t* vstart,
+                       uint32_t* slot, uint32_t* sorted, const double4* contrib,
+                       double* dxyz, double* dr, hipStream_t s);
 void canonical_rows(int K, int64_t m, int32_t* rows, int idbits,
                     uint32_t* idx, uint32_t* key, uint32_t* idx2,
                     uint32_t* key2, void* rtmp, size_t rtb, int32_t* copy,

@@ -603,6 +603,7 @@ static void autotune(const float* xyzr, int64_t n, const int64_t* offsets,
     static const int blocks[] = {64, 128, 256};
     static const int chunks[] = {64, 256, 1024};
     const pac_options tuned = pick;
+    best = 1e300; /* a shape of the set, also if none beats the default's time */
     for (int bl : blocks)
       for (int ch : chunks) {
         pac_options t = tuned;

@@ -267,7 +267,7 @@ __global__ __launch_bounds__(kBlock) void k_tet_ac2_quick(
 /* What an emptiness kernel walks: every simplex (one per thread), or those
  * a pass before it listed, up to the phase-one budget; or the ones the
  * first phase left. */
-enum { PH_ALL = 0, PH_LIST = 1, PH_REST = 2 };
+enum { PH_ALL = 0, PH_LIST = 1, PH_REST = 2, PH_PACK = 3 };
 /* Phase A (budget > 0): at most `budget` pair tests per tet, in scan order;
  * tets not settled within the budget are appended to `rest`.  Phase B
  * (persistent, over `rest`): the remaining pairs of those tets, skipping the
@@ -768,82 +768,36 @@ __device__ __forceinline__ int low_known(int64_t id, const uint32_t* tkd,
   if (KIND == 0) return (tkd[id] & kDeadBit) ? 0 : -1;
   return edead && edead[id] ? 0 : -1;
 }
-/* The flags of the simplices decided without a scan, and the list of the
- * others: on the 100k globule 2.4M of 11.4M triangles and 0.4M of 2.2M
- * edges.  Scanned in place, the few of each wave keep all of it busy:
- * triangle phase A 280 us against 33 us for the list and 116 us for its
- * scans. */
-template <int KIND>
-__global__ __launch_bounds__(kBlock) void k_low_list(
-    Stage S, Cnt c_n, const uint32_t* tkd, const uint8_t* edead,
-    const uint8_t* in_flag, uint8_t* flag, uint32_t* next, unsigned* nnext) {
-  /* kListRun items a thread, 256 apart (coalesced), one append for all */
-  const int64_t n = c_n.get();
-  const int64_t i0 = (int64_t)blockIdx.x * (kBlock * kListRun) + threadIdx.x;
-  int c[kListRun];
-#pragma unroll
-  for (int q = 0; q < kListRun; ++q) {
-    const int64_t id = i0 + q * kBlock;
-    c[q] = id < n ? low_known<KIND>(id, tkd, edead, in_flag) : 0;
-  }
-#pragma unroll
-  for (int q = 0; q < kListRun; ++q) {
-    const int64_t id = i0 + q * kBlock;
-    if (id < n && c[q] >= 0) flag[id] = (uint8_t)c[q];
-  }
-  /* positions: by thread within the wave, then by wave; a wave's items stay
-   * together, neighbours in the list share their surroundings */
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  __shared__ unsigned s_w[kBlock / 64], s_base;
-  unsigned wtot = 0;
-  uint64_t m[kListRun];
-#pragma unroll
-  for (int q = 0; q < kListRun; ++q) {
-    m[q] = __ballot(c[q] < 0);
-    wtot += (unsigned)__popcll(m[q]);
-  }
-  if (lane == 0) s_w[w] = wtot;
-  __syncthreads();
-  const unsigned k = blockIdx.x & (LSLOTS - 1);
-  if (threadIdx.x == 0) {
-    unsigned t = 0;
-    for (int q = 0; q < kBlock / 64; ++q) t += s_w[q];
-    s_base = t ? atomicAdd(nnext + k * kSlotWords, t) : 0u;
-  }
-  __syncthreads();
-  unsigned at = s_base;
-  for (int q = 0; q < w; ++q) at += s_w[q];
-  const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-#pragma unroll
-  for (int q = 0; q < kListRun; ++q) {
-    const unsigned o = at + (unsigned)__popcll(m[q] & lt);
-    if (c[q] < 0 && o < S.lcap)
-      next[(uint64_t)k * S.lcap + o] = (uint32_t)(i0 + q * kBlock);
-    at += (unsigned)__popcll(m[q]);
-  }
-}
-
-/* Same phase A / phase B split as the tet kernel; phase A runs over the
- * listed simplices (items), or over all, deciding the known ones itself. */
+/* Same phase A / phase B split as the tet kernel.  Phase A scans what it
+ * cannot decide at once: one simplex a thread (PH_ALL), or (PH_PACK) a block
+ * looks at kPack x 256, of which usually a quarter are left (on the 100k
+ * globule 2.4M of 11.4M triangles, 0.4M of 2.2M edges), and its threads take
+ * one of those each; a block's few past 256 go to phase B untested
+ * (kRestWhole).  Phase A of the triangles at 100k: 280 us in place; 33 + 116
+ * with a listing pass before it, 40 of them for the blocks that found the
+ * list's end; 101 packed, and 10 more in phase B. */
+constexpr uint32_t kRestWhole = 0x80000000u;
 template <class R, int KIND, int PH, bool FINE, bool MOL>
 __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
-    Stage S0, Cnt c_nitems, const uint32_t* items, const unsigned* nitems,
-    const uint32_t* ecol, const uint32_t* eleft,
+    Stage S0, Cnt c_nitems, const uint32_t* ecol, const uint32_t* eleft,
     const uint32_t* tkd, const uint32_t* tedge, const uint8_t* edead,
     const uint8_t* in_flag, uint8_t* flag, Queue q1, uint32_t* rest,
     unsigned* nrest, int budget) {
   unsigned evals = 0, pairs = 0;
   __shared__ uint32_t s_pre[LSLOTS + 1];
-  if (PH != PH_ALL) list_table(PH == PH_REST ? nrest : nitems, S0.lcap, s_pre);
+  if (PH == PH_REST) list_table(nrest, S0.lcap, s_pre);
   const int64_t total =
-      PH != PH_ALL ? (int64_t)s_pre[LSLOTS] : c_nitems.get();
+      PH == PH_REST ? (int64_t)s_pre[LSLOTS] : c_nitems.get();
   uint32_t rest_id = 0xffffffffu; /* phase A: the item left for phase B */
   auto item = [&](int64_t w) {
     const Stage& S = fresh_stage();
-    const int64_t id =
-        PH == PH_ALL ? w
-                     : (int64_t)list_at(PH == PH_REST ? rest : items, S.lcap,
-                                        s_pre, (uint32_t)w);
+    int64_t id = w;
+    int tested = budget; /* phase B: the pairs that phase A tested */
+    if (PH == PH_REST) {
+      const uint32_t x = list_at(rest, S.lcap, s_pre, (uint32_t)w);
+      id = x & ~kRestWhole;
+      if (x & kRestWhole) tested = 0;
+    }
     if (PH == PH_ALL) {
       const int c = low_known<KIND>(id, tkd, edead, in_flag);
       if (c >= 0) {
@@ -867,7 +821,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     PairSS<R> P;
     typename std::conditional<FINE, SphBox, CellBox>::type box;
     if (!low_setup<R, KIND>(g, v, P, box)) {
-      if (PH != PH_REST) {
+      if (PH != PH_REST || !tested) {
         push_q(q1, (uint32_t)id, 0xffffffffu);
         flag[id] = 2;
       }
@@ -879,7 +833,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     auto visit = [&](uint32_t j, const Ball& E) {
       if (!FINE && (j == vid[0] || j == vid[1] || j == vid[2])) return false;
       if (PH == PH_REST) {
-        if (seen < budget) {
+        if (seen < tested) {
           ++seen;
           return false;
         }
@@ -907,7 +861,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     /* fine grid: four balls at a time, as in k_tet_ac2_hot */
     auto group = [&](uint32_t p, uint32_t n) -> bool {
       if (PH == PH_REST) {
-        if (seen < budget) {
+        if (seen < tested) {
           seen += (int)n;
           return false;
         }
@@ -943,7 +897,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
       scan_sph_flat(g, S.fstart, box, group);
     else
       scan_box4(g, S.cstart, S.ball, box, visit);
-    if (PH == PH_REST) {
+    if (PH == PH_REST && tested) {
       if (stop == 1)
         flag[id] = 0;
       else if (pending)
@@ -956,10 +910,58 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
   if constexpr (PH == PH_REST) {
     for_work(S0.bchunk, total, item); /* persistent launch */
   } else {
-    /* (a list's grid covers all simplices: its length is known only on the
-     * device, and a loop over it costs 30 VGPRs, 7 -> 4 waves per SIMD) */
-    if ((int64_t)blockIdx.x * kBlock >= total) return;
-    if (gtid() < total) item(gtid());
+    if constexpr (PH == PH_PACK) {
+      const int64_t i0 = (int64_t)blockIdx.x * (kBlock * kPack);
+      if (i0 >= total) return;
+      __shared__ uint32_t s_live[kBlock];
+      __shared__ unsigned s_w[kBlock / 64], s_over;
+      const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+      const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+      /* kPack items a thread, 256 apart (coalesced); a wave's items stay
+       * together, neighbours share their surroundings */
+      int c[kPack];
+      unsigned wtot = 0;
+#pragma unroll
+      for (int q = 0; q < kPack; ++q) {
+        const int64_t id = i0 + q * kBlock + threadIdx.x;
+        c[q] = id < total ? low_known<KIND>(id, tkd, edead, in_flag) : 0;
+      }
+#pragma unroll
+      for (int q = 0; q < kPack; ++q) {
+        const int64_t id = i0 + q * kBlock + threadIdx.x;
+        if (id < total && c[q] >= 0) flag[id] = (uint8_t)c[q];
+        wtot += (unsigned)__popcll(__ballot(c[q] < 0));
+      }
+      if (lane == 0) s_w[wv] = wtot;
+      __syncthreads();
+      unsigned at = 0, live = 0;
+      for (int q = 0; q < kBlock / 64; ++q) {
+        if (q < wv) at += s_w[q];
+        live += s_w[q];
+      }
+      const unsigned k = blockIdx.x & (LSLOTS - 1);
+      if (live > kBlock && threadIdx.x == 0)
+        s_over = atomicAdd(nrest + k * kSlotWords, live - kBlock);
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < kPack; ++q) {
+        const uint64_t m = __ballot(c[q] < 0);
+        const unsigned o = at + (unsigned)__popcll(m & lt);
+        const uint32_t id = (uint32_t)(i0 + q * kBlock + threadIdx.x);
+        if (c[q] < 0) {
+          if (o < kBlock)
+            s_live[o] = id;
+          else if (s_over + (o - kBlock) < S0.lcap)
+            rest[(uint64_t)k * S0.lcap + s_over + (o - kBlock)] =
+                id | kRestWhole;
+        }
+        at += (unsigned)__popcll(m);
+      }
+      __syncthreads();
+      if (threadIdx.x < live) item(s_live[threadIdx.x]);
+    } else {
+      if (gtid() < total) item(gtid());
+    }
     list_append(rest, nrest, S0.lcap, rest_id != 0xffffffffu, rest_id);
   }
   (void)evals;
@@ -1339,31 +1341,27 @@ static void low_hot4(const Stage& S, Cnt nitems, const uint32_t* ecol,
                      const uint32_t* eleft, const uint32_t* tkd,
                      const uint32_t* tedge, const uint8_t* edead,
                      const uint8_t* in_flag, uint8_t* flag, Queue q1,
-                     uint32_t* rest, unsigned* nrest, uint32_t* next,
-                     unsigned* nnext, int budget, PipeLaunch L) {
+                     uint32_t* rest, unsigned* nrest, int budget,
+                     PipeLaunch L) {
   const dim3 gr((unsigned)((nitems.cap + kBlock - 1) / kBlock)),
       gb(rest_grid(S, nitems));
-  if (nitems.cap >= kListItems) {
-    const int64_t per = kBlock * kListRun;
-    hipLaunchKernelGGL(k_low_list<KIND>,
+  if (S.pack && nitems.cap >= kPackItems && nitems.cap < ((int64_t)1 << 31) &&
+      budget > 0) {
+    const int64_t per = kBlock * kPack;
+    hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, PH_PACK, FINE, MOL>),
                        dim3((unsigned)((nitems.cap + per - 1) / per)),
-                       dim3(kBlock), 0, L.s, S, nitems, tkd, edead, in_flag,
-                       flag, next, nnext);
-    hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, PH_LIST, FINE, MOL>), gr,
-                       dim3(kBlock), 0, L.s, S, nitems, next,
-                       nnext, ecol, eleft, tkd, tedge, edead, in_flag, flag, q1,
-                       rest, nrest, budget);
+                       dim3(kBlock), 0, L.s, S, nitems, ecol, eleft, tkd, tedge,
+                       edead, in_flag, flag, q1, rest, nrest, budget);
   } else {
     hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, PH_ALL, FINE, MOL>), gr,
-                       dim3(kBlock), 0, L.s, S, nitems, next, nnext, ecol,
-                       eleft, tkd, tedge, edead, in_flag, flag, q1, rest, nrest,
-                       budget);
+                       dim3(kBlock), 0, L.s, S, nitems, ecol, eleft, tkd, tedge,
+                       edead, in_flag, flag, q1, rest, nrest, budget);
   }
   if (budget > 0) {
     hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, PH_REST, FINE, MOL>), gb,
-                       dim3((unsigned)S.bblock), 0, L.s, S, nitems, next, nnext,
-                       ecol, eleft, tkd, tedge, edead, in_flag, flag, q1, rest,
-                       nrest, budget);
+                       dim3((unsigned)S.bblock), 0, L.s, S, nitems, ecol, eleft,
+                       tkd, tedge, edead, in_flag, flag, q1, rest, nrest,
+                       budget);
   }
 }
 template <class R, int KIND, bool FINE>
@@ -1371,57 +1369,56 @@ static void low_hot3(const Stage& S, Cnt nitems, const uint32_t* ecol,
                      const uint32_t* eleft, const uint32_t* tkd,
                      const uint32_t* tedge, const uint8_t* edead,
                      const uint8_t* in_flag, uint8_t* flag, Queue q1,
-                     uint32_t* rest, unsigned* nrest, uint32_t* next,
-                     unsigned* nnext, int budget, PipeLaunch L) {
+                     uint32_t* rest, unsigned* nrest, int budget,
+                     PipeLaunch L) {
   if (S.mol)
     low_hot4<R, KIND, FINE, true>(S, nitems, ecol, eleft, tkd, tedge, edead,
-                                  in_flag, flag, q1, rest, nrest, next, nnext,
-                                  budget, L);
+                                  in_flag, flag, q1, rest, nrest, budget,
+                                  L);
   else
     low_hot4<R, KIND, FINE, false>(S, nitems, ecol, eleft, tkd, tedge, edead,
-                                   in_flag, flag, q1, rest, nrest, next, nnext,
-                                   budget, L);
+                                   in_flag, flag, q1, rest, nrest, budget,
+                                  L);
 }
 template <class R, int KIND>
 static void low_hot2(const Stage& S, Cnt nitems, const uint32_t* ecol,
                      const uint32_t* eleft, const uint32_t* tkd,
                      const uint32_t* tedge, const uint8_t* edead,
                      const uint8_t* in_flag, uint8_t* flag, Queue q1,
-                     uint32_t* rest, unsigned* nrest, uint32_t* next,
-                     unsigned* nnext, int budget, PipeLaunch L) {
+                     uint32_t* rest, unsigned* nrest, int budget,
+                     PipeLaunch L) {
   if (S.fine)
     low_hot3<R, KIND, true>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
-                            flag, q1, rest, nrest, next, nnext, budget, L);
+                            flag, q1, rest, nrest, budget, L);
   else
     low_hot3<R, KIND, false>(S, nitems, ecol, eleft, tkd, tedge, edead,
-                             in_flag, flag, q1, rest, nrest, next, nnext,
-                             budget, L);
+                             in_flag, flag, q1, rest, nrest, budget,
+                                  L);
 }
 void launch_low_ac2_hot(const Stage& S, int kind, Cnt nitems,
                         const uint32_t* ecol, const uint32_t* eleft,
                         const uint32_t* tkd, const uint32_t* tedge,
                         const uint8_t* edead, const uint8_t* in_flag,
                         uint8_t* flag, Queue q1, uint32_t* rest,
-                        unsigned* nrest, uint32_t* next, unsigned* nnext,
-                        int budget, PipeLaunch L) {
+                        unsigned* nrest, int budget, PipeLaunch L) {
   if (nitems.cap <= 0) return;
   if constexpr (!kBallF64) {
     if (S.staged) {
       if (kind == 0)
         low_hot2<float, 0>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
-                           flag, q1, rest, nrest, next, nnext, budget, L);
+                           flag, q1, rest, nrest, budget, L);
       else
         low_hot2<float, 1>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
-                           flag, q1, rest, nrest, next, nnext, budget, L);
+                           flag, q1, rest, nrest, budget, L);
       return;
     }
   }
   if (kind == 0)
     low_hot2<double, 0>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
-                        flag, q1, rest, nrest, next, nnext, budget, L);
+                        flag, q1, rest, nrest, budget, L);
   else
     low_hot2<double, 1>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
-                        flag, q1, rest, nrest, next, nnext, budget, L);
+                        flag, q1, rest, nrest, budget, L);
 }
 void launch_low_ac2_esc(const Stage& S, int kind, QRef q,
                         const uint32_t* ecol, const uint32_t* eleft,

@@ -184,11 +184,11 @@ constexpr int QSLOTS = 32;
  * in one 128-byte line: appending 44,600 blocks' items took 262 us, with a
  * line for each counter 53 us. */
 constexpr int LSLOTS = 32;
-constexpr int kListRun = 8; /* items a thread of a listing pass takes */
+constexpr int kPack = 4; /* items a thread of a packing block looks at */
 inline uint32_t list_slot_cap(int64_t blocks) {
-  /* blocks of kBlock items, or of kListRun times as many */
-  return (uint32_t)((blocks + LSLOTS * kListRun - 1) / (LSLOTS * kListRun) *
-                    (kBlock * kListRun));
+  /* blocks of kBlock items, or of kPack times as many */
+  return (uint32_t)((blocks + LSLOTS * kPack - 1) / (LSLOTS * kPack) *
+                    (kBlock * kPack));
 }
 /* queue counters of a run: slot k's line of kSlotWords words holds the
  * fills of sub-queue k of the hot (QK_HOT) and escalation (QK_ESC) queues
@@ -436,6 +436,9 @@ struct Stage {
   const Ball* fball;     /* balls in fine-cell order */
   const uint32_t* fid;   /* their ball (cell-sorted) ids */
   const uint32_t* fstart;
+  /* covered edges are marked: most triangles and edges are decided without
+   * a scan */
+  int pack;
   /* chunk != 0: a chunk's sub-input, whose output keeps only the simplices
    * with lowest vertex in [own_lo, own_hi) (cell-sorted ids).  Emptiness
    * tests that cannot change one of those are skipped: tets with none of
@@ -561,13 +564,12 @@ void launch_filter_exact(const Stage& S, int kind, CandCtx C, QRef q, const uint
  * number of items); budget = phase A pair budget (0: single phase) */
 /* next / nnext: scratch list (capacity = number of items) of the simplices
  * phase A scans, where a pass before it left only some: the quick
- * rejection pass (tets, fine scan grid), a chunk sub-input's needed tets,
- * the triangles / edges neither in the closure nor covered (kListItems).
+ * rejection pass (tets, fine scan grid), a chunk sub-input's needed tets.
  * Both lists' counters come cleared (the ladder's last kernel does it). */
-/* triangles / edges from this many on are listed before their scans: the
- * dead and closed ones leave most lanes of a wave idle otherwise; below it
- * the extra launch costs more than the idle lanes do */
-constexpr int64_t kListItems = 1 << 17;
+/* triangles / edges from this many on are packed by the blocks that scan
+ * them: the dead and closed ones leave most lanes of a wave idle otherwise;
+ * fewer do not fill the chip as they are */
+constexpr int64_t kPackItems = 1 << 17;
 /* chunk sub-input: in_flag[id] = 1 (pass untested) for the triangles
  * (kind 0) / edges (kind 1) no owned simplex depends on */
 void launch_own_mark(const Stage& S, int kind, Cnt n, const uint32_t* ecol,
@@ -597,8 +599,7 @@ void launch_low_ac2_hot(const Stage& S, int kind, Cnt nitems,
                         const uint32_t* tkd, const uint32_t* tedge,
                         const uint8_t* edead, const uint8_t* in_flag,
                         uint8_t* flag, Queue q1, uint32_t* rest,
-                        unsigned* nrest, uint32_t* next, unsigned* nnext,
-                        int budget, PipeLaunch L);
+                        unsigned* nrest, int budget, PipeLaunch L);
 void launch_low_ac2_esc(const Stage& S, int kind, QRef q,
                         const uint32_t* ecol, const uint32_t* eleft,
                         const uint32_t* tk, const uint32_t* tedge,

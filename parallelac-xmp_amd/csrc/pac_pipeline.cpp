@@ -538,6 +538,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
    * whose scans see every ball (the reference's stencil may miss the
    * covering one), and where tets are tested */
   const bool prune = opt.cell_policy == PAC_CELL_EXACT && !opt.skip_tet_ac2;
+  SG.pack = prune;
   DBuf<uint8_t> edead, edge_in; /* edge_in, tri_in: the closure's marks */
   CandCtx C0{nullptr, nullptr, nullptr, nullptr, nullptr};
   if (!no_edges) {
@@ -886,8 +887,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           [&](Queue q) {
             launch_low_ac2_hot(SG, 0, Talpha, ecol.get(), eleft.get(), tkm,
                                tedge.get(), nullptr, tri_skip, tflag.get(), q,
-                               rest.get(), nrest, next.get(), nnext,
-                               budget(Talpha), L);
+                               rest.get(), nrest, budget(Talpha), L);
           },
           [&](QRef q, Queue q2) {
             launch_low_ac2_esc(SG, 0, q, ecol.get(), eleft.get(), tk.get(),
@@ -954,8 +954,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           [&](Queue q) {
             launch_low_ac2_hot(SG, 1, Ealpha, ecol.get(), eleft.get(), nullptr,
                                nullptr, dead, edge_skip, eflag.get(), q,
-                               rest.get(), nrest, next.get(), nnext,
-                               budget(Ealpha), L);
+                               rest.get(), nrest, budget(Ealpha), L);
           },
           [&](QRef q, Queue q2) {
             launch_low_ac2_esc(SG, 1, q, ecol.get(), eleft.get(), nullptr,

@@ -53,10 +53,13 @@ typedef struct pac_options {
   int32_t ac2_budget;    /* emptiness phase-one pair budget: > 0 splits
                             each scan after that many balls, the rest
                             finished by the persistent second phase
-                            (0 = 4); < 0: one phase, every scan to its end */
+                            (0 = 6, or 4 with the reference's cells or
+                            skip_tet_ac2, and one phase below 65,536
+                            simplices); < 0: one phase, every scan to its
+                            end                                          */
   int32_t batch_balls;   /* batch: max balls per pipeline pass (0 = 4Mi;
                             a recorded batch, pac_graph_create: 2Mi)      */
-  int32_t ac2_grid;      /* blocks of the second emptiness phase (0=2048) */
+  int32_t ac2_grid;      /* blocks of the second emptiness phase (0=4096) */
   int32_t ac2_fine;      /* exact policy: emptiness scans over the grid's
                             cells split in ac2_fine (2..8) along x
                             (0 = 2, < 0 or 1: the grid's own cells)       */

@@ -316,7 +316,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   SG.ex.alpha = pl.alpha_wi;
   /* FP64 balls are not exact in FP32: their ladder starts at FP64 */
   SG.staged = opt.precision == PAC_PREC_STAGED && !kBallF64;
-  SG.bgrid = opt.ac2_grid > 0 ? std::min(opt.ac2_grid, 1 << 16) : 2048;
+  SG.bgrid = opt.ac2_grid > 0 ? std::min(opt.ac2_grid, 1 << 16) : 4096;
   /* persistent second emptiness phase: block shape and hand-out size */
   SG.bblock = opt.block == 64 || opt.block == 128 ? opt.block : kBlock;
   SG.bchunk = opt.ac2_chunk > 0
@@ -782,7 +782,11 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
 
   /* ---- tet emptiness ---- */
   /* phase-one budget: 0 = the default, < 0 = no second phase.  The default
-   * is 4 where the items fill the chip many times over, and one phase below
+   * is 6 (4 without the covered simplices gone, which were the quickly
+   * rejected ones) where the items fill the chip many times over: with 4,096
+   * blocks in phase two, 1M balls 12.85 ms, 12.90 at 8, 13.0 at 16, and
+   * 13.41 at 4 and 2,048 blocks; 100k balls 1572 us, 1588, 1604, 1607; the
+   * reference's cells on 60k balls 646 at 6, 639 at 4.  One phase below
    * kOnePhase items: then no wave waits for a slot, the run is as long as
    * its longest scan either way, and the second phase's launch comes on top
    * (262 balls, 8,000 tets: 11 us in one phase, 11 + 21 in two). */
@@ -790,7 +794,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   auto budget = [&](Cnt items) {
     return opt.ac2_budget > 0
                ? opt.ac2_budget
-               : (opt.ac2_budget < 0 || items.cap < kOnePhase ? 0 : 4);
+               : (opt.ac2_budget < 0 || items.cap < kOnePhase ? 0
+                                                           : (prune ? 6 : 4));
   };
   /* the left-over and quick-pass lists: LSLOTS sub-lists sized for the
    * largest first-phase grid */

@@ -759,13 +759,13 @@ __device__ __forceinline__ bool low_setup(const GridP& g, const Ball* v,
 /* KIND 0: triangles (items = alpha triangle ids), 1: edges (alpha edge
  * ids).  What is decided without a scan: 1 for a simplex already in the
  * closure (in_flag), 0 for one with an edge that one ball covers (kDeadBit
- * in tkd, edead), else -1. */
+ * in tk, edead), else -1. */
 template <int KIND>
-__device__ __forceinline__ int low_known(int64_t id, const uint32_t* tkd,
+__device__ __forceinline__ int low_known(int64_t id, const uint32_t* tk,
                                          const uint8_t* edead,
                                          const uint8_t* in_flag) {
   if (in_flag[id]) return 1;
-  if (KIND == 0) return (tkd[id] & kDeadBit) ? 0 : -1;
+  if (KIND == 0) return (tk[id] & kDeadBit) ? 0 : -1;
   return edead && edead[id] ? 0 : -1;
 }
 /* Same phase A / phase B split as the tet kernel.  Phase A scans what it
@@ -780,7 +780,7 @@ constexpr uint32_t kRestWhole = 0x80000000u;
 template <class R, int KIND, int PH, bool FINE, bool MOL>
 __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     Stage S0, Cnt c_nitems, const uint32_t* ecol, const uint32_t* eleft,
-    const uint32_t* tkd, const uint32_t* tedge, const uint8_t* edead,
+    const uint32_t* tk, const uint32_t* tedge, const uint8_t* edead,
     const uint8_t* in_flag, uint8_t* flag, Queue q1, uint32_t* rest,
     unsigned* nrest, int budget) {
   unsigned evals = 0, pairs = 0;
@@ -799,7 +799,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
       if (x & kRestWhole) tested = 0;
     }
     if (PH == PH_ALL) {
-      const int c = low_known<KIND>(id, tkd, edead, in_flag);
+      const int c = low_known<KIND>(id, tk, edead, in_flag);
       if (c >= 0) {
         flag[id] = (uint8_t)c;
         return;
@@ -810,7 +810,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
       uint32_t e = tedge[id];
       vid[0] = eleft[e];
       vid[1] = ecol[e];
-      vid[2] = tkd[id] & ~kDeadBit;
+      vid[2] = tk[id] & ~kDeadBit;
     } else {
       vid[0] = eleft[id];
       vid[1] = ecol[id];
@@ -924,7 +924,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
 #pragma unroll
       for (int q = 0; q < kPack; ++q) {
         const int64_t id = i0 + q * kBlock + threadIdx.x;
-        c[q] = id < total ? low_known<KIND>(id, tkd, edead, in_flag) : 0;
+        c[q] = id < total ? low_known<KIND>(id, tk, edead, in_flag) : 0;
       }
 #pragma unroll
       for (int q = 0; q < kPack; ++q) {
@@ -984,7 +984,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_esc(
       uint32_t ed = tedge[e.item];
       vid[0] = eleft[ed];
       vid[1] = ecol[ed];
-      vid[2] = tk[e.item];
+      vid[2] = tk[e.item] & ~kDeadBit;
     } else {
       vid[0] = eleft[e.item];
       vid[1] = ecol[e.item];
@@ -1091,7 +1091,7 @@ __device__ __forceinline__ void low_exact_setup(const Stage& S,
     const uint32_t ed = tedge[item];
     T.vid[0] = eleft[ed];
     T.vid[1] = ecol[ed];
-    T.vid[2] = tk[item];
+    T.vid[2] = tk[item] & ~kDeadBit;
   } else {
     T.vid[0] = eleft[item];
     T.vid[1] = ecol[item];
@@ -1338,7 +1338,7 @@ void launch_tet_ac2_exact_sorted(const Stage& S, const uint32_t* item,
 }
 template <class R, int KIND, bool FINE, bool MOL>
 static void low_hot4(const Stage& S, Cnt nitems, const uint32_t* ecol,
-                     const uint32_t* eleft, const uint32_t* tkd,
+                     const uint32_t* eleft, const uint32_t* tk,
                      const uint32_t* tedge, const uint8_t* edead,
                      const uint8_t* in_flag, uint8_t* flag, Queue q1,
                      uint32_t* rest, unsigned* nrest, int budget,
@@ -1350,54 +1350,54 @@ static void low_hot4(const Stage& S, Cnt nitems, const uint32_t* ecol,
     const int64_t per = kBlock * kPack;
     hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, PH_PACK, FINE, MOL>),
                        dim3((unsigned)((nitems.cap + per - 1) / per)),
-                       dim3(kBlock), 0, L.s, S, nitems, ecol, eleft, tkd, tedge,
+                       dim3(kBlock), 0, L.s, S, nitems, ecol, eleft, tk, tedge,
                        edead, in_flag, flag, q1, rest, nrest, budget);
   } else {
     hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, PH_ALL, FINE, MOL>), gr,
-                       dim3(kBlock), 0, L.s, S, nitems, ecol, eleft, tkd, tedge,
+                       dim3(kBlock), 0, L.s, S, nitems, ecol, eleft, tk, tedge,
                        edead, in_flag, flag, q1, rest, nrest, budget);
   }
   if (budget > 0) {
     hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, PH_REST, FINE, MOL>), gb,
                        dim3((unsigned)S.bblock), 0, L.s, S, nitems, ecol, eleft,
-                       tkd, tedge, edead, in_flag, flag, q1, rest, nrest,
+                       tk, tedge, edead, in_flag, flag, q1, rest, nrest,
                        budget);
   }
 }
 template <class R, int KIND, bool FINE>
 static void low_hot3(const Stage& S, Cnt nitems, const uint32_t* ecol,
-                     const uint32_t* eleft, const uint32_t* tkd,
+                     const uint32_t* eleft, const uint32_t* tk,
                      const uint32_t* tedge, const uint8_t* edead,
                      const uint8_t* in_flag, uint8_t* flag, Queue q1,
                      uint32_t* rest, unsigned* nrest, int budget,
                      PipeLaunch L) {
   if (S.mol)
-    low_hot4<R, KIND, FINE, true>(S, nitems, ecol, eleft, tkd, tedge, edead,
+    low_hot4<R, KIND, FINE, true>(S, nitems, ecol, eleft, tk, tedge, edead,
                                   in_flag, flag, q1, rest, nrest, budget,
                                   L);
   else
-    low_hot4<R, KIND, FINE, false>(S, nitems, ecol, eleft, tkd, tedge, edead,
+    low_hot4<R, KIND, FINE, false>(S, nitems, ecol, eleft, tk, tedge, edead,
                                    in_flag, flag, q1, rest, nrest, budget,
                                   L);
 }
 template <class R, int KIND>
 static void low_hot2(const Stage& S, Cnt nitems, const uint32_t* ecol,
-                     const uint32_t* eleft, const uint32_t* tkd,
+                     const uint32_t* eleft, const uint32_t* tk,
                      const uint32_t* tedge, const uint8_t* edead,
                      const uint8_t* in_flag, uint8_t* flag, Queue q1,
                      uint32_t* rest, unsigned* nrest, int budget,
                      PipeLaunch L) {
   if (S.fine)
-    low_hot3<R, KIND, true>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
+    low_hot3<R, KIND, true>(S, nitems, ecol, eleft, tk, tedge, edead, in_flag,
                             flag, q1, rest, nrest, budget, L);
   else
-    low_hot3<R, KIND, false>(S, nitems, ecol, eleft, tkd, tedge, edead,
+    low_hot3<R, KIND, false>(S, nitems, ecol, eleft, tk, tedge, edead,
                              in_flag, flag, q1, rest, nrest, budget,
                                   L);
 }
 void launch_low_ac2_hot(const Stage& S, int kind, Cnt nitems,
                         const uint32_t* ecol, const uint32_t* eleft,
-                        const uint32_t* tkd, const uint32_t* tedge,
+                        const uint32_t* tk, const uint32_t* tedge,
                         const uint8_t* edead, const uint8_t* in_flag,
                         uint8_t* flag, Queue q1, uint32_t* rest,
                         unsigned* nrest, int budget, PipeLaunch L) {
@@ -1405,19 +1405,19 @@ void launch_low_ac2_hot(const Stage& S, int kind, Cnt nitems,
   if constexpr (!kBallF64) {
     if (S.staged) {
       if (kind == 0)
-        low_hot2<float, 0>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
+        low_hot2<float, 0>(S, nitems, ecol, eleft, tk, tedge, edead, in_flag,
                            flag, q1, rest, nrest, budget, L);
       else
-        low_hot2<float, 1>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
+        low_hot2<float, 1>(S, nitems, ecol, eleft, tk, tedge, edead, in_flag,
                            flag, q1, rest, nrest, budget, L);
       return;
     }
   }
   if (kind == 0)
-    low_hot2<double, 0>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
+    low_hot2<double, 0>(S, nitems, ecol, eleft, tk, tedge, edead, in_flag,
                         flag, q1, rest, nrest, budget, L);
   else
-    low_hot2<double, 1>(S, nitems, ecol, eleft, tkd, tedge, edead, in_flag,
+    low_hot2<double, 1>(S, nitems, ecol, eleft, tk, tedge, edead, in_flag,
                         flag, q1, rest, nrest, budget, L);
 }
 void launch_low_ac2_esc(const Stage& S, int kind, QRef q,

@@ -50,7 +50,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_tets(
    * (i, .); -1 if there is none (a recorded pass over its capacities) */
   auto face = [&](uint32_t e, uint32_t e2, uint32_t v) -> int64_t {
     const uint64_t m = emask[e].x, r0 = trow[e];
-    if (m >> 63) return find_row(tk, r0, trow[e + 1], v);
+    if (m >> 63) return find_row(tk, r0, trow[e + 1], v, ~kDeadBit);
     const uint32_t r = e2 - e - 1u;
     if (r >= 63u || !((m >> r) & 1)) return -1;
     return (int64_t)(r0 + (uint64_t)__popcll(m & ((1ull << r) - 1)));
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_tris(
     edge_in[tejk[t]] = 1;
     out[3 * p] = (int32_t)perm[eleft[e]];
     out[3 * p + 1] = (int32_t)perm[ecol[e]];
-    out[3 * p + 2] = (int32_t)perm[tk[t]];
+    out[3 * p + 2] = (int32_t)perm[tk[t] & ~kDeadBit];
   });
 }
 void launch_tile_tris(Cnt nt, const uint8_t* flag, const uint64_t* offs,

@@ -652,7 +652,7 @@ __global__ __launch_bounds__(kBlock) void k_tail_caps_own(
   int64_t q = gtid();
   if (q >= m) return;
   const uint32_t e = owner[q];
-  const uint32_t i = eleft[e], j = ecol[e], k = tk[q];
+  const uint32_t i = eleft[e], j = ecol[e], k = tk[q] & ~kDeadBit;
   const bool need = (i >= S.own_lo && i < S.own_hi) ||
                     (j >= S.own_lo && j < S.own_hi) ||
                     (k >= S.own_lo && k < S.own_hi);
@@ -914,13 +914,13 @@ constexpr int fam_of(int KIND) {
  * or more edges on: dense inputs) merges the three rows instead, each lane
  * its own, into fourth vertices in LDS (928 of them, the rest in the
  * candidates' own array).
- * At 100k balls 271 us; 395 with all waves merging, whose rounds last as
+ * At 100k balls 266 us; 395 with all waves merging, whose rounds last as
  * long as their longest rows; 523 with blocks of 256 triangles filtering
  * every slot.  200k balls with a lattice block: 1.39 ms against 1.70 and
  * 9.6.  The vector ALU bounds it, the filter's 114 instructions being half
  * of a round.
  * A candidate with a covered edge (kDeadBit of one of its triangles in
- * tkd, carried with the fourth vertex) is filtered like any other, but an
+ * tk, carried with the fourth vertex) is filtered like any other, but an
  * alpha tet among them is only counted (CTR_DROP), not written: it cannot
  * be empty.  On the 100k globule 4.6M of the 19.1M alpha tets are written. */
 /* First slot of alpha triangle q without a per-triangle offset array:
@@ -941,7 +941,7 @@ __device__ __forceinline__ uint64_t tet_slot_off(const uint64_t* roff,
 template <class R, bool BUF>
 __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_filter(
-    Stage S, Cnt c_nt, const uint64_t* trow, const uint32_t* tkd,
+    Stage S, Cnt c_nt, const uint64_t* trow, const uint32_t* tk,
     const uint32_t* tedge, const uint32_t* teik, const uint32_t* tejk,
     const uint32_t* eleft, const uint32_t* ecol, const ulonglong2* emask,
     const uint64_t* off, const uint64_t* roff, const uint32_t* epre,
@@ -971,7 +971,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
       eij = tedge[q];
       eik = teik[q];
       ejk = tejk[q];
-      kd = tkd[q];
+      kd = tk[q];
       i = eleft[eij];
       j = ecol[eij];
       mij = emask[eij];
@@ -1054,9 +1054,9 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
        * its current one (kEnd past the row's end, above every ball id) */
       if (o < oe) {
         if constexpr (BUF) {
-          /* byte offsets into tkd (below 4 GiB): no 64-bit address
+          /* byte offsets into tk (below 4 GiB): no 64-bit address
            * arithmetic per load */
-          const BufU32 K{tkd, (uint32_t)(c_nt.cap * 4)};
+          const BufU32 K{tk, (uint32_t)(c_nt.cap * 4)};
           uint32_t a = ((uint32_t)q + 1u) << 2, ae = (uint32_t)trow[eij + 1] << 2;
           uint32_t b = (uint32_t)trow[eik] << 2, be = (uint32_t)trow[eik + 1] << 2;
           uint32_t c = (uint32_t)trow[ejk] << 2, ce = (uint32_t)trow[ejk + 1] << 2;
@@ -1088,7 +1088,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
           uint32_t b = (uint32_t)trow[eik], be = (uint32_t)trow[eik + 1];
           uint32_t c = (uint32_t)trow[ejk], ce = (uint32_t)trow[ejk + 1];
           while (a < ae && b < be && c < ce) {
-            const uint32_t xd = tkd[a], yd = tkd[b], zd = tkd[c];
+            const uint32_t xd = tk[a], yd = tk[b], zd = tk[c];
             const uint32_t x = xd & kEnd, y = yd & kEnd, z = zd & kEnd;
             const uint32_t m = max(x, max(y, z));
             if (x == m && y == m && z == m) {
@@ -1144,7 +1144,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
             const uint64_t ax = (uint64_t)x.y << 32 | x.x;
             /* (bit b of `after` is set: the count includes it) */
             const uint32_t tl = q0 + t + (uint32_t)__popcll(ax << (63u - b));
-            const uint32_t p = tejk[tl] - z.w, ld = tkd[tl];
+            const uint32_t p = tejk[tl] - z.w, ld = tk[tl];
             const uint32_t mm = p & 32u ? y.y : y.x, md = p & 32u ? y.w : y.z;
             have = p < 63u && ((mm >> (p & 31u)) & 1u);
             dead = (((b & 32u ? x.w : x.z) >> (b & 31u)) | (md >> (p & 31u))) & 1u;
@@ -1216,7 +1216,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
   block_flush(S.ctr, CTR_DROP, dropped);
 }
 void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
-                            const uint32_t* tkd, const uint32_t* tedge,
+                            const uint32_t* tk, const uint32_t* tedge,
                             const uint32_t* teik, const uint32_t* tejk,
                             const uint32_t* eleft, const uint32_t* ecol,
                             const ulonglong2* emask, const uint64_t* off,
@@ -1226,13 +1226,13 @@ void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
                             PipeLaunch L, uint64_t lim) {
   if (nt.cap <= 0) return;
   dim3 gr((unsigned)((nt.cap + kBlock - 1) / kBlock));
-  /* byte offsets into tkd while it stays below 4 GiB */
+  /* byte offsets into tk while it stays below 4 GiB */
   const bool buf = nt.cap < ((int64_t)1 << 30);
   if constexpr (!kBallF64) {
     if (S.staged) {
       auto kf = buf ? k_tet_enum_filter<float, true>
                     : k_tet_enum_filter<float, false>;
-      hipLaunchKernelGGL(kf, gr, dim3(kBlock), 0, L.s, S, nt, trow, tkd, tedge,
+      hipLaunchKernelGGL(kf, gr, dim3(kBlock), 0, L.s, S, nt, trow, tk, tedge,
                          teik, tejk, eleft, ecol, emask, off, roff, epre, bbase, ctet,
                          flag, bcnt, bkeep, q1, lim);
       return;
@@ -1240,7 +1240,7 @@ void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
   }
   auto kd = buf ? k_tet_enum_filter<double, true>
                 : k_tet_enum_filter<double, false>;
-  hipLaunchKernelGGL(kd, gr, dim3(kBlock), 0, L.s, S, nt, trow, tkd, tedge, teik,
+  hipLaunchKernelGGL(kd, gr, dim3(kBlock), 0, L.s, S, nt, trow, tk, tedge, teik,
                      tejk, eleft, ecol, emask, off, roff, epre, bbase, ctet, flag,
                      bcnt, bkeep, q1, lim);
 }
@@ -1365,8 +1365,8 @@ void launch_tet_seg_copy(Cnt nt, const uint64_t* bbase, const uint32_t* bcnt,
 constexpr int kEdgeBallsPerBlock = kBlock / 64;
 template <class R>
 __global__ __launch_bounds__(kBlock) void k_edge_enum_filter(
-    Stage S, const uint64_t* off, uint32_t* cval, uint32_t* cseg,
-    uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep, Queue q1, uint64_t lim) {
+    Stage S, const uint64_t* off, uint32_t* cval, uint8_t* flag,
+    uint32_t* bcnt, uint32_t* bkeep, Queue q1, uint64_t lim) {
   const int64_t iw = (int64_t)blockIdx.x * kEdgeBallsPerBlock + (threadIdx.x >> 6);
   if (iw >= S.n) return; /* a whole wave */
   const uint32_t i = __builtin_amdgcn_readfirstlane((uint32_t)iw);
@@ -1433,7 +1433,6 @@ __global__ __launch_bounds__(kBlock) void k_edge_enum_filter(
         const uint64_t w = o + (uint64_t)__popcll(m & lt);
         if (w < lim) {
           cval[w] = j;
-          cseg[w] = i;
           flag[w] = (uint8_t)code;
           if (code == UNDEC) push_q(q1, (uint32_t)w, i);
         }
@@ -1450,17 +1449,17 @@ __global__ __launch_bounds__(kBlock) void k_edge_enum_filter(
   }
 }
 void launch_edge_enum_filter(const Stage& S, const uint64_t* off,
-                             uint32_t* cval, uint32_t* cseg, uint8_t* flag,
+                             uint32_t* cval, uint8_t* flag,
                              uint32_t* bcnt, uint32_t* bkeep, Queue q1,
                              PipeLaunch L, uint64_t lim) {
   if (S.n <= 0) return;
   dim3 gr((unsigned)((S.n + kEdgeBallsPerBlock - 1) / kEdgeBallsPerBlock));
   if (S.staged)
     hipLaunchKernelGGL(k_edge_enum_filter<float>, gr, dim3(kBlock), 0, L.s, S,
-                       off, cval, cseg, flag, bcnt, bkeep, q1, lim);
+                       off, cval, flag, bcnt, bkeep, q1, lim);
   else
     hipLaunchKernelGGL(k_edge_enum_filter<double>, gr, dim3(kBlock), 0, L.s, S,
-                       off, cval, cseg, flag, bcnt, bkeep, q1, lim);
+                       off, cval, flag, bcnt, bkeep, q1, lim);
 }
 /* ball i's kept edges (one wave per ball) to (ecol, eleft)[erow[i], ...),
  * their marks in edead (if given; for the triangle stage) and edge_in (the
@@ -1509,6 +1508,17 @@ void launch_edge_copy(int64_t n, const uint64_t* off, const uint32_t* bcnt,
       edge_in, ocap);
 }
 
+/* a triangle candidate's edge within its segment, and how far edge (i, k) lies
+ * after it in row(i), in one word (a row of 2^26 edges has more candidate
+ * pairs among its balls than a run accepts) */
+static_assert(kTriSeg == 64, "six bits for the edge");
+__device__ __forceinline__ uint32_t tri_pos(uint32_t edge, uint32_t ahead) {
+  return edge << 26 | ahead;
+}
+__device__ __forceinline__ uint32_t tri_seg_edge(uint32_t x) { return x >> 26; }
+__device__ __forceinline__ uint32_t tri_ahead(uint32_t x) {
+  return x & 0x3ffffffu;
+}
 /* Triangles of alpha edge q = (i, j) -- k in row(i) after j and in row(j),
  * the positions of k in the two rows being the alpha-edge ids of (i, k)
  * and (j, k), recorded for the tet stage and the closure -- fused with the
@@ -1517,9 +1527,9 @@ void launch_edge_copy(int64_t n, const uint64_t* off, const uint32_t* bcnt,
  * (edge, position in row(j)) in LDS and takes them 64 at a time: k's
  * position in row(i) by a binary search in the wave's part of ecol, which is
  * in LDS (none: a false hit), then the filter; the kept and undecided ones
- * are written compacted, in order, from the wave's first slot on, four
- * arrays and the flag.
- * 121 us at 100k balls (30 at 16068), 211 (48) for blocks of 256 edges that
+ * are written compacted, in order, from the wave's first slot on, three
+ * words and the flag.
+ * 113 us at 100k balls (30 at 16068), 211 (48) for blocks of 256 edges that
  * merged the rows into LDS and filtered them from there, waiting for their
  * longest rows and at two barriers a round.
  * A wave with a row too long for the hits or the LDS merges its rows into
@@ -1532,9 +1542,8 @@ template <class R>
 __global__ __launch_bounds__(kBlock) void k_tri_enum_filter(
     Stage S, Cnt c_ne, const uint64_t* erow, const uint32_t* ecol,
     const uint32_t* eleft, const ulonglong2* hits, const uint64_t* off,
-    uint32_t* cval, uint32_t* cseg, uint32_t* cea, uint32_t* ceb,
-    uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep, uint8_t* edead, Queue q1,
-    uint64_t lim) {
+    uint32_t* cval, uint32_t* cpos, uint32_t* ceb, uint8_t* flag,
+    uint32_t* bcnt, uint32_t* bkeep, uint8_t* edead, Queue q1, uint64_t lim) {
   /* with the tables 4,096 bytes of LDS a wave: 8 blocks per CU */
   constexpr uint32_t LIST = 1152, COLS = 192;
   __shared__ uint4 s_tab[kBlock / 64][64];
@@ -1593,8 +1602,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_enum_filter(
                    [&](uint32_t k, uint32_t a, uint32_t bb) {
                      if (o < lim) {
                        cval[o] = k;
-                       cseg[o] = (uint32_t)q;
-                       cea[o] = a;
+                       cpos[o] = tri_pos((uint32_t)lane, a - (uint32_t)q);
                        ceb[o] = bb;
                      }
                      ++o;
@@ -1646,8 +1654,9 @@ __global__ __launch_bounds__(kBlock) void k_tri_enum_filter(
           }
         } else if (have) {
           k = cval[base + d];
-          e = cseg[base + d];
-          ea = cea[base + d];
+          const uint32_t x = cpos[base + d];
+          e = q0 + tri_seg_edge(x);
+          ea = e + tri_ahead(x);
           eb = ceb[base + d];
           vi = eleft[e];
           vj = ecol[e];
@@ -1671,8 +1680,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_enum_filter(
           const uint64_t o = base + run + (uint32_t)__popcll(bm & lt);
           if (o < lim) {
             cval[o] = k;
-            cseg[o] = e;
-            cea[o] = ea;
+            cpos[o] = tri_pos(e - q0, ea - e);
             ceb[o] = eb;
             flag[o] = (uint8_t)r;
             if (r == UNDEC) push_q(q1, (uint32_t)o, e);
@@ -1694,22 +1702,22 @@ __global__ __launch_bounds__(kBlock) void k_tri_enum_filter(
 void launch_tri_enum_filter(const Stage& S, Cnt ne, const uint64_t* erow,
                             const uint32_t* ecol, const uint32_t* eleft,
                             const ulonglong2* hits, const uint64_t* off,
-                            uint32_t* cval, uint32_t* cseg, uint32_t* cea,
-                            uint32_t* ceb, uint8_t* flag, uint32_t* bcnt,
+                            uint32_t* cval, uint32_t* cpos, uint32_t* ceb,
+                            uint8_t* flag, uint32_t* bcnt,
                             uint32_t* bkeep, uint8_t* edead, Queue q1,
                             PipeLaunch L, uint64_t lim) {
   if (ne.cap <= 0) return;
   dim3 gr((unsigned)((ne.cap + kBlock - 1) / kBlock));
   auto kf = S.staged ? k_tri_enum_filter<float> : k_tri_enum_filter<double>;
   hipLaunchKernelGGL(kf, gr, dim3(kBlock), 0, L.s, S, ne, erow, ecol, eleft,
-                     hits, off, cval, cseg, cea, ceb, flag, bcnt, bkeep, edead,
+                     hits, off, cval, cpos, ceb, flag, bcnt, bkeep, edead,
                      q1, lim);
 }
 /* the kept triangles of segment b to (tk, tedge, teik, tejk)[bout[b], ...)
  * in order, a wave each; trow[e] for its edges e (and trow[ne], by the wave
  * holding index ne) = bout[b] + the kept triangles of its edges before e.
- * tkd (if given): tk with kDeadBit set where one of the triangle's edges is
- * marked in edead; tri_in (the closure's marks) cleared.  emask[e], e = (i,j): x has bit r if (i, j, k) is a
+ * tk has kDeadBit set where one of the triangle's edges is marked in edead
+ * (if given); tri_in (the closure's marks) cleared.  emask[e], e = (i,j): x has bit r if (i, j, k) is a
  * triangle and (i, k) the (r + 1)th edge after e, y the bits of those with
  * kDeadBit; bit 63 is set if some r is 63 or more.  spair, epre (if given):
  * the tet slots of the segment's triangles (each one's row tail), and of
@@ -1717,9 +1725,8 @@ void launch_tri_enum_filter(const Stage& S, Cnt ne, const uint64_t* erow,
  * has one entry more than segments. */
 __global__ __launch_bounds__(kBlock) void k_tri_seg_copy(
     Cnt c_ne, const uint64_t* off, const uint32_t* bcnt, const uint32_t* cval,
-    const uint32_t* cseg, const uint32_t* cea, const uint32_t* ceb,
-    const uint8_t* flag, const uint64_t* bout, const uint8_t* edead,
-    uint32_t* tk, uint32_t* tkd, uint32_t* tedge, uint32_t* teik,
+    const uint32_t* cpos, const uint32_t* ceb, const uint8_t* flag,
+    const uint64_t* bout, const uint8_t* edead, uint32_t* tk, uint32_t* tedge, uint32_t* teik,
     uint32_t* tejk, uint64_t* trow, uint64_t* spair, uint32_t* epre,
     ulonglong2* emask, uint8_t* tri_in, uint64_t ocap) {
   __shared__ uint32_t s_cnt[kBlock / 64][64];
@@ -1745,7 +1752,8 @@ __global__ __launch_bounds__(kBlock) void k_tri_seg_copy(
     uint64_t o = o0;
     /* kU entries a lane in flight together: the rounds' chains of loads are
      * what the kernel waits for (139 us at 100k balls one by one, 122 by
-     * two, 115 by four; the bytes moved take 55) */
+     * two, 115 by four; 94 with 12 bytes read and 17 written a triangle for
+     * 16 and 21) */
     constexpr int kU = 4;
     for (uint32_t r0 = 0; r0 < n; r0 += 64 * kU) {
       /* an entry's arrays are read whether or not it is kept (all were
@@ -1757,9 +1765,10 @@ __global__ __launch_bounds__(kBlock) void k_tri_seg_copy(
         const uint32_t t = r0 + 64u * u + (uint32_t)lane;
         const uint64_t at = base + (t < n ? t : n - 1);
         fv[u] = all ? (uint32_t)KEEP : flag[at];
-        sv[u] = cseg[at];
+        const uint32_t x = cpos[at];
+        sv[u] = (uint32_t)q0 + tri_seg_edge(x);
         xv[u] = cval[at];
-        av[u] = cea[at];
+        av[u] = sv[u] + tri_ahead(x);
         bv[u] = ceb[at];
         if (t >= n) fv[u] = REJECT;
       }
@@ -1787,8 +1796,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_seg_copy(
           }
           const uint64_t w = o + (uint64_t)__popcll(bm & lt);
           if (w < ocap) {
-            tk[w] = xv[u];
-            if (tkd) tkd[w] = xv[u] | (dead[u] ? kDeadBit : 0u);
+            tk[w] = xv[u] | (dead[u] ? kDeadBit : 0u);
             tedge[w] = seg;
             teik[w] = av[u];
             tejk[w] = bv[u];
@@ -1824,19 +1832,18 @@ __global__ __launch_bounds__(kBlock) void k_tri_seg_copy(
   }
 }
 void launch_tri_seg_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
-                         const uint32_t* cval, const uint32_t* cseg,
-                         const uint32_t* cea, const uint32_t* ceb,
-                         const uint8_t* flag, const uint64_t* bout,
-                         const uint8_t* edead, uint32_t* tk, uint32_t* tkd,
-                         uint32_t* tedge, uint32_t* teik, uint32_t* tejk,
+                         const uint32_t* cval, const uint32_t* cpos,
+                         const uint32_t* ceb, const uint8_t* flag,
+                         const uint64_t* bout, const uint8_t* edead,
+                         uint32_t* tk, uint32_t* tedge, uint32_t* teik, uint32_t* tejk,
                          uint64_t* trow, uint64_t* spair, uint32_t* epre,
                          ulonglong2* emask, uint8_t* tri_in, PipeLaunch L,
                          uint64_t ocap) {
   const int64_t nseg = (std::max<int64_t>(ne.cap, 0) + kTriSeg - 1) / kTriSeg;
   hipLaunchKernelGGL(k_tri_seg_copy,
                      dim3((unsigned)((nseg + kBlock / 64) / (kBlock / 64))),
-                     dim3(kBlock), 0, L.s, ne, off, bcnt, cval, cseg, cea, ceb,
-                     flag, bout, edead, tk, tkd, tedge, teik, tejk, trow, spair,
+                     dim3(kBlock), 0, L.s, ne, off, bcnt, cval, cpos, ceb,
+                     flag, bout, edead, tk, tedge, teik, tejk, trow, spair,
                      epre, emask, tri_in, ocap);
 }
 

@@ -267,11 +267,13 @@ struct StageOf<FEDD> {
  * eight entries where a binary search waits on every probe (the rows of
  * the alpha edge and triangle CSRs hold a few to a few tens of entries) */
 __device__ __forceinline__ int64_t find_row(const uint32_t* a, uint64_t lo,
-                                            uint64_t hi, uint32_t v) {
+                                            uint64_t hi, uint32_t v,
+                                            uint32_t mask = ~0u) {
   for (uint64_t p = lo; p < hi; p += 8) {
     uint32_t x[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) x[k] = p + k < hi ? a[p + k] : 0xffffffffu;
+    for (int k = 0; k < 8; ++k)
+      x[k] = p + k < hi ? a[p + k] & mask : 0xffffffffu;
     int hit = 8;
 #pragma unroll
     for (int k = 7; k >= 0; --k)

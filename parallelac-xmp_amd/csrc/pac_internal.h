@@ -462,7 +462,7 @@ void launch_edge_count(const Stage& S, uint32_t* cnt, PipeLaunch L);
  * their number to bcnt[i]; undecided ones queued on q1 by position (aux =
  * i) */
 void launch_edge_enum_filter(const Stage& S, const uint64_t* off,
-                             uint32_t* cval, uint32_t* cseg, uint8_t* flag,
+                             uint32_t* cval, uint8_t* flag,
                              uint32_t* bcnt, uint32_t* bkeep, Queue q1, PipeLaunch L,
                              uint64_t lim = ~0ull);
 void launch_edge_copy(int64_t n, const uint64_t* off, const uint32_t* bcnt,
@@ -488,8 +488,8 @@ void launch_tri_hits(Cnt ne, const uint64_t* erow, const uint32_t* ecol,
                      unsigned long long* ts, PipeLaunch L);
 /* triangle candidates of the alpha edges, each filtered by the first
  * precision stage in the same kernel: enumeration segment b (kTriSeg alpha
- * edges) writes its kept and undecided candidates (k, edge, edge(i,k),
- * edge(j,k)) with their flags, in order, compacted from its first slot
+ * edges) writes its kept and undecided candidates (k, the edge and how far
+ * edge(i,k) lies after it, edge(j,k)) with their flags, in order, compacted from its first slot
  * off[b] (the exclusive scan of launch_tri_hits's counts) on and their number to bcnt[b]; undecided ones are queued on
  * q1 by position (aux = their edge).  edead[e] (cleared by the caller;
  * null: not wanted) is set for the alpha edges a rejected candidate shows
@@ -497,22 +497,22 @@ void launch_tri_hits(Cnt ne, const uint64_t* erow, const uint32_t* ecol,
 void launch_tri_enum_filter(const Stage& S, Cnt ne, const uint64_t* erow,
                             const uint32_t* ecol, const uint32_t* eleft,
                             const ulonglong2* hits, const uint64_t* off,
-                            uint32_t* cval, uint32_t* cseg, uint32_t* cea,
-                            uint32_t* ceb, uint8_t* flag, uint32_t* bcnt,
+                            uint32_t* cval, uint32_t* cpos, uint32_t* ceb,
+                            uint8_t* flag, uint32_t* bcnt,
                             uint32_t* bkeep, uint8_t* edead, Queue q1,
                             PipeLaunch L, uint64_t lim = ~0ull);
 /* after the ladder (bkeep by launch_seg_kept over the ne alpha
  * edges, bout its exclusive scan): the kept triangles of each segment to
- * (tk, tedge, teik, tejk) in order (tkd, if given: tk with kDeadBit where one
- * of the three edges is marked in edead), the alpha-triangle row start of
+ * (tk, tedge, teik, tejk) in order (tk with kDeadBit where one of the three
+ * edges is marked in edead), the alpha-triangle row start of
  * every alpha edge, trow[0 .. ne], its third vertices as a mask (emask), and
  * (spair, if given) the segment's tet slots, L (L - 1) / 2 for an edge of L
  * triangles (each one's row tail), with epre[e] those before edge e in it */
 void launch_tri_seg_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
-                         const uint32_t* cval, const uint32_t* cseg,
-                         const uint32_t* cea, const uint32_t* ceb,
-                         const uint8_t* flag, const uint64_t* bout,
-                         const uint8_t* edead, uint32_t* tk, uint32_t* tkd,
+                         const uint32_t* cval, const uint32_t* cpos,
+                         const uint32_t* ceb, const uint8_t* flag,
+                         const uint64_t* bout, const uint8_t* edead,
+                         uint32_t* tk,
                          uint32_t* tedge, uint32_t* teik, uint32_t* tejk,
                          uint64_t* trow, uint64_t* spair, uint32_t* epre,
                          ulonglong2* emask, uint8_t* tri_in, PipeLaunch L,
@@ -522,14 +522,14 @@ void launch_tri_seg_copy(Cnt ne, const uint64_t* off, const uint32_t* bcnt,
  * triangles) writes its kept and undecided tets (i, j, k, l) with their
  * flags, in order, compacted from its first slot on (bbase[b]) and their
  * number to bcnt[b]; undecided ones are queued on q1 by position.  Kept
- * tets one of whose triangles has kDeadBit in tkd are counted (CTR_DROP)
+ * tets one of whose triangles has kDeadBit in tk are counted (CTR_DROP)
  * but not written.  Slot offsets per triangle from off[], or (off null)
  * from roff, the exclusive scan of launch_tri_seg_copy's spair, and epre
  * (each triangle's slots its row's tail: not for chunk sub-inputs, whose
  * unowned triangles get none) */
 constexpr int kTetSeg = 64;
 void launch_tet_enum_filter(const Stage& S, Cnt nt, const uint64_t* trow,
-                            const uint32_t* tkd, const uint32_t* tedge,
+                            const uint32_t* tk, const uint32_t* tedge,
                             const uint32_t* teik, const uint32_t* tejk,
                             const uint32_t* eleft, const uint32_t* ecol,
                             const ulonglong2* emask, const uint64_t* off,
@@ -596,7 +596,7 @@ void launch_tet_ac2_exact_sorted(const Stage& S, const uint32_t* item,
 /* kind 0 triangles, 1 edges */
 void launch_low_ac2_hot(const Stage& S, int kind, Cnt nitems,
                         const uint32_t* ecol, const uint32_t* eleft,
-                        const uint32_t* tkd, const uint32_t* tedge,
+                        const uint32_t* tk, const uint32_t* tedge,
                         const uint8_t* edead, const uint8_t* in_flag,
                         uint8_t* flag, Queue q1, uint32_t* rest,
                         unsigned* nrest, int budget, PipeLaunch L);

@@ -548,7 +548,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       launch_edge_count(SG, cnt.get(), L);
       Ecand = count_scan(cnt.get(), n, off.get(), RC_ECAND, "edge");
     }
-    DBuf<uint32_t> cval(P, Ecand.cap), cseg(P, Ecand.cap);
+    DBuf<uint32_t> cval(P, Ecand.cap);
     DBuf<uint8_t> flag(P, Ecand.cap);
     /* enumeration and first filter stage in one kernel (each ball's kept
      * and undecided candidates compacted from its first slot, their count
@@ -561,8 +561,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     Ealpha = ladder(
         std::min<int64_t>(Ecand.cap, Ecand.cap / 32 + 65536), Ecand.cap / 64, KP_EDGE_FILL, -1,
         [&](Queue qq) {
-          launch_edge_enum_filter(SG, off.get(), cval.get(), cseg.get(),
-                                  flag.get(), bcnt.get(), bkeep.get(), qq, L,
+          launch_edge_enum_filter(SG, off.get(), cval.get(), flag.get(),
+                                  bcnt.get(), bkeep.get(), qq, L,
                                   (uint64_t)Ecand.cap);
         },
         [&](QRef qr, Queue q2) {
@@ -603,7 +603,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   const bool tail_slots = !SG.chunk;
   DBuf<uint64_t> spair(P, tail_slots ? std::max<int64_t>(neseg, 1) : 1);
   DBuf<uint32_t> epre(P, tail_slots ? std::max<int64_t>(Ealpha.cap, 1) : 1);
-  DBuf<uint32_t> tk, tkd, tedge, teik, tejk;
+  DBuf<uint32_t> tk, tedge, teik, tejk;
   DBuf<uint8_t> tri_in;
   /* per alpha edge 128 bits: first its hits, then its mask of third
    * vertices */
@@ -619,8 +619,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       Tslots = count_scan(cnt.get(), Cnt(neseg), off.get(), RC_TSLOTS,
                           "triangle");
     }
-    DBuf<uint32_t> cval(P, Tslots.cap), cseg(P, Tslots.cap),
-        cea(P, Tslots.cap), ceb(P, Tslots.cap);
+    DBuf<uint32_t> cval(P, Tslots.cap), cpos(P, Tslots.cap), ceb(P, Tslots.cap);
     DBuf<uint8_t> flag(P, Tslots.cap);
     /* enumeration and first filter stage in one kernel, each segment's kept
      * and undecided candidates compacted in place (their count in bcnt);
@@ -639,8 +638,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
           if (runs++ && !rec)
             zero_counter(ctr, CTR_CAND + 1, s);
           launch_tri_enum_filter(SG, Ealpha, erow.get(), ecol.get(), eleft.get(),
-                                 emask.get(), off.get(), cval.get(), cseg.get(),
-                                 cea.get(), ceb.get(), flag.get(), bcnt.get(),
+                                 emask.get(), off.get(), cval.get(), cpos.get(),
+                                 ceb.get(), flag.get(), bcnt.get(),
                                  bkeep.get(), dead, qq, L,
                                  (uint64_t)Tslots.cap);
         },
@@ -658,22 +657,18 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
         },
         RC_TALPHA);
     tk = DBuf<uint32_t>(P, Talpha.cap);
-    if (prune) tkd = DBuf<uint32_t>(P, Talpha.cap);
     tedge = DBuf<uint32_t>(P, Talpha.cap);
     teik = DBuf<uint32_t>(P, Talpha.cap);
     tejk = DBuf<uint32_t>(P, Talpha.cap);
     tri_in = DBuf<uint8_t>(P, Talpha.cap);
-    launch_tri_seg_copy(Ealpha, off.get(), bcnt.get(), cval.get(), cseg.get(),
-                        cea.get(), ceb.get(), flag.get(), bout.get(), dead,
-                        tk.get(), tkd.get(), tedge.get(), teik.get(),
+    launch_tri_seg_copy(Ealpha, off.get(), bcnt.get(), cval.get(), cpos.get(),
+                        ceb.get(), flag.get(), bout.get(), dead,
+                        tk.get(), tedge.get(), teik.get(),
                         tejk.get(), trow.get(),
                         tail_slots ? spair.get() : nullptr, epre.get(),
                         emask.get(), tri_in.get(), L, (uint64_t)Talpha.cap);
     KCHK();
   }
-
-  /* the third vertices, marked with kDeadBit where edges are */
-  const uint32_t* const tkm = prune ? tkd.get() : tk.get();
 
   /* ---- tets (AlphaComplexParallel.cu:1381-1442) ---- */
   Cnt Kslots(0), Kalpha(0);
@@ -724,7 +719,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
             zero_counter(ctr, CTR_CAND + 2, s);
             zero_counter(ctr, CTR_DROP, s);
           }
-          launch_tet_enum_filter(SG, Talpha, trow.get(), tkm, tedge.get(),
+          launch_tet_enum_filter(SG, Talpha, trow.get(), tk.get(), tedge.get(),
                                  teik.get(), tejk.get(), eleft.get(), ecol.get(),
                                  emask.get(), tail_slots ? nullptr : off.get(),
                                  tail_slots ? roff.get() : nullptr, epre.get(),
@@ -890,7 +885,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       Tf = ladder(
           ac2_cap(Talpha.cap), Talpha.cap / 4, KP_TRI_AC2, -1,
           [&](Queue q) {
-            launch_low_ac2_hot(SG, 0, Talpha, ecol.get(), eleft.get(), tkm,
+            launch_low_ac2_hot(SG, 0, Talpha, ecol.get(), eleft.get(), tk.get(),
                                tedge.get(), nullptr, tri_skip, tflag.get(), q,
                                rest.get(), nrest, budget(Talpha), L);
           },

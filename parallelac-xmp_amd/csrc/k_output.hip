@@ -553,28 +553,31 @@ void canonical_rows(int K, int64_t m, int32_t* rows, int idbits,
 /* Rows of a batch's list are grouped by molecule in molecule order and the
  * first id of a row lies in its molecule's id range, so "first id >=
  * moff[m]" is monotone over the rows: out[m] = first row of molecule m. */
-__global__ __launch_bounds__(kBlock) void k_mol_rows(const int32_t* rows,
-                                                    Cnt c_m, int K,
+__global__ __launch_bounds__(kBlock) void k_mol_rows(MolLists lists,
                                                     const uint32_t* moff,
                                                     int64_t nmol,
                                                     uint64_t* out) {
-  const int64_t m = c_m.get();
-  int64_t q = gtid();
+  const int d = blockIdx.y;
+  const int32_t* const rows = d == 0 ? lists.rows[0]
+                                     : (d == 1 ? lists.rows[1] : lists.rows[2]);
+  const int64_t m = d == 0 ? lists.m[0].get()
+                           : (d == 1 ? lists.m[1].get() : lists.m[2].get());
+  const int64_t q = gtid();
   if (q > nmol) return;
   uint32_t key = moff[q];
   int64_t lo = 0, hi = m;
   while (lo < hi) {
     int64_t mid = (lo + hi) >> 1;
-    if ((uint32_t)rows[(int64_t)K * mid] < key) lo = mid + 1;
+    if ((uint32_t)rows[(int64_t)(d + 2) * mid] < key) lo = mid + 1;
     else hi = mid;
   }
-  out[q] = (uint64_t)lo;
+  out[d * (nmol + 1) + q] = (uint64_t)lo;
 }
-void launch_mol_rows(const int32_t* rows, Cnt m, int K,
-                     const uint32_t* moff, int64_t nmol, uint64_t* out,
-                     hipStream_t s) {
-  hipLaunchKernelGGL(k_mol_rows, dim3((unsigned)((nmol + 1 + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, s, rows, m, K, moff, nmol, out);
+void launch_mol_rows(const MolLists& lists, const uint32_t* moff, int64_t nmol,
+                     uint64_t* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_mol_rows,
+                     dim3((unsigned)((nmol + 1 + kBlock - 1) / kBlock), 3),
+                     dim3(kBlock), 0, s, lists, moff, nmol, out);
 }
 
 }  // namespace pac

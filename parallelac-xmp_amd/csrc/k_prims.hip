@@ -591,12 +591,13 @@ __global__ __launch_bounds__(64) void k_ladder_rec(unsigned* qn, uint32_t c1,
   unsigned f1 = 0, f2 = 0;
   if (k < QSLOTS) {
     unsigned* const line = qn + k * kSlotWords;
-    f1 = line[QK_HOT];
-    f2 = line[QK_ESC];
-    line[QK_HOT] = 0;
-    line[QK_ESC] = 0;
-    line[QK_REST] = 0;
-    line[QK_NEXT] = 0;
+#pragma unroll
+    for (int t = 0; t < QK_SETS; ++t) {
+      f1 = max(f1, line[t * QK_WORDS + QK_HOT]);
+      f2 = max(f2, line[t * QK_WORDS + QK_ESC]);
+    }
+#pragma unroll
+    for (int t = 0; t < QK_SETS * QK_WORDS; ++t) line[t] = 0;
   }
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) {

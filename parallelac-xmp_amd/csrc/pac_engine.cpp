@@ -158,8 +158,8 @@ static bool is_device_ptr(const void* p) {
  * lists, 134 MB, in 13.3 ms with a pass over them for the base against 9.0
  * here; three of 20 KB in 63 us against 38.  The source's stream has been
  * waited for. */
-static void to_host(Engine* E, void* dst, const void* src, size_t bytes,
-                    int32_t base = 0) {
+void pac::to_host(Engine* E, void* dst, const void* src, size_t bytes,
+                  int32_t base) {
   if (!bytes) return;
   if (base == 0 && memory_of(dst) == hipMemoryTypeHost) { /* pinned: direct */
     HIPCHK(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
@@ -474,9 +474,12 @@ void pac::compute_batch(const float* xyzr, const int64_t* offsets,
       DBuf<uint64_t> rows(&E->pool, 3 * (gm + 1));
       HIPCHK(hipMemcpyAsync(dmo.get(), mo.data(), mo.size() * sizeof(uint32_t),
                             hipMemcpyHostToDevice, s));
-      for (int d = 1; d <= 3; ++d)
-        launch_mol_rows(R->lists[d - 1].get(), R->counts[d], d + 1, dmo.get(),
-                        gm, rows.get() + (d - 1) * (gm + 1), s);
+      MolLists ml;
+      for (int d = 0; d < 3; ++d) {
+        ml.rows[d] = R->lists[d].get();
+        ml.m[d] = Cnt(R->counts[d + 1]);
+      }
+      launch_mol_rows(ml, dmo.get(), gm, rows.get(), s);
       KCHK();
       std::vector<uint64_t> hr(3 * (gm + 1));
       HIPCHK(hipMemcpyAsync(hr.data(), rows.get(), hr.size() * sizeof(uint64_t),

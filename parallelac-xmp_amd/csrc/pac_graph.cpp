@@ -39,9 +39,11 @@ struct GPass {
   int64_t cap[RC_COUNT];
   vf32::PassPlan plan;
   DBuf<Bounds> bref, bnow;
-  DBuf<uint64_t> dcnt;       /* RC_COUNT device counts */
+  DBuf<uint64_t> cnt;        /* RC_COUNT device counts, then rows() */
   DBuf<uint32_t> dmo;        /* rel as uint32, for the row starts */
-  DBuf<uint64_t> rows;       /* 3 x (gm+1) first row of each molecule */
+  /* 3 x (gm+1) first row of each molecule */
+  uint64_t* rows() const { return cnt.get() + RC_COUNT; }
+  size_t words() const { return (size_t)(RC_COUNT + 3 * (gm + 1)); }
   std::unique_ptr<pac_result> R; /* output lists (capacities) */
   pac_stats st;              /* per-pass plan statistics */
 };
@@ -61,9 +63,13 @@ struct pac_graph {
   DBuf<float4> in;               /* owned input copy (host inputs) */
   const float4* raw = nullptr;   /* what the graph reads */
   std::vector<std::unique_ptr<GPass>> passes;
-  DBuf<unsigned> status;         /* [0] REC_* bits, [1..2] largest fills */
+  /* the counters, the status words (REC_* bits, two largest fills), the
+   * queue counters */
   DBuf<unsigned long long> ctr;
-  DBuf<unsigned> qn;
+  static constexpr int kCtrs = CTR_COUNT * CTR_SLOTS, kRead = kCtrs + 2,
+                       kWords = kRead + QN_WORDS / 2;
+  unsigned* status() const { return (unsigned*)(ctr.get() + kCtrs); }
+  unsigned* qn() const { return (unsigned*)(ctr.get() + kRead); }
   DBuf<QEntry> q1, q2;
   uint32_t c1 = 0, c2 = 0;
   hipGraph_t graph = nullptr;
@@ -81,9 +87,7 @@ struct pac_graph {
     if (ev1) (void)hipEventDestroy(ev1);
     passes.clear();
     in.release();
-    status.release();
     ctr.release();
-    qn.release();
     q1.release();
     q2.release();
     pool.trim();
@@ -103,9 +107,7 @@ int64_t with_headroom(int64_t v, double h) {
  * left there and allocates nothing. */
 void record_all(pac_graph* G) {
   hipStream_t s = G->s;
-  zero_u32(G->status.get(), 4, s);
-  zero_u32(G->qn.get(), QN_WORDS, s); /* then kept clear by the ladders */
-  zero_u64(G->ctr.get(), CTR_COUNT * CTR_SLOTS, s);
+  zero_u64(G->ctr.get(), G->kWords, s); /* (queue counters: then by passes) */
   KProf KP;
   for (auto& pp : G->passes) {
     GPass& p = *pp;
@@ -121,11 +123,11 @@ void record_all(pac_graph* G) {
     rec.bref = p.bref.get();
     rec.bnow = p.bnow.get();
     for (int q = 0; q < RC_COUNT; ++q) rec.cap[q] = p.cap[q];
-    rec.dcnt = p.dcnt.get();
-    rec.status = G->status.get();
-    rec.fill = G->status.get() + 1;
+    rec.dcnt = p.cnt.get();
+    rec.status = G->status();
+    rec.fill = G->status() + 1;
     rec.ctr = G->ctr.get();
-    rec.qn = G->qn.get();
+    rec.qn = G->qn();
     rec.q1 = G->q1.get();
     rec.q2 = G->q2.get();
     rec.c1 = G->c1;
@@ -133,17 +135,21 @@ void record_all(pac_graph* G) {
     vf32::run_pipeline(G->E, G->raw + p.b0, p.gn, G->solvent, G->alpha,
                        G->opt, p.R.get(), s, KP, p.rel.data(), p.gm, &rec);
     static const int fin[3] = {RC_EF, RC_TF, RC_KF};
-    for (int d = 1; d <= 3; ++d)
-      launch_mol_rows(p.R->lists[d - 1].get(),
-                      Cnt(p.cap[fin[d - 1]], p.dcnt.get() + fin[d - 1]), d + 1,
-                      p.dmo.get(), p.gm, p.rows.get() + (d - 1) * (p.gm + 1), s);
+    MolLists ml;
+    for (int d = 0; d < 3; ++d) {
+      ml.rows[d] = p.R->lists[d].get();
+      ml.m[d] = Cnt(p.cap[fin[d]], p.cnt.get() + fin[d]);
+    }
+    launch_mol_rows(ml, p.dmo.get(), p.gm, p.rows(), s);
     KCHK();
   }
 }
 
-void check_status(pac_graph* G, const char* when) {
+/* hs: the counters and status words */
+void check_status(pac_graph* G, const unsigned long long* hs,
+                  const char* when) {
   unsigned h[4];
-  HIPCHK(hipMemcpy(h, G->status.get(), sizeof(h), hipMemcpyDeviceToHost));
+  std::memcpy(h, hs + G->kCtrs, sizeof(h));
   if (!h[0]) return;
   std::string w = std::string(when) + ": ";
   if (h[0] & (1u << REC_STALE))
@@ -254,13 +260,12 @@ void graph_create(const float* xyzr, const int64_t* offsets, int64_t nmol,
       p.bnow = DBuf<Bounds>(&G->pool, nb);
       HIPCHK(hipMemcpyAsync(p.bref.get(), p.plan.bounds.data(),
                             nb * sizeof(Bounds), hipMemcpyHostToDevice, s));
-      p.dcnt = DBuf<uint64_t>(&G->pool, RC_COUNT);
       std::vector<uint32_t> mo(p.gm + 1);
       for (int64_t q = 0; q <= p.gm; ++q) mo[q] = (uint32_t)p.rel[q];
       p.dmo = DBuf<uint32_t>(&G->pool, p.gm + 1);
       HIPCHK(hipMemcpyAsync(p.dmo.get(), mo.data(), mo.size() * sizeof(uint32_t),
                             hipMemcpyHostToDevice, s));
-      p.rows = DBuf<uint64_t>(&G->pool, 3 * (p.gm + 1));
+      p.cnt = DBuf<uint64_t>(&G->pool, p.words());
       HIPCHK(hipStreamSynchronize(s));
     }
     G->passes.push_back(std::move(P));
@@ -272,9 +277,7 @@ void graph_create(const float* xyzr, const int64_t* offsets, int64_t nmol,
   G->c1 = (uint32_t)std::min(with_headroom(fill1, headroom) + 256, qmax);
   G->c2 = (uint32_t)std::min(
       std::max(with_headroom(fill2, headroom) + 256, (int64_t)G->c1 + 512), qmax);
-  G->status = DBuf<unsigned>(&G->pool, 4);
-  G->ctr = DBuf<unsigned long long>(&G->pool, CTR_COUNT * CTR_SLOTS);
-  G->qn = DBuf<unsigned>(&G->pool, QN_WORDS);
+  G->ctr = DBuf<unsigned long long>(&G->pool, G->kWords);
   G->q1 = DBuf<QEntry>(&G->pool, (size_t)G->c1 * QSLOTS);
   G->q2 = DBuf<QEntry>(&G->pool, (size_t)G->c2 * QSLOTS);
 
@@ -282,12 +285,15 @@ void graph_create(const float* xyzr, const int64_t* offsets, int64_t nmol,
    * counts exactly */
   record_all(G.get());
   HIPCHK(hipStreamSynchronize(s));
-  check_status(G.get(), "recorded run");
+  std::vector<unsigned long long> hs(G->kRead);
+  HIPCHK(hipMemcpy(hs.data(), G->ctr.get(), G->kRead * sizeof(hs[0]),
+                   hipMemcpyDeviceToHost));
+  check_status(G.get(), hs.data(), "recorded run");
   for (auto& pp : G->passes) {
     GPass& p = *pp;
     if (p.gn == 0) continue;
     uint64_t h[RC_COUNT];
-    HIPCHK(hipMemcpy(h, p.dcnt.get(), sizeof(h), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(h, p.cnt.get(), sizeof(h), hipMemcpyDeviceToHost));
     check_counts(p, h, "recorded run");
     for (int q = 0; q < RC_COUNT; ++q)
       if ((int64_t)h[q] != p.probe[q])
@@ -350,7 +356,9 @@ void graph_result(pac_graph* G, pac_batch_result** out) {
   Engine* E = G->E;
   HIPCHK(hipSetDevice(E->device));
   HIPCHK(hipStreamSynchronize(G->last));
-  check_status(G, "graph launch");
+  std::vector<unsigned long long> hs(G->kRead);
+  to_host(E, hs.data(), G->ctr.get(), G->kRead * sizeof(hs[0]));
+  check_status(G, hs.data(), "graph launch");
   std::unique_ptr<pac_batch_result> B(new pac_batch_result());
   B->eng = E;
   B->nmol = G->nmol;
@@ -367,13 +375,11 @@ void graph_result(pac_graph* G, pac_batch_result** out) {
     R->alpha = G->alpha;
     std::memset(&R->st, 0, sizeof(R->st));
     R->counts[0] = p.gn;
-    std::vector<uint64_t> hr(3 * (p.gm + 1), 0);
+    std::vector<uint64_t> hw(p.words(), 0); /* counts, rows */
+    const uint64_t *const h = hw.data(), *const hr = h + RC_COUNT;
     if (p.gn > 0) {
-      uint64_t h[RC_COUNT];
-      HIPCHK(hipMemcpy(h, p.dcnt.get(), sizeof(h), hipMemcpyDeviceToHost));
+      to_host(E, hw.data(), p.cnt.get(), hw.size() * sizeof(uint64_t));
       check_counts(p, h, "graph launch");
-      HIPCHK(hipMemcpy(hr.data(), p.rows.get(), hr.size() * sizeof(uint64_t),
-                       hipMemcpyDeviceToHost));
       static const int fin[3] = {RC_EF, RC_TF, RC_KF};
       for (int d = 1; d <= 3; ++d) {
         const int64_t m = (int64_t)h[fin[d - 1]];
@@ -402,9 +408,9 @@ void graph_result(pac_graph* G, pac_batch_result** out) {
     }
     for (int d = 1; d <= 3; ++d)
       for (int64_t q = 0; q < p.gm; ++q) {
-        const uint64_t* h = hr.data() + (d - 1) * (p.gm + 1);
-        B->row0[d - 1][p.m0 + q] = h[q];
-        B->counts[4 * (p.m0 + q) + d] = (int64_t)(h[q + 1] - h[q]);
+        const uint64_t* r0 = hr + (d - 1) * (p.gm + 1);
+        B->row0[d - 1][p.m0 + q] = r0[q];
+        B->counts[4 * (p.m0 + q) + d] = (int64_t)(r0[q + 1] - r0[q]);
       }
     for (int64_t q = 0; q < p.gm; ++q) {
       B->counts[4 * (p.m0 + q)] = p.rel[q + 1] - p.rel[q];
@@ -414,9 +420,6 @@ void graph_result(pac_graph* G, pac_batch_result** out) {
     B->group_first.push_back(p.m0);
     B->groups.push_back(std::move(R));
   }
-  std::vector<unsigned long long> hs(CTR_COUNT * CTR_SLOTS);
-  HIPCHK(hipMemcpyAsync(hs.data(), G->ctr.get(), hs.size() * sizeof(hs[0]),
-                        hipMemcpyDeviceToHost, G->s));
   HIPCHK(hipStreamSynchronize(G->s));
   for (int k = 1; k < CTR_SLOTS; ++k) /* the copies' sums, in the first */
     for (int c = 0; c < CTR_COUNT; ++c) hs[c] += hs[k * CTR_COUNT + c];

@@ -228,6 +228,10 @@ struct Engine {
 /* the pool the current run allocates from */
 inline Pool* pool_of(Engine* E) { return E->run_pool ? E->run_pool : &E->pool; }
 /* the per-device engine (created on first use) */
+/* device memory to pageable host memory, words minus base (the source's
+ * stream waited for) */
+void to_host(Engine* E, void* dst, const void* src, size_t bytes,
+             int32_t base = 0);
 Engine* engine_for(int dev);
 
 template <class T>

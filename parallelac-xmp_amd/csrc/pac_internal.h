@@ -198,6 +198,9 @@ inline uint32_t list_slot_cap(int64_t blocks) {
  * first one; counter k is kSlotWords * k words on. */
 constexpr int kSlotWords = 32; /* 128 bytes */
 enum { QK_HOT = 0, QK_ESC = 1, QK_REST = 2, QK_NEXT = 3 };
+/* sets of QK_WORDS counters on a line: one per ladder of a recorded pass */
+constexpr int QK_WORDS = 4, QK_SETS = 6;
+static_assert(QK_WORDS * QK_SETS <= kSlotWords, "the sets fit a line");
 static_assert(QSLOTS == LSLOTS, "the counters share their lines");
 constexpr int QN_WORDS = QSLOTS * kSlotWords;
 struct Queue {
@@ -261,9 +264,9 @@ enum { REC_Q1 = 9,     /* hot queue overflow */
        REC_STALE = 11  /* the input no longer matches the recorded plan */ };
 /* set counter idx of every copy to zero */
 void zero_counter(unsigned long long* ctr, int idx, hipStream_t s);
-/* the end of a recorded ladder: the largest fills of its queues (capacity
- * c1, c2 per sub-queue) into fill[0..1], overflows into *status, and the
- * queue and list counters cleared for the next ladder */
+/* the end of a recorded pass: the largest fills of its ladders' queues
+ * (capacity c1, c2 per sub-queue) into fill[0..1], overflows into *status, and
+ * the queue and list counters cleared for the next pass */
 void launch_ladder_rec(unsigned* qn, uint32_t c1, uint32_t c2, unsigned* status,
                        unsigned* fill, hipStream_t s);
 /* a run's statistics: the counters summed over their copies (CTR_COUNT
@@ -358,10 +361,13 @@ void canonical_rows(int K, int64_t m, int32_t* rows, int idbits,
 
 /* batch: first row of each molecule in a list of m rows of K original ids
  * grouped by molecule (moff: first original id of each molecule);
- * out[nmol+1] */
-void launch_mol_rows(const int32_t* rows, Cnt m, int K,
-                     const uint32_t* moff, int64_t nmol, uint64_t* out,
-                     hipStream_t s);
+ * out[nmol+1] for each list in turn */
+struct MolLists { /* edges, triangles, tets */
+  const int32_t* rows[3];
+  Cnt m[3];
+};
+void launch_mol_rows(const MolLists& lists, const uint32_t* moff, int64_t nmol,
+                     uint64_t* out, hipStream_t s);
 
 
 

@@ -332,9 +332,17 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   unsigned long long* const ctr = SG.ctr;
   unsigned* const qn =
       rec ? rec->qn : (unsigned*)(ctl.p + CTR_COUNT * CTR_SLOTS);
-  unsigned* const nesc = qn + QK_ESC;
-  unsigned* const nrest = qn + QK_REST;
-  unsigned* const nnext = qn + QK_NEXT;
+  /* the counters of the ladder at hand: eager runs clear them after each
+   * ladder, a recorded pass has a set for each (QK_SETS) */
+  unsigned *nhot, *nesc, *nrest, *nnext;
+  int ladders = 0;
+  auto counters = [&](int set) {
+    nhot = qn + set * QK_WORDS + QK_HOT;
+    nesc = qn + set * QK_WORDS + QK_ESC;
+    nrest = qn + set * QK_WORDS + QK_REST;
+    nnext = qn + set * QK_WORDS + QK_NEXT;
+  };
+  counters(0);
 
   /* ---- binning: the balls in the order of (cell, id) ----
    * Cells no more than a few per ball: counted as the keys are made, their
@@ -435,13 +443,13 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   auto ladder = [&](int64_t cap1_total, int64_t esc_items, int kp_hot, int kp_exact, auto&& hot,
                     auto&& esc, auto&& exact, auto&& tail, int q) -> Cnt {
     if (rec) { /* once, over the recorded queues */
-      const Queue h{rec->q1, qn, rec->c1}, e{rec->q2, nesc, rec->c2};
+      counters(ladders++);
+      const Queue h{rec->q1, nhot, rec->c1}, e{rec->q2, nesc, rec->c2};
       hot(h);
       if (staged) esc(queue_ref(h, false, esc_items), e);
       exact(queue_ref(staged ? e : h, false, esc_items));
       KCHK();
       tail(Post());
-      launch_ladder_rec(qn, rec->c1, rec->c2, rec->status, rec->fill, s);
       KCHK();
       return settle(q, Post());
     }
@@ -989,7 +997,11 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     launch_rank_of(perm.get(), n, R->rank.get(), s);
   }
   KCHK();
-  if (rec) return; /* counts and statistics are read after the graph runs */
+  if (rec) { /* counts and statistics are read after the graph runs */
+    launch_ladder_rec(qn, rec->c1, rec->c2, rec->status, rec->fill, s);
+    KCHK();
+    return;
+  }
   R->counts[1] = Ef.cap;
   R->counts[2] = Tf.cap;
   R->counts[3] = Kf.cap;

@@ -772,17 +772,16 @@ __device__ __forceinline__ int low_known(int64_t id, const uint32_t* tk,
  * cannot decide at once: one simplex a thread (PH_ALL), or (PH_PACK) a block
  * looks at kPack x 256, of which usually a quarter are left (on the 100k
  * globule 2.4M of 11.4M triangles, 0.4M of 2.2M edges), and its threads take
- * one of those each; a block's few past 256 go to phase B untested
- * (kRestWhole).  Phase A of the triangles at 100k: 280 us in place; 33 + 116
- * with a listing pass before it, 40 of them for the blocks that found the
- * list's end; 101 packed, and 10 more in phase B. */
-constexpr uint32_t kRestWhole = 0x80000000u;
+ * one of those each; a block's few past 256 go to phase B untested, marked
+ * with `whole` (low_phases).  Phase A of the triangles at 100k: 280 us in
+ * place; 33 + 116 with a listing pass before it, 40 of them for the blocks
+ * that found the list's end; 101 packed, and 10 more in phase B. */
 template <class R, int KIND, int PH, bool FINE, bool MOL>
 __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     Stage S0, Cnt c_nitems, const uint32_t* ecol, const uint32_t* eleft,
     const uint32_t* tk, const uint32_t* tedge, const uint8_t* edead,
     const uint8_t* in_flag, uint8_t* flag, Queue q1, uint32_t* rest,
-    unsigned* nrest, int budget) {
+    unsigned* nrest, int budget, uint32_t whole) {
   unsigned evals = 0, pairs = 0;
   __shared__ uint32_t s_pre[LSLOTS + 1];
   if (PH == PH_REST) list_table(nrest, S0.lcap, s_pre);
@@ -795,8 +794,8 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     int tested = budget; /* phase B: the pairs that phase A tested */
     if (PH == PH_REST) {
       const uint32_t x = list_at(rest, S.lcap, s_pre, (uint32_t)w);
-      id = x & ~kRestWhole;
-      if (x & kRestWhole) tested = 0;
+      id = left_id(x, whole);
+      tested = left_tested(x, whole, budget);
     }
     if (PH == PH_ALL) {
       const int c = low_known<KIND>(id, tk, edead, in_flag);
@@ -953,7 +952,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
             s_live[o] = id;
           else if (s_over + (o - kBlock) < S0.lcap)
             rest[(uint64_t)k * S0.lcap + s_over + (o - kBlock)] =
-                id | kRestWhole;
+                id | whole;
         }
         at += (unsigned)__popcll(m);
       }
@@ -1345,23 +1344,25 @@ static void low_hot4(const Stage& S, Cnt nitems, const uint32_t* ecol,
                      PipeLaunch L) {
   const dim3 gr((unsigned)((nitems.cap + kBlock - 1) / kBlock)),
       gb(rest_grid(S, nitems));
-  if (S.pack && nitems.cap >= kPackItems && nitems.cap < ((int64_t)1 << 31) &&
-      budget > 0) {
+  const LowPhases ph = low_phases(S.pack != 0, nitems.cap, budget);
+  if (ph.pack) {
     const int64_t per = kBlock * kPack;
     hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, PH_PACK, FINE, MOL>),
                        dim3((unsigned)((nitems.cap + per - 1) / per)),
                        dim3(kBlock), 0, L.s, S, nitems, ecol, eleft, tk, tedge,
-                       edead, in_flag, flag, q1, rest, nrest, budget);
+                       edead, in_flag, flag, q1, rest, nrest, budget,
+                       ph.whole);
   } else {
     hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, PH_ALL, FINE, MOL>), gr,
                        dim3(kBlock), 0, L.s, S, nitems, ecol, eleft, tk, tedge,
-                       edead, in_flag, flag, q1, rest, nrest, budget);
+                       edead, in_flag, flag, q1, rest, nrest, budget,
+                       ph.whole);
   }
   if (budget > 0) {
     hipLaunchKernelGGL((k_low_ac2_hot<R, KIND, PH_REST, FINE, MOL>), gb,
                        dim3((unsigned)S.bblock), 0, L.s, S, nitems, ecol, eleft,
                        tk, tedge, edead, in_flag, flag, q1, rest, nrest,
-                       budget);
+                       budget, ph.whole);
   }
 }
 template <class R, int KIND, bool FINE>

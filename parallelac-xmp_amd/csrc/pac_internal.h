@@ -11,6 +11,7 @@
 #include <stdint.h>
 
 #include "pac_arith.h"
+#include "pac_phases.h"
 
 namespace pac {
 
@@ -572,10 +573,6 @@ void launch_filter_exact(const Stage& S, int kind, CandCtx C, QRef q, const uint
  * phase A scans, where a pass before it left only some: the quick
  * rejection pass (tets, fine scan grid), a chunk sub-input's needed tets.
  * Both lists' counters come cleared (the ladder's last kernel does it). */
-/* triangles / edges from this many on are packed by the blocks that scan
- * them: the dead and closed ones leave most lanes of a wave idle otherwise;
- * fewer do not fill the chip as they are */
-constexpr int64_t kPackItems = 1 << 17;
 /* chunk sub-input: in_flag[id] = 1 (pass untested) for the triangles
  * (kind 0) / edges (kind 1) no owned simplex depends on */
 void launch_own_mark(const Stage& S, int kind, Cnt n, const uint32_t* ecol,

@@ -230,18 +230,6 @@ static void copy_to(Engine* E, void* dst, const void* src, size_t bytes) {
     to_host(E, dst, src, bytes);
 }
 
-/* runs f; should it throw, waits for the kernels it left in flight before
- * anyone can take their buffers (the caller holds the engine's lock) */
-template <class F>
-static void drained(hipStream_t s, F&& f) {
-  try {
-    f();
-  } catch (...) {
-    (void)hipStreamSynchronize(s);
-    throw;
-  }
-}
-
 /* one molecule; F is float (FP32 balls, the reference's input) or double
  * (FP64 balls) */
 template <class F>

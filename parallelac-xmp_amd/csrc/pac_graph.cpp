@@ -356,6 +356,10 @@ void graph_result(pac_graph* G, pac_batch_result** out) {
   Engine* E = G->E;
   HIPCHK(hipSetDevice(E->device));
   HIPCHK(hipStreamSynchronize(G->last));
+  /* The lists come from the engine's pool, to which an eager run returns
+   * scratch that its queued kernels still use: only that run's own stream
+   * orders its reuse, so nobody takes blocks beside a run. */
+  std::lock_guard<std::mutex> lk(E->run_mu);
   std::vector<unsigned long long> hs(G->kRead);
   to_host(E, hs.data(), G->ctr.get(), G->kRead * sizeof(hs[0]));
   check_status(G, hs.data(), "graph launch");
@@ -368,58 +372,61 @@ void graph_result(pac_graph* G, pac_batch_result** out) {
   for (auto& r : B->row0) r.assign(G->nmol, 0);
   std::memset(&B->st, 0, sizeof(B->st));
   int64_t ecand = 0;
-  for (auto& pp : G->passes) {
-    GPass& p = *pp;
-    std::unique_ptr<pac_result> R(new pac_result());
-    R->eng = E;
-    R->alpha = G->alpha;
-    std::memset(&R->st, 0, sizeof(R->st));
-    R->counts[0] = p.gn;
-    std::vector<uint64_t> hw(p.words(), 0); /* counts, rows */
-    const uint64_t *const h = hw.data(), *const hr = h + RC_COUNT;
-    if (p.gn > 0) {
-      to_host(E, hw.data(), p.cnt.get(), hw.size() * sizeof(uint64_t));
-      check_counts(p, h, "graph launch");
-      static const int fin[3] = {RC_EF, RC_TF, RC_KF};
-      for (int d = 1; d <= 3; ++d) {
-        const int64_t m = (int64_t)h[fin[d - 1]];
-        R->counts[d] = m;
-        R->lists[d - 1] = DBuf<int32_t>(&E->pool, (size_t)m * (d + 1));
-        if (m)
-          HIPCHK(hipMemcpyAsync(R->lists[d - 1].get(), p.R->lists[d - 1].get(),
-                                (size_t)m * (d + 1) * sizeof(int32_t),
-                                hipMemcpyDeviceToDevice, G->s));
+  drained(G->s, [&] {
+    for (auto& pp : G->passes) {
+      GPass& p = *pp;
+      std::unique_ptr<pac_result> R(new pac_result());
+      R->eng = E;
+      R->alpha = G->alpha;
+      std::memset(&R->st, 0, sizeof(R->st));
+      R->counts[0] = p.gn;
+      std::vector<uint64_t> hw(p.words(), 0); /* counts, rows */
+      const uint64_t *const h = hw.data(), *const hr = h + RC_COUNT;
+      if (p.gn > 0) {
+        to_host(E, hw.data(), p.cnt.get(), hw.size() * sizeof(uint64_t));
+        check_counts(p, h, "graph launch");
+        static const int fin[3] = {RC_EF, RC_TF, RC_KF};
+        for (int d = 1; d <= 3; ++d) {
+          const int64_t m = (int64_t)h[fin[d - 1]];
+          R->counts[d] = m;
+          R->lists[d - 1] = DBuf<int32_t>(&E->pool, (size_t)m * (d + 1));
+          if (m)
+            HIPCHK(hipMemcpyAsync(R->lists[d - 1].get(),
+                                  p.R->lists[d - 1].get(),
+                                  (size_t)m * (d + 1) * sizeof(int32_t),
+                                  hipMemcpyDeviceToDevice, G->s));
+        }
+        for (int q = 0; q < RC_COUNT; ++q) R->sizes[q] = (int64_t)h[q];
+        pac_stats& st = R->st;
+        st.n = p.gn;
+        st.edge_candidates = (int64_t)h[RC_ECAND];
+        st.edge_alpha = (int64_t)h[RC_EALPHA];
+        st.tri_alpha = (int64_t)h[RC_TALPHA];
+        st.tet_alpha = (int64_t)h[RC_KALPHA];
+        st.edges_final = (int64_t)h[RC_EF];
+        st.tris_final = (int64_t)h[RC_TF];
+        st.tets_final = (int64_t)h[RC_KF];
+        st.k_enum = p.st.k_enum;
+        st.k_ac2 = p.st.k_ac2;
+        st.scale_bits = p.st.scale_bits;
+        st.grid_cells = p.st.grid_cells;
+        ecand += st.edge_candidates;
       }
-      for (int q = 0; q < RC_COUNT; ++q) R->sizes[q] = (int64_t)h[q];
-      pac_stats& st = R->st;
-      st.n = p.gn;
-      st.edge_candidates = (int64_t)h[RC_ECAND];
-      st.edge_alpha = (int64_t)h[RC_EALPHA];
-      st.tri_alpha = (int64_t)h[RC_TALPHA];
-      st.tet_alpha = (int64_t)h[RC_KALPHA];
-      st.edges_final = (int64_t)h[RC_EF];
-      st.tris_final = (int64_t)h[RC_TF];
-      st.tets_final = (int64_t)h[RC_KF];
-      st.k_enum = p.st.k_enum;
-      st.k_ac2 = p.st.k_ac2;
-      st.scale_bits = p.st.scale_bits;
-      st.grid_cells = p.st.grid_cells;
-      ecand += st.edge_candidates;
-    }
-    for (int d = 1; d <= 3; ++d)
+      for (int d = 1; d <= 3; ++d)
+        for (int64_t q = 0; q < p.gm; ++q) {
+          const uint64_t* r0 = hr + (d - 1) * (p.gm + 1);
+          B->row0[d - 1][p.m0 + q] = r0[q];
+          B->counts[4 * (p.m0 + q) + d] = (int64_t)(r0[q + 1] - r0[q]);
+        }
       for (int64_t q = 0; q < p.gm; ++q) {
-        const uint64_t* r0 = hr + (d - 1) * (p.gm + 1);
-        B->row0[d - 1][p.m0 + q] = r0[q];
-        B->counts[4 * (p.m0 + q) + d] = (int64_t)(r0[q + 1] - r0[q]);
+        B->counts[4 * (p.m0 + q)] = p.rel[q + 1] - p.rel[q];
+        B->mol_group[p.m0 + q] = (int32_t)B->groups.size();
       }
-    for (int64_t q = 0; q < p.gm; ++q) {
-      B->counts[4 * (p.m0 + q)] = p.rel[q + 1] - p.rel[q];
-      B->mol_group[p.m0 + q] = (int32_t)B->groups.size();
+      add_stats(B->st, R->st);
+      B->group_first.push_back(p.m0);
+      B->groups.push_back(std::move(R));
     }
-    add_stats(B->st, R->st);
-    B->group_first.push_back(p.m0);
-    B->groups.push_back(std::move(R));
-  }
+  });
   HIPCHK(hipStreamSynchronize(G->s));
   for (int k = 1; k < CTR_SLOTS; ++k) /* the copies' sums, in the first */
     for (int c = 0; c < CTR_COUNT; ++c) hs[c] += hs[k * CTR_COUNT + c];

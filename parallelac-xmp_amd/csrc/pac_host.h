@@ -234,6 +234,18 @@ void to_host(Engine* E, void* dst, const void* src, size_t bytes,
              int32_t base = 0);
 Engine* engine_for(int dev);
 
+/* runs f; should it throw, waits for the kernels it left in flight before
+ * anyone can take their buffers (the caller holds the engine's lock) */
+template <class F>
+inline void drained(hipStream_t s, F&& f) {
+  try {
+    f();
+  } catch (...) {
+    (void)hipStreamSynchronize(s);
+    throw;
+  }
+}
+
 template <class T>
 struct DBuf {
   Pool* pool = nullptr;

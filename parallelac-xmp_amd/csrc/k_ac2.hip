@@ -225,7 +225,7 @@ __global__ __launch_bounds__(kBlock) void k_tet_need(Stage S, Cnt c_nk,
                                                      uint8_t* flag,
                                                      uint32_t* next,
                                                      unsigned* nnext) {
-  stamp(S.ts, 5);
+  stamp(S.ts, TS_TET_AC2);
   const int64_t nk = c_nk.get();
   const int64_t id = gtid();
   bool need = false;
@@ -244,7 +244,7 @@ template <class R, bool MOL>
 __global__ __launch_bounds__(kBlock) void k_tet_ac2_quick(
     Stage S, Cnt c_nk, const uint4* tets, uint8_t* flag, uint32_t* next,
     unsigned* nnext) {
-  stamp(S.ts, 5);
+  stamp(S.ts, TS_TET_AC2);
   unsigned pairs = 0;
   const int64_t nk = c_nk.get();
   const int64_t id = gtid();
@@ -283,7 +283,7 @@ __global__ __launch_bounds__(kBlock) void k_tet_ac2_hot(
     Stage S0, Cnt c_nk, const uint32_t* items, const unsigned* nitems,
     const uint4* tets, uint8_t* flag, Queue q1, uint32_t* rest,
     unsigned* nrest, int budget) {
-  if (PH == PH_ALL) stamp(S0.ts, 5);
+  if (PH == PH_ALL) stamp(S0.ts, TS_TET_AC2);
   unsigned evals = 0, pairs = 0;
   /* phase A: the alpha tets, or the list `items` of them (those the quick
    * pass left); phase B: `rest` */

@@ -45,7 +45,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_tets(
     const uint64_t* trow, const uint32_t* tk, const uint32_t* tejk,
     const uint32_t* perm, uint8_t* tri_in, int4* out, uint64_t ocap,
     unsigned long long* ts) {
-  stamp(ts, 6);
+  stamp(ts, TS_TRI_AC2);
   /* the triangle of edge e whose third vertex is v, e2 = (i, v) for e =
    * (i, .); -1 if there is none (a recorded pass over its capacities) */
   auto face = [&](uint32_t e, uint32_t e2, uint32_t v) -> int64_t {
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_tris(
     const uint32_t* eleft, const uint32_t* tk, const uint32_t* tedge,
     const uint32_t* teik, const uint32_t* tejk, const uint32_t* perm,
     uint8_t* edge_in, int32_t* out, uint64_t ocap, unsigned long long* ts) {
-  stamp(ts, 7);
+  stamp(ts, TS_EDGE_AC2);
   tile_each(flag, c_nt.get(), offs, [&](int64_t t, uint64_t p) {
     if (p >= ocap) return;
     const uint32_t e = tedge[t];

@@ -156,7 +156,7 @@ __global__ __launch_bounds__(kBlock) void k_bounds_part(
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   if (ctl) {
     for (int64_t i = gtid(); i < ctl_words; i += stride)
-      ctl[i] = i == ctl_words - kStamps + 1 ? wall_clock64() : 0ull;
+      ctl[i] = i == ctl_words - kStamps + TS_GRID ? wall_clock64() : 0ull;
   }
   BRed b;
   bred_init(b);
@@ -243,7 +243,8 @@ void launch_mol_ids(const uint32_t* moff, int64_t nmol, int64_t n,
 /* computeCellIndex (LD:65-78): FP32 subtract, IEEE divide, truncate; in a
  * batch the molecule's first global cell id is added.  idx: the ball, or
  * with the cells' counts (cleared) its place among the balls of its cell, in
- * the order they arrive. */
+ * the order they arrive, counted a run of lanes at a time: 20,000 balls in one
+ * cell 6 us, 230 with an atomic each. */
 __global__ __launch_bounds__(kBlock) void k_cell_key(const Ball* raw,
                                                      int64_t n, GridP g1,
                                                      const GridP* grids,
@@ -269,7 +270,7 @@ __global__ __launch_bounds__(kBlock) void k_cell_key(const Ball* raw,
   cz = min(max(cz, 0), g.ez - 1);
   const uint32_t c = g.cbase + (uint32_t)(cx + g.ex * cy + g.ex * g.ey * cz);
   key[i] = c;
-  idx[i] = cnt ? atomicAdd(cnt + c, 1u) : (uint32_t)i;
+  idx[i] = cnt ? count_run(cnt, c) : (uint32_t)i;
 }
 void launch_cell_key(const Ball* raw, int64_t n, GridP g,
                      const GridP* grids, const uint32_t* mol, uint32_t* key,
@@ -279,43 +280,72 @@ void launch_cell_key(const Ball* raw, int64_t n, GridP g,
                      dim3(kBlock), 0, L.s, raw, n, g, grids, mol, key, idx, cnt);
 }
 
-/* the balls by cell, in each cell as they arrived */
+/* the balls by cell, in each cell as they arrived, and their cells */
 __global__ __launch_bounds__(kBlock) void k_cell_put(int64_t n,
                                                      const uint32_t* key,
                                                      const uint32_t* place,
                                                      const uint32_t* cstart,
-                                                     uint32_t* sidx) {
+                                                     uint32_t* sidx,
+                                                     uint32_t* cellk) {
   const int64_t i = gtid();
-  if (i < n) sidx[cstart[key[i]] + place[i]] = (uint32_t)i;
+  if (i >= n) return;
+  const uint32_t c = key[i], at = cstart[c] + place[i];
+  sidx[at] = (uint32_t)i;
+  cellk[at] = c;
 }
+void launch_cell_put(int64_t n, const uint32_t* key, const uint32_t* place,
+                     const uint32_t* cstart, uint32_t* sidx, uint32_t* cellk,
+                     PipeLaunch L) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_cell_put, dim3((unsigned)((n + kBlock - 1) / kBlock)),
+                     dim3(kBlock), 0, L.s, n, key, place, cstart, sidx, cellk);
+}
+struct __attribute__((packed, aligned(4))) U4a4 { /* 16 bytes at any word */
+  uint32_t x, y, z, w;
+};
 /* Each ball to its place by cell and id: as many after its cell's start as
- * the cell holds smaller ids (the enumeration tests all pairs of a cell, so
- * a full cell costs no more here). */
+ * the cell holds smaller ids.  A cell of m balls walks m^2 ids and has
+ * m (m - 1) / 2 edge candidates: this runs after the candidates were counted
+ * and found below 2^32, so at most 2^33 ids in all.  A cell of 20,000: 296 us
+ * with 32 ids in flight a thread, 1,496 one by one. */
 __global__ __launch_bounds__(kBlock) void k_cell_order(
-    const Ball* raw, int64_t n, const uint32_t* sidx, const uint32_t* key,
+    const Ball* raw, int64_t n, const uint32_t* sidx, const uint32_t* cellk,
     const uint32_t* cstart, Real solvent, Ball* ball, uint32_t* perm,
-    uint32_t* cellk) {
+    unsigned long long* ts) {
+  stamp(ts, TS_ORDER);
   const int64_t s = gtid();
   if (s >= n) return;
   const uint32_t o = sidx[s];
   const Ball a = raw[o];
-  const uint32_t c = key[o], b = cstart[c], e = cstart[c + 1];
-  uint32_t at = b;
-  for (uint32_t t = b; t < e; ++t) at += sidx[t] < o;
+  const uint32_t c = cellk[s], b = cstart[c], e = cstart[c + 1];
+  uint32_t at = b, t = b;
+  for (; t + 32 <= e; t += 32) {
+    U4a4 x[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      x[k] = *reinterpret_cast<const U4a4*>(sidx + t + 4 * k);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      at += (x[k].x < o) + (x[k].y < o) + (x[k].z < o) + (x[k].w < o);
+  }
+  for (; t < e; t += 8) {
+    uint32_t x[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) x[k] = sidx[t + k < e ? t + k : b];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) at += t + k < e && x[k] < o;
+  }
   ball[at] = Ball{a.x, a.y, a.z, add_r(a.w, solvent)};
   perm[at] = o;
-  cellk[at] = c;
 }
-void launch_cell_order(const Ball* raw, int64_t n, const uint32_t* key,
-                       const uint32_t* place, const uint32_t* cstart,
-                       uint32_t* sidx, Real solvent, Ball* ball, uint32_t* perm,
-                       uint32_t* cellk, PipeLaunch L) {
+void launch_cell_order(const Ball* raw, int64_t n, const uint32_t* sidx,
+                       const uint32_t* cellk, const uint32_t* cstart,
+                       Real solvent, Ball* ball, uint32_t* perm,
+                       unsigned long long* ts, PipeLaunch L) {
   if (n <= 0) return;
-  const dim3 gr((unsigned)((n + kBlock - 1) / kBlock));
-  hipLaunchKernelGGL(k_cell_put, gr, dim3(kBlock), 0, L.s, n, key, place,
-                     cstart, sidx);
-  hipLaunchKernelGGL(k_cell_order, gr, dim3(kBlock), 0, L.s, raw, n, sidx, key,
-                     cstart, solvent, ball, perm, cellk);
+  hipLaunchKernelGGL(k_cell_order, dim3((unsigned)((n + kBlock - 1) / kBlock)),
+                     dim3(kBlock), 0, L.s, raw, n, sidx, cellk, cstart, solvent,
+                     ball, perm, ts);
 }
 
 __global__ __launch_bounds__(kBlock) void k_gather(const Ball* raw,
@@ -593,7 +623,7 @@ __device__ __forceinline__ void cell_xyz(uint32_t c, const GridP& g, int& x,
 }
 
 __global__ __launch_bounds__(kBlock) void k_edge_count(Stage S, uint32_t* cnt) {
-  stamp(S.ts, 2);
+  stamp(S.ts, TS_EDGES);
   int64_t i = gtid();
   if (i >= S.n) return;
   const GridP g = grid_of(S, (uint32_t)i);
@@ -715,9 +745,6 @@ __device__ __forceinline__ void merge_rows(const uint32_t* ecol, uint32_t a,
     b += (y <= x);
   }
 }
-struct __attribute__((packed, aligned(4))) U4a4 { /* 16 bytes at any word */
-  uint32_t x, y, z, w;
-};
 /* Triangle candidates of the alpha edges (computePossibleTriangleCount,
  * Parallel:232-266), a wave per kTriSeg = 64 edges, an edge q = (i, j) a
  * lane: bit t of hits[q] is set if the t-th of row(j) may be in row(i), and
@@ -735,7 +762,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_hits(
     const uint32_t* eleft, ulonglong2* hits, uint32_t* cnt,
     unsigned long long* ts) {
   static_assert(kTriSeg == 64, "an edge a lane");
-  stamp(ts, 3);
+  stamp(ts, TS_TRIS);
   constexpr int W = 512; /* words of a wave's bitmaps */
   __shared__ uint4 s_raw[kBlock / 64][W / 4];
   const int64_t ne = c_ne.get();
@@ -947,7 +974,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
     const uint64_t* off, const uint64_t* roff, const uint32_t* epre,
     uint64_t* bbase, uint4* ctet, uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep, Queue q1, uint64_t lim) {
   static_assert(kTetSeg == 64, "a triangle a lane");
-  stamp(S.ts, 4);
+  stamp(S.ts, TS_TETS);
   /* LDS of a wave, 4,992 bytes (8 blocks per CU): by masks, three rows of
    * 16 bytes a triangle and the listed bits; by merges, the stage of fourth
    * vertices and the lanes' prefix counts */
@@ -1367,6 +1394,7 @@ template <class R>
 __global__ __launch_bounds__(kBlock) void k_edge_enum_filter(
     Stage S, const uint64_t* off, uint32_t* cval, uint8_t* flag,
     uint32_t* bcnt, uint32_t* bkeep, Queue q1, uint64_t lim) {
+  stamp(S.ts, TS_ENUM);
   const int64_t iw = (int64_t)blockIdx.x * kEdgeBallsPerBlock + (threadIdx.x >> 6);
   if (iw >= S.n) return; /* a whole wave */
   const uint32_t i = __builtin_amdgcn_readfirstlane((uint32_t)iw);

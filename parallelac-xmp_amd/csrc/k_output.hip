@@ -347,22 +347,6 @@ void filtration_order(int64_t m, const uint64_t* key, const int64_t counts[4],
  * so d rho / d p_q = 2 lam_q (p_q - c) and d rho / d r_q = -2 lam_q r_q.
  * Contributions are written per (simplex, vertex) slot and summed per ball
  * in slot order after a stable sort by ball: the result is deterministic. */
-/* this lane's place among those counted so far for v: one atomic for a run
- * of lanes with the same v (rows come by their first vertex), by its first
- * lane (the lanes at work are the wave's first ones) */
-__device__ __forceinline__ uint32_t count_run(uint32_t* cnt, uint32_t v) {
-  const int lane = threadIdx.x & 63;
-  const uint32_t prev = (uint32_t)__shfl_up((int)v, 1, 64);
-  const uint64_t act = __ballot(true);
-  const uint64_t heads = __ballot(lane == 0 || prev != v);
-  const uint64_t upto = ~0ull >> (63 - lane);
-  const int head = 63 - __builtin_clzll(heads & upto);
-  const uint64_t later = lane == 63 ? 0ull : heads >> (lane + 1);
-  const int end = later ? lane + 1 + __builtin_ctzll(later) : __popcll(act);
-  uint32_t base = 0;
-  if (head == lane) base = atomicAdd(cnt + v, (uint32_t)(end - lane));
-  return (uint32_t)__shfl((int)base, head, 64) + (uint32_t)(lane - head);
-}
 template <int DIM>
 __global__ __launch_bounds__(kBlock) void k_adj_contrib(
     int64_t m, const int32_t* rows, const double4* balls, const double* g,

@@ -635,7 +635,7 @@ __global__ __launch_bounds__(kSumsBlock) void k_post_stats(
     out[c] = v;
   }
   if (c < kStamps)
-    out[CTR_COUNT + c] = c == kStamps - 1 ? wall_clock64() : ts[c];
+    out[CTR_COUNT + c] = c == TS_END ? wall_clock64() : ts[c];
   do_post(post, 0);
 }
 void launch_post_stats(const unsigned long long* ctr,

@@ -132,6 +132,22 @@ struct StageCnt {
   }
 };
 
+/* this lane's place among those counted so far for v: one atomic for a run
+ * of lanes with the same v, by its first lane (the lanes at work are the
+ * wave's first ones) */
+__device__ __forceinline__ uint32_t count_run(uint32_t* cnt, uint32_t v) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t prev = (uint32_t)__shfl_up((int)v, 1, 64);
+  const uint64_t act = __ballot(true);
+  const uint64_t heads = __ballot(lane == 0 || prev != v);
+  const uint64_t upto = ~0ull >> (63 - lane);
+  const int head = 63 - __builtin_clzll(heads & upto);
+  const uint64_t later = lane == 63 ? 0ull : heads >> (lane + 1);
+  const int end = later ? lane + 1 + __builtin_ctzll(later) : __popcll(act);
+  uint32_t base = 0;
+  if (head == lane) base = atomicAdd(cnt + v, (uint32_t)(end - lane));
+  return (uint32_t)__shfl((int)base, head, 64) + (uint32_t)(lane - head);
+}
 /* a phase's time stamp, by the first thread of its first kernel */
 __device__ __forceinline__ void stamp(unsigned long long* ts, int k) {
   if (ts && blockIdx.x == 0 && threadIdx.x == 0) ts[k] = wall_clock64();

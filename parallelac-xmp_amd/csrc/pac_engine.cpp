@@ -72,12 +72,12 @@ __global__ void k_fill_u8(uint8_t* p, int64_t n, uint8_t v) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
-__global__ void k_zero_u32(unsigned* p, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void k_zero_u32(unsigned* p, int64_t n) {
+  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
 }
-__global__ void k_zero_u64(unsigned long long* p, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void k_zero_u64(unsigned long long* p, int64_t n) {
+  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
 }
 void fill_u8(uint8_t* p, int64_t n, uint8_t v, hipStream_t s) {
@@ -85,13 +85,14 @@ void fill_u8(uint8_t* p, int64_t n, uint8_t v, hipStream_t s) {
   hipLaunchKernelGGL(k_fill_u8, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                      s, p, n, v);
 }
-void zero_u32(unsigned* p, int n, hipStream_t s) {
-  hipLaunchKernelGGL(k_zero_u32, dim3((n + 255) / 256), dim3(256), 0, s, p, n);
+void zero_u32(unsigned* p, int64_t n, hipStream_t s) {
+  hipLaunchKernelGGL(k_zero_u32, dim3((unsigned)((n + 255) / 256)), dim3(256),
+                     0, s, p, n);
 }
 void zero_u64(unsigned long long* p, int64_t n, hipStream_t s) {
   if (n <= 0) return;
   hipLaunchKernelGGL(k_zero_u64, dim3((unsigned)((n + 255) / 256)), dim3(256),
-                     0, s, p, (int)n);
+                     0, s, p, n);
 }
 }  // namespace pac
 
@@ -332,7 +333,7 @@ static void alpha_adjoint(const pac_result* r, const double* gtri,
     DBuf<uint32_t> key(P, F + 1), place(P, F + 1), slot(P, F + 1),
         sorted(P, F + 1), deg(P, n), vstart(P, n + 1);
     DBuf<double4> contrib(P, F + 1);
-    zero_u32(deg.get(), (int)n, s);
+    zero_u32(deg.get(), n, s);
     launch_adj_contrib(2, T, r->lists[1].get(), r->balls.get(), g.get(), 0,
                        key.get(), place.get(), deg.get(), contrib.get(), s);
     launch_adj_contrib(3, K, r->lists[2].get(), r->balls.get(), g.get() + T,

@@ -137,7 +137,7 @@ size_t radix_tmp_bytes(int64_t n);
 /* small fills on a stream (kernels, not hipMemsetAsync: they may be
  * captured into graphs) */
 void fill_u8(uint8_t* p, int64_t n, uint8_t v, hipStream_t s);
-void zero_u32(unsigned* p, int n, hipStream_t s);
+void zero_u32(unsigned* p, int64_t n, hipStream_t s);
 void zero_u64(unsigned long long* p, int64_t n, hipStream_t s);
 
 /* ---- chunked driver (k_chunk.hip) ---- */
@@ -272,7 +272,10 @@ void launch_ladder_rec(unsigned* qn, uint32_t c1, uint32_t c2, unsigned* status,
                        unsigned* fill, hipStream_t s);
 /* a run's statistics: the counters summed over their copies (CTR_COUNT
  * u64) and the time stamps (kStamps u64) to the box's data words */
-constexpr int kStamps = 9;
+enum { TS_GRID = 1, TS_EDGES, TS_TRIS, TS_TETS, TS_TET_AC2, TS_TRI_AC2,
+       TS_EDGE_AC2, TS_END, /* (set when the statistics are posted) */
+       TS_ORDER, TS_ENUM,   /* the ordering within the edge phase's counts */
+       kStamps };
 void launch_post_stats(const unsigned long long* ctr,
                        const unsigned long long* ts, Post post, hipStream_t s);
 void launch_plan_check(const Bounds* now, const Bounds* ref, int64_t m,
@@ -392,10 +395,13 @@ void launch_mol_ids(const uint32_t* moff, int64_t nmol, int64_t n,
 void launch_cell_key(const Ball* raw, int64_t n, GridP g,
                      const GridP* grids, const uint32_t* mol, uint32_t* key,
                      uint32_t* idx, uint32_t* cnt, PipeLaunch L);
-void launch_cell_order(const Ball* raw, int64_t n, const uint32_t* key,
-                       const uint32_t* place, const uint32_t* cstart,
-                       uint32_t* sidx, Real solvent, Ball* ball, uint32_t* perm,
-                       uint32_t* cellk, PipeLaunch L);
+void launch_cell_put(int64_t n, const uint32_t* key, const uint32_t* place,
+                     const uint32_t* cstart, uint32_t* sidx, uint32_t* cellk,
+                     PipeLaunch L);
+void launch_cell_order(const Ball* raw, int64_t n, const uint32_t* sidx,
+                       const uint32_t* cellk, const uint32_t* cstart,
+                       Real solvent, Ball* ball, uint32_t* perm,
+                       unsigned long long* ts, PipeLaunch L);
 void launch_gather(const Ball* raw, const uint32_t* sidx,
                    const uint32_t* skey, int64_t n, Real solvent,
                    Ball* ball, uint32_t* perm, uint32_t* cellk,
@@ -421,9 +427,7 @@ struct Stage {
   Real alpha;
   ExactScale ex;
   unsigned long long* ctr;
-  /* time stamps (kStamps), set by the first kernel of each phase: 1 bounds,
-   * 2 edges, 3 triangles, 4 tets, 5 - 7 the emptiness tests, 8 the end
-   * (null: none) */
+  /* time stamps (TS_*), set by the first kernel of each phase (null: none) */
   unsigned long long* ts;
   int staged;
   /* second emptiness phase: a persistent launch of bgrid blocks of bblock

@@ -349,19 +349,24 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
    * starts scanned, the balls put by cell and ranked by id within it.  A grid
    * mostly of empty cells: a stable radix sort of the keys and a search per
    * cell, whose memory and time do not grow with it.  (16068 balls: 30 us in
-   * five launches against 60 in ten.) */
+   * five launches against 60 in ten.)  The ranks cost a crowded cell the
+   * square of its balls, as its edge candidates do: they wait until those
+   * are counted, and an input refused for their number is never ranked; nor
+   * one without any, which nothing bounds. */
   DBuf<Ball> ball(P, n);
-  DBuf<uint32_t> perm(P, n), cellk(P, n), cstart(P, G + 1);
+  DBuf<uint32_t> perm(P, n), cellk(P, n), cstart(P, G + 1), sidx;
+  const bool counted = !no_edges && G <= 4 * n + 65536;
   KP.begin(KP_SORT);
-  if (G <= 4 * n + 65536) {
-    DBuf<uint32_t> key(P, n), place(P, n), sidx(P, n), cnt(P, G);
+  if (counted) {
+    DBuf<uint32_t> key(P, n), place(P, n), cnt(P, G);
+    sidx = DBuf<uint32_t>(P, n);
     auto tmp = DBuf<uint8_t>(P, scan_tmp_bytes(G) + 64);
     zero_u32(cnt.get(), G, s);
     launch_cell_key(raw, n, SG.g, SG.grids, SG.mol, key.get(), place.get(),
                     cnt.get(), L);
     scan_u32(cnt.get(), cstart.get(), Cnt(G), tmp.get(), s);
-    launch_cell_order(raw, n, key.get(), place.get(), cstart.get(), sidx.get(),
-                      solvent, ball.get(), perm.get(), cellk.get(), L);
+    launch_cell_put(n, key.get(), place.get(), cstart.get(), sidx.get(),
+                    cellk.get(), L);
   } else {
     DBuf<uint32_t> key(P, n), idx(P, n), key2(P, n), idx2(P, n);
     launch_cell_key(raw, n, SG.g, SG.grids, SG.mol, key.get(), idx.get(),
@@ -384,10 +389,19 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   SG.cellk = cellk.get();
   SG.cstart = cstart.get();
 
-  /* ---- fine scan grid: reference cells split along x ---- */
+  /* ---- the ranks; the fine scan grid: reference cells split along x ---- */
   DBuf<Ball> fball;
   DBuf<uint32_t> fid, fstart;
-  if (pl.kf) {
+  auto order_balls = [&] {
+    if (counted) {
+      KP.begin(KP_SORT);
+      launch_cell_order(raw, n, sidx.get(), cellk.get(), cstart.get(), solvent,
+                        ball.get(), perm.get(), ts, L);
+      KP.end();
+      sidx.release();
+    }
+    KCHK();
+    if (!pl.kf) return;
     const GridP* dsg = nmol > 1 ? pl.dsgrids.get() : nullptr;
     fball = DBuf<Ball>(P, n);
     fid = DBuf<uint32_t>(P, n);
@@ -402,7 +416,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     SG.fball = fball.get();
     SG.fid = fid.get();
     SG.fstart = fstart.get();
-  }
+  };
+  if (!counted) order_balls();
 
   auto scan_tmp = [&](int64_t m) { return DBuf<uint8_t>(P, scan_tmp_bytes(m) + 64); };
   const bool staged = SG.staged != 0;
@@ -556,6 +571,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       launch_edge_count(SG, cnt.get(), L);
       Ecand = count_scan(cnt.get(), n, off.get(), RC_ECAND, "edge");
     }
+    if (counted) order_balls();
     DBuf<uint32_t> cval(P, Ecand.cap);
     DBuf<uint8_t> flag(P, Ecand.cap);
     /* enumeration and first filter stage in one kernel (each ball's kept
@@ -1028,10 +1044,15 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
   stats_from_counters(hs, SG.staged != 0, host_evals[0], st);
   /* a phase without work left no stamp: it takes no time */
   unsigned long long* const t = hs + CTR_COUNT;
-  for (int q = kStamps - 2; q >= 1; --q)
+  for (int q = TS_END - 1; q >= 1; --q)
     if (!t[q]) t[q] = t[q + 1];
-  for (int q = 1; q < kStamps - 1; ++q)
+  for (int q = 1; q < TS_END; ++q)
     st.phase_ms[q] = (double)(t[q + 1] - t[q]) / E->clock_khz;
+  if (t[TS_ORDER]) { /* the ordering is the grid's, not the edges' */
+    const double d = (double)(t[TS_ENUM] - t[TS_ORDER]) / E->clock_khz;
+    st.phase_ms[TS_GRID] += d;
+    st.phase_ms[TS_EDGES] -= d;
+  }
 }
 
 /* The LD driver (AlphaComplexLargeData.cu:1227-1992).  The cell-sorted

@@ -753,10 +753,14 @@ __device__ __forceinline__ void merge_rows(const uint32_t* ecol, uint32_t a,
  * bitmap over the ids modulo its size (512 words shared by the wave's i, so
  * usually 4,096 bits for the ~20 ids of a row), and a lane tests its row(j),
  * four ids a load, instead of merging it with row(i).  The few false hits
- * are dropped by the enumeration; they cost a slot each.
+ * are dropped by the enumeration; they cost a slot each.  EXACT: they are
+ * looked up in row(i) and dropped here, for a recorded pass, whose capacity
+ * is one of triangles: how many hits are false also depends on which rows
+ * share a wave.
  * A wave with a row(j) of more than 128 ids counts by merges and leaves no
  * bits.  39 us at 100k balls (10.6 at 16068), 85 (20) with every lane
  * merging its rows; the loads of the rows and the LDS reads bound it.  ecol is readable up to kEcolPad words past its end. */
+template <bool EXACT>
 __global__ __launch_bounds__(kBlock) void k_tri_hits(
     Cnt c_ne, const uint64_t* erow, const uint32_t* ecol,
     const uint32_t* eleft, ulonglong2* hits, uint32_t* cnt,
@@ -826,6 +830,21 @@ __global__ __launch_bounds__(kBlock) void k_tri_hits(
       /* (the ids past the row's end) */
       const uint32_t left = len > 32u * w ? len - 32u * w : 0u;
       h[w] = left >= 32u ? x : x & ((1u << left) - 1u);
+      if constexpr (EXACT) {
+        const uint32_t end = act ? (uint32_t)erow[i + 1] : 0u;
+        for (uint32_t m = h[w]; m; m &= m - 1) {
+          const uint32_t t = (uint32_t)__builtin_ctz(m);
+          const uint32_t k = ecol[b + 32u * w + t];
+          uint32_t lo = (uint32_t)q + 1u, hi = end;
+          while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            const bool c = ecol[mid] < k;
+            lo = c ? mid + 1u : lo;
+            hi = c ? hi : mid;
+          }
+          if (lo >= end || ecol[lo] != k) h[w] &= ~(1u << t);
+        }
+      }
       n += (uint32_t)__popc(h[w]);
     }
     if (act)
@@ -837,9 +856,10 @@ __global__ __launch_bounds__(kBlock) void k_tri_hits(
 }
 void launch_tri_hits(Cnt ne, const uint64_t* erow, const uint32_t* ecol,
                      const uint32_t* eleft, ulonglong2* hits, uint32_t* cnt,
-                     unsigned long long* ts, PipeLaunch L) {
+                     bool exact, unsigned long long* ts, PipeLaunch L) {
   if (ne.cap <= 0) return;
-  hipLaunchKernelGGL(k_tri_hits, dim3((unsigned)((ne.cap + kBlock - 1) / kBlock)),
+  auto kf = exact ? k_tri_hits<true> : k_tri_hits<false>;
+  hipLaunchKernelGGL(kf, dim3((unsigned)((ne.cap + kBlock - 1) / kBlock)),
                      dim3(kBlock), 0, L.s, ne, erow, ecol, eleft, hits, cnt, ts);
 }
 

@@ -240,12 +240,13 @@ void graph_create(const float* xyzr, const int64_t* offsets, int64_t nmol,
     for (int64_t q = 0; q <= p.gm; ++q) p.rel[q] = offsets[p.m0 + q] - p.b0;
     const pac_result& pr = *probe->groups[g];
     for (int q = 0; q < RC_COUNT; ++q) {
-      p.probe[q] = pr.sizes[q];
+      /* triangle slots: one a candidate (the eager run has a few more) */
+      p.probe[q] = q == RC_TSLOTS ? pr.st.tri_candidates : pr.sizes[q];
       /* alpha tets: room for all of them, also those a covered edge kept
        * out of the list, so that a changed input is accepted as long as
        * its alpha tets keep within the headroom */
       p.cap[q] = with_headroom(
-          q == RC_KALPHA ? pr.st.tet_alpha : pr.sizes[q], headroom);
+          q == RC_KALPHA ? pr.st.tet_alpha : p.probe[q], headroom);
       if (p.cap[q] >= ((int64_t)1 << 32) - 1)
         p.cap[q] = ((int64_t)1 << 32) - 2; /* survivors index with uint32 */
     }

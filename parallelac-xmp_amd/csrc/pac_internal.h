@@ -491,12 +491,12 @@ void launch_tet_caps(const Stage& S, Cnt m, const uint64_t* trow,
                      const uint32_t* ecol, const uint32_t* tk, uint32_t* cap,
                      PipeLaunch L);
 /* the triangle candidates of each segment of kTriSeg alpha edges, or a few
- * more (cnt), and per edge the positions of its own in row(j) (hits);
+ * more unless `exact` (cnt), and per edge the positions of its own in row(j) (hits);
  * ecol has kEcolPad readable words past its edges */
 constexpr int kTriSeg = 64, kEcolPad = 3;
 void launch_tri_hits(Cnt ne, const uint64_t* erow, const uint32_t* ecol,
                      const uint32_t* eleft, ulonglong2* hits, uint32_t* cnt,
-                     unsigned long long* ts, PipeLaunch L);
+                     bool exact, unsigned long long* ts, PipeLaunch L);
 /* triangle candidates of the alpha edges, each filtered by the first
  * precision stage in the same kernel: enumeration segment b (kTriSeg alpha
  * edges) writes its kept and undecided candidates (k, the edge and how far

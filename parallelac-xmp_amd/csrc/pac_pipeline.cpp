@@ -639,7 +639,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     {
       DBuf<uint32_t> cnt(P, std::max<int64_t>(neseg, 1));
       launch_tri_hits(Ealpha, erow.get(), ecol.get(), eleft.get(), emask.get(),
-                      cnt.get(), ts, L);
+                      cnt.get(), rec != nullptr, ts, L);
       Tslots = count_scan(cnt.get(), Cnt(neseg), off.get(), RC_TSLOTS,
                           "triangle");
     }

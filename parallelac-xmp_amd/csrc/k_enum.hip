@@ -733,17 +733,37 @@ __device__ __forceinline__ uint32_t cut_at(uint32_t n, uint64_t base,
   return n < room ? n : (uint32_t)room;
 }
 /* the third vertices of alpha edge (i, j) are row(i) after j, from a on,
- * merged with row(j): hit(k, a, b) for each */
+ * merged with row(j): hit(k, a, b) for each; two steps a round, each row's
+ * next id loaded with its current one (~0 past the end) */
 template <class F>
 __device__ __forceinline__ void merge_rows(const uint32_t* ecol, uint32_t a,
                                            uint32_t ae, uint32_t b,
                                            uint32_t be, F&& hit) {
   while (a < ae && b < be) {
-    const uint32_t x = ecol[a], y = ecol[b];
-    if (x == y) hit(x, a, b);
+    const uint32_t x0 = ecol[a], y0 = ecol[b];
+    const uint32_t x1 = a + 1u < ae ? ecol[a + 1u] : ~0u;
+    const uint32_t y1 = b + 1u < be ? ecol[b + 1u] : ~0u;
+    if (x0 == y0) hit(x0, a, b);
+    const bool sa = x0 <= y0, sb = y0 <= x0;
+    a += sa;
+    b += sb;
+    const uint32_t x = sa ? x1 : x0, y = sb ? y1 : y0;
+    if (x == y && x != ~0u) hit(x, a, b);
     a += (x <= y);
     b += (y <= x);
   }
+}
+/* the first of the ascending ids at(lo), .. at(hi - 1) not below v, or hi */
+template <class F>
+__device__ __forceinline__ uint32_t first_from(uint32_t lo, uint32_t hi,
+                                               uint32_t v, F&& at) {
+  while (lo < hi) {
+    const uint32_t m = (lo + hi) >> 1;
+    const bool c = at(m) < v;
+    lo = c ? m + 1u : lo;
+    hi = c ? hi : m;
+  }
+  return lo;
 }
 /* Triangle candidates of the alpha edges (computePossibleTriangleCount,
  * Parallel:232-266), a wave per kTriSeg = 64 edges, an edge q = (i, j) a
@@ -757,8 +777,8 @@ __device__ __forceinline__ void merge_rows(const uint32_t* ecol, uint32_t a,
  * looked up in row(i) and dropped here, for a recorded pass, whose capacity
  * is one of triangles: how many hits are false also depends on which rows
  * share a wave.
- * A wave with a row(j) of more than 128 ids counts by merges and leaves no
- * bits.  39 us at 100k balls (10.6 at 16068), 85 (20) with every lane
+ * A wave with a row(j) of more than 128 ids counts by merges and leaves its
+ * edges' counts for bits.  39 us at 100k balls (10.6 at 16068), 85 (20) with every lane
  * merging its rows; the loads of the rows and the LDS reads bound it.  ecol is readable up to kEcolPad words past its end. */
 template <bool EXACT>
 __global__ __launch_bounds__(kBlock) void k_tri_hits(
@@ -789,6 +809,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_hits(
     if (act)
       merge_rows(ecol, (uint32_t)q + 1u, (uint32_t)erow[i + 1], b, b + len,
                  [&](uint32_t, uint32_t, uint32_t) { ++n; });
+    if (act) hits[q] = make_ulonglong2(n, 0);
   } else {
     /* the wave's different i: this lane's is number `rank` of them */
     const uint32_t pi = (uint32_t)__shfl_up((int)i, 1, 64);
@@ -835,14 +856,9 @@ __global__ __launch_bounds__(kBlock) void k_tri_hits(
         for (uint32_t m = h[w]; m; m &= m - 1) {
           const uint32_t t = (uint32_t)__builtin_ctz(m);
           const uint32_t k = ecol[b + 32u * w + t];
-          uint32_t lo = (uint32_t)q + 1u, hi = end;
-          while (lo < hi) {
-            const uint32_t mid = (lo + hi) >> 1;
-            const bool c = ecol[mid] < k;
-            lo = c ? mid + 1u : lo;
-            hi = c ? hi : mid;
-          }
-          if (lo >= end || ecol[lo] != k) h[w] &= ~(1u << t);
+          const uint32_t a = first_from((uint32_t)q + 1u, end, k,
+                                        [&](uint32_t c) { return ecol[c]; });
+          if (a >= end || ecol[a] != k) h[w] &= ~(1u << t);
         }
       }
       n += (uint32_t)__popc(h[w]);
@@ -1574,13 +1590,16 @@ __device__ __forceinline__ uint32_t tri_ahead(uint32_t x) {
  * A wave takes the kTriSeg edges and hits of k_tri_hits: it lists the hits
  * (edge, position in row(j)) in LDS and takes them 64 at a time: k's
  * position in row(i) by a binary search in the wave's part of ecol, which is
- * in LDS (none: a false hit), then the filter; the kept and undecided ones
+ * in LDS unless a row is long (none: a false hit), then the filter; the kept and undecided ones
  * are written compacted, in order, from the wave's first slot on, three
  * words and the flag.
  * 113 us at 100k balls (30 at 16068), 211 (48) for blocks of 256 edges that
  * merged the rows into LDS and filtered them from there, waiting for their
  * longest rows and at two barriers a round.
- * A wave with a row too long for the hits or the LDS merges its rows into
+ * A ball with 4,000 edges to small ones of short rows: 45 us (and 18 for the
+ * hits), 1,948 with its waves, whose rows do not fit the LDS, merging; merges
+ * throughout took 889 and 341.
+ * A wave with a row too long for the hits merges its rows into
  * the slots themselves and filters them from there: each round's 64 are read
  * before any is written, to positions not past them.
  * edead (alpha edges, cleared; may be null): set for the edges a rejected
@@ -1616,7 +1635,9 @@ __global__ __launch_bounds__(kBlock) void k_tri_enum_filter(
       ae = (uint32_t)erow[i + 1];
       h = hits[q];
     }
-    const bool listed = __ballot(len > 128u || (q < ne && ae - q0 > COLS)) == 0;
+    const bool listed = __ballot(len > 128u) == 0;
+    /* the wave's rows end within the LDS */
+    const bool near = __ballot(q < ne && ae - q0 > COLS) == 0;
     const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
     uint32_t w4[4] = {0u, 0u, 0u, 0u};
     uint32_t total, step, at = 0;
@@ -1635,13 +1656,11 @@ __global__ __launch_bounds__(kBlock) void k_tri_enum_filter(
       /* the rest of the last row */
       const int last = ne - q0 < 64 ? (int)(ne - q0) - 1 : 63;
       const uint32_t end = (uint32_t)__builtin_amdgcn_readlane((int)ae, last);
-      for (uint32_t t = 64u + (uint32_t)lane; q0 + t < end; t += 64)
-        s_col[wv][t] = ecol[q0 + t];
+      if (near)
+        for (uint32_t t = 64u + (uint32_t)lane; q0 + t < end; t += 64)
+          s_col[wv][t] = ecol[q0 + t];
     } else {
-      uint32_t n = 0;
-      if (q < ne)
-        merge_rows(ecol, (uint32_t)q + 1u, ae, b, b + len,
-                   [&](uint32_t, uint32_t, uint32_t) { ++n; });
+      const uint32_t n = (uint32_t)h.x;
       const uint32_t incl = wave_prefix(n);
       total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
       uint64_t o = base + (incl - n);
@@ -1687,14 +1706,16 @@ __global__ __launch_bounds__(kBlock) void k_tri_enum_filter(
             eb = T.w + (x & 127u);
             k = ecol[eb];
             /* k among the ids after (i, j) in row(i) */
-            uint32_t lo = t + 1u, hi = T.z;
-            while (lo < hi) {
-              const uint32_t m = (lo + hi) >> 1;
-              const bool c = s_col[wv][m] < k;
-              lo = c ? m + 1u : lo;
-              hi = c ? hi : m;
+            uint32_t lo;
+            if (near) {
+              lo = first_from(t + 1u, T.z, k,
+                              [&](uint32_t m) { return s_col[wv][m]; });
+              have = lo < T.z && s_col[wv][lo] == k;
+            } else {
+              lo = first_from(t + 1u, T.z, k,
+                              [&](uint32_t m) { return ecol[q0 + m]; });
+              have = lo < T.z && ecol[q0 + lo] == k;
             }
-            have = lo < T.z && s_col[wv][lo] == k;
             vi = T.x;
             vj = T.y;
             e = q0 + t;

@@ -833,6 +833,20 @@ __global__ __launch_bounds__(kBlock) void k_tri_hits(
     }
     wave_sync();
     const uint32_t* const mine = bm + (act ? rank << sh : 0);
+    /* EXACT: where the row's ids in the bitmap, from the wave's first one on,
+     * span fewer than its bits, no two of them share one, and a hit up to the
+     * last of them is true */
+    uint32_t end = 0, last = ~0u;
+    bool wide = false;
+    if constexpr (EXACT) {
+      const int head = 63 - __builtin_clzll(heads & (~0ull >> (63 - lane)));
+      const uint32_t first = (uint32_t)__shfl((int)j, head, 64);
+      if (act) {
+        end = (uint32_t)erow[i + 1];
+        last = ecol[end - 1u];
+        wide = last - first >= 32u << sh;
+      }
+    }
     uint32_t h[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
@@ -842,18 +856,20 @@ __global__ __launch_bounds__(kBlock) void k_tri_hits(
         U4a4 y = {0u, 0u, 0u, 0u};
         if (32u * w + t < len)
           y = *reinterpret_cast<const U4a4*>(ecol + b + 32u * w + t);
-        x |= (((mine[(y.x >> 5) & wm] >> (y.x & 31u)) & 1u) |
-              ((mine[(y.y >> 5) & wm] >> (y.y & 31u)) & 1u) << 1 |
-              ((mine[(y.z >> 5) & wm] >> (y.z & 31u)) & 1u) << 2 |
-              ((mine[(y.w >> 5) & wm] >> (y.w & 31u)) & 1u) << 3)
-             << t;
+        uint32_t in = ((mine[(y.x >> 5) & wm] >> (y.x & 31u)) & 1u) |
+                      ((mine[(y.y >> 5) & wm] >> (y.y & 31u)) & 1u) << 1 |
+                      ((mine[(y.z >> 5) & wm] >> (y.z & 31u)) & 1u) << 2 |
+                      ((mine[(y.w >> 5) & wm] >> (y.w & 31u)) & 1u) << 3;
+        if (EXACT)
+          in &= (uint32_t)(y.x <= last) | (uint32_t)(y.y <= last) << 1 |
+                (uint32_t)(y.z <= last) << 2 | (uint32_t)(y.w <= last) << 3;
+        x |= in << t;
       }
       /* (the ids past the row's end) */
       const uint32_t left = len > 32u * w ? len - 32u * w : 0u;
       h[w] = left >= 32u ? x : x & ((1u << left) - 1u);
       if constexpr (EXACT) {
-        const uint32_t end = act ? (uint32_t)erow[i + 1] : 0u;
-        for (uint32_t m = h[w]; m; m &= m - 1) {
+        for (uint32_t m = wide ? h[w] : 0u; m; m &= m - 1) {
           const uint32_t t = (uint32_t)__builtin_ctz(m);
           const uint32_t k = ecol[b + 32u * w + t];
           const uint32_t a = first_from((uint32_t)q + 1u, end, k,

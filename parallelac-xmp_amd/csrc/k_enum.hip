@@ -202,7 +202,9 @@ void launch_bounds(const Ball* raw, int64_t n, Real solvent, Bounds* part,
 __global__ __launch_bounds__(kBlock) void k_bounds_mol(const Ball* raw,
                                                        const uint32_t* moff,
                                                        Real solvent,
-                                                       Bounds* out) {
+                                                       Bounds* out,
+                                                       unsigned long long* ts) {
+  stamp(ts, TS_GRID);
   __shared__ BRed sh[kBlock];
   const uint32_t m = blockIdx.x, b0 = moff[m], b1 = moff[m + 1];
   BRed b;
@@ -213,10 +215,11 @@ __global__ __launch_bounds__(kBlock) void k_bounds_mol(const Ball* raw,
   if (threadIdx.x == 0) out[m] = bred_out(b);
 }
 void launch_bounds_mol(const Ball* raw, const uint32_t* moff, int64_t nmol,
-                       Real solvent, Bounds* out, PipeLaunch L) {
+                       Real solvent, Bounds* out, unsigned long long* ts,
+                       PipeLaunch L) {
   if (nmol <= 0) return;
   hipLaunchKernelGGL(k_bounds_mol, dim3((unsigned)nmol), dim3(kBlock), 0, L.s,
-                     raw, moff, solvent, out);
+                     raw, moff, solvent, out, ts);
 }
 
 __global__ __launch_bounds__(kBlock) void k_mol_ids(const uint32_t* moff,

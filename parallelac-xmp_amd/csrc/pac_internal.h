@@ -387,7 +387,8 @@ void launch_bounds(const Ball* raw, int64_t n, Real solvent, Bounds* part,
                    int ctl_words, Post post, PipeLaunch L);
 /* per-molecule bounds of a batch: one block per molecule, moff[nmol+1] */
 void launch_bounds_mol(const Ball* raw, const uint32_t* moff, int64_t nmol,
-                       Real solvent, Bounds* out, PipeLaunch L);
+                       Real solvent, Bounds* out, unsigned long long* ts,
+                       PipeLaunch L);
 /* mol[i] = molecule of ball i (same for input and cell-sorted order) */
 void launch_mol_ids(const uint32_t* moff, int64_t nmol, int64_t n,
                     uint32_t* mol, PipeLaunch L);

@@ -138,7 +138,8 @@ void plan_pass(Engine* E, const Ball* raw, int64_t n, Real solvent,
                           hipMemcpyHostToDevice, s));
     DBuf<Bounds> bout(P, nmol);
     if (ctl) zero_u64(ctl->p, ctl->words, s);
-    launch_bounds_mol(raw, pl.dmoff.get(), nmol, solvent, bout.get(), L);
+    launch_bounds_mol(raw, pl.dmoff.get(), nmol, solvent, bout.get(),
+                      ctl ? ctl->p + ctl->words - kStamps : nullptr, L);
     KCHK();
     HIPCHK(hipMemcpyAsync(hb.data(), bout.get(), nmol * sizeof(Bounds),
                           hipMemcpyDeviceToHost, s));
@@ -286,7 +287,8 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     zero_u64((unsigned long long*)dcnt, RC_COUNT, s);
     /* does the current input still fit the recorded plan? */
     if (nmol > 1) {
-      launch_bounds_mol(raw, pl.dmoff.get(), nmol, solvent, rec->bnow, L);
+      launch_bounds_mol(raw, pl.dmoff.get(), nmol, solvent, rec->bnow, nullptr,
+                        L);
     } else {
       DBuf<Bounds> bpart(P, 1024 * 2 + 4);
       launch_bounds(raw, n, solvent, bpart.get(), rec->bnow, nullptr, nullptr, 0,

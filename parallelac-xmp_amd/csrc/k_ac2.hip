@@ -782,6 +782,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     const uint32_t* tk, const uint32_t* tedge, const uint8_t* edead,
     const uint8_t* in_flag, uint8_t* flag, Queue q1, uint32_t* rest,
     unsigned* nrest, int budget, uint32_t whole) {
+  if (PH != PH_REST) stamp(S0.low_ts, KIND == 0 ? TS_TRI_AC2 : TS_EDGE_AC2);
   unsigned evals = 0, pairs = 0;
   __shared__ uint32_t s_pre[LSLOTS + 1];
   if (PH == PH_REST) list_table(nrest, S0.lcap, s_pre);

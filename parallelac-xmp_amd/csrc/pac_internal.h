@@ -430,6 +430,9 @@ struct Stage {
   unsigned long long* ctr;
   /* time stamps (TS_*), set by the first kernel of each phase (null: none) */
   unsigned long long* ts;
+  /* the same for the triangle or edge emptiness where no tets or triangles
+   * were closed before it, whose kernel would have set the phase's stamp */
+  unsigned long long* low_ts;
   int staged;
   /* second emptiness phase: a persistent launch of bgrid blocks of bblock
    * threads whose waves take bchunk entries of the left-over list at a

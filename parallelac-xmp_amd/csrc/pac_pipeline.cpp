@@ -908,6 +908,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       KCHK();
       Tf = settle(RC_TF, post);
     } else {
+      SG.low_ts = Kalpha.cap ? nullptr : ts;
       Tf = ladder(
           ac2_cap(Talpha.cap), Talpha.cap / 4, KP_TRI_AC2, -1,
           [&](Queue q) {
@@ -975,6 +976,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
       KCHK();
       Ef = settle(RC_EF, post);
     } else {
+      SG.low_ts = Talpha.cap ? nullptr : ts;
       Ef = ladder(
           ac2_cap(Ealpha.cap), Ealpha.cap / 4, KP_EDGE_AC2, -1,
           [&](Queue q) {

@@ -22,3 +22,32 @@ def test_batch(batch_balls):
                                  batch_balls=batch_balls).stats())
     assert all(t[k] > 0 for k in pac.PHASE_LABELS[1:]), t
     assert sum(t.values()) < 100
+
+
+def test_no_tets():
+    """balls of one plane: the triangles' test is most of the run"""
+    print("case: no tets", flush=True)
+    b = pac.synth_globule(1500, seed=2)
+    b[:, 2] = 0
+    pac.compute(b, 1.4, 0.0)
+    st = pac.compute(b, 1.4, 0.0).stats()
+    t = phases(st)
+    assert st.tri_alpha > 0 and st.tet_alpha == 0
+    assert t["AC2 test for triangles"] > t["AC2 test for tetrahedra"]
+    assert t["AC2 test for edges"] > 0
+
+
+def test_no_triangles():
+    """separate pairs: the edges' test has a time of its own"""
+    print("case: no triangles", flush=True)
+    b = np.zeros((40000, 4), np.float32)
+    k = np.arange(20000)
+    b[0::2, 0], b[0::2, 1], b[0::2, 2] = 8 * (k % 30), 8 * (k // 30 % 30), 8 * (k // 900)
+    b[1::2] = b[0::2]
+    b[1::2, 0] += 1
+    b[:, 3] = 1.5
+    pac.compute(b, 0.0, 0.0)
+    st = pac.compute(b, 0.0, 0.0).stats()
+    t = phases(st)
+    assert st.edge_alpha == 20000 and st.tri_alpha == 0
+    assert t["AC2 test for edges"] > 0 and t["Potential triangles"] > 0

@@ -124,10 +124,14 @@ __device__ void bred_block(BRed& mine, BRed* sh) {
 
 /* the reduced bounds to `out`, and posted */
 __device__ __forceinline__ void bounds_done(const BRed& b, Bounds* out,
-                                            const Post& post, Bounds* s_b) {
+                                            const Post& post, Bounds* s_b,
+                                            unsigned long long began) {
   if (threadIdx.x == 0) {
     *s_b = bred_out(b);
     *out = *s_b;
+    if (post.box)
+      *reinterpret_cast<unsigned long long*>(post.box + kBoxSpan) =
+          wall_clock64() - began;
   }
   if (!post.box) return;
   __syncthreads();
@@ -153,10 +157,11 @@ __global__ __launch_bounds__(kBlock) void k_bounds_part(
     double4* orig, unsigned long long* ctl, int ctl_words, Post post) {
   __shared__ BRed sh[kBlock];
   __shared__ Bounds s_b;
+  const unsigned long long began = wall_clock64();
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   if (ctl) {
     for (int64_t i = gtid(); i < ctl_words; i += stride)
-      ctl[i] = i == ctl_words - kStamps + TS_GRID ? wall_clock64() : 0ull;
+      ctl[i] = i == ctl_words - kStamps + TS_GRID ? began : 0ull;
   }
   BRed b;
   bred_init(b);
@@ -168,20 +173,22 @@ __global__ __launch_bounds__(kBlock) void k_bounds_part(
   }
   bred_block(b, sh);
   if (gridDim.x == 1)
-    bounds_done(b, out, post, &s_b);
+    bounds_done(b, out, post, &s_b, began);
   else if (threadIdx.x == 0)
     part[blockIdx.x] = b;
 }
 __global__ __launch_bounds__(kBlock) void k_bounds_final(const BRed* part,
                                                          int np, Bounds* out,
+                                                         const unsigned long long* ts,
                                                          Post post) {
   __shared__ BRed sh[kBlock];
   __shared__ Bounds s_b;
+  const unsigned long long began = ts ? ts[TS_GRID] : wall_clock64();
   BRed b;
   bred_init(b);
   for (int i = threadIdx.x; i < np; i += blockDim.x) bred_merge(b, part[i]);
   bred_block(b, sh);
-  bounds_done(b, out, post, &s_b);
+  bounds_done(b, out, post, &s_b, began);
 }
 void launch_bounds(const Ball* raw, int64_t n, Real solvent, Bounds* part,
                    Bounds* out, double4* orig, unsigned long long* ctl,
@@ -194,7 +201,8 @@ void launch_bounds(const Ball* raw, int64_t n, Real solvent, Bounds* part,
                      solvent, (BRed*)part, out, orig, ctl, ctl_words, post);
   if (nb > 1)
     hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlock), 0, L.s,
-                       (const BRed*)part, nb, out, post);
+                       (const BRed*)part, nb, out,
+                       ctl ? ctl + ctl_words - kStamps : nullptr, post);
 }
 
 /* Per-molecule bounds of a batch: block m reduces the balls of molecule m

@@ -263,8 +263,8 @@ static void compute_one(const F* xyzr, int64_t n, F solvent, F alpha,
   KP.on = opt.profile != 0;
   KP.s = s;
   using clk = std::chrono::steady_clock;
-  auto since = [](clk::time_point t) {
-    return std::chrono::duration<double, std::milli>(clk::now() - t).count();
+  auto ms = [](clk::duration d) {
+    return std::chrono::duration<double, std::milli>(d).count();
   };
   const auto t_host0 = clk::now();
   DBuf<B> raw_own;
@@ -275,7 +275,6 @@ static void compute_one(const F* xyzr, int64_t n, F solvent, F alpha,
                           hipMemcpyHostToDevice, s));
     raw = raw_own.get();
   }
-  const double t_in = since(t_host0);
   if (n > 0) {
     /* filled by the run's first kernel, or here for a chunked one */
     R->balls = DBuf<double4>(&E->pool, n);
@@ -290,8 +289,10 @@ static void compute_one(const F* xyzr, int64_t n, F solvent, F alpha,
   HIPCHK(hipStreamSynchronize(s));
   pac_stats& st = R->st;
   for (int q = 0; q < 8; ++q) st.phase_ms[q] += R->phase_add[q];
-  st.phase_ms[0] += t_in;
-  st.total_ms = since(t_host0);
+  /* the input's copy, up to the first kernel behind it */
+  if (raw_own.get())
+    st.phase_ms[0] += std::max(ms(R->began - t_host0), 0.0);
+  st.total_ms = ms(clk::now() - t_host0);
   KP.collect(st.kernel_ms);
   *out = R.release();
 }

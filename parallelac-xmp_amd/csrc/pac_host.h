@@ -213,6 +213,13 @@ struct Engine {
     if (__atomic_load_n(t, __ATOMIC_ACQUIRE) != p.ticket)
       fail(PAC_ERR_DEVICE, "internal: a post is missing");
   }
+  /* the time from the first bounds kernel to its post */
+  std::chrono::steady_clock::duration posted_span() const {
+    uint64_t v;
+    std::memcpy(&v, box + kBoxSpan, sizeof(v));
+    return std::chrono::duration_cast<std::chrono::steady_clock::duration>(
+        std::chrono::duration<double, std::milli>((double)v / clock_khz));
+  }
   uint64_t posted_count() const {
     uint64_t v;
     std::memcpy(&v, box + kBoxCount, sizeof(v));
@@ -288,6 +295,8 @@ struct pac_result {
   pac_stats st;
   /* phase times (ms) measured outside the run's own timer (chunked runs) */
   double phase_add[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  /* when the device began with the input, on this side's clock */
+  std::chrono::steady_clock::time_point began;
   /* filtration (pac_options.filtration): per output edge / triangle, 1 if
    * its smallest orthosphere is empty (it enters at its own rho); rank of
    * each ball in cell-sorted order; filtration keys, made on first use */
@@ -483,6 +492,7 @@ struct PassPlan {
   WI alpha_wi;
   bool no_edges = true;
   int k_enum = 0, k_ac2 = 0;
+  std::chrono::steady_clock::time_point began; /* (of one molecule) */
   DBuf<uint32_t> dmoff, dmol;
   DBuf<GridP> dgrids;
 };

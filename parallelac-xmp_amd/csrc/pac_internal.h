@@ -96,8 +96,9 @@ enum { FAM_EDGE = 0, FAM_TRI = 1, FAM_TET = 2, FAM_TET_AC2 = 3,
  * through a copy and a stream synchronisation left the GPU idle for ~20 us
  * (copy kernel, completion signal, wake-up), a post for ~8.
  * Box words: the ticket (u64), the count (u64), the sub-queue fills of the
- * hot and of the escalation queue (QSLOTS each), then kBoxData words of
- * data (bounds, statistics). */
+ * hot and of the escalation queue (QSLOTS each), with the bounds the clock
+ * ticks since their first kernel began (u64), then kBoxData words of data
+ * (bounds, statistics). */
 struct Post {
   unsigned* box = nullptr; /* null: nothing is posted */
   unsigned long long ticket = 0;
@@ -105,7 +106,7 @@ struct Post {
                              are read, then cleared for the next ladder */
 };
 constexpr int kBoxTicket = 0, kBoxCount = 2, kBoxQ1 = 4, kBoxQ2 = 36,
-              kBoxData = 128, kBoxWords = 2048;
+              kBoxSpan = 68, kBoxData = 128, kBoxWords = 2048;
 
 /* ---- primitives (k_prims.hip) ---- */
 /* exclusive scan; out has n+1 entries, out[n] = total */

@@ -129,6 +129,7 @@ void plan_pass(Engine* E, const Ball* raw, int64_t n, Real solvent,
                   ctl ? ctl->words : 0, post, L);
     KCHK();
     E->wait(post, s);
+    pl.began = std::chrono::steady_clock::now() - E->posted_span();
     std::memcpy(&hb[0], E->box + kBoxData, sizeof(Bounds));
   } else {
     std::vector<uint32_t> mo(nmol + 1);
@@ -274,6 +275,7 @@ void run_pipeline(Engine* E, const Ball* raw, int64_t n, Real solvent,
     ts = ctl.p + ctl.words - kStamps;
     plan_pass(E, raw, n, solvent, alpha, opt, s, moff, nmol, own,
               sub ? &sub->grid : nullptr, &ctl);
+    R->began = own.began;
   }
   const PassPlan& pl = rec ? *(const PassPlan*)rec->plan : own;
   /* counts left on the device by the scans (RC_*) */
@@ -1100,6 +1102,7 @@ void run_chunked(Engine* E, const Ball* raw, int64_t n, Real solvent,
   RunCtl keep;
   keep.orig = R->balls.get();
   plan_pass(E, raw, n, solvent, alpha, opt, s, nullptr, 1, gp, nullptr, &keep);
+  R->began = gp.began;
   const GridP g = gp.grids[0];
   const Bounds gb = gp.bounds[0];
   DBuf<uint32_t> rank(P, n);

@@ -51,3 +51,24 @@ def test_no_triangles():
     t = phases(st)
     assert st.edge_alpha == 20000 and st.tri_alpha == 0
     assert t["AC2 test for edges"] > 0 and t["Potential triangles"] > 0
+
+
+def test_transfer():
+    """pinned memory is copied behind the call: 32 MB take the bus at least
+    0.2 ms (160 GB/s would), however soon the copy's call returns"""
+    print("case: transfer", flush=True)
+    import torch
+    n = 2000000
+    b = np.zeros((n, 4), np.float32)
+    k = np.arange(n)
+    b[:, 0], b[:, 1], b[:, 2] = 4 * (k % 128), 4 * (k // 128 % 128), 4 * (k // 16384)
+    b[:, 3] = 1.0
+    pinned = torch.from_numpy(b).pin_memory()
+    for x in (b, pinned.numpy()):
+        pac.compute(x, 0.0, 0.0)
+        t = phases(pac.compute(x, 0.0, 0.0).stats())
+        assert 0.2 < t["Data transfer"] < 50, t
+    dev = pinned.cuda()
+    torch.cuda.synchronize()
+    r = pac.compute_device(dev.data_ptr(), n, 0.0, 0.0)
+    assert phases(r.stats())["Data transfer"] == 0

@@ -292,7 +292,7 @@ __global__ __launch_bounds__(kBlock) void k_tet_ac2_hot(
   const int64_t total =
       PH != PH_ALL ? (int64_t)s_pre[LSLOTS] : c_nk.get();
   uint32_t rest_id = 0xffffffffu; /* phase A: the item left for phase B */
-  auto item = [&](int64_t w) {
+  auto item = [&](int64_t w) __attribute__((always_inline)) {
     const Stage& S = fresh_stage();
     const int64_t id =
         PH == PH_ALL ? w
@@ -789,7 +789,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
   const int64_t total =
       PH == PH_REST ? (int64_t)s_pre[LSLOTS] : c_nitems.get();
   uint32_t rest_id = 0xffffffffu; /* phase A: the item left for phase B */
-  auto item = [&](int64_t w) {
+  auto item = [&](int64_t w) __attribute__((always_inline)) {
     const Stage& S = fresh_stage();
     int64_t id = w;
     int tested = budget; /* phase B: the pairs that phase A tested */

@@ -33,16 +33,27 @@ PEAK_TFLOPS = {"f32": WORK_MODEL["peaks"]["valu_f32_TFLOPs"],
 KERNEL_KEYS = ("edge_fill", "tri_fill", "tet_fill", "tet_ac2", "tri_ac2", "edge_ac2")
 
 
-def kernel_flops(key, units, alpha_tets, fp64):
+def work_units(st):
+    """({kernel: work units}, tets whose emptiness scan was certainly set up) of
+    a run's statistics.  Alpha tets with an edge that one ball covers are
+    counted but not scanned, and how many the statistics do not say: the final
+    tets, all of them scanned to the end, are a lower bound."""
+    return ({"edge_fill": st.edge_candidates, "tri_fill": st.tri_candidates,
+             "tet_fill": st.tet_candidates, "tet_ac2": st.ac2_pairs[0],
+             "tri_ac2": st.ac2_pairs[1], "edge_ac2": st.ac2_pairs[2]},
+            st.tets_final)
+
+
+def kernel_flops(key, units, setups, fp64):
     """(FP32 flops, FP64 flops) of one launch of kernel `key` over `units`
-    work units; the tet emptiness scan adds its per-alpha-tet setup.  On the
-    plain FP64 path every FP32 flop runs in FP64."""
+    work units; the tet emptiness scan adds the set-up of `setups` tets.  On
+    the plain FP64 path every FP32 flop runs in FP64."""
     f = WORK_MODEL["flops"][key]
     f32, f64 = f["f32"] * units, f["f64"] * units
     if key == "tet_ac2":
         su = WORK_MODEL["flops"]["tet_ac2_setup"]
-        f32 += su["f32"] * alpha_tets
-        f64 += su["f64"] * alpha_tets
+        f32 += su["f32"] * setups
+        f64 += su["f64"] * setups
     return (0.0, f32 + f64) if fp64 else (float(f32), float(f64))
 
 
@@ -204,30 +215,27 @@ def main():
     p_st = run(pac.PREC_STAGED, profile=True).stats()
     p_pl = run(pac.PREC_PLAIN_FP64, profile=True).stats()
     kms = {pac.KERNELS[i]: p_st.kernel_ms[i] for i in range(8)}
-    units = {"edge_fill": s_st.edge_candidates, "tri_fill": s_st.tri_candidates,
-             "tet_fill": s_st.tet_candidates, "tet_ac2": s_st.ac2_pairs[0],
-             "tri_ac2": s_st.ac2_pairs[1], "edge_ac2": s_st.ac2_pairs[2]}
+    units, setups = work_units(s_st)
     dom = max(KERNEL_KEYS, key=lambda k: kms[k])
-    f32, f64 = kernel_flops(dom, units[dom], s_st.tet_alpha, fp64=False)
+    f32, f64 = kernel_flops(dom, units[dom], setups, fp64=False)
     achieved, peak = valu_roofline(f32, f64, kms[dom])
     # the same model for every filter kernel (vector FP32/FP64 rate), both paths
     kms_pl = {pac.KERNELS[i]: p_pl.kernel_ms[i] for i in range(8)}
-    units_pl = {"edge_fill": s_pl.edge_candidates, "tri_fill": s_pl.tri_candidates,
-                "tet_fill": s_pl.tet_candidates, "tet_ac2": s_pl.ac2_pairs[0],
-                "tri_ac2": s_pl.ac2_pairs[1], "edge_ac2": s_pl.ac2_pairs[2]}
+    units_pl, setups_pl = work_units(s_pl)
     rates, fracs = {}, {}
     for k in KERNEL_KEYS:
-        for tag, km, un, fp64 in (("staged", kms, units, False),
-                                  ("plain", kms_pl, units_pl, True)):
-            a32, a64 = kernel_flops(k, un[k], (s_st if not fp64 else s_pl).tet_alpha, fp64)
+        for tag, km, un, su, fp64 in (
+                ("staged", kms, units, setups, False),
+                ("plain", kms_pl, units_pl, setups_pl, True)):
+            a32, a64 = kernel_flops(k, un[k], su, fp64)
             ach, pk = valu_roofline(a32, a64, km[k])
             rates.setdefault(k, {})[tag] = round(ach, 3) if km[k] > 0 else None
             fracs.setdefault(k, {})[tag] = round(ach / pk, 4) if km[k] > 0 else None
     traffic, traffic_src = None, None
     tpath = os.path.join(ROOT, "profiles", "hbm_traffic_globule100k.json")
-    if os.path.exists(tpath) and dom in ("tet_ac2",):
-        tj = json.load(open(tpath))
-        traffic = tj.get("bytes_per_run", {}).get(dom)
+    if os.path.exists(tpath):
+        traffic = json.load(open(tpath)).get("bytes_per_run", {}).get(dom)
+    if traffic is not None:
         traffic_src = "profiles/hbm_traffic_globule100k.json (rocprofv3 --pmc " \
                       "FETCH_SIZE / WRITE_SIZE, scaled by a 1 GiB copy)"
     roofline = {"bound": "valu", "achieved": achieved, "peak": peak,
@@ -236,7 +244,7 @@ def main():
                 "kernel": dom, "kernel_ms": kms[dom],
                 "work_units": int(units[dom]),
                 "flops_per_unit": WORK_MODEL["flops"][dom],
-                "setup_units": int(s_st.tet_alpha) if dom == "tet_ac2" else 0,
+                "setup_units": int(setups) if dom == "tet_ac2" else 0,
                 "flops_per_setup": WORK_MODEL["flops"]["tet_ac2_setup"]
                 if dom == "tet_ac2" else None,
                 "flops_f32": f32, "flops_f64": f64,

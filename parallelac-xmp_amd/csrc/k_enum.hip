@@ -785,9 +785,11 @@ __device__ __forceinline__ uint32_t first_from(uint32_t lo, uint32_t hi,
  * usually 4,096 bits for the ~20 ids of a row), and a lane tests its row(j),
  * four ids a load, instead of merging it with row(i).  The few false hits
  * are dropped by the enumeration; they cost a slot each.  EXACT: they are
- * looked up in row(i) and dropped here, for a recorded pass, whose capacity
- * is one of triangles: how many hits are false also depends on which rows
- * share a wave.
+ * dropped here, for a recorded pass, whose capacity is one of triangles (how
+ * many hits are false also depends on which rows share a wave): an id's bits
+ * above its word's place in the bitmap are compared too, and only hits in
+ * words that ids of several such values share are looked up in row(i); 61 us
+ * for 42 at 100k balls, 120 with every hit of a long row looked up.
  * A wave with a row(j) of more than 128 ids counts by merges and leaves its
  * edges' counts for bits.  39 us at 100k balls (10.6 at 16068), 85 (20) with every lane
  * merging its rows; the loads of the rows and the LDS reads bound it.  ecol is readable up to kEcolPad words past its end. */
@@ -799,7 +801,8 @@ __global__ __launch_bounds__(kBlock) void k_tri_hits(
   static_assert(kTriSeg == 64, "an edge a lane");
   stamp(ts, TS_TRIS);
   constexpr int W = 512; /* words of a wave's bitmaps */
-  __shared__ uint4 s_raw[kBlock / 64][W / 4];
+  constexpr int E = EXACT ? 2 : 1; /* words of an entry */
+  __shared__ uint4 s_raw[kBlock / 64][W * E / 4];
   const int64_t ne = c_ne.get();
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int64_t seg = gtid() >> 6, q = gtid();
@@ -830,59 +833,68 @@ __global__ __launch_bounds__(kBlock) void k_tri_hits(
     const int sh = nd > 1 ? 9 - (32 - __builtin_clz((unsigned)nd - 1u)) : 9;
     const uint32_t wm = (1u << sh) - 1u;
     uint32_t* const bm = reinterpret_cast<uint32_t*>(s_raw[wv]);
-    s_raw[wv][lane] = s_raw[wv][64 + lane] = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+    for (int t = 0; t < W * E / 256; ++t)
+      s_raw[wv][64 * t + lane] = make_uint4(0u, 0u, 0u, 0u);
     wave_sync();
-    if (act) atomicOr(&bm[(rank << sh) + ((j >> 5) & wm)], 1u << (j & 31u));
-    if (seg * kTriSeg + 64 < ne) { /* the rest of the last row */
-      const uint32_t il = (uint32_t)__builtin_amdgcn_readlane((int)i, 63);
-      const uint32_t ae = (uint32_t)erow[il + 1];
-      for (uint32_t a = (uint32_t)(seg * kTriSeg) + 64u + (uint32_t)lane; a < ae;
-           a += 64) {
-        const uint32_t y = ecol[a];
-        atomicOr(&bm[((nd - 1) << sh) + ((y >> 5) & wm)], 1u << (y & 31u));
+    /* the wave's ids of each row: this lane's, and the rest of the last row */
+    auto each_id = [&](auto&& f) {
+      if (act) f(rank << sh, j);
+      if (seg * kTriSeg + 64 < ne) {
+        const uint32_t il = (uint32_t)__builtin_amdgcn_readlane((int)i, 63);
+        const uint32_t ae = (uint32_t)erow[il + 1];
+        for (uint32_t a = (uint32_t)(seg * kTriSeg) + 64u + (uint32_t)lane;
+             a < ae; a += 64)
+          f((nd - 1) << sh, ecol[a]);
       }
-    }
+    };
+    /* EXACT: beside each word the ids' bits above it, or kMixed where two ids
+     * of the row in that word differ there */
+    constexpr uint32_t kMixed = ~0u;
+    each_id([&](int row, uint32_t y) {
+      const uint32_t at = (uint32_t)row + ((y >> 5) & wm);
+      atomicOr(&bm[E * at], 1u << (y & 31u));
+      if (EXACT) bm[E * at + 1] = y >> (5 + sh);
+    });
     wave_sync();
-    const uint32_t* const mine = bm + (act ? rank << sh : 0);
-    /* EXACT: where the row's ids in the bitmap, from the wave's first one on,
-     * span fewer than its bits, no two of them share one, and a hit up to the
-     * last of them is true */
-    uint32_t end = 0, last = ~0u;
-    bool wide = false;
     if constexpr (EXACT) {
-      const int head = 63 - __builtin_clzll(heads & (~0ull >> (63 - lane)));
-      const uint32_t first = (uint32_t)__shfl((int)j, head, 64);
-      if (act) {
-        end = (uint32_t)erow[i + 1];
-        last = ecol[end - 1u];
-        wide = last - first >= 32u << sh;
-      }
+      each_id([&](int row, uint32_t y) {
+        const uint32_t at = (uint32_t)row + ((y >> 5) & wm);
+        if (bm[E * at + 1] != y >> (5 + sh)) bm[E * at + 1] = kMixed;
+      });
+      wave_sync();
     }
+    const uint32_t* const mine = bm + (act ? E * (rank << sh) : 0);
+    /* bit 0: a hit; bit 16: a hit in a mixed word */
+    auto test = [&](uint32_t y) -> uint32_t {
+      const uint32_t at = (y >> 5) & wm;
+      if (!EXACT) return (mine[at] >> (y & 31u)) & 1u;
+      const uint2 m = reinterpret_cast<const uint2*>(mine)[at];
+      const uint32_t in = (m.x >> (y & 31u)) & 1u, p = m.y;
+      return p == y >> (5 + sh) ? in : (p == kMixed ? in | in << 16 : 0u);
+    };
     uint32_t h[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       if (__ballot(len > 32u * w) == 0) break;
-      uint32_t x = 0;
+      uint32_t x = 0, mixed = 0;
       for (uint32_t t = 0; t < 32 && __ballot(len > 32u * w + t) != 0; t += 4) {
         U4a4 y = {0u, 0u, 0u, 0u};
         if (32u * w + t < len)
           y = *reinterpret_cast<const U4a4*>(ecol + b + 32u * w + t);
-        uint32_t in = ((mine[(y.x >> 5) & wm] >> (y.x & 31u)) & 1u) |
-                      ((mine[(y.y >> 5) & wm] >> (y.y & 31u)) & 1u) << 1 |
-                      ((mine[(y.z >> 5) & wm] >> (y.z & 31u)) & 1u) << 2 |
-                      ((mine[(y.w >> 5) & wm] >> (y.w & 31u)) & 1u) << 3;
-        if (EXACT)
-          in &= (uint32_t)(y.x <= last) | (uint32_t)(y.y <= last) << 1 |
-                (uint32_t)(y.z <= last) << 2 | (uint32_t)(y.w <= last) << 3;
-        x |= in << t;
+        const uint32_t in =
+            test(y.x) | test(y.y) << 1 | test(y.z) << 2 | test(y.w) << 3;
+        x |= (in & 15u) << t;
+        if (EXACT) mixed |= (in >> 16) << t;
       }
       /* (the ids past the row's end) */
       const uint32_t left = len > 32u * w ? len - 32u * w : 0u;
-      h[w] = left >= 32u ? x : x & ((1u << left) - 1u);
+      const uint32_t in_row = left >= 32u ? ~0u : (1u << left) - 1u;
+      h[w] = x & in_row;
       if constexpr (EXACT) {
-        for (uint32_t m = wide ? h[w] : 0u; m; m &= m - 1) {
+        for (uint32_t m = mixed & in_row; m; m &= m - 1) {
           const uint32_t t = (uint32_t)__builtin_ctz(m);
-          const uint32_t k = ecol[b + 32u * w + t];
+          const uint32_t k = ecol[b + 32u * w + t], end = (uint32_t)erow[i + 1];
           const uint32_t a = first_from((uint32_t)q + 1u, end, k,
                                         [&](uint32_t c) { return ecol[c]; });
           if (a >= end || ecol[a] != k) h[w] &= ~(1u << t);

@@ -241,9 +241,9 @@ void pac_graph_free(pac_graph* g);
  * quick rejection pass on or off), then opt->ac2_budget / opt->ac2_grid
  * (one phase, or a phase-one pair budget of 2, 4, 8 or 16 x second-phase
  * grid, over the chosen scan grid), then, with a second phase,
- * opt->block / opt->ac2_chunk (its block shape and queue granularity);
- * the other fields of *opt
- * are used as given.  offsets ==
+ * opt->block / opt->ac2_chunk (its block shape and queue granularity).
+ * Where *opt as given is more than 2% faster than all of these, these
+ * fields stay as they are; the others are used as given.  offsets ==
  * NULL: the n balls are one molecule; otherwise they are a batch
  * (offsets[n_mol+1]) and the leading molecules, up to about 2^20 balls,
  * are the sample.  best_ms (may be NULL) receives the fastest wall time

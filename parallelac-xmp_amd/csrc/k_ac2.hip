@@ -284,7 +284,7 @@ __global__ __launch_bounds__(kBlock) void k_tet_ac2_hot(
     const uint4* tets, uint8_t* flag, Queue q1, uint32_t* rest,
     unsigned* nrest, int budget) {
   if (PH == PH_ALL) stamp(S0.ts, TS_TET_AC2);
-  unsigned evals = 0, pairs = 0;
+  unsigned pairs = 0;
   /* phase A: the alpha tets, or the list `items` of them (those the quick
    * pass left); phase B: `rest` */
   __shared__ uint32_t s_pre[LSLOTS + 1];
@@ -330,7 +330,6 @@ __global__ __launch_bounds__(kBlock) void k_tet_ac2_hot(
         ++seen;
       }
       ++pairs;
-      ++evals;
       int s = pairss_sign(P, E);
       if (s == 0) {
         const uint32_t p = FINE ? S.fid[j] : j;
@@ -409,16 +408,10 @@ __global__ __launch_bounds__(kBlock) void k_tet_ac2_hot(
     if (gtid() < total) item(gtid());
     list_append(rest, nrest, S0.lcap, rest_id != 0xffffffffu, rest_id);
   }
-  (void)evals;
   block_flush(S0.ctr, CTR_PAIRS + 0, pairs);
 }
 
 /* FP64 then double-double for queued pairs / uncertified tets */
-template <class T>
-__device__ __forceinline__ int tet_pair_code_T(const TetQ<T>& t, int sD,
-                                               const Ball& e) {
-  return tet_pair_code(t, sD, e);
-}
 __global__ __launch_bounds__(kBlock) void k_tet_ac2_esc(
     Stage S, QRef qr, const uint4* tets, uint8_t* flag,
     Queue q2) {
@@ -783,7 +776,7 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     const uint8_t* in_flag, uint8_t* flag, Queue q1, uint32_t* rest,
     unsigned* nrest, int budget, uint32_t whole) {
   if (PH != PH_REST) stamp(S0.low_ts, KIND == 0 ? TS_TRI_AC2 : TS_EDGE_AC2);
-  unsigned evals = 0, pairs = 0;
+  unsigned pairs = 0;
   __shared__ uint32_t s_pre[LSLOTS + 1];
   if (PH == PH_REST) list_table(nrest, S0.lcap, s_pre);
   const int64_t total =
@@ -844,7 +837,6 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
         ++seen;
       }
       ++pairs;
-      ++evals;
       int s = pairss_sign(P, E);
       if (s < 0) { /* power <= rho strictly: violator */
         stop = 1;
@@ -964,7 +956,6 @@ __global__ __launch_bounds__(kBlock) void k_low_ac2_hot(
     }
     list_append(rest, nrest, S0.lcap, rest_id != 0xffffffffu, rest_id);
   }
-  (void)evals;
   block_flush(S0.ctr, CTR_PAIRS + 1 + KIND, pairs);
 }
 

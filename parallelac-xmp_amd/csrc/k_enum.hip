@@ -3,9 +3,9 @@
  *
  * Waves enumerate the candidates of a ball or of 64 alpha edges or
  * triangles (cells of the stencil, rows in each other by bitmaps and masks),
- * 64 at a time whatever item they belong to, classify each with one precision stage (FP32 on the staged
- * path, FP64 on the plain path) and append undecided candidates to a
- * queue.  The escalation kernel re-decides them in FP64 then double-double;
+ * 64 at a time whatever item they belong to, classify each with one precision
+ * stage (FP32 on the staged path, FP64 on the plain path) and append undecided
+ * candidates to a queue.  The escalation kernel re-decides them in FP64 then double-double;
  * what is still undecided goes to the wide-integer kernel.
  *
  * Reference kernels restated (AlphaComplexLargeData.cu unless noted):
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(kBlock) void k_bounds_part(
 }
 __global__ __launch_bounds__(kBlock) void k_bounds_final(const BRed* part,
                                                          int np, Bounds* out,
-                                                         const unsigned long long* ts,
+                                                         const uint64_t* ts,
                                                          Post post) {
   __shared__ BRed sh[kBlock];
   __shared__ Bounds s_b;
@@ -202,7 +202,8 @@ void launch_bounds(const Ball* raw, int64_t n, Real solvent, Bounds* part,
   if (nb > 1)
     hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlock), 0, L.s,
                        (const BRed*)part, nb, out,
-                       ctl ? ctl + ctl_words - kStamps : nullptr, post);
+                       ctl ? (const uint64_t*)ctl + ctl_words - kStamps
+                           : nullptr, post);
 }
 
 /* Per-molecule bounds of a batch: block m reduces the balls of molecule m
@@ -662,29 +663,13 @@ void launch_edge_count(const Stage& S, uint32_t* cnt, PipeLaunch L) {
 }
 
 /* ------------------------------------------------------------------ */
-/* triangles: k in row(i) after j, intersected with row(j)             */
+/* triangles: k in row(i) after j and in row(j); tets: l in T(i,j)     */
+/* after k, T(i,k), T(j,k)                                             */
 /* ------------------------------------------------------------------ */
-/* ------------------------------------------------------------------ */
-/* tets: l in T(i,j) after k, T(i,k), T(j,k)                           */
-/* ------------------------------------------------------------------ */
-/* ------------------------------------------------------------------ */
-/* enumeration: candidates as (segment, new vertex) pairs              */
-/* ------------------------------------------------------------------ */
-/* Slot capacities that need no merge: a triangle from alpha edge (i,j) has
- * its third vertex in row(i) after j, a tet from alpha triangle (i,j,k) has
- * its fourth vertex in T(i,j) after k.  Unused slots carry seg = ~0. */
-__global__ __launch_bounds__(kBlock) void k_tail_caps(Cnt c_m,
-                                                      const uint64_t* row,
-                                                      const uint32_t* owner,
-                                                      uint32_t* cap) {
-  const int64_t m = c_m.get();
-  int64_t q = gtid();
-  if (q >= m) return;
-  cap[q] = (uint32_t)(row[owner[q] + 1] - (uint64_t)q - 1);
-}
-/* chunk sub-input: no slots for the triangles (i,j,k) none of whose
- * vertices is owned -- every tet they start has its three lowest vertices
- * unowned, and no owned simplex depends on it */
+/* Tet slots of the alpha triangles of a chunk sub-input: the row tail of each,
+ * but no slots for the triangles (i,j,k) none of whose vertices is owned --
+ * every tet they start has its three lowest vertices unowned, and no owned
+ * simplex depends on it */
 __global__ __launch_bounds__(kBlock) void k_tail_caps_own(
     Stage S, Cnt c_m, const uint64_t* row, const uint32_t* owner,
     const uint32_t* eleft, const uint32_t* ecol, const uint32_t* tk,
@@ -699,21 +684,11 @@ __global__ __launch_bounds__(kBlock) void k_tail_caps_own(
                     (k >= S.own_lo && k < S.own_hi);
   cap[q] = need ? (uint32_t)(row[e + 1] - (uint64_t)q - 1) : 0u;
 }
-void launch_tail_caps(Cnt m, const uint64_t* row, const uint32_t* owner,
-                      uint32_t* cap, PipeLaunch L) {
-  if (m.cap <= 0) return;
-  hipLaunchKernelGGL(k_tail_caps, dim3((unsigned)((m.cap + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, m, row, owner, cap);
-}
 void launch_tet_caps(const Stage& S, Cnt m, const uint64_t* trow,
                      const uint32_t* tedge, const uint32_t* eleft,
                      const uint32_t* ecol, const uint32_t* tk, uint32_t* cap,
                      PipeLaunch L) {
   if (m.cap <= 0) return;
-  if (!S.chunk) {
-    launch_tail_caps(m, trow, tedge, cap, L);
-    return;
-  }
   hipLaunchKernelGGL(k_tail_caps_own,
                      dim3((unsigned)((m.cap + kBlock - 1) / kBlock)),
                      dim3(kBlock), 0, L.s, S, m, trow, tedge, eleft, ecol, tk,
@@ -791,8 +766,9 @@ __device__ __forceinline__ uint32_t first_from(uint32_t lo, uint32_t hi,
  * words that ids of several such values share are looked up in row(i); 61 us
  * for 42 at 100k balls, 120 with every hit of a long row looked up.
  * A wave with a row(j) of more than 128 ids counts by merges and leaves its
- * edges' counts for bits.  39 us at 100k balls (10.6 at 16068), 85 (20) with every lane
- * merging its rows; the loads of the rows and the LDS reads bound it.  ecol is readable up to kEcolPad words past its end. */
+ * edges' counts for bits.  39 us at 100k balls (10.6 at 16068), 85 (20) with
+ * every lane merging its rows; the loads of the rows and the LDS reads bound
+ * it.  ecol is readable up to kEcolPad words past its end. */
 template <bool EXACT>
 __global__ __launch_bounds__(kBlock) void k_tri_hits(
     Cnt c_ne, const uint64_t* erow, const uint32_t* ecol,
@@ -1047,7 +1023,8 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 8 : 1))) void k_tet_enum_fil
     const uint32_t* tedge, const uint32_t* teik, const uint32_t* tejk,
     const uint32_t* eleft, const uint32_t* ecol, const ulonglong2* emask,
     const uint64_t* off, const uint64_t* roff, const uint32_t* epre,
-    uint64_t* bbase, uint4* ctet, uint8_t* flag, uint32_t* bcnt, uint32_t* bkeep, Queue q1, uint64_t lim) {
+    uint64_t* bbase, uint4* ctet, uint8_t* flag, uint32_t* bcnt,
+    uint32_t* bkeep, Queue q1, uint64_t lim) {
   static_assert(kTetSeg == 64, "a triangle a lane");
   stamp(S.ts, TS_TETS);
   /* LDS of a wave, 4,992 bytes (8 blocks per CU): by masks, three rows of
@@ -1452,7 +1429,8 @@ void launch_tet_seg_copy(Cnt nt, const uint64_t* bbase, const uint32_t* bcnt,
   const int64_t nseg = (nt.cap + kTetSeg - 1) / kTetSeg;
   hipLaunchKernelGGL(
       k_tet_seg_copy,
-      dim3((unsigned)((nseg * kSegLanes + kBlock - 1) / kBlock)), dim3(kBlock), 0, L.s, nt, bbase, bcnt, ctet, flag, bout, tets, ocap);
+      dim3((unsigned)((nseg * kSegLanes + kBlock - 1) / kBlock)), dim3(kBlock),
+      0, L.s, nt, bbase, bcnt, ctet, flag, bout, tets, ocap);
 }
 
 /* Edge candidates of ball i (j > i in the stencil rows, Parallel:122-201)
@@ -1629,9 +1607,9 @@ __device__ __forceinline__ uint32_t tri_ahead(uint32_t x) {
  * A wave takes the kTriSeg edges and hits of k_tri_hits: it lists the hits
  * (edge, position in row(j)) in LDS and takes them 64 at a time: k's
  * position in row(i) by a binary search in the wave's part of ecol, which is
- * in LDS unless a row is long (none: a false hit), then the filter; the kept and undecided ones
- * are written compacted, in order, from the wave's first slot on, three
- * words and the flag.
+ * in LDS unless a row is long (none: a false hit), then the filter; the kept
+ * and undecided ones are written compacted, in order, from the wave's first
+ * slot on, three words and the flag.
  * 113 us at 100k balls (30 at 16068), 211 (48) for blocks of 256 edges that
  * merged the rows into LDS and filtered them from there, waiting for their
  * longest rows and at two barriers a round.
@@ -1825,9 +1803,9 @@ void launch_tri_enum_filter(const Stage& S, Cnt ne, const uint64_t* erow,
  * in order, a wave each; trow[e] for its edges e (and trow[ne], by the wave
  * holding index ne) = bout[b] + the kept triangles of its edges before e.
  * tk has kDeadBit set where one of the triangle's edges is marked in edead
- * (if given); tri_in (the closure's marks) cleared.  emask[e], e = (i,j): x has bit r if (i, j, k) is a
- * triangle and (i, k) the (r + 1)th edge after e, y the bits of those with
- * kDeadBit; bit 63 is set if some r is 63 or more.  spair, epre (if given):
+ * (if given); tri_in (the closure's marks) cleared.  emask[e], e = (i,j): x
+ * has bit r if (i, j, k) is a triangle and (i, k) the (r + 1)th edge after e,
+ * y the bits of those with kDeadBit; bit 63 is set if some r is 63 or more.  spair, epre (if given):
  * the tet slots of the segment's triangles (each one's row tail), and of
  * those of its edges before e.  Grid: a wave per segment and one more; bout
  * has one entry more than segments. */
@@ -2074,9 +2052,5 @@ void launch_filter_exact(const Stage& S, int kind, CandCtx C, QRef q, const uint
                        cval, flag);
 }
 
-/* ------------------------------------------------------------------ */
-/* survivors: segment starts and flat stable compaction                */
-/* ------------------------------------------------------------------ */
-/* orow[s] = number of survivors before segment s = pos[off[s]] */
 }  // namespace PAC_V
 }  // namespace pac

@@ -345,8 +345,9 @@ void filtration_order(int64_t m, const uint64_t* key, const int64_t counts[4],
  * differentials with weights lam_q removes dc:
  *     drho = sum_q lam_q (2 (p_q - c) . dp_q - dw_q),   dw_q = 2 r_q dr_q,
  * so d rho / d p_q = 2 lam_q (p_q - c) and d rho / d r_q = -2 lam_q r_q.
- * Contributions are written per (simplex, vertex) slot and summed per ball
- * in slot order after a stable sort by ball: the result is deterministic. */
+ * Contributions are written per (simplex, vertex) slot; each ball's slots are
+ * counted, put together and ranked, and eight partial sums over every eighth
+ * of them in slot order added pairwise: the result is deterministic. */
 template <int DIM>
 __global__ __launch_bounds__(kBlock) void k_adj_contrib(
     int64_t m, const int32_t* rows, const double4* balls, const double* g,

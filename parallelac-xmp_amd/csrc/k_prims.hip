@@ -32,18 +32,16 @@ __device__ __forceinline__ void do_post(const Post& P, uint64_t count) {
                        P.ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-template <class TIn, bool kFlag>
+template <class TIn>
 __device__ __forceinline__ uint64_t load_val(const TIn* in, int64_t i,
                                              int64_t n) {
-  if (i >= n) return 0;
-  if (kFlag) return in[i] != 0 ? 1 : 0;
-  return (uint64_t)in[i];
+  return i < n ? (uint64_t)in[i] : 0;
 }
 
 /* Tiles of kTile items are read and written striped across the block
  * (coalesced), and transposed through LDS so that each thread scans
  * kScanItems consecutive items. */
-template <class TIn, bool kFlag>
+template <class TIn>
 __global__ __launch_bounds__(kBlock) void k_tile_sums(const TIn* in, Cnt cn,
                                                       uint64_t* sums) {
   const int64_t n = cn.get();
@@ -51,7 +49,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_sums(const TIn* in, Cnt cn,
   uint64_t s = 0;
 #pragma unroll
   for (int q = 0; q < kScanItems; ++q)
-    s += load_val<TIn, kFlag>(in, base + (int64_t)q * kBlock + threadIdx.x, n);
+    s += load_val(in, base + (int64_t)q * kBlock + threadIdx.x, n);
   uint64_t tot;
   block_excl_scan_u64(s, &tot);
   if (threadIdx.x == 0) sums[blockIdx.x] = tot;
@@ -88,7 +86,7 @@ __device__ __forceinline__ uint64_t sum_before(const TIn* in, int64_t m) {
  * offset: for small arrays two launches fewer (~4 us each) for ~2 us more
  * of reading. */
 constexpr int64_t kFewTiles = 16;
-template <class TIn, bool kFlag, class TOut, bool FEW>
+template <class TIn, class TOut, bool FEW>
 __global__ __launch_bounds__(kBlock) void k_tile_scan(const TIn* in, Cnt cn,
                                                       const uint64_t* tile_off,
                                                       TOut* out,
@@ -99,7 +97,6 @@ __global__ __launch_bounds__(kBlock) void k_tile_scan(const TIn* in, Cnt cn,
   const int64_t n = cn.get();
   int64_t base = (int64_t)blockIdx.x * kTile;
   uint64_t before = 0;
-  static_assert(!kFlag, "flags have scans of their own");
   if constexpr (FEW) {
     if (base < n) before = sum_before(in, base);
   } else {
@@ -108,7 +105,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_scan(const TIn* in, Cnt cn,
 #pragma unroll
   for (int q = 0; q < kScanItems; ++q) {
     int t = q * kBlock + threadIdx.x;
-    tile[t] = load_val<TIn, kFlag>(in, base + t, n);
+    tile[t] = load_val(in, base + t, n);
   }
   __syncthreads();
   uint64_t v[kScanItems];
@@ -232,7 +229,7 @@ __global__ __launch_bounds__(kSumsBlock) void k_scan_sums(const uint64_t* in,
 static void scan_u64_rec(const uint64_t* in, uint64_t* out, int64_t n,
                          uint64_t* tmp, hipStream_t s);
 
-template <class TIn, bool kFlag, class TOut = uint64_t>
+template <class TIn, class TOut>
 static void scan_impl(const TIn* in, TOut* out, Cnt n, uint64_t* tmp,
                       hipStream_t s, uint64_t* total64 = nullptr,
                       Post post = Post()) {
@@ -243,14 +240,14 @@ static void scan_impl(const TIn* in, TOut* out, Cnt n, uint64_t* tmp,
   }
   int64_t tiles = (n.cap + kTile - 1) / kTile;
   if (tiles <= kFewTiles) {
-    hipLaunchKernelGGL((k_tile_scan<TIn, kFlag, TOut, true>),
+    hipLaunchKernelGGL((k_tile_scan<TIn, TOut, true>),
                        dim3((unsigned)tiles), dim3(kBlock), 0, s, in, n,
                        (const uint64_t*)nullptr, out, total64, post);
     return;
   }
   uint64_t* sums = tmp;
   uint64_t* offs = tmp + (tiles + 1);
-  hipLaunchKernelGGL((k_tile_sums<TIn, kFlag>), dim3((unsigned)tiles),
+  hipLaunchKernelGGL(k_tile_sums<TIn>, dim3((unsigned)tiles),
                      dim3(kBlock), 0, s, in, n, sums);
   if (tiles <= kSumsMax) { /* the tile sums in one block: three launches */
     hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kSumsBlock), 0, s,
@@ -260,27 +257,27 @@ static void scan_impl(const TIn* in, TOut* out, Cnt n, uint64_t* tmp,
   } else {
     scan_u64_rec(sums, offs, tiles, tmp + 2 * (tiles + 1), s);
   }
-  hipLaunchKernelGGL((k_tile_scan<TIn, kFlag, TOut, false>),
+  hipLaunchKernelGGL((k_tile_scan<TIn, TOut, false>),
                      dim3((unsigned)tiles), dim3(kBlock), 0, s, in, n,
                      (const uint64_t*)offs, out, total64, post);
 }
 
 static void scan_u64_rec(const uint64_t* in, uint64_t* out, int64_t n,
                          uint64_t* tmp, hipStream_t s) {
-  scan_impl<uint64_t, false>(in, out, n, tmp, s);
+  scan_impl(in, out, n, tmp, s);
 }
 
 void scan_u32_to_u64(const uint32_t* in, uint64_t* out, Cnt n, void* tmp,
                      hipStream_t s, uint64_t* total64, Post post) {
-  scan_impl<uint32_t, false>(in, out, n, (uint64_t*)tmp, s, total64, post);
+  scan_impl(in, out, n, (uint64_t*)tmp, s, total64, post);
 }
 void scan_u32(const uint32_t* in, uint32_t* out, Cnt n, void* tmp,
               hipStream_t s) {
-  scan_impl<uint32_t, false>(in, out, n, (uint64_t*)tmp, s);
+  scan_impl(in, out, n, (uint64_t*)tmp, s);
 }
 void scan_u64_to_u64(const uint64_t* in, uint64_t* out, Cnt n, void* tmp,
                      hipStream_t s, uint64_t* total64, Post post) {
-  scan_impl<uint64_t, false>(in, out, n, (uint64_t*)tmp, s, total64, post);
+  scan_impl(in, out, n, (uint64_t*)tmp, s, total64, post);
 }
 /* Flag scans (u8 flags, nonzero = 1 -> u32 positions), the scan every
  * compaction runs: a thread owns kScanItems (8) consecutive flags, read as
@@ -563,7 +560,7 @@ void radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
   for (int shift = 0; shift < bits; shift += 8) {
     hipLaunchKernelGGL(k_radix_hist, dim3((unsigned)ntiles), dim3(kBlock), 0,
                        s, ki, n, shift, ntiles, hist);
-    scan_impl<uint32_t, false>(hist, hoff, (int64_t)h, stmp, s);
+    scan_impl(hist, hoff, (int64_t)h, stmp, s);
     hipLaunchKernelGGL(k_radix_scatter, dim3((unsigned)ntiles), dim3(kBlock),
                        0, s, ki, vi, n, shift, ntiles, hoff, ko, vo);
     uint32_t* t = ki;
@@ -580,9 +577,10 @@ void radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
 /* ------------------------------------------------------------------ */
 /* recorded (fixed-capacity) pipelines                                 */
 /* ------------------------------------------------------------------ */
-/* The end of a recorded ladder, one wave, lane k for slot k: the largest
- * fills, overflows (counters past the capacity: entries were dropped) into
- * the status, every counter cleared for the next ladder. */
+/* The end of a recorded pass, one wave, lane k for slot k: over the counters
+ * of all its ladders the largest fills, and overflows (counters past the
+ * capacity: entries were dropped) into the status; every counter cleared for
+ * the next pass. */
 __global__ __launch_bounds__(64) void k_ladder_rec(unsigned* qn, uint32_t c1,
                                                    uint32_t c2,
                                                    unsigned* status,

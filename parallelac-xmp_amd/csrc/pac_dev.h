@@ -261,22 +261,6 @@ enum { REJECT = 0, KEEP = 1, UNDEC = 2 };
 __device__ __forceinline__ int code_of(int s) {
   return s > 0 ? KEEP : (s < 0 ? REJECT : UNDEC);
 }
-/* stage index of the precision type */
-template <class T>
-struct StageOf;
-template <>
-struct StageOf<FE<float>> {
-  static constexpr int v = 0;
-};
-template <>
-struct StageOf<FE<double>> {
-  static constexpr int v = 1;
-};
-template <>
-struct StageOf<FEDD> {
-  static constexpr int v = 2;
-};
-
 /* ---- CSR lookups ---- */
 /* Position of v in the sorted row a[lo, hi) or -1, reading the row eight
  * entries at a time: the eight loads issue together, one round trip per
@@ -642,13 +626,10 @@ __device__ __forceinline__ bool place_box(const GridP& g, C reach, const C c[3],
                                           const C e[3], SphBox& b) {
   return make_sph<C>(g, reach, c, e, b);
 }
-__device__ __forceinline__ GridP sgrid_of(const Stage& S, uint32_t b) {
-  return S.sgrids ? S.sgrids[S.mol[b]] : S.sg;
-}
-/* The same with the choice made at compile time: MOL (a batch) reads the
+/* The grid of a ball, the choice made at compile time: MOL (a batch) reads the
  * molecule's grid from its table; otherwise the single grid is read from
- * the kernel's arguments (scalar loads, once per wave).  The run-time
- * choice above becomes one generic (flat) pointer whose 88-byte grid is
+ * the kernel's arguments (scalar loads, once per wave).  A run-time
+ * choice (grid_of) becomes one generic (flat) pointer whose 88-byte grid is
  * reloaded per item through the vector memory path. */
 template <bool MOL>
 __device__ __forceinline__ GridP grid_at(const Stage& S, uint32_t b) {

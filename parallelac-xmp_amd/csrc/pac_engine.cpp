@@ -6,8 +6,8 @@
  * 1126-1806): one HIP stream per call, device-resident intermediates taken
  * from a caching pool (no hipMalloc in steady state), counts posted by the
  * kernels between stages only where a buffer must be sized, time stamps by
- * the first kernel of each of the reference's eight phases.  Errors are returned as status codes, never
- * printed (the reference prints and continues: :55-61).
+ * the first kernel of each of the reference's eight phases.  Errors are
+ * returned as status codes, never printed (the reference prints and continues: :55-61).
  */
 #include <hip/hip_runtime.h>
 

@@ -6,10 +6,10 @@
  * front: an eager run of the batch (compute_batch) measures each pass's
  * counts and largest queue fills, each count gets a capacity of that size
  * plus headroom, and run_pipeline records the pass against those
- * capacities (PassRec): item counts stay on the device (Cnt), queue views
- * are built by a kernel, each precision ladder runs once, and overflows or
- * an input that no longer fits the plan set status bits instead of being
- * retried.  All passes go into one stream capture, so a run of the whole
+ * capacities (PassRec): item counts stay on the device (Cnt), queues are
+ * read through their own counters, each precision ladder runs once, and
+ * overflows or an input that no longer fits the plan set status bits instead
+ * of being retried.  All passes go into one stream capture, so a run of the whole
  * batch is one hipGraphLaunch.  Passes run one after another and share one
  * set of scratch buffers (the graph's own pool, whose blocks the capture
  * hands out in stream order); each pass keeps its own output lists, counts

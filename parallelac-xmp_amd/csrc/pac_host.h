@@ -68,7 +68,8 @@ struct Pool {
   /* Arena mode (set_arena): blocks are carved from one fixed device range
    * instead of hipMalloc, 256-byte aligned, from the first hole that
    * fits or the top of the stack; a block freed while it is the topmost is
-   * popped with any freed blocks below it.  Exhausting the range fails with PAC_ERR_NOMEM. */
+   * popped with any freed blocks below it.  Exhausting the range fails with
+   * PAC_ERR_NOMEM. */
   char* abase = nullptr;
   size_t acap = 0, atop = 0, ahigh = 0;
   std::vector<std::pair<size_t, size_t>> ablk; /* (offset, 1 = freed) */

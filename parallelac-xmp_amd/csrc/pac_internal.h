@@ -353,8 +353,8 @@ void launch_rho(int dim, int64_t m, const int32_t* rows, const double4* balls,
  * the slots sorted by vertex */
 void launch_adj_contrib(int dim, int64_t m, const int32_t* rows,
                         const double4* balls, const double* g, int64_t slot0,
-                        uint32_t* key, uint32_t* place, uint32_t* cnt, double4* contrib,
-                        hipStream_t s);
+                        uint32_t* key, uint32_t* place, uint32_t* cnt,
+                        double4* contrib, hipStream_t s);
 void launch_adj_gather(int64_t n, int64_t m, const uint32_t* key,
                        const uint32_t* place, const uint32_t* vstart,
                        uint32_t* slot, uint32_t* sorted, const double4* contrib,
@@ -486,18 +486,15 @@ void launch_edge_copy(int64_t n, const uint64_t* off, const uint32_t* bcnt,
                       uint64_t* erow, uint32_t* ecol, uint32_t* eleft,
                       uint8_t* edead, uint8_t* edge_in, PipeLaunch L,
                       uint64_t ocap = ~0ull);
-/* slot capacity of item q = row[owner[q] + 1] - q - 1 */
-void launch_tail_caps(Cnt m, const uint64_t* row, const uint32_t* owner,
-                      uint32_t* cap, PipeLaunch L);
-/* tet slots of each alpha triangle: launch_tail_caps over its edge's row,
- * or none for the triangles a chunk sub-input does not need */
+/* chunk sub-input: tet slots of each alpha triangle, the tail of its edge's
+ * row after it, or none for a triangle it does not need */
 void launch_tet_caps(const Stage& S, Cnt m, const uint64_t* trow,
                      const uint32_t* tedge, const uint32_t* eleft,
                      const uint32_t* ecol, const uint32_t* tk, uint32_t* cap,
                      PipeLaunch L);
 /* the triangle candidates of each segment of kTriSeg alpha edges, or a few
- * more unless `exact` (cnt), and per edge the positions of its own in row(j) (hits);
- * ecol has kEcolPad readable words past its edges */
+ * more unless `exact` (cnt), and per edge the positions of its own in row(j)
+ * (hits); ecol has kEcolPad readable words past its edges */
 constexpr int kTriSeg = 64, kEcolPad = 3;
 void launch_tri_hits(Cnt ne, const uint64_t* erow, const uint32_t* ecol,
                      const uint32_t* eleft, ulonglong2* hits, uint32_t* cnt,
@@ -505,9 +502,10 @@ void launch_tri_hits(Cnt ne, const uint64_t* erow, const uint32_t* ecol,
 /* triangle candidates of the alpha edges, each filtered by the first
  * precision stage in the same kernel: enumeration segment b (kTriSeg alpha
  * edges) writes its kept and undecided candidates (k, the edge and how far
- * edge(i,k) lies after it, edge(j,k)) with their flags, in order, compacted from its first slot
- * off[b] (the exclusive scan of launch_tri_hits's counts) on and their number to bcnt[b]; undecided ones are queued on
- * q1 by position (aux = their edge).  edead[e] (cleared by the caller;
+ * edge(i,k) lies after it, edge(j,k)) with their flags, in order, compacted
+ * from its first slot off[b] (the exclusive scan of launch_tri_hits's counts)
+ * on and their number to bcnt[b]; undecided ones are queued on q1 by position
+ * (aux = their edge).  edead[e] (cleared by the caller;
  * null: not wanted) is set for the alpha edges a rejected candidate shows
  * covered by one ball: no simplex with such an edge is empty. */
 void launch_tri_enum_filter(const Stage& S, Cnt ne, const uint64_t* erow,
